@@ -5,7 +5,9 @@ it binds the HIP runtime and hipRTC with dlopen) and the device sources
 csrc/spio_hip_scratch.hip and csrc/spio_hip_fill.hip (hipcc, gfx950: the static
 device workspace with the launch that uses it, and the zero-fill kernel; they
 link the HIP runtime by its soname, so the copy a host framework has already
-mapped is the one used).  hipcc cross-compiles, so this builds on machines
+mapped is the one used).  `build_extension()` builds _native.so from
+csrc/spio_torch.cpp, the operators' call path on torch's C++ interface, which
+links that library.  hipcc cross-compiles, so this builds on machines
 without a GPU.  Loading is another matter: because of the device translation
 units the library has libamdhip64 as a link-time dependency and registers its
 code objects when it is dlopen'ed, so every process that loads it, the
@@ -21,11 +23,13 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC_DIR = os.path.join(_HERE, "csrc")
 REPO_INCLUDE_DIR = os.path.join(os.path.dirname(_HERE), "include")
 LIB_PATH = os.path.join(CSRC_DIR, "libspio_hip.so")
+EXTENSION_PATH = os.path.join(_HERE, "_native.so")
 ROCM_HOME = os.environ.get("ROCM_PATH") or os.environ.get("ROCM_HOME") or "/opt/rocm"
 
 # Device translation units of libspio_hip.so.
@@ -93,6 +97,36 @@ def build_native(force: bool = True, verbose: bool = False) -> str:
     return LIB_PATH
 
 
+def build_extension(verbose: bool = False) -> str:
+    """Compile _native.so, the operators' call path on torch's C++ interface; returns its path.
+
+    Host C++ only.  It links libspio_hip.so (found beside it at run time) and torch's own
+    libraries, which a process that imports torch has loaded already."""
+    import torch  # pylint: disable=import-outside-toplevel
+
+    build_native(force=False)
+    cxx = os.environ.get("CXX") or shutil.which("g++") or shutil.which("c++")
+    if cxx is None:
+        raise RuntimeError("no host C++ compiler found to build _native.so")
+    root = os.path.dirname(torch.__file__)
+    includes = [_include_dir(), os.path.join(root, "include"),
+                os.path.join(root, "include", "torch", "csrc", "api", "include"),
+                os.path.join(ROCM_HOME, "include"), sysconfig.get_paths()["include"]]  # fmt: skip
+    tmp = f"{EXTENSION_PATH}.tmp{os.getpid()}"
+    try:
+        _run([cxx, "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__=1",
+              "-DUSE_ROCM=1", "-DTORCH_EXTENSION_NAME=_native", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}",
+              *[f"-I{d}" for d in includes], os.path.join(CSRC_DIR, "spio_torch.cpp"), "-o", tmp,
+              f"-L{os.path.join(root, 'lib')}", "-lc10", "-lc10_hip", "-ltorch", "-ltorch_cpu", "-ltorch_hip",
+              "-ltorch_python", f"-L{CSRC_DIR}", "-l:libspio_hip.so", "-Wl,-rpath,$ORIGIN/csrc"],
+             "compiling spio_torch.cpp", verbose)  # fmt: skip
+        os.replace(tmp, EXTENSION_PATH)
+    finally:
+        if os.path.exists(tmp):
+            os.remove(tmp)
+    return EXTENSION_PATH
+
+
 def hipcc_compile_check(source_path: str, defines: dict, out_dir: str, tag: str) -> str:
     """Compile one kernel source to a gfx950 code object with hipcc."""
     hipcc = shutil.which("hipcc") or os.path.join(ROCM_HOME, "bin", "hipcc")
@@ -108,4 +142,5 @@ def hipcc_compile_check(source_path: str, defines: dict, out_dir: str, tag: str)
 
 if __name__ == "__main__":
     print(build_native(verbose=True))
+    print(build_extension(verbose=True))
     sys.exit(0)

@@ -84,8 +84,11 @@ def fused_backward_kernel(params: Conv2dGw8Params, device):
 
 def reset_fused_backward_choices():
     """Forget which shapes run the fused backward kernel (after the tuning records changed)."""
+    from ..native import forget_plans
+
     with _fused_choice_lock:
         _fused_choice.clear()
+    forget_plans()
 
 
 def _is_unit(value) -> bool:

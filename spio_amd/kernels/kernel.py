@@ -63,14 +63,20 @@ class LaunchTimer:
 
     def __init__(self):
         self.events = {}
+        self._bypass = None
 
     def __enter__(self):
+        from ..native import Bypass
+
+        self._bypass = self._bypass or Bypass()
         LaunchTimer.active = self
         self.events = {}
         return self
 
     def __exit__(self, exc_type, exc_val, exc_tb):
         LaunchTimer.active = None
+        self._bypass.release()
+        self._bypass = None
         return False
 
     def averages(self, skip: int = 0):
@@ -133,7 +139,10 @@ class Kernel:
 
     def unload(self):
         """Drop the module; load() may be called again if the code was kept."""
+        from ..native import forget_plans
+
         if self.module is not None:
+            forget_plans()
             self.module.unload()
             self.module = None
         self.function = None

@@ -32,19 +32,30 @@ class KernelCache:
         self._cache: Dict[KernelKey, Kernel] = {}
         self._cache_overlay: Dict[KernelKey, Kernel] = {}
         self._lock = threading.RLock()
+        self._bypass = None  # held while the overlay has entries: every call must look at it
 
     def update_overlay(self, overlay: Dict[KernelKey, Kernel]):
         """Kernels that take precedence over (and hide) the main cache."""
+        from ..native import Bypass
+
         with self._lock:
             self._cache_overlay.update(overlay)
+            if self._cache_overlay and self._bypass is None:
+                self._bypass = Bypass()
 
     def clear_overlay(self):
         with self._lock:
             self._cache_overlay.clear()
+            if self._bypass is not None:
+                self._bypass.release()
+                self._bypass = None
 
     def clear_cache(self):
+        from ..native import forget_plans
+
         with self._lock:
             self._cache.clear()
+        forget_plans()
 
     @log_kernel_params
     def get(self, kernel_factory, params, device, **kernel_kwargs) -> Kernel:

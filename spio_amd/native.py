@@ -1,0 +1,110 @@
+"""The operators' native call path: loading it, its launch plans, and when it stands aside.
+
+`_native.so` (csrc/spio_torch.cpp) runs a call of `conv2d_gw8` or `layernorm_2d` on plain GPU tensors
+without going through the Python definition of the operator, which costs several times what the
+kernels take at ordinary sizes.  It asks `_make_plan` once per shape for the kernels to launch
+(tuner, compiler and caches are the Python side's) and keeps the answer until `forget_plans()`.
+Whoever wants to see or choose every launch (overlay caches, KernelParamsLogger, LaunchTimer)
+holds a `Bypass` meanwhile: all calls then take the Python path.
+"""
+
+import importlib
+import os
+import struct
+import threading
+
+import torch
+from torch._library.custom_ops import CustomOpDef
+
+from .build import EXTENSION_PATH, build_extension
+
+if not os.path.exists(EXTENSION_PATH):
+    build_extension()
+_native = importlib.import_module(f"{__package__}._native")
+
+_kernels = {}  # what the native plans point into stays loaded as long as they live
+_kernels_lock = threading.Lock()
+
+
+def forget_plans():
+    """Drop every launch plan (kernels were unloaded, caches or choices cleared)."""
+    _native.forget()
+    with _kernels_lock:
+        _kernels.clear()
+
+
+class Bypass:
+    """While one of these is held, the native path declines every call."""
+
+    def __init__(self):
+        self._held = True
+        _native.bypass(1)
+        forget_plans()
+
+    def release(self):
+        """Let calls take the native path again (idempotent)."""
+        if self._held:
+            self._held = False
+            _native.bypass(-1)
+
+    __del__ = release
+
+
+def _stage(function, launch_params):
+    return [function.handle, *launch_params.grid, *launch_params.block, launch_params.shared_mem_bytes]
+
+
+def _make_plan(values):
+    """(stages, workspace bytes, overwrites) of the kernel a key of csrc/spio_torch.cpp stands for."""
+    from . import kernels
+    from .functional.conv2d_gw8_function import fused_backward_kernel
+
+    kind, ordinal = values[:2]
+    device = torch.device("cuda", ordinal)
+    if kind < 4:
+        n, c, h, w, r, s, py, px, bias, _mode = values[2:]
+        params = kernels.Conv2dGw8Params(n=n, c=c, h=h, w=w, r=r, s=s, padding=(py, px), has_bias=bool(bias))
+        params.validate()
+        if kind == 3:
+            kernel = fused_backward_kernel(params, device)
+        elif kind == 2:
+            kernel = kernels.conv2d_gw8_wgrad_kernel_factory.get_kernel(params, device)
+        else:
+            kernel = kernels.conv2d_gw8_kernel_factory.get_kernel(params, device, **({"igrad": True} if kind else {}))
+    else:
+        n, c, h, w, eps, weight, bias = values[2:9]
+        params = kernels.LayerNorm2dParams(n=n, c=c, h=h, w=w, eps=struct.unpack("<d", struct.pack("<q", eps))[0],
+                                           has_weight=bool(weight), has_bias=bool(bias))  # fmt: skip
+        factory = kernels.layernorm_2d_kernel_factory if kind == 4 else kernels.layernorm_2d_bwd_kernel_factory
+        kernel = factory.get_kernel(params, device)
+    if kernel is None:
+        return None
+    with _kernels_lock:
+        _kernels[values] = kernel
+    spec = kernel.kernel_spec
+    stages = [_stage(kernel.function, spec.launch_params)]
+    if kernel.epilogue_function is not None:
+        stages.append(_stage(kernel.epilogue_function, spec.epilogue_launch_params))
+    return stages, spec.workspace_bytes, spec.overwrites_output
+
+
+class NativeOp(CustomOpDef):
+    """A custom operator whose plain calls take the native path."""
+
+    def __call__(self, *args, **kwargs):
+        if torch.compiler.is_compiling():  # the graph records the operator
+            return self._opoverload(*args, **kwargs)
+        result = self.native(*args, **kwargs)
+        return super().__call__(*args, **kwargs) if result is NotImplemented else result
+
+
+def adopt(op, native_name):
+    """Give the custom operator `op` the native path `native_name`."""
+    op.__class__ = NativeOp
+    op.native = getattr(_native, native_name)
+
+
+def configure(backward_op, norm_backward_op):
+    """Switch the native path on; the operators it hands double differentiation to."""
+    _native.configure(_make_plan, backward_op, norm_backward_op)
+    _native.bypass(-1)
