@@ -249,25 +249,13 @@ SPIO_KERNEL_NAME(spio_uint4* __restrict__ grad_input, float* __restrict__ grad_w
     const int wg = wave % GB;
     const int ws = wave / GB;
 
-    // Workgroup ids are dealt round-robin to the 8 XCDs: runs of SPIO_XCD_CHUNK consecutive tiles
-    // go to one XCD (row blocks share halo rows through its L2) while the tiles in flight on the
-    // device form one compact range of addresses; 0 = one contiguous range of tiles per XCD.
-    int b = block_id();
-    {
-        constexpr int CH = SPIO_XCD_CHUNK;
-        if (CH == 0) {
-            if (NUM_BLOCKS % 8 == 0) b = (b & 7) * (NUM_BLOCKS / 8) + (b >> 3);
-        } else if (CH > 1 && NUM_BLOCKS % (8 * CH) == 0) {
-            const int x8 = b & 7;
-            const int k = b >> 3;
-            b = (k / CH) * (8 * CH) + x8 * CH + k % CH;
-        }
-    }
-    // Tile order: row blocks fastest, so that neighbours in a run share halo rows.  Where a
-    // workgroup covers only part of a pixel's 128-byte lines (GB * 16 bytes per pixel), the channel
-    // blocks that share those lines go fastest instead: dealt to different XCDs, every one of
-    // them would fetch the whole lines from memory (measured: twice the algorithmic reads).
-    constexpr bool kSplitLines = GBLKS > 1 && (GB * 16) % 128 != 0;
+    // Tile order: row blocks fastest, so that neighbours in a run of SPIO_XCD_CHUNK tiles share halo
+    // rows through one XCD's L2.  Where channel blocks share lines they go fastest instead, a run
+    // holding all of a pixel's: dealt to different XCDs, every one of them would fetch the whole lines
+    // from memory (measured: twice the algorithmic reads).
+    constexpr bool kSplitLines = splits_lines(GB, GBLKS);
+    constexpr int RUN = kSplitLines ? line_run(SPIO_XCD_CHUNK, GBLKS) : SPIO_XCD_CHUNK;
+    const int b = xcd_tile<RUN, NUM_BLOCKS>(block_id());
     // Column blocks go before the row blocks: neighbours share S - 1 columns of every row.
     constexpr int TILES = QBLKS * PBLKS;
     const int tile = kSplitLines ? (b / GBLKS) % TILES : b % TILES;

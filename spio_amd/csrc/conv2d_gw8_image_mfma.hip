@@ -206,8 +206,12 @@ SPIO_DEVICE void static_for(F&& f) {
 
 // Workgroup -> (channel block, run of ITERS image blocks); channel block fastest, so the
 // workgroups in flight cover whole pixels (all channels) of a compact range of images.
-SPIO_DEVICE int channel_block() { return block_id() % GBLKS; }
-SPIO_DEVICE int first_block() { return (block_id() / GBLKS) * ITERS; }
+// Channel blocks go fastest.  Where they share lines all of a pixel's run on one XCD, so that its L2 joins
+// their parts of a line; dealt round-robin to the XCDs every one would fetch and write the line by itself.
+constexpr int RUN = splits_lines(GB, GBLKS) ? GBLKS : 1;
+SPIO_DEVICE int tile_index() { return xcd_tile<RUN, GBLKS * WGBLKS>(block_id()); }
+SPIO_DEVICE int channel_block() { return tile_index() % GBLKS; }
+SPIO_DEVICE int first_block() { return (tile_index() / GBLKS) * ITERS; }
 
 // ---- the filters: global memory -> registers -> LDS (the output region, free until the first
 //      block is multiplied) -> fragments.  Every multiplying thread takes a share; every

@@ -603,23 +603,13 @@ SPIO_KERNEL_NAME(spio_uint4* __restrict__ dst, const spio_uint4* __restrict__ sr
     // their workgroups run on the same XCD and share their halo rows.
     const int raw = block_id();
     const bool second = BP2 > 0 && raw >= HALF_BLOCKS;
-    int b = second ? raw - HALF_BLOCKS : raw;
-    {
-        constexpr int CH = SPIO_XCD_CHUNK;
-        if (CH == 0) {
-            if (HALF_BLOCKS % 8 == 0) b = (b & 7) * (HALF_BLOCKS / 8) + (b >> 3);
-        } else if (CH > 1 && HALF_BLOCKS % (8 * CH) == 0) {
-            const int x = b & 7;   // XCD
-            const int k = b >> 3;  // position in that XCD's sequence
-            b = (k / CH) * (8 * CH) + x * CH + k % CH;
-        }
-    }
-    // Tile order: row blocks fastest, so that neighbours in a run share halo rows.  Where a
-    // workgroup covers only part of a pixel's 128-byte lines (GB * 16 bytes per pixel), the channel
-    // blocks that share those lines go fastest instead: dealt to different XCDs, every one of
-    // them would fetch the whole lines from memory (measured: twice the algorithmic reads).
-    // Column blocks go before the row blocks: neighbours share S - 1 columns of every row.
-    constexpr bool kSplitLines = GBLKS > 1 && (GB * 16) % 128 != 0;
+    // Tile order: row blocks fastest, so that neighbours in a run share halo rows.  Where channel
+    // blocks share lines they go fastest instead, a run holding all of a pixel's: dealt to different XCDs,
+    // every one of them would fetch the whole lines from memory (measured: twice the algorithmic
+    // reads).  Column blocks go before the row blocks: neighbours share S - 1 columns of every row.
+    constexpr bool kSplitLines = splits_lines(GB, GBLKS);
+    constexpr int RUN = kSplitLines ? line_run(SPIO_XCD_CHUNK, GBLKS) : SPIO_XCD_CHUNK;
+    const int b = xcd_tile<RUN, HALF_BLOCKS>(second ? raw - HALF_BLOCKS : raw);
     constexpr int TILES = QBLKS * PBLKS;  // tiles of one image and channel block
     const int t = kSplitLines ? (b / GBLKS) % TILES : b % TILES;
     const int cb = kSplitLines ? b % GBLKS : (b / TILES) % GBLKS;

@@ -223,13 +223,18 @@ SPIO_KERNEL_NAME(float* __restrict__ grad_weight, const spio_uint4* __restrict__
     const int wg = wave % GB;  // group within the workgroup
     const int ws = wave / GB;  // which share of the 32-pixel chunks this wave multiplies
 
-    int b = block_id();
-    if (NUM_BLOCKS % 8 == 0) b = (b & 7) * (NUM_BLOCKS / 8) + (b >> 3);
-    const int qb = b % QBLKS;  // column blocks fastest: neighbours share S - 1 columns of x
+    // One contiguous range of tiles per XCD; column blocks fastest (neighbours share S - 1 columns of x),
+    // then row blocks.  Where channel blocks share lines they go fastest, so that the lines are fetched
+    // from memory once.
+    const int b = xcd_tile<0, NUM_BLOCKS>(block_id());
+    constexpr bool kSplitLines = splits_lines(GB, GBLKS);
+    constexpr int TILES = QBLKS * PBLKS;
+    const int tile = kSplitLines ? (b / GBLKS) % TILES : b % TILES;
+    const int cb = kSplitLines ? b % GBLKS : (b / TILES) % GBLKS;
+    const int nbk = b / (TILES * GBLKS);
+    const int qb = tile % QBLKS;
     const int q0 = qb * BQ;
-    const int pb = PBLKS == 1 ? 0 : (b / QBLKS) % PBLKS;
-    const int cb = (b / (QBLKS * PBLKS)) % GBLKS;
-    const int nbk = b / (QBLKS * PBLKS * GBLKS);
+    const int pb = tile / QBLKS;
     const int p0 = pb * BH;
     const int bh_eff = imin(BH, kP - p0);  // dy rows that exist in this block
     const int gglob = cb * GB + wg;

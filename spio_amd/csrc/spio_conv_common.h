@@ -73,6 +73,30 @@ SPIO_DEVICE void wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// Whether neighbouring channel blocks of `gb` groups share 128-byte lines of the activations: their
+// boundary lies inside a line unless both the block (gb * 16 bytes) and the pixel (2 C bytes) are whole
+// lines.  With C = 296 (592 bytes a pixel) every boundary does, whatever gb is.
+constexpr bool splits_lines(int gb, int gblks) { return gblks > 1 && ((gb * 16) % 128 != 0 || (kC * 2) % 128 != 0); }
+
+// Tile of workgroup `id` in a grid of TILES: workgroup ids are dealt round-robin to the 8 XCDs, here runs
+// of RUN consecutive tiles go to one XCD (what neighbours share, halo rows and lines, they share in that
+// XCD's L2) before the next run goes to the next XCD.  0 = one contiguous range of tiles per XCD.  The
+// tiles behind the last whole turn of 8 runs are dealt as 8 contiguous ranges, so every tile count gets
+// the order, not only multiples of 8 * RUN.
+constexpr int kXcds = 8;
+template <int RUN, int TILES>
+SPIO_DEVICE int xcd_tile(int id) {
+    constexpr int TURN = kXcds * RUN;
+    constexpr int WHOLE = RUN > 0 ? TILES / TURN * TURN : 0;
+    const int x = id % kXcds, k = id / kXcds;  // XCD, position in its sequence
+    if (RUN == 1) return id;
+    if (RUN > 0 && id < WHOLE) return k / (RUN > 0 ? RUN : 1) * TURN + x * RUN + k % (RUN > 0 ? RUN : 1);
+    constexpr int REST = TILES - WHOLE;
+    return WHOLE + x * (REST / kXcds) + imin(x, REST % kXcds) + k - WHOLE / kXcds;
+}
+// Run length where channel blocks share lines and go fastest in the tile order: whole pixels.
+constexpr int line_run(int run, int gblks) { return run <= 1 ? run : (run + gblks - 1) / gblks * gblks; }
+
 // Streaming accesses: activations are touched once per kernel, so they are
 // loaded and stored with the non-temporal hint (measured on MI355X: a plain
 // 16-byte-per-lane copy gains about 10% from it).

@@ -84,6 +84,26 @@ def test_two_tile_heights_and_prefetch_ramp():
         run_grad_kernel_test(conv2d_gw8_kernel_factory, params, configs=configs, igrad=True)
 
 
+@pytest.mark.parametrize("chunk", [0, 4])
+@pytest.mark.parametrize("params", [Conv2dGw8Params(n=7, c=72, h=9, w=10, padding=1, has_bias=True),
+                                    Conv2dGw8Params(n=5, c=296, h=6, w=7, r=5, s=5, padding=2)], ids=lambda p: p.encode())  # fmt: skip
+def test_channel_blocks_that_share_lines(params, chunk):
+    """Channel blocks whose boundary lies inside a 128-byte line: they go fastest in the tile order and a
+    run of tiles on one XCD holds a pixel's blocks.  Tile counts below and above a turn of the 8 XCDs,
+    none of them a multiple of it: every tile has to be computed, by one workgroup."""
+    for gb in (2, 4, 8):
+        mfma = [Conv2dGw8Config(groups=gb, block_p=bp, prefetch=2, xcd_chunk=chunk) for bp in (2, params.p)]
+        images = [Conv2dGw8Config(groups=gb, block_p=params.p, block_n=nb, variant="image", prefetch=2, block_n_iters=2)
+                  for nb in (1, 2) if nb * gb < 16]  # fmt: skip
+        run_kernel_test(conv2d_gw8_kernel_factory, params, configs=mfma + images)
+        run_grad_kernel_test(conv2d_gw8_kernel_factory, params, configs=mfma + images, igrad=True)
+        run_grad_kernel_test(conv2d_gw8_wgrad_kernel_factory, params,
+                             configs=[Conv2dGw8WgradConfig(groups=gb, block_h=4, block_n=1, block_n_iters=2, prefetch=2, two_stage=two)
+                                      for two in (0, 1)])  # fmt: skip
+        run_bgrad_kernel_test(conv2d_gw8_bgrad_kernel_factory, params,
+                              configs=[Conv2dGw8BgradConfig(groups=min(gb, 4), block_h=3, prefetch=2, xcd_chunk=chunk)])
+
+
 def test_column_blocks():
     """Workgroups that own a block of output columns (block_q) and stage block_q + S - 1 source
     columns: widths that are and are not multiples of the block, blocks wider than what is left
