@@ -206,7 +206,13 @@ static_assert(NB * X_IMAGE_BYTES < (1ll << 31) && NB * D_IMAGE_BYTES < (1ll << 3
 constexpr int X_ROW_BYTES = kW * kC * 2;
 constexpr int D_ROW_BYTES = kQ * kC * 2;
 constexpr unsigned OOB = 0x80000000u;  // offset of a lane without data: beyond every descriptor
-constexpr int AUX_NT = SPIO_NT ? 2 : 0;
+// Cache-policy operands of the buffer instructions: streamed (2) unless several channel blocks share the
+// lines, then loaded with the default policy so that the second block finds them in L2 (50n 152c 21x41 17.3
+// -> 15.7 us, 94n 296c 43x47 125 -> 115, 128n 96c 56x56 56.1 -> 54.9).  SPIO_NT = 0 stores with the
+// default policy: L2 then joins the parts of a line that different blocks store, see the configurations.
+constexpr bool kSplitLines = splits_lines(GB, GBLKS);
+constexpr int AUX_LD = kSplitLines ? 0 : 2;
+constexpr int AUX_ST = SPIO_NT ? 2 : 0;
 
 typedef __amdgpu_buffer_rsrc_t rsrc_t;
 SPIO_DEVICE rsrc_t make_rsrc(const void* base, int bytes) {
@@ -253,7 +259,6 @@ SPIO_KERNEL_NAME(spio_uint4* __restrict__ grad_input, float* __restrict__ grad_w
     // rows through one XCD's L2.  Where channel blocks share lines they go fastest instead, a run
     // holding all of a pixel's: dealt to different XCDs, every one of them would fetch the whole lines
     // from memory (measured: twice the algorithmic reads).
-    constexpr bool kSplitLines = splits_lines(GB, GBLKS);
     constexpr int RUN = kSplitLines ? line_run(SPIO_XCD_CHUNK, GBLKS) : SPIO_XCD_CHUNK;
     const int b = xcd_tile<RUN, NUM_BLOCKS>(block_id());
     // Column blocks go before the row blocks: neighbours share S - 1 columns of every row.
@@ -404,7 +409,7 @@ SPIO_KERNEL_NAME(spio_uint4* __restrict__ grad_input, float* __restrict__ grad_w
             for (int l = 0; l < LPTX; ++l) {
                 Pack16 v;
                 v.i = (SPIO_HALO_CACHED && xhalo) ? __builtin_amdgcn_raw_buffer_load_b128(rx, (int)x_voff[l], sx, 0)
-                                                  : __builtin_amdgcn_raw_buffer_load_b128(rx, (int)x_voff[l], sx, AUX_NT);
+                                                  : __builtin_amdgcn_raw_buffer_load_b128(rx, (int)x_voff[l], sx, AUX_LD);
                 xr[l] = v.u;
             }
             const int pr = p0 - PB + t;
@@ -415,7 +420,7 @@ SPIO_KERNEL_NAME(spio_uint4* __restrict__ grad_input, float* __restrict__ grad_w
             for (int l = 0; l < LPTD; ++l) {
                 Pack16 v;
                 v.i = (SPIO_HALO_CACHED && dhalo) ? __builtin_amdgcn_raw_buffer_load_b128(rd, (int)d_voff[l], sd, 0)
-                                                  : __builtin_amdgcn_raw_buffer_load_b128(rd, (int)d_voff[l], sd, AUX_NT);
+                                                  : __builtin_amdgcn_raw_buffer_load_b128(rd, (int)d_voff[l], sd, AUX_LD);
                 dr[l] = v.u;
             }
         };
@@ -496,7 +501,7 @@ SPIO_KERNEL_NAME(spio_uint4* __restrict__ grad_input, float* __restrict__ grad_w
             for (int l = 0; l < LPTO; ++l) {
                 Pack16 v;
                 v.u = *reinterpret_cast<const spio_uint4*>(ostage + obuf * OUT_ROW_BYTES + o_lds[l]);
-                __builtin_amdgcn_raw_buffer_store_b128(v.i, rs, (int)(o_voff[l] + row_off), 0, AUX_NT);
+                __builtin_amdgcn_raw_buffer_store_b128(v.i, rs, (int)(o_voff[l] + row_off), 0, AUX_ST);
             }
             store_group_end();
         };

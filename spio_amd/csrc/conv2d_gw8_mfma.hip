@@ -184,9 +184,14 @@ constexpr int rows_requested(int t, int steps) { return cmin(cmin(steps, t + 1 +
 #endif
 // Cache-policy operands of the buffer instructions (gfx950: 1 = sc0, 2 = nt, 16 = sc1), one for
 // the interior source rows, one for the rows shared with neighbouring row blocks, one for the
-// stores.  SPIO_NT = 1 streams with the non-temporal hint unless a policy is given explicitly.
+// stores.  SPIO_NT = 1 streams with the non-temporal hint unless a policy is given explicitly;
+// source rows whose lines several channel blocks share are loaded with the default policy all the
+// same: the block that comes second finds the line in L2.  Forward, non-temporal -> default loads:
+// 64n 160c 40x40 22.5 -> 14.4 us, 46n 1072c 17x17 17.7 -> 15.0, 94n 296c 43x47 83.2 -> 76.7, 128n 96c
+// 56x56 29.7 -> 29.1; where the blocks are whole lines the hint is worth 15 %.
+constexpr bool kSplitLines = splits_lines(GB, GBLKS);
 #ifndef SPIO_LD_POLICY
-#define SPIO_LD_POLICY (SPIO_NT ? 2 : 0)
+#define SPIO_LD_POLICY (SPIO_NT && !kSplitLines ? 2 : 0)
 #endif
 #ifndef SPIO_ST_POLICY
 #define SPIO_ST_POLICY (SPIO_NT ? 2 : 0)
@@ -607,7 +612,6 @@ SPIO_KERNEL_NAME(spio_uint4* __restrict__ dst, const spio_uint4* __restrict__ sr
     // blocks share lines they go fastest instead, a run holding all of a pixel's: dealt to different XCDs,
     // every one of them would fetch the whole lines from memory (measured: twice the algorithmic
     // reads).  Column blocks go before the row blocks: neighbours share S - 1 columns of every row.
-    constexpr bool kSplitLines = splits_lines(GB, GBLKS);
     constexpr int RUN = kSplitLines ? line_run(SPIO_XCD_CHUNK, GBLKS) : SPIO_XCD_CHUNK;
     const int b = xcd_tile<RUN, HALF_BLOCKS>(second ? raw - HALF_BLOCKS : raw);
     constexpr int TILES = QBLKS * PBLKS;  // tiles of one image and channel block

@@ -19,7 +19,7 @@ from typing import Dict, List, Tuple
 import torch
 
 from ..util.math import divup
-from .conv2d_gw8_kernel import _shape_defines
+from .conv2d_gw8_kernel import _shape_defines, with_joined_stores
 from .conv2d_gw8_params import Conv2dGw8Params
 from .conv2d_stats import Conv2dStats
 from .kernel import KernelSpec
@@ -62,6 +62,7 @@ class Conv2dGw8BgradConfig:
         block_q: columns per workgroup (0: the whole width; else a multiple of 32 with
             block_n = 1).  The workgroup stages block_q + S - 1 columns of x and of grad_output, so
             rows of any width fit.
+        nontemporal: 1 = store grad_input with the non-temporal hint.
     """
 
     groups: int = 4
@@ -74,6 +75,7 @@ class Conv2dGw8BgradConfig:
     xcd_chunk: int = 4
     block_q: int = 0
     two_stage: int = 0
+    nontemporal: int = 1
 
 
 def bgrad_is_supported(params: Conv2dGw8Params) -> bool:
@@ -241,7 +243,7 @@ def _get_configs(params: Conv2dGw8Params, device_attr=None) -> List[Conv2dGw8Bgr
     # ... and two-stage publishing for the leaders of every height
     configs += [replace(cfg, two_stage=1) for cfg in list(configs) if cfg.prefetch == 4 and cfg.halo_cached == 1
                 and cfg.xcd_chunk == 4][:2 * GEOMETRIES_PER_HEIGHT]  # fmt: skip
-    return configs
+    return with_joined_stores(params, configs)
 
 
 def _get_kernel_spec(params: Conv2dGw8Params, config: Conv2dGw8BgradConfig, _device_attr=None) -> KernelSpec:
@@ -253,7 +255,7 @@ def _get_kernel_spec(params: Conv2dGw8Params, config: Conv2dGw8BgradConfig, _dev
                    SPIO_ITERS=config.block_n_iters,
                    SPIO_PF=config.prefetch, SPIO_TS=config.split,
                    SPIO_HALO_CACHED=config.halo_cached, SPIO_XCD_CHUNK=config.xcd_chunk,
-                   SPIO_HAS_BIAS=int(params.has_bias))  # fmt: skip
+                   SPIO_NT=config.nontemporal, SPIO_HAS_BIAS=int(params.has_bias))  # fmt: skip
     if config.block_q:
         defines["SPIO_BQ"] = config.block_q
     spec = KernelSpec(defines, LaunchParams(grid=g["NUM_BLOCKS"], block=g["THREADS"]), SOURCE, notes=g)

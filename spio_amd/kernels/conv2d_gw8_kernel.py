@@ -49,7 +49,8 @@ class Conv2dGw8Config:
         block_n: images whose rows are laid side by side in one staged row.
         split: waves sharing the 16-pixel tiles of one group.
         prefetch: rows of global loads in flight ahead of the computed row.
-        nontemporal: 1 = stream activations with the non-temporal hint.
+        nontemporal: 1 = stream activations with the non-temporal hint (loads only where no
+            two channel blocks share lines).
         halo_cached: 1 = load rows shared with neighbouring row blocks with the default
             cache policy so the second reader can hit in L2.
         xcd_chunk: consecutive tiles that go to the same XCD (they share halo rows through its
@@ -376,6 +377,7 @@ def _get_configs(params: Conv2dGw8Params, device_attr=None, igrad: bool = False)
             for hc, ch in ((0, 4), (1, 0), (0, 0)):
                 configs.append(replace(cfg, halo_cached=hc, xcd_chunk=ch))
     configs += _two_height_configs(params, configs, igrad, num_cus)
+    configs = with_joined_stores(params, configs)
     # small images: the whole-image kernel; its two best candidates go first, so that the capped
     # sweep an operator runs on an unrecorded shape sees both kernels
     image = _image_configs(params, igrad, num_cus)
@@ -385,6 +387,23 @@ def _get_configs(params: Conv2dGw8Params, device_attr=None, igrad: bool = False)
         configs = configs[:2] + image[:2] + configs[2:] + image[2:]
     configs.append(Conv2dGw8Config(groups=1, block_p=1, block_n=1, split=1, variant="direct"))
     return configs
+
+
+def with_joined_stores(params: Conv2dGw8Params, configs: list) -> list:
+    """`configs` with a second version of the leading eight, right behind each, that stores through L2.
+
+    With an odd number of groups the boundary between two channel blocks is not even 32-byte aligned and
+    memory has to merge the parts of a sector that two blocks store, unless L2 does it first.  Measured,
+    non-temporal -> default stores: 60n 216c 56x56 68 -> 48 us, 94n 296c 43x47 77 -> 64, 30n 184c 60x60
+    26 -> 23; on small images it costs instead (32n 808c 20x20 11.4 -> 13.7), so the sweep decides; a capped one
+    does not count the second versions, whose geometry it tries anyway.  With an even number the hint is
+    the better one or equal (128n 96c 56x56 29.1 against 35.0)."""
+    out = []
+    for i, cfg in enumerate(configs):
+        out.append(cfg)
+        if i < 8 and params.groups % 2 and cfg.groups < params.groups:
+            out.append(replace(cfg, nontemporal=0))
+    return out
 
 
 def _shape_defines(params: Conv2dGw8Params) -> Dict[str, object]:

@@ -56,6 +56,17 @@ def _on_miss_limit() -> int:
         return DEFAULT_ON_MISS_CONFIGS
 
 
+def _leading(configs, count: int) -> int:
+    """Length of the part of `configs` that holds the first `count` geometries; one that differs from its
+    predecessor in the store policy alone (nontemporal = 0) belongs to it."""
+    for i, config in enumerate(configs):
+        if getattr(config, "nontemporal", 1):
+            if count == 0:
+                return i
+            count -= 1
+    return len(configs)
+
+
 def _stream_is_capturing() -> bool:
     try:
         import torch  # pylint: disable=import-outside-toplevel
@@ -193,7 +204,7 @@ class Tuner:
             # inside an operator call: only the best-ranked few, so that a model with many new
             # shapes does not stall (the last entry of a list is its any-shape kernel: keep it as
             # the independent implementation the winner is checked against)
-            limit = _on_miss_limit()
+            limit = _leading(configs, _on_miss_limit())
             if len(configs) > limit + 1:
                 configs = configs[:limit] + [configs[-1]]
             return self.sweep(kernel_factory, params, ordinal, device_attr, configs, **kernel_kwargs)

@@ -4,6 +4,7 @@ record store.  CPU only."""
 
 import json
 import os
+from dataclasses import replace
 
 import pytest
 
@@ -413,3 +414,18 @@ def test_weight_gradient_mfma_kernel_is_not_offered_past_its_32_bit_indices():
     assert {c.variant for c in conv2d_gw8_wgrad_kernel_factory.configs(past, attr)} == {"direct"}
     assert conv2d_gw8_kernel_factory.configs(past, attr)[0].variant == "mfma"
     assert conv2d_gw8_bgrad_kernel_factory.configs(past, attr)
+
+
+def test_second_store_policies_do_not_shorten_a_capped_sweep():
+    """With an odd number of groups in several channel blocks the leading configurations come in two store
+    policies; the first `count` geometries of a capped sweep are the same as without them."""
+    from spio_amd.kernels.tuner import _leading
+
+    for factory in (conv2d_gw8_kernel_factory, conv2d_gw8_bgrad_kernel_factory):
+        odd = list(factory.configs(Conv2dGw8Params(n=50, c=152, h=21, w=41, padding=1), DeviceAttributes()))
+        both = odd[:_leading(odd, 8)]
+        assert sum(c.nontemporal for c in both) == 8 and any(not c.nontemporal for c in both)
+        for before, c in zip(both, both[1:]):
+            assert c.nontemporal or replace(c, nontemporal=1) == before
+        even = list(factory.configs(Conv2dGw8Params(n=50, c=160, h=21, w=41, padding=1), DeviceAttributes()))
+        assert all(c.nontemporal for c in even) and _leading(even, 8) == 8 and _leading(even, 10**6) == len(even)
