@@ -199,11 +199,13 @@ constexpr int LDS_UNITS = max3(STREAM_UNITS, FILTER_UNITS, (PUBLISH_FLOATS + 3) 
 static_assert(LDS_UNITS * 16 <= 160 * 1024, "LDS overflow");
 static_assert(PF >= 2 && PF % 2 == 0 && WAVES <= 16, "bad configuration");
 
-constexpr long long X_IMAGE_BYTES = (long long)kH * kW * kC * 2;  // of x and dx
+constexpr long long X_IMAGE_BYTES = (long long)kH * kW * kC * 2;  // of x
+constexpr long long DX_IMAGE_BYTES = (long long)kH * kW * kC * kDstBytes;  // of dx
 constexpr long long D_IMAGE_BYTES = (long long)kP * kQ * kC * 2;  // of dy
-static_assert(NB * X_IMAGE_BYTES < (1ll << 31) && NB * D_IMAGE_BYTES < (1ll << 31),
+static_assert(NB * DX_IMAGE_BYTES < (1ll << 31) && NB * D_IMAGE_BYTES < (1ll << 31),
               "an image block must stay below 2 GiB (32-bit buffer offsets)");
 constexpr int X_ROW_BYTES = kW * kC * 2;
+constexpr int DX_ROW_BYTES = kW * kC * kDstBytes;
 constexpr int D_ROW_BYTES = kQ * kC * 2;
 constexpr unsigned OOB = 0x80000000u;  // offset of a lane without data: beyond every descriptor
 // Cache-policy operands of the buffer instructions: streamed (2) unless several channel blocks share the
@@ -339,8 +341,8 @@ SPIO_KERNEL_NAME(spio_uint4* __restrict__ grad_input, float* __restrict__ grad_w
                                       (int)(images * X_IMAGE_BYTES));
         const rsrc_t rs_dy = make_rsrc(reinterpret_cast<const unsigned char*>(dy) + n0 * D_IMAGE_BYTES,
                                        (int)(images * D_IMAGE_BYTES));
-        const rsrc_t rs_dx = make_rsrc(reinterpret_cast<const unsigned char*>(grad_input) + n0 * X_IMAGE_BYTES,
-                                       (int)(images * X_IMAGE_BYTES));
+        const rsrc_t rs_dx = make_rsrc(reinterpret_cast<const unsigned char*>(grad_input) + n0 * DX_IMAGE_BYTES,
+                                       (int)(images * DX_IMAGE_BYTES));
 
         // ---- loop-invariant addressing (cells without data carry the out-of-range offset: they
         //      load zeros, which is what halo and gap cells must hold) ----
@@ -393,7 +395,7 @@ SPIO_KERNEL_NAME(spio_uint4* __restrict__ grad_input, float* __restrict__ grad_w
                 o_lds[l] = (img * WPI + q) * OSTRIDE + g * 16;
                 const int wx = q0 + q - XOX;  // column of dx
                 if (q0 + q < DW && wx >= 0 && wx < kW && cb * GB + g < kGroups)
-                    o_voff[l] = (unsigned)(((img * kH * kW + wx) * kGroups + cb * GB + g) * 16);
+                    o_voff[l] = (unsigned)(((img * kH * kW + wx) * kGroups + cb * GB + g) * (8 * kDstBytes));
             }
         }
 
@@ -496,12 +498,24 @@ SPIO_KERNEL_NAME(spio_uint4* __restrict__ grad_input, float* __restrict__ grad_w
             // instructions from writing them: with the row offset in a scalar register a result
             // moved into the first data register right behind the store was stored in its place
             // (seen on gfx950 as stray values in the first two channels of some pixels).
-            const unsigned row_off = (unsigned)(imin(imax(h - XOY, 0), kH - 1) * X_ROW_BYTES);
+            const unsigned row_off = (unsigned)(imin(imax(h - XOY, 0), kH - 1) * DX_ROW_BYTES);
 #pragma unroll
             for (int l = 0; l < LPTO; ++l) {
-                Pack16 v;
-                v.u = *reinterpret_cast<const spio_uint4*>(ostage + obuf * OUT_ROW_BYTES + o_lds[l]);
-                __builtin_amdgcn_raw_buffer_store_b128(v.i, rs, (int)(o_voff[l] + row_off), 0, AUX_ST);
+                const unsigned char* row = ostage + obuf * OUT_ROW_BYTES;
+                if (SPIO_DST_F32) {
+                    const int half = lane & 1;
+                    auto store_half = [&](int voff, int from) {
+                        const spio_uint2 v = *reinterpret_cast<const spio_uint2*>(row + from + 8 * half);
+                        __builtin_amdgcn_raw_buffer_store_b128(widen(v), rs, (int)((unsigned)voff + 16 * half + row_off),
+                                                               0, AUX_ST);
+                    };
+                    store_half(quad_lane<0>((int)o_voff[l]), quad_lane<0>(o_lds[l]));
+                    store_half(quad_lane<1>((int)o_voff[l]), quad_lane<1>(o_lds[l]));
+                } else {
+                    Pack16 v;
+                    v.u = *reinterpret_cast<const spio_uint4*>(row + o_lds[l]);
+                    __builtin_amdgcn_raw_buffer_store_b128(v.i, rs, (int)(o_voff[l] + row_off), 0, AUX_ST);
+                }
             }
             store_group_end();
         };

@@ -94,7 +94,13 @@ SPIO_KERNEL_NAME(spio_uint4* __restrict__ dst, const spio_uint4* __restrict__ sr
     Pack16 o;
 #pragma unroll
     for (int k = 0; k < 8; ++k) o.h[k] = (spio_half)acc[k];
+#if SPIO_DST_F32
+    const spio_uint2 halves[2] = {{o.u[0], o.u[1]}, {o.u[2], o.u[3]}};
+#pragma unroll
+    for (int i = 0; i < 2; ++i) dst[2 * idx + i] = widen(halves[i]);
+#else
     dst[idx] = o.u;
+#endif
 }
 
 #else  // SPIO_WGRAD

@@ -142,9 +142,9 @@ static_assert(LDS_UNITS * 16 <= 160 * 1024, "LDS overflow");
 static_assert(OUT_ROW_BYTES % 16 == 0, "output rows are read in 16-byte units");
 
 constexpr long long SRC_IMAGE_BYTES = (long long)SH * SW * kC * 2;
-constexpr long long DST_IMAGE_BYTES = (long long)DH * DW * kC * 2;
+constexpr long long DST_IMAGE_BYTES = (long long)DH * DW * kC * kDstBytes;
 static_assert(NB * SRC_IMAGE_BYTES < (1ll << 30) && NB * DST_IMAGE_BYTES < (1ll << 30) &&
-                  (long long)(LPT > SPT ? LPT : SPT) * CELL_STEP < (1ll << 30),
+                  (long long)(LPT > SPT ? LPT : SPT) * CELL_STEP * (kDstBytes / 2) < (1ll << 30),
               "an image block must stay far below 2 GiB (32-bit buffer offsets)");
 constexpr unsigned OOB = 0x80000000u;    // offset of a lane without data: beyond every descriptor
 // Cache-policy operands of the buffer instructions: streamed (2) unless several channel blocks share the
@@ -380,11 +380,28 @@ struct BlockMover {
     //  of a 16-byte buffer store untouched for the wait states the hardware needs.)
     SPIO_DEVICE void store(int blk, bool enabled, lds_bytep out) const {
         const rsrc_t rs = block_rsrc(dst, DST_IMAGE_BYTES, blk, enabled);
+        if (SPIO_DST_F32) {
+            // the thread's offset in a block of twice the bytes; OOB stays beyond every descriptor
+            const int half = thread_id() & 1;
+            const int wide = (int)(voff == OOB ? OOB : 2 * voff);
+            auto store_half = [&](int base, int from, int s) {
+                typedef __attribute__((address_space(3))) spio_uint2* lds_u2p;
+                __builtin_amdgcn_raw_buffer_store_b128(widen(*(lds_u2p)(out + from + 8 * half)), rs,
+                                                       (int)((unsigned)base + 16 * half + (unsigned)(2 * CELL_STEP * s)),
+                                                       0, AUX_ST);
+            };
 #pragma unroll
-        for (int s = 0; s < SPT; ++s) {
-            Pack16 v;
-            v.u = *(lds_u4p)(out + out_lds[s]);
-            __builtin_amdgcn_raw_buffer_store_b128(v.i, rs, (int)(voff + (unsigned)(CELL_STEP * s)), 0, AUX_ST);
+            for (int s = 0; s < SPT; ++s) {
+                store_half(quad_lane<0>(wide), quad_lane<0>(out_lds[s]), s);
+                store_half(quad_lane<1>(wide), quad_lane<1>(out_lds[s]), s);
+            }
+        } else {
+#pragma unroll
+            for (int s = 0; s < SPT; ++s) {
+                Pack16 v;
+                v.u = *(lds_u4p)(out + out_lds[s]);
+                __builtin_amdgcn_raw_buffer_store_b128(v.i, rs, (int)(voff + (unsigned)(CELL_STEP * s)), 0, AUX_ST);
+            }
         }
         // (not in the mover waves: a scheduling fence after every block's stores costs them 8 % at
         //  384 channels 14x14; their stores keep the constant-offset form above, for which the

@@ -165,7 +165,7 @@ static_assert(LDS_UNITS * 16 <= 160 * 1024, "LDS overflow");
 
 // Byte extents of the NB-image block a workgroup addresses through one buffer descriptor.
 constexpr long long SRC_IMAGE_BYTES = (long long)SH * SW * kC * 2;
-constexpr long long DST_IMAGE_BYTES = (long long)DH * DW * kC * 2;
+constexpr long long DST_IMAGE_BYTES = (long long)DH * DW * kC * kDstBytes;
 static_assert(NB * SRC_IMAGE_BYTES < (1ll << 31) && NB * DST_IMAGE_BYTES < (1ll << 31),
               "an image block must stay below 2 GiB (32-bit buffer offsets)");
 constexpr unsigned OOB = 0x80000000u;  // offset of a lane without data: beyond every descriptor
@@ -263,7 +263,7 @@ SPIO_DEVICE void conv_rows(spio_uint4* __restrict__ dst, const spio_uint4* __res
         }
     }
     constexpr int SRC_ROW_BYTES = SW * kC * 2;
-    constexpr int DST_ROW_BYTES = DW * kC * 2;
+    constexpr int DST_ROW_BYTES = DW * kC * kDstBytes;
 
     // Source row `t` of this workgroup (image row p0 + t - EPY) for every cell of the thread.
     // Rows outside the image read through the empty descriptor: zeros, the vertical padding.
@@ -346,7 +346,7 @@ SPIO_DEVICE void conv_rows(spio_uint4* __restrict__ dst, const spio_uint4* __res
             const int img = cell / (GB * BQ);
             out_lds[s] = (img * WPI + q) * OSTRIDE + g * 16;
             if (cb * GB + g < kGroups && q0 + q < DW)
-                out_voff[s] = (unsigned)(((img * DH * DW + q0 + q) * kGroups + cb * GB + g) * 16);
+                out_voff[s] = (unsigned)(((img * DH * DW + q0 + q) * kGroups + cb * GB + g) * (8 * kDstBytes));
         }
     }
 
@@ -465,9 +465,21 @@ SPIO_DEVICE void conv_rows(spio_uint4* __restrict__ dst, const spio_uint4* __res
         const unsigned row_off = (unsigned)(imin(imax(p, 0), DH - 1) * DST_ROW_BYTES);
 #pragma unroll
         for (int s = 0; s < SPT; ++s) {
-            Pack16 v;
-            v.u = *(lds_u4p)(ostage + obuf * OUT_ROW_BYTES + out_lds[s]);
-            __builtin_amdgcn_raw_buffer_store_b128(v.i, rs, (int)(out_voff[s] + row_off), 0, AUX_ST);
+            const lds_bytep row = ostage + obuf * OUT_ROW_BYTES;
+            if (SPIO_DST_F32) {
+                typedef __attribute__((address_space(3))) spio_uint2* lds_u2p;
+                const int half = lane & 1;
+                auto store_half = [&](int voff, int from) {
+                    __builtin_amdgcn_raw_buffer_store_b128(widen(*(lds_u2p)(row + from + 8 * half)), rs,
+                                                           (int)((unsigned)voff + 16 * half + row_off), 0, AUX_ST);
+                };
+                store_half(quad_lane<0>((int)out_voff[s]), quad_lane<0>(out_lds[s]));
+                store_half(quad_lane<1>((int)out_voff[s]), quad_lane<1>(out_lds[s]));
+            } else {
+                Pack16 v;
+                v.u = *(lds_u4p)(row + out_lds[s]);
+                __builtin_amdgcn_raw_buffer_store_b128(v.i, rs, (int)(out_voff[s] + row_off), 0, AUX_ST);
+            }
         }
         store_group_end();
     };

@@ -118,6 +118,36 @@ SPIO_DEVICE void store_stream(spio_uint4 v, spio_uint4* p) {
 #endif
 }
 
+// Kernels that write activations can store them as fp32 (SPIO_DST_F32): the same values, rounded to fp16
+// once and widened on the way out, for a caller whose tensors are fp32.  A pass of its own over the result
+// reads 2 bytes and writes 4 per element behind the 2 written here; stored wide at once it is 4 written.
+#ifndef SPIO_DST_F32
+#define SPIO_DST_F32 0
+#endif
+constexpr int kDstBytes = SPIO_DST_F32 ? 4 : 2;
+// A finished row leaves LDS as 16-byte units of 8 channels, one per lane, which widen to 32 bytes: two
+// stores.  In store j the lanes 2i and 2i+1 of a quad write the halves of the unit of the quad's lane
+// 2j + i, so that every quad fills 64 consecutive bytes; a lane that wrote its own two halves would leave
+// every second 16 bytes of a line to the other store.  quad_lane<j> is that lane's value of `v`.
+template <int J>
+SPIO_DEVICE int quad_lane(int v) {
+    return __builtin_amdgcn_update_dpp(0, v, J ? 0xFA : 0x50, 0xf, 0xf, false);  // quad_perm [2,2,3,3] / [0,0,1,1]
+}
+SPIO_DEVICE spio_uint4 widen(spio_uint2 v) {
+    union {
+        spio_float4 f;
+        spio_uint4 u;
+    } o;
+    union {
+        spio_uint2 u;
+        spio_half4 h;
+    } i;
+    i.u = v;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o.f[e] = (float)i.h[e];
+    return o.u;
+}
+
 // Closes a group of 16-byte buffer stores.  Such a store reads its data registers for a few
 // cycles after it issues; an instruction that writes one of them in the very next slot can have
 // its value stored instead (seen on gfx950 as stray values in the first two channels of some

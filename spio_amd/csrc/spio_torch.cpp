@@ -71,7 +71,7 @@ struct Stage {
 struct Plan {
     Stage main, second;         // `second` of two-stage kernels
     int64_t workspace = 0;      // bytes of partial results between the stages
-    bool present = false;       // false: the shape does not use this kind (no fused backward)
+    bool present = false;       // false: the shape does not use this kind (no fused backward, no float32 output)
     bool overwrites = false;    // the kernel stores its sums whole instead of adding to them
 };
 using PlanPtr = std::shared_ptr<const Plan>;
@@ -193,9 +193,18 @@ int64_t fused_mode() {
 
 // ---- convolution ----------------------------------------------------------------------------
 
-Tensor conv_forward(const Conv& cv, const Tensor& x, const Tensor& w, const Tensor& bias) {
-    const auto plan = find_plan(cv.key(FPROP, x.get_device()));
-    Tensor y = empty_cl({cv.n, cv.c, cv.p(), cv.q()}, at::kHalf, x);
+constexpr int64_t WIDE = 4;  // bit of a key's mode: the kernel stores its activations as float32
+
+// `dtype`: what the caller wants; float32 comes from the kernel itself where it has such a version,
+// else the result is float16 and the caller converts it.
+Tensor conv_forward(const Conv& cv, const Tensor& x, const Tensor& w, const Tensor& bias, at::ScalarType dtype) {
+    PlanPtr plan;
+    if (dtype == at::kFloat) plan = find_plan(cv.key(FPROP, x.get_device(), WIDE));
+    if (!plan || !plan->present) {
+        dtype = at::kHalf;
+        plan = find_plan(cv.key(FPROP, x.get_device()));
+    }
+    Tensor y = empty_cl({cv.n, cv.c, cv.p(), cv.q()}, dtype, x);
     launch(plan->main, c10::hip::getCurrentHIPStream(x.get_device()), {ptr(y), ptr(x), ptr(w), ptr(bias)});
     return y;
 }
@@ -207,8 +216,15 @@ struct ConvGrads {
 // The backward operator on channels_last tensors: one fused kernel where the shape uses it and
 // both gradients are wanted, else the weight and the data gradient one after the other.
 ConvGrads conv_backward(const Conv& cv, const Tensor& x, const Tensor& w, const Tensor& dy, bool need_x,
-                        bool need_w, bool need_b) {
+                        bool need_w, bool need_b, at::ScalarType x_dtype) {
     ConvGrads g;
+    // the version of a kernel whose grad_input is float32, where that is wanted and there is one
+    auto wide_or = [&](const PlanPtr& plan, Kind kind, int64_t mode) {
+        const auto wide = x_dtype == at::kFloat ? find_plan(cv.key(kind, dy.get_device(), mode | WIDE)) : nullptr;
+        const bool use = wide && wide->present;
+        g.x = empty_cl({cv.n, cv.c, cv.h, cv.w}, use ? at::kFloat : at::kHalf, dy);
+        return use ? wide : plan;
+    };
     const auto device = dy.get_device();
     hipStream_t stream = c10::hip::getCurrentHIPStream(device);
     // atomic kernels add into zeroed sums, two-stage ones store them whole
@@ -225,10 +241,10 @@ ConvGrads conv_backward(const Conv& cv, const Tensor& x, const Tensor& w, const 
         const int64_t mode = fused_mode();
         if (mode != 0) fused = find_plan(cv.key(BGRAD, device, mode));
         if (fused && !fused->present) fused.reset();
+        if (fused) fused = wide_or(fused, BGRAD, mode);
     }
     if (fused) {
         sums(*fused, cv.bias && need_b, fused->overwrites);
-        g.x = empty_cl({cv.n, cv.c, cv.h, cv.w}, at::kHalf, dy);
         Tensor workspace;
         if (fused->second.function) workspace = empty_1d(fused->workspace, at::kByte, dy);
         const void* dw = workspace.defined() ? ptr(workspace) : ptr(g.w);
@@ -251,8 +267,7 @@ ConvGrads conv_backward(const Conv& cv, const Tensor& x, const Tensor& w, const 
     }
     if (need_b && !g.b.defined()) g.b = dy.sum({0, 2, 3}, /*keepdim=*/false, at::kFloat);
     if (need_x && !g.x.defined()) {
-        const auto plan = find_plan(cv.key(DGRAD, device));
-        g.x = empty_cl({cv.n, cv.c, cv.h, cv.w}, at::kHalf, dy);
+        const auto plan = wide_or(find_plan(cv.key(DGRAD, device)), DGRAD, 0);
         launch(plan->main, stream, {ptr(g.x), ptr(dy), ptr(w), nullptr});
     }
     return g;
@@ -276,7 +291,7 @@ struct ConvFunction : torch::autograd::Function<ConvFunction> {
                           const std::optional<Tensor>& bias_arg, const Conv& cv) {
         const Tensor bias = bias_arg.value_or(Tensor());
         const Tensor xh = to_half_cl(x), wh = to_half_cl(w);
-        Tensor y = conv_forward(cv, xh, wh, to_float_1d(bias));
+        Tensor y = conv_forward(cv, xh, wh, to_float_1d(bias), x.scalar_type());
         ctx->save_for_backward({xh, wh});
         ctx->saved_data["v"] = std::vector<int64_t>{
             cv.n, cv.c, cv.h, cv.w, cv.r, cv.s, cv.py, cv.px, cv.bias, static_cast<int64_t>(x.scalar_type()),
@@ -302,7 +317,8 @@ struct ConvFunction : torch::autograd::Function<ConvFunction> {
             auto get = [&](int i) { return r[i].is_none() ? Tensor() : r[i].cast<Tensor>(); };
             g = {get(0), get(1), get(2)};
         } else {
-            g = conv_backward(cv, x, w, to_half_cl(grads[0]), need_x, need_w, need_b);
+            g = conv_backward(cv, x, w, to_half_cl(grads[0]), need_x, need_w, need_b,
+                              static_cast<at::ScalarType>(v[9]));
         }
         auto typed = [&](const Tensor& t, int i) {
             return t.defined() ? t.to(static_cast<at::ScalarType>(v[i])) : t;
@@ -459,7 +475,7 @@ PyObject* conv2d_gw8(PyObject*, PyObject* const* args, Py_ssize_t nargs, PyObjec
             y = ConvFunction::apply(x, w, optional(bias), cv);
         } else {
             at::AutoDispatchBelowADInplaceOrView below;
-            y = conv_forward(cv, to_half_cl(x), to_half_cl(w), to_float_1d(bias)).to(x.scalar_type());
+            y = conv_forward(cv, to_half_cl(x), to_half_cl(w), to_float_1d(bias), x.scalar_type()).to(x.scalar_type());
         }
     }
     return THPVariable_Wrap(y);

@@ -19,7 +19,7 @@ from typing import Dict, List, Tuple
 import torch
 
 from ..util.math import divup
-from .conv2d_gw8_kernel import _shape_defines, with_joined_stores
+from .conv2d_gw8_kernel import _shape_defines, fits_float32_output, with_joined_stores
 from .conv2d_gw8_params import Conv2dGw8Params
 from .conv2d_stats import Conv2dStats
 from .kernel import KernelSpec
@@ -246,11 +246,20 @@ def _get_configs(params: Conv2dGw8Params, device_attr=None) -> List[Conv2dGw8Bgr
     return with_joined_stores(params, configs)
 
 
-def _get_kernel_spec(params: Conv2dGw8Params, config: Conv2dGw8BgradConfig, _device_attr=None) -> KernelSpec:
+def _get_kernel_name(out_f32: bool = False) -> str:
+    return "spio_conv2d_gw8_bgrad" + ("_f32" if out_f32 else "")
+
+
+def _get_kernel_spec(params: Conv2dGw8Params, config: Conv2dGw8BgradConfig, _device_attr=None,
+                     out_f32: bool = False) -> KernelSpec:  # fmt: skip
+    """Macros and launch geometry; `out_f32`: grad_input is a float32 tensor."""
     params.validate()
     assert _config_is_legal(params, config), f"illegal configuration {config} for {params}"
     g = bgrad_geometry(params, config)
     defines = _shape_defines(params)
+    if out_f32:
+        assert fits_float32_output(params, config), f"no float32 output for {config} and {params}"
+        defines["SPIO_DST_F32"] = 1
     defines.update(SPIO_GB=config.groups, SPIO_BH=g["BH"], SPIO_NB=config.block_n,
                    SPIO_ITERS=config.block_n_iters,
                    SPIO_PF=config.prefetch, SPIO_TS=config.split,
@@ -290,7 +299,7 @@ conv2d_gw8_bgrad_kernel_factory = KernelFactory(
     Conv2dGw8Params,
     Conv2dGw8BgradConfig,
     Conv2dStats,
-    kernel_name="spio_conv2d_gw8_bgrad",
+    kernel_name=_get_kernel_name,
     configs=_get_configs,
     kernel_spec=_get_kernel_spec,
     make_test_args=_make_test_args,

@@ -414,11 +414,22 @@ def _shape_defines(params: Conv2dGw8Params) -> Dict[str, object]:
     }  # fmt: skip
 
 
+def fits_float32_output(params: Conv2dGw8Params, config) -> bool:
+    """Whether a configuration can store its activations as float32: an image block of four bytes an
+    element has to stay within the 32-bit buffer offsets, as one of two bytes does."""
+    block_n = getattr(config, "block_n", 1)
+    return block_n * params.c * max(params.h * params.w, params.p * params.q) * 4 < 2**30
+
+
 def _get_kernel_spec(params: Conv2dGw8Params, config: Conv2dGw8Config, _device_attr=None,
-                     igrad: bool = False) -> KernelSpec:  # fmt: skip
-    """Macros and launch geometry for one (params, config, direction)."""
+                     igrad: bool = False, out_f32: bool = False) -> KernelSpec:  # fmt: skip
+    """Macros and launch geometry for one (params, config, direction); `out_f32`: the destination is a
+    float32 tensor (the same values, widened when they are stored)."""
     params.validate()
     defines = _shape_defines(params)
+    if out_f32:
+        assert fits_float32_output(params, config), f"no float32 output for {config} and {params}"
+        defines["SPIO_DST_F32"] = 1
     defines["SPIO_IGRAD"] = int(igrad)
     defines["SPIO_HAS_BIAS"] = int(params.has_bias and not igrad)
     if config.variant == "direct":
@@ -461,8 +472,8 @@ def _get_kernel_spec(params: Conv2dGw8Params, config: Conv2dGw8Config, _device_a
     )
 
 
-def _get_kernel_name(igrad: bool = False) -> str:
-    return "spio_conv2d_gw8_dgrad" if igrad else "spio_conv2d_gw8_fprop"
+def _get_kernel_name(igrad: bool = False, out_f32: bool = False) -> str:
+    return ("spio_conv2d_gw8_dgrad" if igrad else "spio_conv2d_gw8_fprop") + ("_f32" if out_f32 else "")
 
 
 def _make_test_args(params: Conv2dGw8Params, device, igrad: bool = False):

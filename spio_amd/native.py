@@ -54,6 +54,22 @@ def _stage(function, launch_params):
     return [function.handle, *launch_params.grid, *launch_params.block, launch_params.shared_mem_bytes]
 
 
+WIDE = 4  # bit of a key's mode: the kernel stores its activations as float32
+
+
+def _widened(kernel, factory, params, device, **kwargs):
+    """The version of `kernel` that stores float32, in the configuration chosen for the float16 one (it reads
+    and multiplies the same); None where that has no such version."""
+    from .hip.driver import get_device_attributes
+    from .kernels.conv2d_gw8_kernel import fits_float32_output
+    from .kernels.kernel_cache import compile_and_load_kernel
+
+    if not fits_float32_output(params, kernel.config):
+        return None
+    return compile_and_load_kernel(factory, params, kernel.config, device.index, get_device_attributes(device.index),
+                                   out_f32=True, **kwargs)  # fmt: skip
+
+
 def _make_plan(values):
     """(stages, workspace bytes, overwrites) of the kernel a key of csrc/spio_torch.cpp stands for."""
     from . import kernels
@@ -62,15 +78,19 @@ def _make_plan(values):
     kind, ordinal = values[:2]
     device = torch.device("cuda", ordinal)
     if kind < 4:
-        n, c, h, w, r, s, py, px, bias, _mode = values[2:]
+        n, c, h, w, r, s, py, px, bias, mode = values[2:]
         params = kernels.Conv2dGw8Params(n=n, c=c, h=h, w=w, r=r, s=s, padding=(py, px), has_bias=bool(bias))
         params.validate()
+        factory, direction = kernels.conv2d_gw8_kernel_factory, {"igrad": True} if kind == 1 else {}
         if kind == 3:
+            factory = kernels.conv2d_gw8_bgrad_kernel_factory
             kernel = fused_backward_kernel(params, device)
         elif kind == 2:
             kernel = kernels.conv2d_gw8_wgrad_kernel_factory.get_kernel(params, device)
         else:
-            kernel = kernels.conv2d_gw8_kernel_factory.get_kernel(params, device, **({"igrad": True} if kind else {}))
+            kernel = factory.get_kernel(params, device, **direction)
+        if kernel is not None and mode & WIDE:
+            kernel = _widened(kernel, factory, params, device, **direction)
     else:
         n, c, h, w, eps, weight, bias = values[2:9]
         params = kernels.LayerNorm2dParams(n=n, c=c, h=h, w=w, eps=struct.unpack("<d", struct.pack("<q", eps))[0],

@@ -7,8 +7,11 @@ sentinel.
 """
 
 import pytest
+import torch
 
-from helpers import run_bgrad_kernel_test, run_grad_kernel_test, run_kernel_test, sample_params
+from helpers import gpu_args, run_bgrad_kernel_test, run_grad_kernel_test, run_kernel_test, sample_params, to_gpu
+from spio_amd.compiler.compiler_pool import compile_kernel_configs
+from spio_amd.hip import get_device_attributes
 from spio_amd.kernels import (
     Conv2dGw8BgradConfig,
     Conv2dGw8Config,
@@ -102,6 +105,56 @@ def test_channel_blocks_that_share_lines(params, chunk):
                                       for two in (0, 1)])  # fmt: skip
         run_bgrad_kernel_test(conv2d_gw8_bgrad_kernel_factory, params,
                               configs=[Conv2dGw8BgradConfig(groups=min(gb, 4), block_h=3, prefetch=2, xcd_chunk=chunk)])
+
+
+_F32_CASES = [
+    # cells that do not fill the last wave, odd group counts, images side by side, a ragged batch
+    (Conv2dGw8Params(n=5, c=24, h=9, w=11, padding=1, has_bias=True),
+     [Conv2dGw8Config(groups=3, block_p=4, block_n=2, prefetch=2), Conv2dGw8Config(groups=2, block_p=9, split=1, prefetch=4, nontemporal=0),
+      Conv2dGw8Config(groups=1, block_p=1, variant="direct")],
+     [Conv2dGw8BgradConfig(groups=3, block_h=4, block_n=2, prefetch=2), Conv2dGw8BgradConfig(groups=2, prefetch=2, nontemporal=0)]),
+    (Conv2dGw8Params(n=5, c=72, h=7, w=7, r=5, s=5, padding=2),
+     [Conv2dGw8Config(groups=4, block_p=7, block_n=nb, variant="image", prefetch=pf, block_n_iters=2, movers=mv)
+      for nb, pf, mv in ((1, 2, 0), (2, 2, 4), (1, 1, 0))],
+     [Conv2dGw8BgradConfig(groups=4, block_n=2, block_n_iters=2, prefetch=2)]),
+    # the image size changes; column blocks with a ragged last one
+    (Conv2dGw8Params(n=2, c=16, h=7, w=150, padding=(0, 2)),
+     [Conv2dGw8Config(groups=2, block_p=3, block_q=64, prefetch=4), Conv2dGw8Config(groups=2, block_p=3, block_p2=2, split=2, prefetch=2)],
+     [Conv2dGw8BgradConfig(groups=2, block_h=3, block_q=64, prefetch=2)]),
+]  # fmt: skip
+
+
+@pytest.mark.parametrize("params,configs,fused", _F32_CASES, ids=lambda v: v.encode() if hasattr(v, "encode") else "")
+def test_float32_outputs_are_the_float16_ones_widened(params, configs, fused):
+    """The versions that store activations as float32: every element of the tensor is written and holds
+    exactly the value that the float16 version stores."""
+    x, w, bias, dy = [to_gpu(t) for t in gpu_args(params)]
+    attr = get_device_attributes(0)
+
+    def activations(factory, config, shape, args, **kw):
+        results = []
+        for out_f32 in (False, True):
+            (kernel,) = compile_kernel_configs(factory, params, configs=[config], device_attr=attr, out_f32=out_f32, **kw)
+            kernel.load(0)
+            out = torch.full(shape, -42.0, device="cuda", dtype=torch.float32 if out_f32 else torch.float16)
+            out = out.contiguous(memory_format=torch.channels_last)
+            kernel(out, *args())
+            torch.cuda.synchronize()
+            kernel.unload()
+            results.append(out)
+        assert not (results[1] == -42.0).all(dim=1).any()
+        assert torch.equal(results[1], results[0].float()), f"{params.encode()} {config}"
+
+    for config in configs:
+        activations(conv2d_gw8_kernel_factory, config, params.output_shape, lambda: (x, w, bias))
+        if config.variant != "image" or config.block_p == params.h:
+            activations(conv2d_gw8_kernel_factory, config, params.input_shape, lambda: (dy, w, None), igrad=True)
+    for config in fused:
+        def sums():
+            dw = torch.zeros(params.weight_shape, device="cuda").contiguous(memory_format=torch.channels_last)
+            return (dw, x, dy, w) + ((torch.zeros(params.c, device="cuda"),) if params.has_bias else ())
+
+        activations(conv2d_gw8_bgrad_kernel_factory, config, params.input_shape, sums)
 
 
 def test_column_blocks():
