@@ -162,6 +162,10 @@ int spio_hip_launch_scratch(void* function,
  * under HIP graph capture like any other kernel launch. */
 int spio_hip_zero_fill_async(void* device_ptr, size_t bytes, void* stream);
 
+/* The same for two buffers in one launch (either may be empty). */
+int spio_hip_zero_fill_pair_async(void* first, size_t first_bytes, void* second, size_t second_bytes,
+                              void* stream);
+
 /* Replace get_device_attributes, ctx_synchronize, get_driver_version
  * (driver.pyx:284-303, 360-369) and PrimaryContextGuard.set_device (259-265). */
 int spio_hip_device_count(int* count);

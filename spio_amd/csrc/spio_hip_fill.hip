@@ -1,4 +1,4 @@
-// spio_hip_zero_fill_async -- clear a device buffer with a kernel.
+// spio_hip_zero_fill_async, spio_hip_zero_fill_pair_async -- clear one or two device buffers with a kernel.
 //
 // The weight-gradient kernels add into grad_weight, so the buffer has to hold
 // zeros when they start.  Callers without a tensor library clear it through
@@ -18,35 +18,54 @@ namespace {
 constexpr int kFillThreads = 256;
 constexpr unsigned kMaxFillBlocks = 2048;  // 8 workgroups per CU; the kernel strides over the rest
 
+// A buffer, cut at its 16-byte boundaries: `head` bytes, `vectors` times 16 bytes, the rest.
+struct Range {
+    unsigned char* ptr;
+    size_t bytes, head, vectors;
+};
+
+Range make_range(void* ptr, size_t bytes) {
+    size_t head = static_cast<size_t>((16 - reinterpret_cast<uintptr_t>(ptr) % 16) % 16);
+    if (head > bytes) head = bytes;
+    return {static_cast<unsigned char*>(ptr), bytes, head, (bytes - head) / 16};
+}
+
 // Bytes before the first and after the last 16-byte boundary are written one by one (by the
 // first lanes of block 0); everything between as 16-byte vectors, grid-strided.
-__global__ void __launch_bounds__(kFillThreads)
-zero_fill_kernel(unsigned char* ptr, size_t bytes, size_t head, size_t vectors) {
+__device__ void clear(const Range& r, size_t tid, size_t stride) {
+    uint4* body = reinterpret_cast<uint4*>(r.ptr + r.head);
+    for (size_t i = tid; i < r.vectors; i += stride) body[i] = uint4{0u, 0u, 0u, 0u};
+    const size_t tail_begin = r.head + r.vectors * 16;
+    if (tid < r.head) r.ptr[tid] = 0;
+    if (tid < r.bytes - tail_begin) r.ptr[tail_begin + tid] = 0;
+}
+
+// Bound by its launch: the sums it clears are kilobytes.  Two buffers of one layer (the sums of the weight
+// and of the bias gradient) therefore go in one launch; an empty second range costs a few scalar compares.
+// Measured per training step with a bias, two launches -> one: 32n 48c 224x224 126.8 -> 125.1 us, 128n 96c 56x56
+// with its norm 162.9 -> 161.6 us, 128n 384c 14x14 on float32 activations 94.6 -> 89.3 us.
+__global__ void __launch_bounds__(kFillThreads) zero_fill_kernel(Range a, Range b) {
     const size_t tid = static_cast<size_t>(blockIdx.x) * kFillThreads + threadIdx.x;
     const size_t stride = static_cast<size_t>(gridDim.x) * kFillThreads;
-    uint4* body = reinterpret_cast<uint4*>(ptr + head);
-    for (size_t i = tid; i < vectors; i += stride) body[i] = uint4{0u, 0u, 0u, 0u};
-    const size_t tail_begin = head + vectors * 16;
-    if (tid < head) ptr[tid] = 0;
-    if (tid < bytes - tail_begin) ptr[tail_begin + tid] = 0;
+    clear(a, tid, stride);
+    clear(b, tid, stride);
 }
 
 }  // namespace
 
-extern "C" int spio_hip_zero_fill_async(void* device_ptr, size_t bytes, void* stream) {
-    if (!device_ptr && bytes) return spio_hip_set_error(SPIO_HIP_ERR_ARGUMENT, "zero fill: null pointer");
-    if (!bytes) return SPIO_HIP_OK;
-    const uintptr_t address = reinterpret_cast<uintptr_t>(device_ptr);
-    size_t head = static_cast<size_t>((16 - address % 16) % 16);
-    if (head > bytes) head = bytes;
-    const size_t vectors = (bytes - head) / 16;
+extern "C" int spio_hip_zero_fill_pair_async(void* first, size_t first_bytes, void* second, size_t second_bytes,
+                                         void* stream) {
+    if ((!first && first_bytes) || (!second && second_bytes))
+        return spio_hip_set_error(SPIO_HIP_ERR_ARGUMENT, "zero fill: null pointer");
+    if (!first_bytes && !second_bytes) return SPIO_HIP_OK;
+    const Range a = make_range(first, first_bytes), b = make_range(second, second_bytes);
     // head and tail are shorter than 16 bytes each: the first 16 threads cover them
+    const size_t vectors = a.vectors > b.vectors ? a.vectors : b.vectors;
     size_t blocks = (vectors + kFillThreads - 1) / kFillThreads;
     if (blocks < 1) blocks = 1;
     if (blocks > kMaxFillBlocks) blocks = kMaxFillBlocks;
     hipLaunchKernelGGL(zero_fill_kernel, dim3(static_cast<unsigned>(blocks)), dim3(kFillThreads), 0,
-                       static_cast<hipStream_t>(stream), static_cast<unsigned char*>(device_ptr), bytes,
-                       head, vectors);
+                       static_cast<hipStream_t>(stream), a, b);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) {
         char buf[256];
@@ -55,4 +74,8 @@ extern "C" int spio_hip_zero_fill_async(void* device_ptr, size_t bytes, void* st
         return spio_hip_set_error(SPIO_HIP_ERR_HIP_BASE + static_cast<int>(e), buf);
     }
     return SPIO_HIP_OK;
+}
+
+extern "C" int spio_hip_zero_fill_async(void* device_ptr, size_t bytes, void* stream) {
+    return spio_hip_zero_fill_pair_async(device_ptr, bytes, nullptr, 0, stream);
 }

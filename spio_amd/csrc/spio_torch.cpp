@@ -141,8 +141,10 @@ Tensor empty_cl(at::IntArrayRef sizes, at::ScalarType dtype, const Tensor& like)
 Tensor empty_1d(int64_t n, at::ScalarType dtype, const Tensor& like) {
     return at::detail::empty_cuda({n}, dtype, like.device(), std::nullopt);
 }
-void zero(const Tensor& t, hipStream_t stream) {
-    if (spio_hip_zero_fill_async(t.data_ptr(), t.nbytes(), stream))
+// Clears one or two tensors (undefined: none) in one launch.
+void zero(const Tensor& a, const Tensor& b, hipStream_t stream) {
+    auto bytes = [](const Tensor& t) { return t.defined() ? static_cast<size_t>(t.nbytes()) : 0; };
+    if (spio_hip_zero_fill_pair_async(const_cast<void*>(ptr(a)), bytes(a), const_cast<void*>(ptr(b)), bytes(b), stream))
         throw py::value_error(std::string("zero fill failed: ") + spio_hip_last_error());
 }
 
@@ -230,11 +232,9 @@ ConvGrads conv_backward(const Conv& cv, const Tensor& x, const Tensor& w, const 
     // atomic kernels add into zeroed sums, two-stage ones store them whole
     auto sums = [&](const Plan& plan, bool with_bias, bool bias_is_stored) {
         g.w = empty_cl({cv.c, 8, cv.r, cv.s}, at::kFloat, dy);
-        if (!plan.overwrites) zero(g.w, stream);
-        if (with_bias) {
-            g.b = empty_1d(cv.c, at::kFloat, dy);
-            if (!bias_is_stored) zero(g.b, stream);
-        }
+        if (with_bias) g.b = empty_1d(cv.c, at::kFloat, dy);
+        // one launch for both: a launch is all that the fill of such small sums costs
+        zero(plan.overwrites ? Tensor() : g.w, bias_is_stored ? Tensor() : g.b, stream);
     };
     PlanPtr fused;
     if (need_x && need_w) {

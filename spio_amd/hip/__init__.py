@@ -22,5 +22,6 @@ from .driver import (
     stream_synchronize,
     set_device,
     zero_fill_async,
+    zero_fill_pair_async,
     launch_sequence_timed,
 )

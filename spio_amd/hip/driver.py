@@ -106,6 +106,7 @@ _SIGNATURES = {
         ctypes.c_int,
     ),
     "spio_hip_zero_fill_async": ([_vp, ctypes.c_size_t, _vp], ctypes.c_int),
+    "spio_hip_zero_fill_pair_async": ([_vp, ctypes.c_size_t, _vp, ctypes.c_size_t, _vp], ctypes.c_int),
     "spio_hip_device_count": ([ctypes.POINTER(ctypes.c_int)], ctypes.c_int),
     "spio_hip_device_attrs": ([ctypes.c_int, ctypes.POINTER(_DeviceAttrsStruct)], ctypes.c_int),
     "spio_hip_set_device": ([ctypes.c_int], ctypes.c_int),
@@ -509,3 +510,9 @@ def zero_fill_async(ptr: int, nbytes: int, stream: int = 0):
     alignment, any size; safe to record under HIP graph capture)."""
     init()
     _check(_lib.spio_hip_zero_fill_async(ptr, nbytes, stream or None))
+
+
+def zero_fill_pair_async(first: int, first_bytes: int, second: int, second_bytes: int, stream: int = 0):
+    """`zero_fill_async` of two buffers in one launch; either may be empty."""
+    init()
+    _check(_lib.spio_hip_zero_fill_pair_async(first or None, first_bytes, second or None, second_bytes, stream or None))

@@ -20,6 +20,19 @@ def test_zero_fill_covers_exactly_the_requested_bytes():
         assert bool((buf[:offset] == 0xAB).all()) and bool((buf[offset + size :] == 0xAB).all()), (offset, size)
 
 
+@pytest.mark.parametrize("first,second", [((0, 0), (0, 0)), ((3, 5), (0, 0)), ((0, 0), (7, 4099)), ((16, 16), (15, 17)),
+                                          ((5, 27648), (1, 192)), ((13, 40), (0, 1 << 20)), ((0, 1 << 20), (9, 1))])  # fmt: skip
+def test_zero_fill_of_two_buffers(first, second):
+    """Both ranges are zero, whichever is the longer or empty; their neighbours are untouched."""
+    stream = torch.cuda.current_stream().cuda_stream
+    bufs = [torch.full(((1 << 20) + 32,), 0xAB, dtype=torch.uint8, device="cuda") for _ in range(2)]
+    driver.zero_fill_pair_async(bufs[0].data_ptr() + first[0], first[1], bufs[1].data_ptr() + second[0], second[1], stream)
+    for buf, (offset, size) in zip(bufs, (first, second)):
+        expected = torch.full_like(buf, 0xAB)
+        expected[offset : offset + size] = 0
+        assert torch.equal(buf, expected), (offset, size)
+
+
 def test_zero_fill_replays_from_a_hip_graph():
     """Recorded under stream capture (it is a kernel launch, not a memset node) and replayed
     three times with eager work and synchronisations between the replays."""
