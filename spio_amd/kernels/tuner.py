@@ -15,7 +15,8 @@ Environment:
   SPIO_TUNE=force  sweep even when a record exists
   SPIO_TUNE_DB     path of the record file (default: <cache dir>/tune/<arch>_<CUs>cu.json)
   SPIO_TUNE_MAX_CONFIGS  how many configurations (the first ones of the ranked list) a sweep that
-                   starts inside an operator call may try (default 8); `python -m spio_amd.tune`
+                   starts inside an operator call may try (without it the first 8, not counting
+                   versions that differ in the store policy alone); `python -m spio_amd.tune`
                    and `tune_model` always try all of them
 
 A sweep never starts while the current stream is being captured into a HIP graph (it allocates
@@ -49,11 +50,13 @@ DEFAULT_ON_MISS_CONFIGS = 8
 FINALISTS = 6  # leaders of a sweep that are timed again before one is chosen
 
 
-def _on_miss_limit() -> int:
+def _on_miss_limit(configs) -> int:
+    """How many of `configs` a sweep inside an operator call takes: SPIO_TUNE_MAX_CONFIGS is a bound on all of
+    them, without it the default number of geometries in each store policy they come in."""
     try:
-        return max(1, int(os.environ.get("SPIO_TUNE_MAX_CONFIGS", DEFAULT_ON_MISS_CONFIGS)))
-    except ValueError:
-        return DEFAULT_ON_MISS_CONFIGS
+        return max(1, int(os.environ["SPIO_TUNE_MAX_CONFIGS"]))
+    except (KeyError, ValueError):
+        return _leading(configs, DEFAULT_ON_MISS_CONFIGS)
 
 
 def _leading(configs, count: int) -> int:
@@ -204,7 +207,7 @@ class Tuner:
             # inside an operator call: only the best-ranked few, so that a model with many new
             # shapes does not stall (the last entry of a list is its any-shape kernel: keep it as
             # the independent implementation the winner is checked against)
-            limit = _leading(configs, _on_miss_limit())
+            limit = _on_miss_limit(configs)
             if len(configs) > limit + 1:
                 configs = configs[:limit] + [configs[-1]]
             return self.sweep(kernel_factory, params, ordinal, device_attr, configs, **kernel_kwargs)

@@ -416,10 +416,10 @@ def test_weight_gradient_mfma_kernel_is_not_offered_past_its_32_bit_indices():
     assert conv2d_gw8_bgrad_kernel_factory.configs(past, attr)
 
 
-def test_second_store_policies_do_not_shorten_a_capped_sweep():
+def test_second_store_policies_do_not_shorten_a_capped_sweep(monkeypatch):
     """With an odd number of groups in several channel blocks the leading configurations come in two store
     policies; the first `count` geometries of a capped sweep are the same as without them."""
-    from spio_amd.kernels.tuner import _leading
+    from spio_amd.kernels.tuner import _leading, _on_miss_limit
 
     for factory in (conv2d_gw8_kernel_factory, conv2d_gw8_bgrad_kernel_factory):
         odd = list(factory.configs(Conv2dGw8Params(n=50, c=152, h=21, w=41, padding=1), DeviceAttributes()))
@@ -429,3 +429,7 @@ def test_second_store_policies_do_not_shorten_a_capped_sweep():
             assert c.nontemporal or replace(c, nontemporal=1) == before
         even = list(factory.configs(Conv2dGw8Params(n=50, c=160, h=21, w=41, padding=1), DeviceAttributes()))
         assert all(c.nontemporal for c in even) and _leading(even, 8) == 8 and _leading(even, 10**6) == len(even)
+        monkeypatch.delenv("SPIO_TUNE_MAX_CONFIGS", raising=False)
+        assert _on_miss_limit(odd) == len(both) and _on_miss_limit(even) == 8
+        monkeypatch.setenv("SPIO_TUNE_MAX_CONFIGS", "4")  # a bound that the caller states counts every version
+        assert _on_miss_limit(odd) == 4 and _on_miss_limit(even) == 4
