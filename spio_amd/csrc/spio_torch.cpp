@@ -278,6 +278,11 @@ Tensor to_half_cl(const Tensor& t) {
     if (t.scalar_type() == at::kHalf) return t.is_contiguous(CL) ? t : t.contiguous(CL);
     return t.to(at::kHalf, /*non_blocking=*/false, /*copy=*/false, CL).contiguous(CL);
 }
+// Whether a saved tensor still is what the forward pass saved, up to its layout: hooks on saved tensors may
+// unpack it with other strides (a copy packed into host memory, say) or elsewhere altogether.
+bool is_again(const Tensor& t, const Tensor& grad, at::IntArrayRef sizes, at::ScalarType dtype = at::kHalf) {
+    return is_plain(t) && t.sizes() == sizes && t.device() == grad.device() && t.scalar_type() == dtype;
+}
 // A float32 vector of channels.
 Tensor to_float_1d(const Tensor& t) {
     if (!t.defined() || (t.scalar_type() == at::kFloat && t.is_contiguous())) return t;
@@ -305,11 +310,13 @@ struct ConvFunction : torch::autograd::Function<ConvFunction> {
         const Conv cv{v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7], v[8] != 0};
         const auto saved = ctx->get_saved_variables();
         const Tensor &x = saved[0], &w = saved[1];
+        const bool native = is_again(x, grads[0], {cv.n, cv.c, cv.h, cv.w}) && is_again(w, grads[0], {cv.c, 8, cv.r, cv.s});
         const bool need_x = ctx->needs_input_grad(0), need_w = ctx->needs_input_grad(1),
                    need_b = cv.bias && ctx->needs_input_grad(2);
         ConvGrads g;
-        if (at::GradMode::is_enabled()) {
-            // create_graph=True: the Python operator, which says what it thinks of second derivatives
+        if (!native || at::GradMode::is_enabled()) {
+            // tensors the kernels do not take, which it refuses, and create_graph=True: the Python operator,
+            // which says what it thinks of second derivatives
             py::gil_scoped_acquire gil;
             py::object b = cv.bias ? py::cast(at::empty({cv.c}, x.options().dtype(at::kFloat))) : py::none();
             py::tuple r = py::reinterpret_borrow<py::object>(g_backward_op)(
@@ -317,7 +324,7 @@ struct ConvFunction : torch::autograd::Function<ConvFunction> {
             auto get = [&](int i) { return r[i].is_none() ? Tensor() : r[i].cast<Tensor>(); };
             g = {get(0), get(1), get(2)};
         } else {
-            g = conv_backward(cv, x, w, to_half_cl(grads[0]), need_x, need_w, need_b,
+            g = conv_backward(cv, to_half_cl(x), to_half_cl(w), to_half_cl(grads[0]), need_x, need_w, need_b,
                               static_cast<at::ScalarType>(v[9]));
         }
         auto typed = [&](const Tensor& t, int i) {
@@ -356,7 +363,9 @@ struct NormFunction : torch::autograd::Function<NormFunction> {
         const Tensor xc = to_half_cl(x);
         Tensor y = norm_forward(nm, xc, to_float_1d(weight), to_float_1d(bias));
         ctx->save_for_backward({xc, weight});
-        ctx->saved_data["v"] = std::vector<int64_t>{nm.n, nm.c, nm.h, nm.w, bias.defined()};
+        ctx->saved_data["v"] = std::vector<int64_t>{
+            nm.n, nm.c, nm.h, nm.w, bias.defined(),
+            weight.defined() ? static_cast<int64_t>(weight.scalar_type()) : static_cast<int64_t>(at::kFloat)};
         ctx->saved_data["eps"] = nm.eps;
         return y;
     }
@@ -366,15 +375,17 @@ struct NormFunction : torch::autograd::Function<NormFunction> {
         const Norm nm{v[0], v[1], v[2], v[3], ctx->saved_data["eps"].toDouble()};
         const auto saved = ctx->get_saved_variables();
         const Tensor &x = saved[0], &weight = saved[1];
+        const bool native = is_again(x, grads[0], {nm.n, nm.c, nm.h, nm.w}) &&
+                            (!weight.defined() || is_again(weight, grads[0], {nm.c}, static_cast<at::ScalarType>(v[5])));
         Tensor dx, sums;
-        if (at::GradMode::is_enabled()) {  // create_graph=True
+        if (!native || at::GradMode::is_enabled()) {  // as in ConvFunction
             py::gil_scoped_acquire gil;
             py::object wt = weight.defined() ? py::cast(weight) : py::none();
             py::tuple r = py::reinterpret_borrow<py::object>(g_norm_backward_op)(x, grads[0], wt, nm.eps);
             dx = r[0].cast<Tensor>();
             sums = r[1].cast<Tensor>();
         } else {
-            const Tensor dy = to_half_cl(grads[0]);
+            const Tensor dy = to_half_cl(grads[0]), xc = to_half_cl(x);
             const Tensor w = to_float_1d(weight);
             const auto device = dy.get_device();
             hipStream_t stream = c10::hip::getCurrentHIPStream(device);
@@ -382,7 +393,7 @@ struct NormFunction : torch::autograd::Function<NormFunction> {
             dx = empty_cl({nm.n, nm.c, nm.h, nm.w}, at::kHalf, dy);
             sums = at::detail::empty_cuda({2, nm.c}, at::kFloat, dy.device(), std::nullopt);
             const Tensor workspace = empty_1d(plan->workspace, at::kByte, dy);
-            launch(plan->main, stream, {ptr(workspace), ptr(dx), ptr(x), ptr(dy), ptr(w)});
+            launch(plan->main, stream, {ptr(workspace), ptr(dx), ptr(xc), ptr(dy), ptr(w)});
             launch(plan->second, stream, {ptr(sums), ptr(workspace)});
         }
         // absent tensors have no edge: the bias's follows the weight's or the input's

@@ -1,0 +1,63 @@
+"""Gradients recorded by the operators' native call path (csrc/spio_torch.cpp): what they do when something
+between the forward and the backward pass changes the saved tensors, asks for second derivatives or wants to see
+the launches."""
+
+import pytest
+import torch
+
+from spio_amd import native
+from spio_amd.functional import conv2d_gw8, layernorm_2d
+
+pytestmark = pytest.mark.gpu
+CL = torch.channels_last
+
+
+def _leaves(op, dtype=torch.float16, layout=CL, affine=True):
+    """Leaves and a call of a small convolution ("conv", "autocast") or norm ("norm")."""
+    torch.manual_seed(11)
+    x = torch.randn(3, 24, 9, 7, device="cuda").to(dtype).contiguous(memory_format=layout).requires_grad_()
+    if op == "norm":
+        vectors = [torch.randn(24, device="cuda").requires_grad_() for _ in range(2 if affine else 0)]
+        return [x, *vectors], lambda x, *v: layernorm_2d(x, *v, eps=1e-5) if v else layernorm_2d(x, eps=1e-5)
+    w = (torch.randn(24, 8, 3, 3, device="cuda") * 0.1).to(dtype).contiguous(memory_format=layout).requires_grad_()
+    b = [torch.randn(24, device="cuda").requires_grad_()] if affine else []
+
+    def call(x, w, b=None):
+        with torch.autocast("cuda", dtype=torch.float16, enabled=op == "autocast"):
+            return conv2d_gw8(x, w, b, padding_y=1, padding_x=1, groups=3)
+
+    return [x, w, *b], call
+
+
+def _assert_near(got, expected, tol=2e-3):
+    for a, e in zip(got, expected):
+        assert a.dtype == e.dtype and a.shape == e.shape
+        torch.testing.assert_close(a.float(), e.float(), rtol=tol, atol=tol * float(e.detach().float().abs().max()))
+
+
+def _repack(t):
+    return t.detach().clone(memory_format=torch.contiguous_format)
+
+
+_HOOKS = {
+    "relaid": lambda: torch.autograd.graph.saved_tensors_hooks(_repack, lambda t: t),
+    "pinned": lambda: torch.autograd.graph.save_on_cpu(pin_memory=True),
+    "transposed": lambda: torch.autograd.graph.saved_tensors_hooks(
+        lambda t: t.detach().transpose(0, -1).contiguous(), lambda t: t.transpose(0, -1)),
+}  # fmt: skip
+
+
+@pytest.mark.parametrize("hooks", list(_HOOKS))
+@pytest.mark.parametrize("op,dtype,fused", [("conv", torch.float16, "0"), ("conv", torch.float16, "1"),
+                                            ("autocast", torch.float32, "0"), ("autocast", torch.float32, "1"),
+                                            ("norm", torch.float16, "auto")])  # fmt: skip
+def test_saved_tensors_may_come_back_in_another_layout(op, dtype, fused, hooks, monkeypatch):
+    """Hooks on saved tensors keep values and sizes, not strides: the gradients are those without hooks."""
+    monkeypatch.setenv("SPIO_FUSED_BACKWARD", fused)
+    leaves, call = _leaves(op, dtype)
+    plain = call(*leaves)
+    dy = torch.randn_like(plain)
+    expected = torch.autograd.grad(plain, leaves, dy)
+    with _HOOKS[hooks]():
+        y = call(*leaves)
+    _assert_near(torch.autograd.grad(y, leaves, dy), expected)
