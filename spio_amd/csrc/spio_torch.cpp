@@ -73,11 +73,13 @@ struct Plan {
     int64_t workspace = 0;      // bytes of partial results between the stages
     bool present = false;       // false: the shape does not use this kind (no fused backward, no float32 output)
     bool overwrites = false;    // the kernel stores its sums whole instead of adding to them
+    std::shared_ptr<PyObject> kernel;  // the Python kernel whose code object `main` and `second` point into
 };
 using PlanPtr = std::shared_ptr<const Plan>;
 
 std::shared_mutex g_plans_mutex;
-std::unordered_map<Key, PlanPtr, KeyHash> g_plans;
+using Plans = std::unordered_map<Key, PlanPtr, KeyHash>;
+Plans& g_plans = *new Plans;            // never destroyed: the plans hold Python objects
 std::atomic<int64_t> g_bypass{1};      // > 0: every call takes the Python path
 std::atomic<uint64_t> g_generation{0};  // of the plans: a plan made before a forget() is not kept
 PyObject* g_make_plan = nullptr;        // Python: (key values) -> plan description
@@ -97,7 +99,7 @@ PlanPtr find_plan(const Key& key) {
         for (int i = 0; i < 12; ++i) values[i] = py::int_(key.v[i]);
         py::object made = py::reinterpret_borrow<py::object>(g_make_plan)(values);
         if (!made.is_none()) {
-            auto t = made.cast<py::tuple>();  // (stages, workspace bytes, overwrites)
+            auto t = made.cast<py::tuple>();  // (stages, workspace bytes, overwrites, kernel)
             auto stages = t[0].cast<py::list>();
             for (size_t i = 0; i < stages.size(); ++i) {
                 auto s = stages[i].cast<std::vector<uint64_t>>();
@@ -112,6 +114,11 @@ PlanPtr find_plan(const Key& key) {
             plan->workspace = t[1].cast<int64_t>();
             plan->overwrites = t[2].cast<bool>();
             plan->present = true;
+            // the last owner may be a thread without the GIL
+            plan->kernel = {py::object(t[3]).release().ptr(), [](PyObject* kernel) {
+                                py::gil_scoped_acquire gil;
+                                Py_DECREF(kernel);
+                            }};
         }
     }
     std::unique_lock<std::shared_mutex> lock(g_plans_mutex);
@@ -549,8 +556,9 @@ PYBIND11_MODULE(_native, m) {
     m.def("bypass", [](int64_t change) { g_bypass.fetch_add(change); });
     m.def("forget", [] {
         g_generation.fetch_add(1);
+        Plans dropped;  // destroyed behind the lock: a kernel that goes with its plan runs Python code
         std::unique_lock<std::shared_mutex> lock(g_plans_mutex);
-        g_plans.clear();
+        dropped.swap(g_plans);
     });
     m.def("plans", [] {
         std::shared_lock<std::shared_mutex> lock(g_plans_mutex);

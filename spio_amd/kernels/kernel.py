@@ -104,6 +104,7 @@ class Kernel:
         self.function = None
         self.epilogue_function = None
         self.device_ordinal: Optional[int] = None
+        self.in_plans = False  # launch plans of the native call path point into the module
 
     @property
     def kernel_source_file(self) -> str:
@@ -142,7 +143,9 @@ class Kernel:
         from ..native import forget_plans
 
         if self.module is not None:
-            forget_plans()
+            if self.in_plans:
+                forget_plans()
+                self.in_plans = False
             self.module.unload()
             self.module = None
         self.function = None

@@ -7,7 +7,7 @@ it.  A lock makes get() safe from several threads.
 """
 
 import threading
-from typing import Dict
+from typing import Any, Dict, Tuple
 
 import torch
 
@@ -32,6 +32,7 @@ class KernelCache:
         self._cache: Dict[KernelKey, Kernel] = {}
         self._cache_overlay: Dict[KernelKey, Kernel] = {}
         self._lock = threading.RLock()
+        self._in_config: Dict[Tuple[KernelKey, Any], Kernel] = {}
         self._bypass = None  # held while the overlay has entries: every call must look at it
 
     def update_overlay(self, overlay: Dict[KernelKey, Kernel]):
@@ -55,6 +56,7 @@ class KernelCache:
 
         with self._lock:
             self._cache.clear()
+            self._in_config.clear()
         forget_plans()
 
     @log_kernel_params
@@ -87,6 +89,18 @@ class KernelCache:
             self._cache[key] = kernel
             if logger_enabled:
                 print(f"spio: compiled kernel {kernel} for device {device}.")
+            return kernel
+
+    def get_in_config(self, kernel_factory, params, device, config, **kernel_kwargs) -> Kernel:
+        """The kernel for `params` on `device` in a configuration chosen elsewhere; compiles on first use."""
+        ordinal = _ordinal(device)
+        key = (KernelKey(device_ordinal=ordinal, params=params), config)
+        with self._lock:
+            kernel = self._in_config.get(key)
+            if kernel is None:
+                kernel = self._in_config[key] = compile_and_load_kernel(
+                    kernel_factory, params, config, ordinal, get_device_attributes(ordinal), **kernel_kwargs
+                )
             return kernel
 
 

@@ -66,6 +66,10 @@ class KernelFactory:
         """Cached best kernel for the params on the device (tunes/compiles on a miss)."""
         return self.get_kernel_cache(**kwargs).get(self, params, device, **kwargs)
 
+    def get_kernel_in_config(self, params, device, config, **kwargs) -> Kernel:
+        """Cached kernel for the params on the device in the given configuration (compiles on a miss)."""
+        return self.get_kernel_cache(**kwargs).get_in_config(self, params, device, config, **kwargs)
+
     def make_kernel(self, params, config, device_attr=None, **kwargs) -> Kernel:
         """A new, not yet compiled Kernel for one configuration."""
         return Kernel(

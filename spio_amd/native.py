@@ -11,7 +11,6 @@ holds a `Bypass` meanwhile: all calls then take the Python path.
 import importlib
 import os
 import struct
-import threading
 
 import torch
 from torch._library.custom_ops import CustomOpDef
@@ -22,15 +21,11 @@ if not os.path.exists(EXTENSION_PATH):
     build_extension()
 _native = importlib.import_module(f"{__package__}._native")
 
-_kernels = {}  # what the native plans point into stays loaded as long as they live
-_kernels_lock = threading.Lock()
-
 
 def forget_plans():
-    """Drop every launch plan (kernels were unloaded, caches or choices cleared)."""
+    """Drop every launch plan (a kernel of one was unloaded, caches or choices cleared).  The kernels stay
+    with their caches: graphs, queued work and other threads may still launch them."""
     _native.forget()
-    with _kernels_lock:
-        _kernels.clear()
 
 
 class Bypass:
@@ -60,18 +55,15 @@ WIDE = 4  # bit of a key's mode: the kernel stores its activations as float32
 def _widened(kernel, factory, params, device, **kwargs):
     """The version of `kernel` that stores float32, in the configuration chosen for the float16 one (it reads
     and multiplies the same); None where that has no such version."""
-    from .hip.driver import get_device_attributes
     from .kernels.conv2d_gw8_kernel import fits_float32_output
-    from .kernels.kernel_cache import compile_and_load_kernel
 
     if not fits_float32_output(params, kernel.config):
         return None
-    return compile_and_load_kernel(factory, params, kernel.config, device.index, get_device_attributes(device.index),
-                                   out_f32=True, **kwargs)  # fmt: skip
+    return factory.get_kernel_in_config(params, device, kernel.config, out_f32=True, **kwargs)
 
 
 def _make_plan(values):
-    """(stages, workspace bytes, overwrites) of the kernel a key of csrc/spio_torch.cpp stands for."""
+    """(stages, workspace bytes, overwrites, kernel) for a key of csrc/spio_torch.cpp; the plan owns the kernel."""
     from . import kernels
     from .functional.conv2d_gw8_function import fused_backward_kernel
 
@@ -99,13 +91,12 @@ def _make_plan(values):
         kernel = factory.get_kernel(params, device)
     if kernel is None:
         return None
-    with _kernels_lock:
-        _kernels[values] = kernel
+    kernel.in_plans = True
     spec = kernel.kernel_spec
     stages = [_stage(kernel.function, spec.launch_params)]
     if kernel.epilogue_function is not None:
         stages.append(_stage(kernel.epilogue_function, spec.epilogue_launch_params))
-    return stages, spec.workspace_bytes, spec.overwrites_output
+    return stages, spec.workspace_bytes, spec.overwrites_output, kernel
 
 
 class NativeOp(CustomOpDef):

@@ -2,6 +2,8 @@
 between the forward and the backward pass changes the saved tensors, asks for second derivatives or wants to see
 the launches."""
 
+import gc
+
 import pytest
 import torch
 
@@ -61,3 +63,32 @@ def test_saved_tensors_may_come_back_in_another_layout(op, dtype, fused, hooks, 
     with _HOOKS[hooks]():
         y = call(*leaves)
     _assert_near(torch.autograd.grad(y, leaves, dy), expected)
+
+
+def test_a_captured_graph_outlives_the_launch_plans():
+    """A graph captured over a call on float32 activations replays whatever drops the plans meanwhile."""
+    leaves, call = _leaves("autocast", torch.float32)
+    dy = torch.randn(3, 24, 9, 7, device="cuda").contiguous(memory_format=CL)
+
+    def step():
+        y = call(*leaves)
+        return [y.detach(), *torch.autograd.grad(y, leaves, dy)]
+
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        step()
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        captured = step()
+    for seed in range(3):
+        native.Bypass().release()
+        native.forget_plans()
+        gc.collect()
+        torch.manual_seed(seed)
+        with torch.no_grad():
+            leaves[0].copy_(torch.randn(3, 24, 9, 7, device="cuda"))
+        graph.replay()
+        torch.cuda.synchronize()
+        _assert_near(captured, step())
