@@ -23,6 +23,8 @@
 #include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/custom_function.h>
+#include <torch/csrc/autograd/functions/basic_ops.h>
+#include <torch/csrc/autograd/functions/utils.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <atomic>
@@ -298,13 +300,28 @@ Tensor to_float_1d(const Tensor& t) {
 
 PyObject* g_backward_op = nullptr;  // the Python operator: gradients that are differentiated again
 
+// A saved copy (`cast`) of input number `input` of the node that is running, made to depend on that input
+// again: the forward pass cast it with gradients off.  What is computed from it then leads back to the input,
+// by way of a node that refuses to be run, so that a gradient of it is never taken for a constant.
+Tensor with_history(const Tensor& copy, bool cast, size_t input) {
+    const auto node = torch::autograd::get_current_node();
+    if (!cast || !node || input >= node->num_outputs() || !node->next_edge(input).is_valid()) return copy;
+    Tensor t = copy.variable_data();
+    torch::autograd::set_history(t, std::make_shared<torch::autograd::Error>(
+        "spio::conv2d_gw8: second derivatives have no autograd formula", torch::autograd::edge_list{node->next_edge(input)}));
+    return t;
+}
+
 struct ConvFunction : torch::autograd::Function<ConvFunction> {
     static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& w,
                           const std::optional<Tensor>& bias_arg, const Conv& cv) {
         const Tensor bias = bias_arg.value_or(Tensor());
-        const Tensor xh = to_half_cl(x), wh = to_half_cl(w);
-        Tensor y = conv_forward(cv, xh, wh, to_float_1d(bias), x.scalar_type());
-        ctx->save_for_backward({xh, wh});
+        const Tensor xh = to_half_cl(x), wh = to_half_cl(w), bf = to_float_1d(bias);
+        Tensor y = conv_forward(cv, xh, wh, bf, x.scalar_type());
+        // the caller's own tensors unless their type was cast: with their history and their version, which
+        // a second differentiation and a write to one of them before the backward pass are noticed by
+        ctx->save_for_backward({x.scalar_type() == at::kHalf ? x : xh, w.scalar_type() == at::kHalf ? w : wh,
+                                bias.defined() && bias.scalar_type() == at::kFloat ? bias : bf});
         ctx->saved_data["v"] = std::vector<int64_t>{
             cv.n, cv.c, cv.h, cv.w, cv.r, cv.s, cv.py, cv.px, cv.bias, static_cast<int64_t>(x.scalar_type()),
             static_cast<int64_t>(w.scalar_type()),
@@ -324,10 +341,12 @@ struct ConvFunction : torch::autograd::Function<ConvFunction> {
         if (!native || at::GradMode::is_enabled()) {
             // tensors the kernels do not take, which it refuses, and create_graph=True: the Python operator,
             // which says what it thinks of second derivatives
+            const Tensor xa = with_history(x, v[9] != static_cast<int64_t>(at::kHalf), 0),
+                         wa = with_history(w, v[10] != static_cast<int64_t>(at::kHalf), 1),
+                         ba = with_history(saved[2], v[11] != static_cast<int64_t>(at::kFloat), 2);
             py::gil_scoped_acquire gil;
-            py::object b = cv.bias ? py::cast(at::empty({cv.c}, x.options().dtype(at::kFloat))) : py::none();
             py::tuple r = py::reinterpret_borrow<py::object>(g_backward_op)(
-                x, w, b, grads[0].to(at::kHalf), cv.py, cv.px, need_x, need_w, need_b);
+                xa, wa, ba.defined() ? py::cast(ba) : py::none(), grads[0].to(at::kHalf), cv.py, cv.px, need_x, need_w, need_b);
             auto get = [&](int i) { return r[i].is_none() ? Tensor() : r[i].cast<Tensor>(); };
             g = {get(0), get(1), get(2)};
         } else {
@@ -369,7 +388,7 @@ struct NormFunction : torch::autograd::Function<NormFunction> {
         const Tensor weight = weight_arg.value_or(Tensor()), bias = bias_arg.value_or(Tensor());
         const Tensor xc = to_half_cl(x);
         Tensor y = norm_forward(nm, xc, to_float_1d(weight), to_float_1d(bias));
-        ctx->save_for_backward({xc, weight});
+        ctx->save_for_backward({x, weight});  // as in ConvFunction
         ctx->saved_data["v"] = std::vector<int64_t>{
             nm.n, nm.c, nm.h, nm.w, bias.defined(),
             weight.defined() ? static_cast<int64_t>(weight.scalar_type()) : static_cast<int64_t>(at::kFloat)};

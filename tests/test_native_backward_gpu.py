@@ -92,3 +92,41 @@ def test_a_captured_graph_outlives_the_launch_plans():
         graph.replay()
         torch.cuda.synchronize()
         _assert_near(captured, step())
+
+
+@pytest.mark.parametrize("op,dtype,layout,affine", [
+    ("conv", torch.float16, CL, True), ("conv", torch.float16, torch.contiguous_format, True),
+    ("autocast", torch.float32, CL, True), ("autocast", torch.float32, torch.contiguous_format, False),
+    ("norm", torch.float16, CL, False), ("norm", torch.float16, torch.contiguous_format, False),
+    ("norm", torch.float16, torch.contiguous_format, True),
+])  # fmt: skip
+def test_second_derivatives_are_refused(op, dtype, layout, affine):
+    """A gradient made with create_graph=True depends on the inputs whatever was cast or laid out anew on the
+    way, and differentiating it raises: a penalty on it is never dropped from a sum."""
+    leaves, call = _leaves(op, dtype, layout, affine)
+    for wanted in leaves:
+        y = call(*leaves)
+        (g,) = torch.autograd.grad(y.sum(), wanted, create_graph=True)  # a grad_output that needs no gradient
+        assert g.requires_grad
+        loss = g.float().square().sum() + y.float().sum()
+        with pytest.raises(RuntimeError, match="autograd formula"):
+            loss.backward(retain_graph=True)
+        for leaf in leaves[: 2 if op == "norm" else 3]:  # no gradient of the norm depends on its bias
+            with pytest.raises(RuntimeError, match="autograd formula"):
+                loss.backward(inputs=[leaf], retain_graph=True)
+
+
+@pytest.mark.parametrize("op,dtype,layout,which", [
+    ("conv", torch.float16, CL, 0), ("conv", torch.float16, torch.contiguous_format, 0),
+    ("conv", torch.float16, torch.contiguous_format, 1), ("conv", torch.float16, CL, 2),
+    ("autocast", torch.float16, torch.contiguous_format, 0), ("autocast", torch.float32, CL, 2),
+    ("norm", torch.float16, torch.contiguous_format, 0), ("norm", torch.float16, CL, 1),
+])  # fmt: skip
+def test_saved_inputs_must_not_change(op, dtype, layout, which):
+    """The operators save their own arguments: writing to one before the backward pass is an error, in any layout."""
+    leaves, call = _leaves(op, dtype, layout)
+    y = call(*leaves)
+    with torch.no_grad():
+        leaves[which].add_(1)
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        y.sum().backward()
