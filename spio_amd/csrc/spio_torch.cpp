@@ -175,6 +175,12 @@ bool eager_mode() {
            !at::impl::torch_function_mode_enabled();
 }
 
+// Whether a backward pass goes to the Python operators: somebody has come to see every launch, or to trace or
+// transform the call, since the forward pass, or its gradients are to be differentiated (create_graph=True).
+bool stands_aside(const Tensor& grad) {
+    return g_bypass.load(std::memory_order_relaxed) != 0 || !eager_mode() || !is_plain(grad) || at::GradMode::is_enabled();
+}
+
 bool wants_grad(const Tensor& t) { return t.defined() && t.requires_grad(); }
 
 std::optional<Tensor> optional(const Tensor& t) { return t.defined() ? std::optional<Tensor>(t) : std::nullopt; }
@@ -334,13 +340,12 @@ struct ConvFunction : torch::autograd::Function<ConvFunction> {
         const Conv cv{v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7], v[8] != 0};
         const auto saved = ctx->get_saved_variables();
         const Tensor &x = saved[0], &w = saved[1];
-        const bool native = is_again(x, grads[0], {cv.n, cv.c, cv.h, cv.w}) && is_again(w, grads[0], {cv.c, 8, cv.r, cv.s});
+        const bool native = !stands_aside(grads[0]) && is_again(x, grads[0], {cv.n, cv.c, cv.h, cv.w}) &&
+                            is_again(w, grads[0], {cv.c, 8, cv.r, cv.s});
         const bool need_x = ctx->needs_input_grad(0), need_w = ctx->needs_input_grad(1),
                    need_b = cv.bias && ctx->needs_input_grad(2);
         ConvGrads g;
-        if (!native || at::GradMode::is_enabled()) {
-            // tensors the kernels do not take, which it refuses, and create_graph=True: the Python operator,
-            // which says what it thinks of second derivatives
+        if (!native) {  // the Python operator, which refuses second derivatives and tensors it does not take
             const Tensor xa = with_history(x, v[9] != static_cast<int64_t>(at::kHalf), 0),
                          wa = with_history(w, v[10] != static_cast<int64_t>(at::kHalf), 1),
                          ba = with_history(saved[2], v[11] != static_cast<int64_t>(at::kFloat), 2);
@@ -401,10 +406,10 @@ struct NormFunction : torch::autograd::Function<NormFunction> {
         const Norm nm{v[0], v[1], v[2], v[3], ctx->saved_data["eps"].toDouble()};
         const auto saved = ctx->get_saved_variables();
         const Tensor &x = saved[0], &weight = saved[1];
-        const bool native = is_again(x, grads[0], {nm.n, nm.c, nm.h, nm.w}) &&
+        const bool native = !stands_aside(grads[0]) && is_again(x, grads[0], {nm.n, nm.c, nm.h, nm.w}) &&
                             (!weight.defined() || is_again(weight, grads[0], {nm.c}, static_cast<at::ScalarType>(v[5])));
         Tensor dx, sums;
-        if (!native || at::GradMode::is_enabled()) {  // as in ConvFunction
+        if (!native) {
             py::gil_scoped_acquire gil;
             py::object wt = weight.defined() ? py::cast(weight) : py::none();
             py::tuple r = py::reinterpret_borrow<py::object>(g_norm_backward_op)(x, grads[0], wt, nm.eps);

@@ -6,9 +6,12 @@ import gc
 
 import pytest
 import torch
+from torch.utils._python_dispatch import TorchDispatchMode
 
 from spio_amd import native
 from spio_amd.functional import conv2d_gw8, layernorm_2d
+from spio_amd.kernels import KernelParamsLogger
+from spio_amd.kernels.kernel import LaunchTimer
 
 pytestmark = pytest.mark.gpu
 CL = torch.channels_last
@@ -114,6 +117,47 @@ def test_second_derivatives_are_refused(op, dtype, layout, affine):
         for leaf in leaves[: 2 if op == "norm" else 3]:  # no gradient of the norm depends on its bias
             with pytest.raises(RuntimeError, match="autograd formula"):
                 loss.backward(inputs=[leaf], retain_graph=True)
+
+
+@pytest.mark.parametrize("op,dtype", [("conv", torch.float16), ("autocast", torch.float32), ("norm", torch.float16)])
+def test_backward_stands_aside(op, dtype):
+    """A backward pass whose forward ran natively takes the Python operator where a timer, a logger or a
+    dispatch mode was entered in between, with the same gradients."""
+    leaves, call = _leaves(op, dtype)
+    y = call(*leaves)
+    dy = torch.randn_like(y)
+    expected = torch.autograd.grad(y, leaves, dy, retain_graph=True)
+    plans = native._native.plans()
+    assert plans > 0
+
+    with LaunchTimer() as timer:
+        _assert_near(torch.autograd.grad(y, leaves, dy, retain_graph=True), expected)
+    assert any("grad" in str(k) or "_bwd" in str(k) for k in timer.events)
+
+    with KernelParamsLogger() as logger:
+        _assert_near(torch.autograd.grad(y, leaves, dy, retain_graph=True), expected)
+    assert logger.get_logged_params() and native._native.plans() == 0
+
+    seen = []
+
+    class Mode(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            seen.append(str(func))
+            return func(*args, **(kwargs or {}))
+
+    with Mode():
+        _assert_near(torch.autograd.grad(y, leaves, dy, retain_graph=True), expected)
+    assert any("_backward" in f and f.startswith("spio") for f in seen)
+
+
+@pytest.mark.parametrize("op,dtype", [("conv", torch.float16), ("autocast", torch.float32), ("norm", torch.float16)])
+def test_batched_gradients(op, dtype):
+    """Several gradients of one output at once, as jacobian(vectorize=True) asks for them."""
+    leaves, call = _leaves(op, dtype)
+    y = call(*leaves)
+    dys = torch.randn(3, *y.shape, device="cuda", dtype=y.dtype)
+    expected = [torch.stack(g) for g in zip(*[torch.autograd.grad(y, leaves, dy, retain_graph=True) for dy in dys])]
+    _assert_near(torch.autograd.grad(y, leaves, dys, is_grads_batched=True), expected)
 
 
 @pytest.mark.parametrize("op,dtype,layout,which", [
