@@ -385,7 +385,7 @@ Tensor norm_forward(const Norm& nm, const Tensor& x, const Tensor& weight, const
 }
 
 constexpr int64_t NORM_BACKWARD_MAX_CHANNELS = 1024;  // of the backward kernel
-PyObject* g_norm_backward_op = nullptr;
+PyObject* g_norm_gradients = nullptr;  // Python: the gradients, by kernel or torch operations
 
 struct NormFunction : torch::autograd::Function<NormFunction> {
     static Tensor forward(AutogradContext* ctx, const Tensor& x, const std::optional<Tensor>& weight_arg,
@@ -406,32 +406,32 @@ struct NormFunction : torch::autograd::Function<NormFunction> {
         const Norm nm{v[0], v[1], v[2], v[3], ctx->saved_data["eps"].toDouble()};
         const auto saved = ctx->get_saved_variables();
         const Tensor &x = saved[0], &weight = saved[1];
-        const bool native = !stands_aside(grads[0]) && is_again(x, grads[0], {nm.n, nm.c, nm.h, nm.w}) &&
+        const bool native = !stands_aside(grads[0]) && !std::getenv("SPIO_LAYERNORM_BACKWARD") &&
+                            is_again(x, grads[0], {nm.n, nm.c, nm.h, nm.w}) &&
                             (!weight.defined() || is_again(weight, grads[0], {nm.c}, static_cast<at::ScalarType>(v[5])));
-        Tensor dx, sums;
+        // absent tensors have no edge: the bias's follows the weight's or the input's
+        const bool has_weight = weight.defined();
+        const bool need_x = ctx->needs_input_grad(0), need_w = has_weight && ctx->needs_input_grad(1),
+                   need_b = v[4] != 0 && ctx->needs_input_grad(has_weight ? 2 : 1);
         if (!native) {
             py::gil_scoped_acquire gil;
-            py::object wt = weight.defined() ? py::cast(weight) : py::none();
-            py::tuple r = py::reinterpret_borrow<py::object>(g_norm_backward_op)(x, grads[0], wt, nm.eps);
-            dx = r[0].cast<Tensor>();
-            sums = r[1].cast<Tensor>();
-        } else {
-            const Tensor dy = to_half_cl(grads[0]), xc = to_half_cl(x);
-            const Tensor w = to_float_1d(weight);
-            const auto device = dy.get_device();
-            hipStream_t stream = c10::hip::getCurrentHIPStream(device);
-            const auto plan = find_plan(nm.key(NORM_BWD, device, w.defined(), false));
-            dx = empty_cl({nm.n, nm.c, nm.h, nm.w}, at::kHalf, dy);
-            sums = at::detail::empty_cuda({2, nm.c}, at::kFloat, dy.device(), std::nullopt);
-            const Tensor workspace = empty_1d(plan->workspace, at::kByte, dy);
-            launch(plan->main, stream, {ptr(workspace), ptr(dx), ptr(xc), ptr(dy), ptr(w)});
-            launch(plan->second, stream, {ptr(sums), ptr(workspace)});
+            py::tuple r = py::reinterpret_borrow<py::object>(g_norm_gradients)(
+                x, has_weight ? py::cast(weight) : py::none(), grads[0], nm.eps, need_x, need_w, need_b);
+            auto get = [&](int i) { return r[i].is_none() ? Tensor() : r[i].cast<Tensor>(); };
+            return {get(0), get(1), get(2), Tensor()};
         }
-        // absent tensors have no edge: the bias's follows the weight's or the input's
-        const bool has_weight = weight.defined(), has_bias = v[4] != 0;
-        return {ctx->needs_input_grad(0) ? dx : Tensor(),
-                has_weight && ctx->needs_input_grad(1) ? sums.select(0, 0).to(weight.scalar_type()) : Tensor(),
-                has_bias && ctx->needs_input_grad(has_weight ? 2 : 1) ? sums.select(0, 1) : Tensor(), Tensor()};
+        const Tensor dy = to_half_cl(grads[0]), xc = to_half_cl(x);
+        const Tensor w = to_float_1d(weight);
+        const auto device = dy.get_device();
+        hipStream_t stream = c10::hip::getCurrentHIPStream(device);
+        const auto plan = find_plan(nm.key(NORM_BWD, device, w.defined(), false));
+        const Tensor dx = empty_cl({nm.n, nm.c, nm.h, nm.w}, at::kHalf, dy);
+        const Tensor sums = at::detail::empty_cuda({2, nm.c}, at::kFloat, dy.device(), std::nullopt);
+        const Tensor workspace = empty_1d(plan->workspace, at::kByte, dy);
+        launch(plan->main, stream, {ptr(workspace), ptr(dx), ptr(xc), ptr(dy), ptr(w)});
+        launch(plan->second, stream, {ptr(sums), ptr(workspace)});
+        return {need_x ? dx : Tensor(), need_w ? sums.select(0, 0).to(weight.scalar_type()) : Tensor(),
+                need_b ? sums.select(0, 1) : Tensor(), Tensor()};
     }
 };
 
@@ -545,7 +545,7 @@ PyObject* layernorm_2d(PyObject*, PyObject* const* args, Py_ssize_t nargs, PyObj
     if (nm.n < 1 || nm.h < 1 || nm.w < 1 || nm.c < 8 || nm.c % 8 || !(nm.eps > 0)) return not_implemented();
     const bool record = at::GradMode::is_enabled() && (wants_grad(x) || wants_grad(weight) || wants_grad(bias));
     // the backward pass by torch operations is the Python operator's
-    if (record && (nm.c > NORM_BACKWARD_MAX_CHANNELS || std::getenv("SPIO_LAYERNORM_BACKWARD"))) return not_implemented();
+    if (record && nm.c > NORM_BACKWARD_MAX_CHANNELS) return not_implemented();
     Tensor y;
     {
         py::gil_scoped_release no_gil;
@@ -572,10 +572,10 @@ PyMethodDef g_methods[] = {
 }  // namespace
 
 PYBIND11_MODULE(_native, m) {
-    m.def("configure", [](py::object make_plan, py::object backward_op, py::object norm_backward_op) {
+    m.def("configure", [](py::object make_plan, py::object backward_op, py::object norm_gradients) {
         g_make_plan = make_plan.release().ptr();
         g_backward_op = backward_op.release().ptr();
-        g_norm_backward_op = norm_backward_op.release().ptr();
+        g_norm_gradients = norm_gradients.release().ptr();
     });
     m.def("bypass", [](int64_t change) { g_bypass.fetch_add(change); });
     m.def("forget", [] {

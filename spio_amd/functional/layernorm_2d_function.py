@@ -79,33 +79,38 @@ def _layernorm_2d_backward_fake(inputs, grad_output, weight, eps):
             inputs.new_empty((2, c), dtype=torch.float32))  # fmt: skip
 
 
-def _backward(ctx, grad_output) -> Tuple[Optional[torch.Tensor], ...]:
-    x, weight = ctx.saved_tensors
+def layernorm_2d_gradients(x, weight, grad_output, eps, needs_input, needs_weight, needs_bias):
+    """Gradients of layernorm_2d, None where not needed; by the kernel, or by torch operations where it does
+    not take the shape or SPIO_LAYERNORM_BACKWARD=torch asks for them."""
     n, c, h, w = (int(v) for v in x.shape)
     use_kernel = (os.environ.get("SPIO_LAYERNORM_BACKWARD", "hip") != "torch" and x.device.type == "cuda"
                   and layernorm_2d_bwd_is_supported(LayerNorm2dParams(n=n, c=c, h=h, w=w)))  # fmt: skip
     if use_kernel:
-        grad_input, sums = layernorm_2d_backward(x, grad_output, weight, ctx.eps)
+        grad_input, sums = layernorm_2d_backward(x, grad_output, weight, eps)
         return (
-            grad_input if ctx.needs_input_grad[0] else None,
-            sums[0].to(weight.dtype) if weight is not None and ctx.needs_input_grad[1] else None,
-            sums[1] if ctx.has_bias and ctx.needs_input_grad[2] else None,
-            None,
+            grad_input if needs_input else None,
+            sums[0].to(weight.dtype) if needs_weight else None,
+            sums[1] if needs_bias else None,
         )
     xf = x.float().permute(0, 2, 3, 1)  # [n, h, w, c] view of the channels_last tensor
     dy = grad_output.float().permute(0, 2, 3, 1)
     mean = xf.mean(-1, keepdim=True)
     var = (xf - mean).pow(2).mean(-1, keepdim=True)
-    rstd = torch.rsqrt(var + ctx.eps)
+    rstd = torch.rsqrt(var + eps)
     xhat = (xf - mean) * rstd
     g = dy if weight is None else dy * weight.float()
     dx = rstd * (g - g.mean(-1, keepdim=True) - xhat * (g * xhat).mean(-1, keepdim=True))
-    grad_input = dx.permute(0, 3, 1, 2).to(x.dtype) if ctx.needs_input_grad[0] else None
-    grad_weight = None
-    if weight is not None and ctx.needs_input_grad[1]:
-        grad_weight = (dy * xhat).sum((0, 1, 2)).to(weight.dtype)
-    grad_bias = dy.sum((0, 1, 2)) if ctx.has_bias and ctx.needs_input_grad[2] else None
-    return grad_input, grad_weight, grad_bias, None
+    grad_input = dx.permute(0, 3, 1, 2).to(x.dtype) if needs_input else None
+    grad_weight = (dy * xhat).sum((0, 1, 2)).to(weight.dtype) if needs_weight else None
+    grad_bias = dy.sum((0, 1, 2)) if needs_bias else None
+    return grad_input, grad_weight, grad_bias
+
+
+def _backward(ctx, grad_output) -> Tuple[Optional[torch.Tensor], ...]:
+    x, weight = ctx.saved_tensors
+    needs = ctx.needs_input_grad
+    return (*layernorm_2d_gradients(x, weight, grad_output, ctx.eps, needs[0], weight is not None and needs[1],
+                                    ctx.has_bias and needs[2]), None)  # fmt: skip
 
 
 layernorm_2d.register_autograd(_backward, setup_context=_setup_context)

@@ -115,7 +115,7 @@ def adopt(op, native_name):
     op.native = getattr(_native, native_name)
 
 
-def configure(backward_op, norm_backward_op):
-    """Switch the native path on; the operators it hands double differentiation to."""
-    _native.configure(_make_plan, backward_op, norm_backward_op)
+def configure(backward_op, norm_gradients):
+    """Switch the native path on; what its backward passes hand over to where they stand aside."""
+    _native.configure(_make_plan, backward_op, norm_gradients)
     _native.bypass(-1)

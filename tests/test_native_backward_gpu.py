@@ -174,3 +174,25 @@ def test_saved_inputs_must_not_change(op, dtype, layout, which):
         leaves[which].add_(1)
     with pytest.raises(RuntimeError, match="modified by an inplace operation"):
         y.sum().backward()
+
+
+def test_norm_backward_choice_is_read_in_the_backward_pass(monkeypatch):
+    """SPIO_LAYERNORM_BACKWARD=torch set behind the forward pass: no plan of the backward kernel is made, and
+    the gradients can be differentiated, with the results of the Python operator."""
+    leaves, call = _leaves("norm")
+    y = call(*leaves)
+    dy = torch.randn_like(y)
+    expected = torch.autograd.grad(y, leaves, dy, retain_graph=True)
+    native.forget_plans()
+    monkeypatch.setenv("SPIO_LAYERNORM_BACKWARD", "torch")
+    _assert_near(torch.autograd.grad(y, leaves, dy, retain_graph=True), expected)
+    assert native._native.plans() == 0
+
+    def second(y):
+        (g,) = torch.autograd.grad(y, leaves[0], dy, create_graph=True)
+        return torch.autograd.grad(g.float().square().sum(), leaves[:2])
+
+    results = second(call(*leaves))
+    held = native.Bypass()
+    _assert_near(results, second(call(*leaves)))
+    held.release()
