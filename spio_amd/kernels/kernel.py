@@ -63,20 +63,19 @@ class LaunchTimer:
 
     def __init__(self):
         self.events = {}
-        self._bypass = None
+        self._bypasses = []  # one for each time it is entered
 
     def __enter__(self):
         from ..native import Bypass
 
-        self._bypass = self._bypass or Bypass()
+        self._bypasses.append(Bypass())
         LaunchTimer.active = self
         self.events = {}
         return self
 
     def __exit__(self, exc_type, exc_val, exc_tb):
         LaunchTimer.active = None
-        self._bypass.release()
-        self._bypass = None
+        self._bypasses.pop().release()
         return False
 
     def averages(self, skip: int = 0):

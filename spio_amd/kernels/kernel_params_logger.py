@@ -25,13 +25,13 @@ class KernelParamsLogger(ContextDecorator):
     def __init__(self):
         self.logged_params: List[KernelParams] = []
         self._lock = threading.Lock()
-        self._bypass = None
+        self._bypasses = []  # one for each time it is entered: a decorated function may call itself
 
     def __enter__(self):
         global _active
         from ..native import Bypass
 
-        self._bypass = self._bypass or Bypass()
+        self._bypasses.append(Bypass())
         with _active_lock:
             _active = self
         self.logged_params = []
@@ -41,8 +41,7 @@ class KernelParamsLogger(ContextDecorator):
         global _active
         with _active_lock:
             _active = None
-        self._bypass.release()
-        self._bypass = None
+        self._bypasses.pop().release()
         return False
 
     def get_logged_params(self) -> List[KernelParams]:

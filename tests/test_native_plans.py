@@ -8,8 +8,8 @@ import pytest
 
 from spio_amd import native
 from spio_amd.hip import DeviceAttributes
-from spio_amd.kernels import Conv2dGw8Config, KernelSpec, LaunchParams, conv2d_gw8_kernel_factory, kernel_cache
-from spio_amd.kernels.kernel import Kernel
+from spio_amd.kernels import Conv2dGw8Config, KernelParamsLogger, KernelSpec, LaunchParams, conv2d_gw8_kernel_factory, kernel_cache
+from spio_amd.kernels.kernel import Kernel, LaunchTimer
 
 WIDE_FORWARD = (0, 0, 2, 64, 8, 8, 3, 3, 1, 1, 0, native.WIDE)  # a key: float32-storing forward kernel on device 0
 
@@ -98,3 +98,15 @@ def test_unloading_a_kernel_outside_the_plans_forgets_none(made, monkeypatch):
     assert not calls
     native._make_plan(WIDE_FORWARD)[3].unload()
     assert calls
+
+
+@pytest.mark.parametrize("recorder", [KernelParamsLogger, LaunchTimer])
+def test_recorders_may_be_entered_again(recorder, monkeypatch):
+    """One instance, inside itself: the native path stays off until the outer block ends."""
+    held = []
+    monkeypatch.setattr(native._native, "bypass", held.append)
+    with recorder() as outer:
+        with outer:
+            assert sum(held) == 2
+        assert sum(held) == 1
+    assert sum(held) == 0
