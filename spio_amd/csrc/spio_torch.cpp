@@ -137,9 +137,9 @@ void launch(const Stage& stage, hipStream_t stream, std::initializer_list<const 
         params[n] = &values[n];
         ++n;
     }
-    if (spio_hip_launch(stage.function, stage.grid[0], stage.grid[1], stage.grid[2], stage.block[0],
-                        stage.block[1], stage.block[2], stage.lds, stream, params, n))
-        throw py::value_error(std::string("kernel launch failed: ") + spio_hip_last_error());
+    const int rc = spio_hip_launch(stage.function, stage.grid[0], stage.grid[1], stage.grid[2], stage.block[0],
+                                   stage.block[1], stage.block[2], stage.lds, stream, params, n);
+    TORCH_CHECK_VALUE(rc == 0, "kernel launch failed: ", spio_hip_last_error());
 }
 
 const void* ptr(const Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; }
@@ -153,8 +153,8 @@ Tensor empty_1d(int64_t n, at::ScalarType dtype, const Tensor& like) {
 // Clears one or two tensors (undefined: none) in one launch.
 void zero(const Tensor& a, const Tensor& b, hipStream_t stream) {
     auto bytes = [](const Tensor& t) { return t.defined() ? static_cast<size_t>(t.nbytes()) : 0; };
-    if (spio_hip_zero_fill_pair_async(const_cast<void*>(ptr(a)), bytes(a), const_cast<void*>(ptr(b)), bytes(b), stream))
-        throw py::value_error(std::string("zero fill failed: ") + spio_hip_last_error());
+    const int rc = spio_hip_zero_fill_pair_async(const_cast<void*>(ptr(a)), bytes(a), const_cast<void*>(ptr(b)), bytes(b), stream);
+    TORCH_CHECK_VALUE(rc == 0, "zero fill failed: ", spio_hip_last_error());
 }
 
 // ---- which calls take this path -------------------------------------------------------------

@@ -9,7 +9,7 @@ import torch
 from torch.utils._python_dispatch import TorchDispatchMode
 
 from spio_amd import native
-from spio_amd.functional import conv2d_gw8, layernorm_2d
+from spio_amd.functional import conv2d_gw8, conv2d_gw8_backward_op, layernorm_2d, layernorm_2d_gradients
 from spio_amd.kernels import KernelParamsLogger
 from spio_amd.kernels.kernel import LaunchTimer
 
@@ -196,3 +196,18 @@ def test_norm_backward_choice_is_read_in_the_backward_pass(monkeypatch):
     held = native.Bypass()
     _assert_near(results, second(call(*leaves)))
     held.release()
+
+
+@pytest.mark.parametrize("in_backward", [False, True])
+def test_a_launch_that_fails_raises_value_error(in_backward):
+    """The error of the kernels' Python launch; here the library refuses a plan without a function."""
+    leaves, call = _leaves("conv")
+    y = call(*leaves)
+    native.forget_plans()
+    native._native.configure(lambda values: ([[0, 1, 1, 1, 64, 1, 1, 0]], 0, False, None), conv2d_gw8_backward_op, None)
+    try:
+        with pytest.raises(ValueError, match="launch"):
+            y.sum().backward() if in_backward else call(*leaves)
+    finally:
+        native.forget_plans()
+        native._native.configure(native._make_plan, conv2d_gw8_backward_op, layernorm_2d_gradients)
