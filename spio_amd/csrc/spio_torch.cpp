@@ -472,6 +472,9 @@ bool int_arg(PyObject* o, int64_t* v) {
 
 PyObject* not_implemented() { Py_RETURN_NOTIMPLEMENTED; }
 
+// Paddings above this are the Python operator's to refuse: twice one near 2^63 would wrap around to a small image.
+constexpr int64_t MAX_PADDING = 1 << 24;
+
 // conv2d_gw8(inputs, weight, bias=None, stride=1, padding_y=0, padding_x=0, dilation=1, groups=1)
 PyObject* conv2d_gw8(PyObject*, PyObject* const* args, Py_ssize_t nargs, PyObject* kwnames) {
     HANDLE_TH_ERRORS
@@ -495,8 +498,8 @@ PyObject* conv2d_gw8(PyObject*, PyObject* const* args, Py_ssize_t nargs, PyObjec
         return not_implemented();
     const Conv cv{x.size(0), x.size(1), x.size(2), x.size(3), w.size(2), w.size(3), py, px, bias.defined()};
     if (stride != 1 || dilation != 1 || groups != cv.c / 8 || cv.c % 8 || w.size(0) != cv.c || w.size(1) != 8 || py < 0 ||
-        px < 0 || cv.r < 1 || cv.r > 7 || cv.s < 1 || cv.s > 7 || cv.n < 1 || cv.c < 8 || cv.h < 1 || cv.w < 1 ||
-        cv.p() < 1 || cv.q() < 1)
+        px < 0 || py > MAX_PADDING || px > MAX_PADDING || cv.r < 1 || cv.r > 7 || cv.s < 1 || cv.s > 7 || cv.n < 1 ||
+        cv.c < 8 || cv.h < 1 || cv.w < 1 || cv.p() < 1 || cv.q() < 1)
         return not_implemented();
     const bool autocast = at::autocast::is_autocast_enabled(at::kCUDA);
     auto floating = [](const Tensor& t) { return t.scalar_type() == at::kFloat || t.scalar_type() == at::kHalf; };

@@ -108,3 +108,14 @@ def test_it_stands_aside():
         y = call(*args)
         (g,) = torch.autograd.grad(y.float().square().sum(), args[0], create_graph=True)
         torch.autograd.grad(g.float().square().sum(), args[0])
+
+
+@pytest.mark.parametrize("padding", [2**63 - 1, 2**62, 2**40])
+@pytest.mark.parametrize("side", ["padding_y", "padding_x"])
+def test_paddings_without_a_possible_output_are_refused(side, padding):
+    """The Python operator raises when it allocates the output; a size that wraps around is never launched."""
+    args, _ = _conv_args(Conv2dGw8Params(2, 16, 8, 8), grads=(False,) * 3)
+    native.forget_plans()
+    with pytest.raises((TypeError, RuntimeError)):
+        conv2d_gw8(args[0], args[1], None, groups=2, **{side: padding})
+    assert native._native.plans() == 0
