@@ -181,6 +181,13 @@ bool stands_aside(const Tensor& grad) {
     return g_bypass.load(std::memory_order_relaxed) != 0 || !eager_mode() || !is_plain(grad) || at::GradMode::is_enabled();
 }
 
+// What a profiler that records shapes is told of a call; evaluated only if one is active.
+std::vector<c10::IValue> tensors(std::initializer_list<Tensor> args) {
+    std::vector<c10::IValue> values;
+    for (const Tensor& t : args) values.emplace_back(t);
+    return values;
+}
+
 bool wants_grad(const Tensor& t) { return t.defined() && t.requires_grad(); }
 
 std::optional<Tensor> optional(const Tensor& t) { return t.defined() ? std::optional<Tensor>(t) : std::nullopt; }
@@ -355,6 +362,7 @@ struct ConvFunction : torch::autograd::Function<ConvFunction> {
             auto get = [&](int i) { return r[i].is_none() ? Tensor() : r[i].cast<Tensor>(); };
             g = {get(0), get(1), get(2)};
         } else {
+            RECORD_FUNCTION("spio::conv2d_gw8_backward", tensors({x, w, saved[2], grads[0]}));
             g = conv_backward(cv, to_half_cl(x), to_half_cl(w), to_half_cl(grads[0]), need_x, need_w, need_b,
                               static_cast<at::ScalarType>(v[9]));
         }
@@ -420,6 +428,7 @@ struct NormFunction : torch::autograd::Function<NormFunction> {
             auto get = [&](int i) { return r[i].is_none() ? Tensor() : r[i].cast<Tensor>(); };
             return {get(0), get(1), get(2), Tensor()};
         }
+        RECORD_FUNCTION("spio::layernorm_2d_backward", tensors({x, grads[0], weight}));
         const Tensor dy = to_half_cl(grads[0]), xc = to_half_cl(x);
         const Tensor w = to_float_1d(weight);
         const auto device = dy.get_device();
@@ -513,7 +522,7 @@ PyObject* conv2d_gw8(PyObject*, PyObject* const* args, Py_ssize_t nargs, PyObjec
     {
         py::gil_scoped_release no_gil;
         c10::DeviceGuard device(x.device());
-        RECORD_FUNCTION("spio::conv2d_gw8", std::vector<c10::IValue>());
+        RECORD_FUNCTION("spio::conv2d_gw8", tensors({x, w, bias}));
         // the casts and copies inside are the operator's own, whatever autocast thinks of them
         c10::impl::ExcludeDispatchKeyGuard no_autocast(c10::autocast_dispatch_keyset);
         if (at::GradMode::is_enabled() && (wants_grad(x) || wants_grad(w) || wants_grad(bias))) {
@@ -553,7 +562,7 @@ PyObject* layernorm_2d(PyObject*, PyObject* const* args, Py_ssize_t nargs, PyObj
     {
         py::gil_scoped_release no_gil;
         c10::DeviceGuard device(x.device());
-        RECORD_FUNCTION("spio::layernorm_2d", std::vector<c10::IValue>());
+        RECORD_FUNCTION("spio::layernorm_2d", tensors({x, weight, bias}));
         if (record) {
             y = NormFunction::apply(x, optional(weight), optional(bias), nm);
         } else {

@@ -211,3 +211,24 @@ def test_a_launch_that_fails_raises_value_error(in_backward):
     finally:
         native.forget_plans()
         native._native.configure(native._make_plan, conv2d_gw8_backward_op, layernorm_2d_gradients)
+
+
+def _profiled(op, dtype):
+    """{operator: shapes of its tensor arguments} of a pass as torch's profiler sees it."""
+    leaves, call = _leaves(op, dtype)
+    y = call(*leaves)
+    torch.autograd.grad(y, leaves, torch.randn_like(y))
+    with torch.autograd.profiler.profile(record_shapes=True, use_device=None) as profile:
+        y = call(*leaves)
+        torch.autograd.grad(y, leaves, torch.randn_like(y))
+    return {e.name: [s for s in e.input_shapes if s] for e in profile.function_events if e.name.startswith("spio::")}
+
+
+@pytest.mark.parametrize("op,dtype", [("conv", torch.float16), ("autocast", torch.float32), ("norm", torch.float16)])
+def test_profiles_show_the_operators(op, dtype):
+    """Forward and backward operators appear under their names with the shapes of their tensors."""
+    seen = _profiled(op, dtype)
+    held = native.Bypass()
+    expected = _profiled(op, dtype)
+    held.release()
+    assert len(expected) == 2 and seen == expected
