@@ -19,6 +19,7 @@ a list of representative shape specialisations; at run time the same sources
 are specialised per shape with hipRTC instead.
 """
 
+import hashlib
 import os
 import shutil
 import subprocess
@@ -97,6 +98,27 @@ def build_native(force: bool = True, verbose: bool = False) -> str:
     return LIB_PATH
 
 
+def extension_digest() -> str:
+    """What a _native.so is built from: its source, the header of the library it calls and torch's version."""
+    import torch  # pylint: disable=import-outside-toplevel
+
+    digest = hashlib.sha256(torch.__version__.encode())
+    for path in (os.path.join(CSRC_DIR, "spio_torch.cpp"), os.path.join(_include_dir(), "spio_hip.h")):
+        with open(path, "rb") as f:
+            digest.update(f.read())
+    return digest.hexdigest()[:32]
+
+
+def extension_is_current() -> bool:
+    """Whether _native.so is there and was built from the present source and for the present torch: it holds
+    the digest of both (not their dates, which a copy of the tree may not keep)."""
+    try:
+        with open(EXTENSION_PATH, "rb") as f:
+            return f"spio-built-from:{extension_digest()}".encode() in f.read()
+    except OSError:
+        return False
+
+
 def build_extension(verbose: bool = False) -> str:
     """Compile _native.so, the operators' call path on torch's C++ interface; returns its path.
 
@@ -115,7 +137,8 @@ def build_extension(verbose: bool = False) -> str:
     tmp = f"{EXTENSION_PATH}.tmp{os.getpid()}"
     try:
         _run([cxx, "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__=1",
-              "-DUSE_ROCM=1", "-DTORCH_EXTENSION_NAME=_native", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}",
+              "-DUSE_ROCM=1", "-DTORCH_EXTENSION_NAME=_native", f"-DSPIO_BUILT_FROM={extension_digest()}",
+              f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}",
               *[f"-I{d}" for d in includes], os.path.join(CSRC_DIR, "spio_torch.cpp"), "-o", tmp,
               f"-L{os.path.join(root, 'lib')}", "-lc10", "-lc10_hip", "-ltorch", "-ltorch_cpu", "-ltorch_hip",
               "-ltorch_python", f"-L{CSRC_DIR}", "-l:libspio_hip.so", "-Wl,-rpath,$ORIGIN/csrc"],

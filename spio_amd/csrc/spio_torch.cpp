@@ -583,7 +583,13 @@ PyMethodDef g_methods[] = {
 
 }  // namespace
 
+// Found in the built file by spio_amd/build.py.
+#define SPIO_TEXT_(x) #x
+#define SPIO_TEXT(x) SPIO_TEXT_(x)
+
 PYBIND11_MODULE(_native, m) {
+    m.attr("built_from") = "spio-built-from:" SPIO_TEXT(SPIO_BUILT_FROM);
+    m.attr("WIDE") = WIDE;
     m.def("configure", [](py::object make_plan, py::object backward_op, py::object norm_gradients) {
         g_make_plan = make_plan.release().ptr();
         g_backward_op = backward_op.release().ptr();

@@ -4,37 +4,45 @@
 without going through the Python definition of the operator, which costs several times what the
 kernels take at ordinary sizes.  It asks `_make_plan` once per shape for the kernels to launch
 (tuner, compiler and caches are the Python side's) and keeps the answer until `forget_plans()`.
+Where the file cannot be built or loaded the Python definitions run every call.
 Whoever wants to see or choose every launch (overlay caches, KernelParamsLogger, LaunchTimer)
 holds a `Bypass` meanwhile: all calls then take the Python path.
 """
 
 import importlib
-import os
 import struct
+import warnings
 
 import torch
 from torch._library.custom_ops import CustomOpDef
 
-from .build import EXTENSION_PATH, build_extension
+from .build import build_extension, extension_is_current
 
-if not os.path.exists(EXTENSION_PATH):
-    build_extension()
-_native = importlib.import_module(f"{__package__}._native")
+try:
+    if not extension_is_current():
+        build_extension()
+    _native = importlib.import_module(f"{__package__}._native")
+except (ImportError, OSError, RuntimeError) as error:
+    _native = None
+    warnings.warn(f"spio_amd._native could not be built or loaded; every call pays for the Python path: {error}",
+                  RuntimeWarning, stacklevel=2)  # fmt: skip
 
 
 def forget_plans():
     """Drop every launch plan (a kernel of one was unloaded, caches or choices cleared).  The kernels stay
     with their caches: graphs, queued work and other threads may still launch them."""
-    _native.forget()
+    if _native is not None:
+        _native.forget()
 
 
 class Bypass:
     """While one of these is held, the native path declines every call."""
 
     def __init__(self):
-        self._held = True
-        _native.bypass(1)
-        forget_plans()
+        self._held = _native is not None
+        if self._held:
+            _native.bypass(1)
+            forget_plans()
 
     def release(self):
         """Let calls take the native path again (idempotent)."""
@@ -49,7 +57,7 @@ def _stage(function, launch_params):
     return [function.handle, *launch_params.grid, *launch_params.block, launch_params.shared_mem_bytes]
 
 
-WIDE = 4  # bit of a key's mode: the kernel stores its activations as float32
+WIDE = 0 if _native is None else _native.WIDE  # bit of a key's mode: the kernel stores its activations as float32
 
 
 def _widened(kernel, factory, params, device, **kwargs):
@@ -111,11 +119,15 @@ class NativeOp(CustomOpDef):
 
 def adopt(op, native_name):
     """Give the custom operator `op` the native path `native_name`."""
+    if _native is None:
+        return
     op.__class__ = NativeOp
     op.native = getattr(_native, native_name)
 
 
 def configure(backward_op, norm_gradients):
     """Switch the native path on; what its backward passes hand over to where they stand aside."""
+    if _native is None:
+        return
     _native.configure(_make_plan, backward_op, norm_gradients)
     _native.bypass(-1)
