@@ -209,9 +209,13 @@ constexpr int DX_ROW_BYTES = kW * kC * kDstBytes;
 constexpr int D_ROW_BYTES = kQ * kC * 2;
 constexpr unsigned OOB = 0x80000000u;  // offset of a lane without data: beyond every descriptor
 // Cache-policy operands of the buffer instructions: streamed (2) unless several channel blocks share the
-// lines, then loaded with the default policy so that the second block finds them in L2 (50n 152c 21x41 17.3
-// -> 15.7 us, 94n 296c 43x47 125 -> 115, 128n 96c 56x56 56.1 -> 54.9).  SPIO_NT = 0 stores with the
-// default policy: L2 then joins the parts of a line that different blocks store, see the configurations.
+// lines, then loaded with the default policy so that the second block finds them in L2.  Streamed -> default
+// loads, best of four configurations: 94n 296c 43x47 129 -> 112 us, 50n 152c 21x41 17.1 -> 15.1, 64n 72c 56x56
+// 41 -> 38, 32n 320c 28x28 17.8 -> 15.6, 16n 256c 56x56 38 -> 35, 128n 96c 56x56 equal.  Where a pixel is whole lines
+// it can cost instead (64n 192c 28x28 18.6 -> 19.3, 8n 128c 112x112 35.6 -> 38.1); offering the sweep both
+// there made a shape's first use 1 to 3 s longer and chose the same on the shapes tried.  SPIO_NT = 0 stores
+// with the default policy: L2 then joins the parts of a line that different blocks store, see the
+// configurations.
 constexpr bool kSplitLines = splits_lines(GB, GBLKS);
 constexpr int AUX_LD = kSplitLines ? 0 : 2;
 constexpr int AUX_ST = SPIO_NT ? 2 : 0;

@@ -393,9 +393,10 @@ def with_joined_stores(params: Conv2dGw8Params, configs: list) -> list:
     """`configs` with a second version of the leading eight, right behind each, that stores through L2.
 
     With an odd number of groups the boundary between two channel blocks is not even 32-byte aligned and
-    memory has to merge the parts of a sector that two blocks store, unless L2 does it first.  Measured,
-    non-temporal -> default stores: 60n 216c 56x56 68 -> 48 us, 94n 296c 43x47 77 -> 64, 30n 184c 60x60
-    26 -> 23; on small images it costs instead (32n 808c 20x20 11.4 -> 13.7), so the sweep decides; a capped one
+    memory has to merge the parts of a sector that two blocks store, unless L2 does it first.  Measured, best
+    of the pairs, non-temporal -> default stores: 60n 216c 56x56 61 -> 48 us, 94n 296c 43x47 83 -> 66 (fused
+    backward 110 -> 94); on smaller tensors it costs instead (30n 184c 60x60 20.4 -> 21.8, 32n 808c 20x20
+    11.0 -> 11.5), so the sweep decides; a capped one
     does not count the second versions, whose geometry it tries anyway.  With an even number the hint is
     the better one or equal (128n 96c 56x56 29.1 against 35.0)."""
     out = []
