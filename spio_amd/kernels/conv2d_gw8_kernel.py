@@ -222,10 +222,22 @@ def _image_score(params, config, igrad, num_cus: int) -> float:
     split = 1.0 + 0.05 * (config.split - 1)
     single = 1.0 if config.prefetch >= 2 else 1.03
     # mover waves pay where moving a block takes longer than multiplying it (measured: 3x3 on
-    # 14x14 0.73x, 7x7 on 14x14 1.05x)
-    movers = 1.0 if not config.movers else (0.9 if params.r * params.s < 25 else 1.05)
+    # 14x14 0.73x, 5x5 on 9x9 and 14x14 0.97x, 7x7 on 14x14 1.05x)
+    movers = 1.0 if not config.movers else (0.9 if params.r * params.s <= 25 else 1.05)
     ragged = g["WGBLKS"] * config.block_n_iters * config.block_n / params.n
     return quant * ragged * split_line * setup * split * single * movers / (tile_eff * group_eff)
+
+
+def _whole_round_iters(params, config, igrad, num_cus: int) -> List[int]:
+    """Image blocks per workgroup with which the grid is one or two whole rounds of the device.
+
+    A workgroup's set-up (filters through LDS, pipeline fill) costs about two image blocks, so fewer and
+    longer workgroups are better until they leave compute units idle.  128n 1392c 9x9 5x5: 22 channel blocks
+    leave 11 workgroups each, 12 images a workgroup; forward 21.3 us with 4 images (704 workgroups, 2.75
+    rounds) and 21.7 with 16 (176, 0.7 rounds) -> 19.1, data gradient 21.2 -> 18.6."""
+    g = image_geometry(params, replace(config, block_n_iters=1), igrad)
+    per_cu = max(1, min(DEVICE_LDS_BYTES // g["LDS_BYTES"], 2048 // g["THREADS"]))
+    return [divup(g["NBLKS"], max(1, num_cus * per_cu * rounds // g["GBLKS"])) for rounds in (1, 2)]
 
 
 def _image_configs(params: Conv2dGw8Params, igrad: bool, num_cus: int) -> List[Conv2dGw8Config]:
@@ -235,16 +247,17 @@ def _image_configs(params: Conv2dGw8Params, igrad: bool, num_cus: int) -> List[C
     for gb in sorted({g for g in (4, 8, 16, G) if g <= min(G, MAX_WAVES)}):
         for nb in (1, 2, 4, 8):
             for ts in (1, 2, 4):
-                for iters in (1, 2, 4, 8, 16):
-                    for buffers, movers in ((2, 0), (1, 0), (2, MOVER_WAVES)):
-                        cfg = Conv2dGw8Config(groups=gb, block_p=direction_geometry(params, igrad)["DH"],
-                                              block_n=nb, split=ts, prefetch=buffers, variant="image",
-                                              halo_cached=0, xcd_chunk=0, block_n_iters=iters,
-                                              movers=movers)  # fmt: skip
+                for buffers, movers in ((2, 0), (1, 0), (2, MOVER_WAVES)):
+                    base = Conv2dGw8Config(groups=gb, block_p=direction_geometry(params, igrad)["DH"],
+                                           block_n=nb, split=ts, prefetch=buffers, variant="image",
+                                           halo_cached=0, xcd_chunk=0, movers=movers)  # fmt: skip
+                    if not _image_config_is_legal(params, base, igrad):
+                        continue
+                    for iters in sorted({1, 2, 4, 8, 16, *_whole_round_iters(params, base, igrad, num_cus)}):
                         if nb * iters > max(params.n, 1) and iters > 1:
                             continue
-                        if _image_config_is_legal(params, cfg, igrad):
-                            found.append((_image_score(params, cfg, igrad, num_cus), cfg))
+                        cfg = replace(base, block_n_iters=iters)
+                        found.append((_image_score(params, cfg, igrad, num_cus), cfg))
     found.sort(key=lambda sc: sc[0])
     return [cfg for _, cfg in found[:MAX_IMAGE_CONFIGS]]
 

@@ -107,6 +107,17 @@ def test_channel_blocks_that_share_lines(params, chunk):
                               configs=[Conv2dGw8BgradConfig(groups=min(gb, 4), block_h=3, prefetch=2, xcd_chunk=chunk)])
 
 
+@pytest.mark.parametrize("movers", [0, 4])
+def test_whole_image_runs_of_any_length(movers):
+    """Image blocks per workgroup that are no power of two: odd and even runs, a last run that is partly or
+    wholly behind the batch's end, a run longer than the batch."""
+    params = Conv2dGw8Params(n=7, c=72, h=9, w=9, r=5, s=5, padding=2, has_bias=True)
+    configs = [Conv2dGw8Config(groups=4, block_p=9, block_n=nb, variant="image", prefetch=2, block_n_iters=it, movers=movers)
+               for nb, it in ((1, 3), (1, 5), (2, 3), (1, 6), (1, 9))]  # fmt: skip
+    run_kernel_test(conv2d_gw8_kernel_factory, params, configs=configs)
+    run_grad_kernel_test(conv2d_gw8_kernel_factory, params, configs=configs, igrad=True)
+
+
 _F32_CASES = [
     # cells that do not fill the last wave, odd group counts, images side by side, a ragged batch
     (Conv2dGw8Params(n=5, c=24, h=9, w=11, padding=1, has_bias=True),

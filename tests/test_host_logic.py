@@ -433,3 +433,22 @@ def test_second_store_policies_do_not_shorten_a_capped_sweep(monkeypatch):
         assert _on_miss_limit(odd) == len(both) and _on_miss_limit(even) == 8
         monkeypatch.setenv("SPIO_TUNE_MAX_CONFIGS", "4")  # a bound that the caller states counts every version
         assert _on_miss_limit(odd) == 4 and _on_miss_limit(even) == 4
+
+
+def test_whole_image_configurations_offer_whole_rounds():
+    """Among the whole-image configurations is one whose workgroups are one round of the device at most and
+    would not be one with fewer image blocks each; every one covers the batch."""
+    from types import SimpleNamespace
+
+    from spio_amd.kernels import conv2d_gw8_kernel as ck
+
+    for n, c, h, k in ((128, 1392, 9, 5), (100, 400, 14, 5), (37, 256, 7, 3)):
+        params = Conv2dGw8Params(n=n, c=c, h=h, w=h, r=k, s=k, padding=k // 2)
+        configs = [q for q in ck._get_configs(params, SimpleNamespace(multiprocessor_count=256)) if q.variant == "image"]
+        geometries = [(q, ck.image_geometry(params, q, False)) for q in configs]
+        assert all(g["WGBLKS"] * q.block_n_iters >= g["NBLKS"] for q, g in geometries)
+        first, g = geometries[0]
+        resident = max(1, min(ck.DEVICE_LDS_BYTES // g["LDS_BYTES"], 2048 // g["THREADS"]))
+        shorter = ck.image_geometry(params, replace(first, block_n_iters=max(1, first.block_n_iters - 1)), False)
+        assert g["NUM_BLOCKS"] <= 2 * 256 * resident
+        assert first.block_n_iters == 1 or shorter["NUM_BLOCKS"] > g["NUM_BLOCKS"]
