@@ -836,19 +836,17 @@ SPIO_KERNEL_NAME(spio_uint4* __restrict__ grad_input, float* __restrict__ grad_w
 #if SPIO_PARTIALS
 // Second stage: grad_weight (and grad_bias) = sum over the workgroups' blocks.  A workgroup of
 // 256 threads owns 8 float4 columns of one channel block (128 contiguous bytes of every block);
-// its 32 slices each add the blocks p = slice, slice + 32, ... with up to 8 loads in flight, the
+// its 32 slices each add the blocks p = slice, slice + 32, ... with up to 16 loads in flight, the
 // slices are added through LDS and slice 0 stores the totals.  A block is laid out like the
 // channel block's part of grad_weight, so column `col` of channel block `cb` is the float4 at
 // grad_weight[cb * GB * GROUP_FLOATS + 4 * col]; the columns behind it are the bias sums.
-#define SPIO_CONCAT2(a, b) a##b
-#define SPIO_CONCAT(a, b) SPIO_CONCAT2(a, b)
-extern "C" __global__ void SPIO_LAUNCH_BOUNDS(256)
-SPIO_CONCAT(SPIO_KERNEL_NAME, _reduce)(float* __restrict__ grad_weight, const spio_float4* __restrict__ partials,
-                                       float* __restrict__ grad_bias) {
+template <class T>
+SPIO_DEVICE void reduce_partials(T* __restrict__ grad_weight, const spio_float4* __restrict__ partials,
+                                 float* __restrict__ grad_bias) {
     constexpr int BLOCK_F4 = PART_FLOATS / 4;  // float4 columns of one block
     constexpr int COLS = 8;
     constexpr int SLICES = 256 / COLS;
-    constexpr int UN = 8;
+    constexpr int UN = NPART <= 8 * SLICES ? 8 : 16;
     constexpr int WGS_PER_CB = (BLOCK_F4 + COLS - 1) / COLS;
     __shared__ spio_float4 red[SLICES][COLS];
     const int tid = thread_id();
@@ -878,11 +876,21 @@ SPIO_CONCAT(SPIO_KERNEL_NAME, _reduce)(float* __restrict__ grad_weight, const sp
         const int f = 4 * col;  // float index inside the block
         if (f < GB * GROUP_FLOATS) {
             if (cb * GB + f / GROUP_FLOATS < kGroups)
-                *reinterpret_cast<spio_float4*>(grad_weight + (long long)cb * GB * GROUP_FLOATS + f) = sum;
+                store_sums(grad_weight + (long long)cb * GB * GROUP_FLOATS + f, sum);
         } else if (grad_bias != nullptr) {
             const int k = cb * GB * 8 + (f - GB * GROUP_FLOATS);
             if (k < kC) *reinterpret_cast<spio_float4*>(grad_bias + k) = sum;
         }
     }
+}
+extern "C" __global__ void SPIO_LAUNCH_BOUNDS(256)
+SPIO_CONCAT(SPIO_KERNEL_NAME, _reduce)(float* __restrict__ grad_weight, const spio_float4* __restrict__ partials,
+                                       float* __restrict__ grad_bias) {
+    reduce_partials(grad_weight, partials, grad_bias);
+}
+extern "C" __global__ void SPIO_LAUNCH_BOUNDS(256)
+SPIO_CONCAT(SPIO_KERNEL_NAME, _reduce_h)(spio_half* __restrict__ grad_weight, const spio_float4* __restrict__ partials,
+                                         float* __restrict__ grad_bias) {
+    reduce_partials(grad_weight, partials, grad_bias);
 }
 #endif

@@ -188,6 +188,9 @@ static_assert(PF >= 2 && PF % 2 == 0, "prefetch distance must be even");
 static_assert(RB == 1 || RB == 2, "one or two rows per step");
 static_assert(LEAD + RB <= NRD, "the dy rows of the prologue fit the ring");
 constexpr int PART_WAVE_FLOATS = kR * NBLK * 4 * 32;  // floats one wave publishes (partial-block layout)
+// Two stages with a bias: behind the partial blocks, every workgroup's bias sums, [block][channel], zeros
+// for channels past the last one.
+constexpr long long BIAS_PARTIALS = (long long)NBLKS * PBLKS * QBLKS * GBLKS * GB * PART_WAVE_FLOATS;
 
 
 SPIO_DEVICE spio_half8 read_tr_pair(const unsigned char* lo, const unsigned char* hi) {
@@ -729,12 +732,15 @@ SPIO_KERNEL_NAME(float* __restrict__ grad_weight, const spio_uint4* __restrict__
                     bslots[wave * 8 + k4 + e] = wave_active ? accb[e] + scratch[e * 32 + lane] : 0.f;
             }
             block_sync();
-            if (wave == 0 && grad_bias != nullptr) {
+            if (wave == 0) {
                 for (int i = lane; i < GB * 8; i += 64) {
                     float v = 0.f;
 #pragma unroll
                     for (int w2 = 0; w2 < TS; ++w2) v += bslots[(w2 * GB + i / 8) * 8 + (i & 7)];
-                    if (cb * GB + i / 8 < kGroups) atomic_add_f32(grad_bias + 8 * cb * GB + i, v);
+#if SPIO_PARTIALS
+                    grad_weight[BIAS_PARTIALS + (((long long)nbk * PBLKS + pb) * QBLKS + qb) * GBLKS * GB * 8 + cb * GB * 8 + i] = v;
+#endif
+                    if (grad_bias != nullptr && cb * GB + i / 8 < kGroups) atomic_add_f32(grad_bias + 8 * cb * GB + i, v);
                 }
             }
         }
@@ -745,24 +751,23 @@ SPIO_KERNEL_NAME(float* __restrict__ grad_weight, const spio_uint4* __restrict__
 
 #if SPIO_PARTIALS
 // Second stage: grad_weight = sum over the partial blocks (stored whole: a caller that runs the
-// two-stage kernel need not zero grad_weight first).  A workgroup owns 32 float4 columns
-// of one channel block (512 contiguous bytes of every partial block: half a wave per load
-// instruction); its 8 slices each add the blocks p = slice, slice + 8, ... with 4 loads in
-// flight, the slices are added through LDS and slice 0 adds the total onto grad_weight.  (With 8
-// columns and 32 slices per workgroup, 3584 workgroups of 128-byte rows for a 7x7 filter on 256
-// channels, the stage took 5.9 us for 14.7 MB; now 5.1 us, of which about 2.2 us are what any
-// kernel costs in a stream.)  Every element of grad_weight has exactly one
+// two-stage kernel need not zero grad_weight first).  A workgroup owns COLS float4 columns
+// of one channel block (COLS * 16 contiguous bytes of every partial block); its slices each add the blocks
+// p = slice, slice + SLICES, ... with UN loads in flight, the slices are added through LDS and slice 0
+// stores the total.  With 32 columns (512 bytes: half a wave per load instruction) where that gives
+// a workgroup per compute unit: with 8 columns, 3584 workgroups of 128-byte rows for a 7x7 filter on 256
+// channels, the stage took 5.9 us for 14.7 MB, with 32 5.1 us, of which about 2.2 us are what any
+// kernel costs in a stream.  With 8 where there are few columns: more workgroups, and more slices each.
+// Every element of grad_weight has exactly one
 // owner, so no atomics are needed and the sum does not depend on timing.  A column is four
 // consecutive lanes of the publishing wave, i.e. four consecutive channels c of one (k, r, s).
-#define SPIO_CONCAT2(a, b) a##b
-#define SPIO_CONCAT(a, b) SPIO_CONCAT2(a, b)
-extern "C" __global__ void SPIO_LAUNCH_BOUNDS(256)
-SPIO_CONCAT(SPIO_KERNEL_NAME, _reduce)(float* __restrict__ grad_weight, const spio_float4* __restrict__ partials) {
+template <class T>
+SPIO_DEVICE void reduce_partials(T* __restrict__ grad_weight, const spio_float4* __restrict__ partials) {
     constexpr int BLOCK_F4 = GB * PART_WAVE_FLOATS / 4;  // float4 columns of one partial block
     constexpr int NPART = NBLKS * PBLKS * QBLKS;
-    constexpr int COLS = 32;
+    constexpr int COLS = SPIO_REDUCE_COLS;
     constexpr int SLICES = 256 / COLS;
-    constexpr int UN = 4;
+    constexpr int UN = NPART <= 4 * SLICES ? 4 : NPART <= 8 * SLICES ? 8 : 16;
     static_assert(BLOCK_F4 % COLS == 0, "a workgroup's columns lie in one channel block");
     __shared__ spio_float4 red[SLICES][COLS];
     const int tid = thread_id();
@@ -796,11 +801,62 @@ SPIO_CONCAT(SPIO_KERNEL_NAME, _reduce)(float* __restrict__ grad_weight, const sp
         const int r = rn / NBLK;
         const int s = 2 * (rn % NBLK) + ((l32 & 15) >> 3);
         const int k = 8 * (cb * GB + g) + 4 * (l32 >> 4) + e;
-        if (cb * GB + g < kGroups && s < kS) {
-            spio_float4* dst =
-                reinterpret_cast<spio_float4*>(grad_weight + (((long long)k * kR + r) * kS + s) * 8 + (l32 & 7));
-            *dst = sum;
-        }
+        if (cb * GB + g < kGroups && s < kS)
+            store_sums(grad_weight + (((long long)k * kR + r) * kS + s) * 8 + (l32 & 7), sum);
     }
+}
+extern "C" __global__ void SPIO_LAUNCH_BOUNDS(256)
+SPIO_CONCAT(SPIO_KERNEL_NAME, _reduce)(float* __restrict__ grad_weight, const spio_float4* __restrict__ partials) {
+    reduce_partials(grad_weight, partials);
+}
+// The version for fp16 weights also sums the bias partials, in a workgroup of its own per channel block
+// behind the others, and stores grad_bias (null = not wanted): nothing is left to clear before the main
+// kernel, which gets a null grad_bias then.
+#if SPIO_HAS_BIAS
+SPIO_DEVICE void reduce_bias(float* __restrict__ grad_bias, const float* __restrict__ bias_partials, int cb) {
+    constexpr int NPART = NBLKS * PBLKS * QBLKS;
+    constexpr int CH = GB * 8;
+    constexpr int SLICES = 256 / CH;
+    constexpr int UN = 8;
+    __shared__ float red[SLICES][CH];
+    const int tid = thread_id();
+    const int ch = tid % CH;
+    const int slice = tid / CH;
+    const int k = cb * CH + ch;
+    float sum = 0.f;
+    if (slice < SLICES) {
+        for (int base = slice; base < NPART; base += SLICES * UN) {
+            float v[UN];
+#pragma unroll
+            for (int i = 0; i < UN; ++i) {
+                const int p = base + i * SLICES;
+                v[i] = p < NPART ? bias_partials[(long long)p * GBLKS * CH + k] : 0.f;
+            }
+#pragma unroll
+            for (int i = 0; i < UN; ++i) sum += v[i];
+        }
+        red[slice][ch] = sum;
+    }
+    block_sync();
+    if (slice == 0 && k < kC && grad_bias != nullptr) {
+        for (int i = 1; i < SLICES; ++i) sum += red[i][ch];
+        grad_bias[k] = sum;
+    }
+}
+#endif
+extern "C" __global__ void SPIO_LAUNCH_BOUNDS(256)
+SPIO_CONCAT(SPIO_KERNEL_NAME, _reduce_h)(spio_half* __restrict__ grad_weight, const spio_float4* __restrict__ partials
+#if SPIO_HAS_BIAS
+                                         , float* __restrict__ grad_bias
+#endif
+) {
+#if SPIO_HAS_BIAS
+    constexpr int WEIGHT_BLOCKS = GBLKS * (GB * PART_WAVE_FLOATS / 4) / SPIO_REDUCE_COLS;
+    if (block_id() >= WEIGHT_BLOCKS) {
+        reduce_bias(grad_bias, reinterpret_cast<const float*>(partials) + BIAS_PARTIALS, block_id() - WEIGHT_BLOCKS);
+        return;
+    }
+#endif
+    reduce_partials(grad_weight, partials);
 }
 #endif

@@ -170,6 +170,18 @@ SPIO_DEVICE void atomic_add_f32(float* address, float value) {
     __hip_atomic_fetch_add(address, value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// Stores four sums of a second stage: as they are, or rounded to fp16 for a caller whose weights are fp16.
+SPIO_DEVICE void store_sums(float* p, spio_float4 v) { *reinterpret_cast<spio_float4*>(p) = v; }
+SPIO_DEVICE void store_sums(spio_half* p, spio_float4 v) {
+    spio_half4 h;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) h[e] = (spio_half)v[e];
+    *reinterpret_cast<spio_half4*>(p) = h;
+}
+// A second stage comes twice: <name>_reduce stores float sums, <name>_reduce_h the same rounded to fp16.
+#define SPIO_CONCAT2(a, b) a##b
+#define SPIO_CONCAT(a, b) SPIO_CONCAT2(a, b)
+
 // Bit-cast helpers between the 16-byte vector views of one (pixel, group).
 union Pack16 {
     spio_uint4 u;

@@ -72,6 +72,7 @@ struct Stage {
 };
 struct Plan {
     Stage main, second;         // `second` of two-stage kernels
+    Stage second_half;          // the second stage that stores grad_weight as float16
     int64_t workspace = 0;      // bytes of partial results between the stages
     bool present = false;       // false: the shape does not use this kind (no fused backward, no float32 output)
     bool overwrites = false;    // the kernel stores its sums whole instead of adding to them
@@ -105,7 +106,7 @@ PlanPtr find_plan(const Key& key) {
             auto stages = t[0].cast<py::list>();
             for (size_t i = 0; i < stages.size(); ++i) {
                 auto s = stages[i].cast<std::vector<uint64_t>>();
-                Stage& stage = i == 0 ? plan->main : plan->second;
+                Stage& stage = i == 0 ? plan->main : i == 1 ? plan->second : plan->second_half;
                 stage.function = reinterpret_cast<void*>(s[0]);
                 for (int d = 0; d < 3; ++d) {
                     stage.grid[d] = static_cast<unsigned>(s[1 + d]);
@@ -217,7 +218,9 @@ int64_t fused_mode() {
 
 // ---- convolution ----------------------------------------------------------------------------
 
-constexpr int64_t WIDE = 4;  // bit of a key's mode: the kernel stores its activations as float32
+// Bits of a key's mode: the kernel stores its activations as float32; the caller's weights, and so their
+// gradient, are float16.
+constexpr int64_t WIDE = 4, HALF_WEIGHT = 8;
 
 // `dtype`: what the caller wants; float32 comes from the kernel itself where it has such a version,
 // else the result is float16 and the caller converts it.
@@ -239,9 +242,12 @@ struct ConvGrads {
 
 // The backward operator on channels_last tensors: one fused kernel where the shape uses it and
 // both gradients are wanted, else the weight and the data gradient one after the other.
+// `x_dtype`, `w_dtype`: what the caller's tensors are; a gradient is stored in that type where the kernel
+// can (a two-stage one's grad_weight), else in the operator's and the caller converts it.
 ConvGrads conv_backward(const Conv& cv, const Tensor& x, const Tensor& w, const Tensor& dy, bool need_x,
-                        bool need_w, bool need_b, at::ScalarType x_dtype) {
+                        bool need_w, bool need_b, at::ScalarType x_dtype, at::ScalarType w_dtype) {
     ConvGrads g;
+    const int64_t weight_mode = w_dtype == at::kHalf ? HALF_WEIGHT : 0;
     // the version of a kernel whose grad_input is float32, where that is wanted and there is one
     auto wide_or = [&](const PlanPtr& plan, Kind kind, int64_t mode) {
         const auto wide = x_dtype == at::kFloat ? find_plan(cv.key(kind, dy.get_device(), mode | WIDE)) : nullptr;
@@ -253,17 +259,20 @@ ConvGrads conv_backward(const Conv& cv, const Tensor& x, const Tensor& w, const 
     hipStream_t stream = c10::hip::getCurrentHIPStream(device);
     // atomic kernels add into zeroed sums, two-stage ones store them whole
     auto sums = [&](const Plan& plan, bool with_bias, bool bias_is_stored) {
-        g.w = empty_cl({cv.c, 8, cv.r, cv.s}, at::kFloat, dy);
+        g.w = empty_cl({cv.c, 8, cv.r, cv.s}, weight_mode && plan.second_half.function ? at::kHalf : at::kFloat, dy);
         if (with_bias) g.b = empty_1d(cv.c, at::kFloat, dy);
         // one launch for both: a launch is all that the fill of such small sums costs
         zero(plan.overwrites ? Tensor() : g.w, bias_is_stored ? Tensor() : g.b, stream);
     };
+    auto second = [&](const Plan& plan) -> const Stage& {
+        return g.w.scalar_type() == at::kHalf ? plan.second_half : plan.second;
+    };
     PlanPtr fused;
     if (need_x && need_w) {
         const int64_t mode = fused_mode();
-        if (mode != 0) fused = find_plan(cv.key(BGRAD, device, mode));
+        if (mode != 0) fused = find_plan(cv.key(BGRAD, device, mode | weight_mode));
         if (fused && !fused->present) fused.reset();
-        if (fused) fused = wide_or(fused, BGRAD, mode);
+        if (fused) fused = wide_or(fused, BGRAD, mode | weight_mode);
     }
     if (fused) {
         sums(*fused, cv.bias && need_b, fused->overwrites);
@@ -274,18 +283,23 @@ ConvGrads conv_backward(const Conv& cv, const Tensor& x, const Tensor& w, const 
             launch(fused->main, stream, {ptr(g.x), dw, ptr(x), ptr(dy), ptr(w), ptr(g.b)});
         else
             launch(fused->main, stream, {ptr(g.x), dw, ptr(x), ptr(dy), ptr(w)});
-        if (workspace.defined()) launch(fused->second, stream, {ptr(g.w), ptr(workspace), ptr(g.b)});
+        if (workspace.defined()) launch(second(*fused), stream, {ptr(g.w), ptr(workspace), ptr(g.b)});
     } else if (need_w) {
-        const auto plan = find_plan(cv.key(WGRAD, device));
-        sums(*plan, cv.bias && need_b, false);
+        const auto plan = find_plan(cv.key(WGRAD, device, weight_mode));
+        // the second stage that stores float16 stores the bias sums as well; the other adds them with atomics
+        const bool half = weight_mode && plan->second_half.function;
+        sums(*plan, cv.bias && need_b, half);
         Tensor workspace;
         if (plan->second.function) workspace = empty_1d(plan->workspace, at::kByte, dy);
         const void* dw = workspace.defined() ? ptr(workspace) : ptr(g.w);
         if (cv.bias)
-            launch(plan->main, stream, {dw, ptr(x), ptr(dy), ptr(g.b)});
+            launch(plan->main, stream, {dw, ptr(x), ptr(dy), half ? nullptr : ptr(g.b)});
         else
             launch(plan->main, stream, {dw, ptr(x), ptr(dy)});
-        if (workspace.defined()) launch(plan->second, stream, {ptr(g.w), ptr(workspace)});
+        if (half && cv.bias)
+            launch(plan->second_half, stream, {ptr(g.w), ptr(workspace), ptr(g.b)});
+        else if (workspace.defined())
+            launch(second(*plan), stream, {ptr(g.w), ptr(workspace)});
     }
     if (need_b && !g.b.defined()) g.b = dy.sum({0, 2, 3}, /*keepdim=*/false, at::kFloat);
     if (need_x && !g.x.defined()) {
@@ -364,7 +378,7 @@ struct ConvFunction : torch::autograd::Function<ConvFunction> {
         } else {
             RECORD_FUNCTION("spio::conv2d_gw8_backward", tensors({x, w, saved[2], grads[0]}));
             g = conv_backward(cv, to_half_cl(x), to_half_cl(w), to_half_cl(grads[0]), need_x, need_w, need_b,
-                              static_cast<at::ScalarType>(v[9]));
+                              static_cast<at::ScalarType>(v[9]), static_cast<at::ScalarType>(v[10]));
         }
         auto typed = [&](const Tensor& t, int i) {
             return t.defined() ? t.to(static_cast<at::ScalarType>(v[i])) : t;
@@ -590,6 +604,7 @@ PyMethodDef g_methods[] = {
 PYBIND11_MODULE(_native, m) {
     m.attr("built_from") = "spio-built-from:" SPIO_TEXT(SPIO_BUILT_FROM);
     m.attr("WIDE") = WIDE;
+    m.attr("HALF_WEIGHT") = HALF_WEIGHT;
     m.def("configure", [](py::object make_plan, py::object backward_op, py::object norm_gradients) {
         g_make_plan = make_plan.release().ptr();
         g_backward_op = backward_op.release().ptr();

@@ -12,7 +12,7 @@ from .kernel_cache import KernelCache
 from .kernel_params_logger import KernelParamsLogger, kernel_params_logging_is_enabled
 from .tuner import tuner, Tuner
 from .conv2d_gw8_kernel import conv2d_gw8_kernel_factory, Conv2dGw8Config
-from .conv2d_gw8_wgrad_kernel import conv2d_gw8_wgrad_kernel_factory, Conv2dGw8WgradConfig
+from .conv2d_gw8_wgrad_kernel import conv2d_gw8_wgrad_kernel_factory, Conv2dGw8WgradConfig, stored_sums
 from .conv2d_gw8_bgrad_kernel import (
     conv2d_gw8_bgrad_kernel_factory,
     Conv2dGw8BgradConfig,

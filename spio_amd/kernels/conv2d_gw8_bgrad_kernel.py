@@ -276,8 +276,10 @@ def _get_kernel_spec(params: Conv2dGw8Params, config: Conv2dGw8BgradConfig, _dev
         spec.workspace_bytes = g["GBLKS"] * npart * part_floats * 4
         spec.workspace_arg = 1  # the workspace takes the place of grad_weight
         spec.epilogue_suffix = "_reduce"
+        spec.epilogue_half_suffix = "_reduce_h"
         spec.epilogue_extra_args = (5,)  # grad_bias, or None where there is none
         spec.epilogue_launch_params = LaunchParams(grid=g["GBLKS"] * divup(part_floats // 4, 8), block=256)
+        spec.epilogue_half_launch_params = spec.epilogue_launch_params
         spec.overwrites_output = True
     return spec
 

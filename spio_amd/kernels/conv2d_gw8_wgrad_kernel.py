@@ -260,13 +260,42 @@ def _get_kernel_spec(params: Conv2dGw8Params, config: Conv2dGw8WgradConfig, _dev
         # float4 columns of the partial blocks of one (image block, row block): per wave
         # [r][tap pair][4][32 lanes] floats
         cols = g["GBLKS"] * config.groups * params.r * g["NBLK"] * 32
-        defines.update(SPIO_PARTIALS=1)
-        spec.workspace_bytes = num_partials * cols * 16
+        # columns per workgroup of the second stage (cols is a multiple of 32 per channel block)
+        reduce_cols = 32 if cols >= 32 * 256 else 8
+        defines.update(SPIO_PARTIALS=1, SPIO_REDUCE_COLS=reduce_cols)
+        bias_floats = num_partials * g["GBLKS"] * config.groups * 8 if params.has_bias else 0
+        spec.workspace_bytes = num_partials * cols * 16 + bias_floats * 4
         spec.epilogue_suffix = "_reduce"
+        spec.epilogue_half_suffix = "_reduce_h"  # with a bias it takes grad_bias as well and stores it
         spec.overwrites_output = True  # the second stage stores grad_weight whole
-        # one workgroup per 32 float4 columns (cols is a multiple of 32 per channel block)
-        spec.epilogue_launch_params = LaunchParams(grid=cols // 32, block=256)
+        spec.epilogue_launch_params = LaunchParams(grid=cols // reduce_cols, block=256)
+        bias_blocks = g["GBLKS"] if params.has_bias else 0
+        spec.epilogue_half_launch_params = LaunchParams(grid=cols // reduce_cols + bias_blocks, block=256)
     return spec
+
+
+# Partial sums up to this many bytes are published in two stages where grad_weight ends as float16: twice
+# this through memory costs about what the two launches do.
+STORED_SUMS_BYTES = 32 * 1024 * 1024
+
+
+def stored_sums(factory, params: Conv2dGw8Params, config):
+    """The configuration to run where grad_weight is wanted as float16: `config`, or its two-stage version.
+
+    A kernel that adds its sums with atomics needs them cleared before and rounded to float16 after it, a
+    launch each; the second stage of a two-stage kernel stores float16 itself.  Fill + kernel + rounding ->
+    two stages, captured in a graph: fused backward 32n 64c 56x56 19.7 -> 17.6 us, 128n 41.1 -> 38.1, 512n
+    131.1 -> 127.6, 128n 96c 64.8 -> 60.1, 2n 1024c 20x20 12.9 -> 12.9; weight gradient 4n 120c 39x39 11.4 ->
+    9.5, 128n 768c 7x7 15.0 -> 12.6.  With float32 sums only the fill is saved and the two are equal (128n 38.0
+    and 38.1), so there the sweep's choice stands."""
+    if config.two_stage or getattr(config, "variant", "mfma") != "mfma":
+        return config
+    stored = replace(config, two_stage=1)
+    try:
+        spec = factory.get_kernel_spec(params, stored)
+    except AssertionError:  # its scratch does not fit
+        return config
+    return stored if spec.workspace_bytes <= STORED_SUMS_BYTES else config
 
 
 def _make_test_args(params: Conv2dGw8Params, device):

@@ -41,6 +41,9 @@ class KernelSpec:
     epilogue_launch_params: Optional[LaunchParams] = None
     workspace_arg: int = 0
     epilogue_extra_args: tuple = ()
+    # The second stage that stores the same sums rounded to float16 (launched by the native call path)
+    epilogue_half_suffix: Optional[str] = None
+    epilogue_half_launch_params: Optional[LaunchParams] = None
     # True: the kernel (its last stage) stores the tensor at `workspace_arg` whole, so the caller
     # need not zero it; False: the kernel adds into it
     overwrites_output: bool = False
@@ -102,6 +105,7 @@ class Kernel:
         self.module = None
         self.function = None
         self.epilogue_function = None
+        self.epilogue_half_function = None
         self.device_ordinal: Optional[int] = None
         self.in_plans = False  # launch plans of the native call path point into the module
 
@@ -132,6 +136,10 @@ class Kernel:
             self.epilogue_function = self.module.get_function(
                 self.kernel_name + self.kernel_spec.epilogue_suffix
             )
+        if self.kernel_spec.epilogue_half_suffix:
+            self.epilogue_half_function = self.module.get_function(
+                self.kernel_name + self.kernel_spec.epilogue_half_suffix
+            )
         if self.kernel_spec.max_dynamic_lds:
             self.function.set_max_dynamic_lds(self.kernel_spec.max_dynamic_lds)
         if clear_code:
@@ -149,6 +157,7 @@ class Kernel:
             self.module = None
         self.function = None
         self.epilogue_function = None
+        self.epilogue_half_function = None
 
     def _prepare(self, args):
         """Check the arguments and return the device they live on."""

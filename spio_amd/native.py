@@ -57,17 +57,25 @@ def _stage(function, launch_params):
     return [function.handle, *launch_params.grid, *launch_params.block, launch_params.shared_mem_bytes]
 
 
-WIDE = 0 if _native is None else _native.WIDE  # bit of a key's mode: the kernel stores its activations as float32
+# bits of a key's mode: the kernel stores its activations as float32; the caller's weights are float16
+WIDE = 0 if _native is None else _native.WIDE
+HALF_WEIGHT = 0 if _native is None else _native.HALF_WEIGHT
 
 
-def _widened(kernel, factory, params, device, **kwargs):
-    """The version of `kernel` that stores float32, in the configuration chosen for the float16 one (it reads
-    and multiplies the same); None where that has no such version."""
+def _adapted(kernel, factory, params, device, mode, **kwargs):
+    """`kernel` or the version of it for the caller's types, in the configuration chosen for the plain one (it
+    reads and multiplies the same); None where that has no such version."""
+    from .kernels import stored_sums
     from .kernels.conv2d_gw8_kernel import fits_float32_output
 
-    if not fits_float32_output(params, kernel.config):
-        return None
-    return factory.get_kernel_in_config(params, device, kernel.config, out_f32=True, **kwargs)
+    config = stored_sums(factory, params, kernel.config) if mode & HALF_WEIGHT else kernel.config
+    if mode & WIDE:
+        if not fits_float32_output(params, config):
+            return None
+        kwargs["out_f32"] = True
+    elif config == kernel.config:
+        return kernel
+    return factory.get_kernel_in_config(params, device, config, **kwargs)
 
 
 def _make_plan(values):
@@ -86,11 +94,12 @@ def _make_plan(values):
             factory = kernels.conv2d_gw8_bgrad_kernel_factory
             kernel = fused_backward_kernel(params, device)
         elif kind == 2:
-            kernel = kernels.conv2d_gw8_wgrad_kernel_factory.get_kernel(params, device)
+            factory = kernels.conv2d_gw8_wgrad_kernel_factory
+            kernel = factory.get_kernel(params, device)
         else:
             kernel = factory.get_kernel(params, device, **direction)
-        if kernel is not None and mode & WIDE:
-            kernel = _widened(kernel, factory, params, device, **direction)
+        if kernel is not None:
+            kernel = _adapted(kernel, factory, params, device, mode, **direction)
     else:
         n, c, h, w, eps, weight, bias = values[2:9]
         params = kernels.LayerNorm2dParams(n=n, c=c, h=h, w=w, eps=struct.unpack("<d", struct.pack("<q", eps))[0],
@@ -104,6 +113,8 @@ def _make_plan(values):
     stages = [_stage(kernel.function, spec.launch_params)]
     if kernel.epilogue_function is not None:
         stages.append(_stage(kernel.epilogue_function, spec.epilogue_launch_params))
+    if kernel.epilogue_half_function is not None:
+        stages.append(_stage(kernel.epilogue_half_function, spec.epilogue_half_launch_params))
     return stages, spec.workspace_bytes, spec.overwrites_output, kernel
 
 

@@ -118,6 +118,52 @@ def test_whole_image_runs_of_any_length(movers):
     run_grad_kernel_test(conv2d_gw8_kernel_factory, params, configs=configs, igrad=True)
 
 
+@pytest.mark.parametrize("params,weight,fused", [
+    # few partial blocks and few columns; more of both than one trip of the loads takes, with a bias and an
+    # idle group; more than 512 partial blocks
+    (Conv2dGw8Params(n=3, c=16, h=6, w=7, padding=1), Conv2dGw8WgradConfig(groups=2, block_h=6, two_stage=1),
+     Conv2dGw8BgradConfig(groups=2, prefetch=2, two_stage=1)),
+    (Conv2dGw8Params(n=70, c=24, h=9, w=8, r=5, s=5, padding=2, has_bias=True),
+     Conv2dGw8WgradConfig(groups=2, block_h=4, two_stage=1), Conv2dGw8BgradConfig(groups=2, block_h=2, prefetch=2, two_stage=1)),
+    (Conv2dGw8Params(n=130, c=8, h=10, w=8, padding=1), Conv2dGw8WgradConfig(groups=1, block_h=2, two_stage=1),
+     Conv2dGw8BgradConfig(groups=1, block_h=2, prefetch=2, two_stage=1)),
+], ids=lambda v: v.encode() if hasattr(v, "encode") else "")  # fmt: skip
+def test_second_stages_round_their_sums(params, weight, fused):
+    """The second stage that stores float16: exactly the float32 one's sums (no atomics: the same in every
+    launch), rounded once, every element written."""
+    x, w, _bias, dy = [to_gpu(t) for t in gpu_args(params)]
+    def empty(shape, dtype=torch.float32):
+        t = torch.full(shape, -42.0, device="cuda", dtype=dtype)
+        return t.contiguous(memory_format=torch.channels_last) if t.dim() == 4 else t
+
+    for factory, config in ((conv2d_gw8_wgrad_kernel_factory, weight), (conv2d_gw8_bgrad_kernel_factory, fused)):
+        kernel = factory.make_kernel(params, config, get_device_attributes(0))
+        kernel.compile()
+        kernel.load(0)
+        single = factory is conv2d_gw8_wgrad_kernel_factory
+
+        def main_args(dw, db):
+            args = (dw, x, dy) if single else (torch.empty_like(x), dw, x, dy, w)
+            return args + ((db,) if params.has_bias else ())
+
+        dw, db = empty(params.weight_shape), torch.zeros(params.c, device="cuda")
+        kernel(*main_args(dw, db))
+        # by hand: the main kernel without a grad_bias, then the second stage, which stores that too
+        dw_half, db_half = empty(params.weight_shape, torch.float16), empty((params.c,))
+        spec, stream = kernel.kernel_spec, torch.cuda.current_stream().cuda_stream
+        workspace = torch.full((spec.workspace_bytes // 4,), float("nan"), device="cuda")
+        kernel.function.launch(spec.launch_params.grid, spec.launch_params.block, main_args(workspace, None), 0, stream)
+        second = [dw_half, workspace] + ([db_half] if params.has_bias else [] if single else [None])
+        lp = spec.epilogue_half_launch_params
+        kernel.epilogue_half_function.launch(lp.grid, lp.block, second, 0, stream)
+        torch.cuda.synchronize()
+        assert torch.equal(dw.half(), dw_half), kernel
+        if params.has_bias:  # the same sums of at most n * p * q float16 values, in another order
+            depth = params.n * params.p * params.q
+            assert torch.allclose(db, db_half, rtol=0, atol=depth * 2.0**-24 * float(dy.float().abs().sum((0, 2, 3)).max()))
+        kernel.unload()
+
+
 _F32_CASES = [
     # cells that do not fill the last wave, odd group counts, images side by side, a ragged batch
     (Conv2dGw8Params(n=5, c=24, h=9, w=11, padding=1, has_bias=True),
