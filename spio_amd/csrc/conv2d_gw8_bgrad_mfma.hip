@@ -201,12 +201,12 @@ static_assert(PF >= 2 && PF % 2 == 0 && WAVES <= 16, "bad configuration");
 
 constexpr long long X_IMAGE_BYTES = (long long)kH * kW * kC * 2;  // of x
 constexpr long long DX_IMAGE_BYTES = (long long)kH * kW * kC * kDstBytes;  // of dx
-constexpr long long D_IMAGE_BYTES = (long long)kP * kQ * kC * 2;  // of dy
+constexpr long long D_IMAGE_BYTES = (long long)kP * kQ * kC * kSrcBytes;  // of dy (SPIO_SRC_F32: fp32)
 static_assert(NB * DX_IMAGE_BYTES < (1ll << 31) && NB * D_IMAGE_BYTES < (1ll << 31),
               "an image block must stay below 2 GiB (32-bit buffer offsets)");
 constexpr int X_ROW_BYTES = kW * kC * 2;
 constexpr int DX_ROW_BYTES = kW * kC * kDstBytes;
-constexpr int D_ROW_BYTES = kQ * kC * 2;
+constexpr int D_ROW_BYTES = kQ * kC * kSrcBytes;
 constexpr unsigned OOB = 0x80000000u;  // offset of a lane without data: beyond every descriptor
 // Cache-policy operands of the buffer instructions: streamed (2) unless several channel blocks share the
 // lines, then loaded with the default policy so that the second block finds them in L2.  Streamed -> default
@@ -369,44 +369,55 @@ SPIO_KERNEL_NAME(spio_uint4* __restrict__ grad_input, float* __restrict__ grad_w
         }
         // dy cells, and the dx cells of the same (image, domain column, group): where dy and x have
         // the same size, the same offset
-        unsigned d_voff[LPTD], o_voff[LPTO];
-        int d_lds[LPTD], o_lds[LPTO];
+        int d_voff[LPTD][kSrcLoads], d_lds[LPTD][kSrcLoads];  // (SPIO_SRC_F32: d_lds in bytes)
+        unsigned o_voff[LPTO][kDstStores];
+        int o_lds[LPTO][kDstStores];
 #pragma unroll
         for (int l = 0; l < LPTD; ++l) {
-            const int cell = tid + THREADS * l;
-            d_voff[l] = OOB;
-            d_lds[l] = DDUMP;
-            if (cell < D_CELLS) {
-                const int g = cell % GB;
-                // whole rows: the cells are the real columns; column blocks: every staged column
-                const int q = kColBlocks ? q0 + (cell / GB) % WPI - PR : (cell / GB) % DW;  // domain column
-                const int img = kColBlocks ? 0 : cell / (GB * DW);
-                d_lds[l] = g * GSD + (kColBlocks ? cell / GB : img * WPI + q + PR);
-                const int qd = q - DOX;  // column of dy
-                if (qd >= 0 && qd < kQ && cb * GB + g < kGroups)
-                    d_voff[l] = (unsigned)(((img * kP * kQ + qd) * kGroups + cb * GB + g) * 16);
+#pragma unroll
+            for (int j = 0; j < kSrcLoads; ++j) {
+                const int cell = moved_unit(tid, j, kSrcLoads) + THREADS * l;
+                unsigned voff = OOB;
+                int unit = DDUMP;
+                if (cell < D_CELLS) {
+                    const int g = cell % GB;
+                    // whole rows: the cells are the real columns; column blocks: every staged column
+                    const int q = kColBlocks ? q0 + (cell / GB) % WPI - PR : (cell / GB) % DW;  // domain column
+                    const int img = kColBlocks ? 0 : cell / (GB * DW);
+                    unit = g * GSD + (kColBlocks ? cell / GB : img * WPI + q + PR);
+                    const int qd = q - DOX;  // column of dy
+                    if (qd >= 0 && qd < kQ && cb * GB + g < kGroups)
+                        voff = (unsigned)(((img * kP * kQ + qd) * kGroups + cb * GB + g) * (8 * kSrcBytes));
+                }
+                d_voff[l][j] = (int)(voff + (unsigned)half_bytes(tid, kSrcLoads, 16));
+                d_lds[l][j] = SPIO_SRC_F32 ? unit * 16 + half_bytes(tid, kSrcLoads, 8) : unit;
             }
         }
 #pragma unroll
         for (int l = 0; l < LPTO; ++l) {
-            const int cell = tid + THREADS * l;
-            o_voff[l] = OOB;
-            o_lds[l] = 0;
-            if (cell < O_CELLS) {
-                const int g = cell % GB;
-                const int q = (cell / GB) % BQ;
-                const int img = cell / (GB * BQ);
-                o_lds[l] = (img * WPI + q) * OSTRIDE + g * 16;
-                const int wx = q0 + q - XOX;  // column of dx
-                if (q0 + q < DW && wx >= 0 && wx < kW && cb * GB + g < kGroups)
-                    o_voff[l] = (unsigned)(((img * kH * kW + wx) * kGroups + cb * GB + g) * (8 * kDstBytes));
+#pragma unroll
+            for (int j = 0; j < kDstStores; ++j) {
+                const int cell = moved_unit(tid, j, kDstStores) + THREADS * l;
+                unsigned voff = OOB;
+                int from = 0;
+                if (cell < O_CELLS) {
+                    const int g = cell % GB;
+                    const int q = (cell / GB) % BQ;
+                    const int img = cell / (GB * BQ);
+                    from = (img * WPI + q) * OSTRIDE + g * 16;
+                    const int wx = q0 + q - XOX;  // column of dx
+                    if (q0 + q < DW && wx >= 0 && wx < kW && cb * GB + g < kGroups)
+                        voff = (unsigned)(((img * kH * kW + wx) * kGroups + cb * GB + g) * (8 * kDstBytes));
+                }
+                o_voff[l][j] = voff + (unsigned)half_bytes(tid, kDstStores, 16);
+                o_lds[l][j] = from + half_bytes(tid, kDstStores, 8);
             }
         }
 
         // Rows `t` of x (domain row p0-(R-1)+t) and of dy (p0-PB+t) for every cell of the thread.
         // Rows the block does not need, and domain rows outside the tensor, read through the empty
         // descriptor (zeros, no traffic).
-        auto load_rows = [&](spio_uint4(&xr)[LPTX], spio_uint4(&dr)[LPTD], int t) {
+        auto load_rows = [&](spio_uint4(&xr)[LPTX], spio_uint4(&dr)[LPTD][kSrcLoads], int t) {
             const int h = p0 - (kR - 1) + t;
             const rsrc_t rx = (h >= xrow_lo && h <= xrow_hi && h >= XOY && h < XOY + kH) ? rs_x : rs_none;
             const int sx = __builtin_amdgcn_readfirstlane(imin(imax(h - XOY, 0), kH - 1) * X_ROW_BYTES);
@@ -424,15 +435,31 @@ SPIO_KERNEL_NAME(spio_uint4* __restrict__ grad_input, float* __restrict__ grad_w
             const bool dhalo = pr < p0 || pr >= p0 + bh_eff;
 #pragma unroll
             for (int l = 0; l < LPTD; ++l) {
-                Pack16 v;
-                v.i = (SPIO_HALO_CACHED && dhalo) ? __builtin_amdgcn_raw_buffer_load_b128(rd, (int)d_voff[l], sd, 0)
-                                                  : __builtin_amdgcn_raw_buffer_load_b128(rd, (int)d_voff[l], sd, AUX_LD);
-                dr[l] = v.u;
+#pragma unroll
+                for (int j = 0; j < kSrcLoads; ++j) {
+                    Pack16 v;
+                    v.i = (SPIO_HALO_CACHED && dhalo) ? __builtin_amdgcn_raw_buffer_load_b128(rd, d_voff[l][j], sd, 0)
+                                                      : __builtin_amdgcn_raw_buffer_load_b128(rd, d_voff[l][j], sd, AUX_LD);
+                    dr[l][j] = v.u;
+                }
+            }
+        };
+        auto dy_to_ring = [&](const spio_uint4(&dr)[LPTD][kSrcLoads], int slot) {
+            spio_uint4* const row = dring + slot * DROW_UNITS;
+#pragma unroll
+            for (int l = 0; l < LPTD; ++l) {
+                if (!SPIO_SRC_F32) {
+                    row[d_lds[l][0]] = dr[l][0];
+                } else {
+#pragma unroll
+                    for (int j = 0; j < kSrcLoads; ++j)
+                        *reinterpret_cast<spio_uint2*>(reinterpret_cast<unsigned char*>(row) + d_lds[l][j]) = narrow(dr[l][j]);
+                }
             }
         };
 
         // ---- prologue: rows 0..PF-1 into registers ----
-        spio_uint4 xpre[PF][LPTX], dpre[PF][LPTD];
+        spio_uint4 xpre[PF][LPTX], dpre[PF][LPTD][kSrcLoads];
 #pragma unroll
         for (int t = 0; t < PF; ++t) load_rows(xpre[t], dpre[t], t);
         __builtin_amdgcn_sched_barrier(0);  // the first loads are on their way before anything waits
@@ -478,8 +505,7 @@ SPIO_KERNEL_NAME(spio_uint4* __restrict__ grad_input, float* __restrict__ grad_w
         block_sync();  // rings zeroed / previous image block finished
 #pragma unroll
         for (int l = 0; l < LPTX; ++l) xring[x_lds[l]] = xpre[0][l];
-#pragma unroll
-        for (int l = 0; l < LPTD; ++l) dring[d_lds[l]] = dpre[0][l];
+        dy_to_ring(dpre[0], 0);
         block_sync();
 
         spio_float4 dacc[TPW][NACC];  // data gradient: rotating row slots
@@ -506,19 +532,12 @@ SPIO_KERNEL_NAME(spio_uint4* __restrict__ grad_input, float* __restrict__ grad_w
 #pragma unroll
             for (int l = 0; l < LPTO; ++l) {
                 const unsigned char* row = ostage + obuf * OUT_ROW_BYTES;
-                if (SPIO_DST_F32) {
-                    const int half = lane & 1;
-                    auto store_half = [&](int voff, int from) {
-                        const spio_uint2 v = *reinterpret_cast<const spio_uint2*>(row + from + 8 * half);
-                        __builtin_amdgcn_raw_buffer_store_b128(widen(v), rs, (int)((unsigned)voff + 16 * half + row_off),
-                                                               0, AUX_ST);
-                    };
-                    store_half(quad_lane<0>((int)o_voff[l]), quad_lane<0>(o_lds[l]));
-                    store_half(quad_lane<1>((int)o_voff[l]), quad_lane<1>(o_lds[l]));
-                } else {
+#pragma unroll
+                for (int j = 0; j < kDstStores; ++j) {
                     Pack16 v;
-                    v.u = *reinterpret_cast<const spio_uint4*>(row + o_lds[l]);
-                    __builtin_amdgcn_raw_buffer_store_b128(v.i, rs, (int)(o_voff[l] + row_off), 0, AUX_ST);
+                    v.u = SPIO_DST_F32 ? widen(*reinterpret_cast<const spio_uint2*>(row + o_lds[l][j]))
+                                       : *reinterpret_cast<const spio_uint4*>(row + o_lds[l][j]);
+                    __builtin_amdgcn_raw_buffer_store_b128(v.i, rs, (int)(o_voff[l][j] + row_off), 0, AUX_ST);
                 }
             }
             store_group_end();
@@ -610,9 +629,7 @@ SPIO_KERNEL_NAME(spio_uint4* __restrict__ grad_input, float* __restrict__ grad_w
 #pragma unroll
                     for (int l = 0; l < LPTX; ++l)
                         xring[((sp + 1) & 1) * XROW_UNITS + x_lds[l]] = xpre[(uu + 1) % PF][l];
-                    const int dslot = (t + 1) % NRD;
-#pragma unroll
-                    for (int l = 0; l < LPTD; ++l) dring[dslot * DROW_UNITS + d_lds[l]] = dpre[(uu + 1) % PF][l];
+                    dy_to_ring(dpre[(uu + 1) % PF], (t + 1) % NRD);
                 }
 
                 // 5. multiply: weight gradient ...

@@ -141,11 +141,17 @@ static_assert(MV == 0 || SPIO_DB, "mover waves work on the other pair of buffers
 static_assert(LDS_UNITS * 16 <= 160 * 1024, "LDS overflow");
 static_assert(OUT_ROW_BYTES % 16 == 0, "output rows are read in 16-byte units");
 
-constexpr long long SRC_IMAGE_BYTES = (long long)SH * SW * kC * 2;
+constexpr long long SRC_IMAGE_BYTES = (long long)SH * SW * kC * kSrcBytes;
 constexpr long long DST_IMAGE_BYTES = (long long)DH * DW * kC * kDstBytes;
 static_assert(NB * SRC_IMAGE_BYTES < (1ll << 30) && NB * DST_IMAGE_BYTES < (1ll << 30) &&
-                  (long long)(LPT > SPT ? LPT : SPT) * CELL_STEP * (kDstBytes / 2) < (1ll << 30),
+                  (long long)(LPT > SPT ? LPT : SPT) * CELL_STEP * (SPIO_SRC_F32 || SPIO_DST_F32 ? 2 : 1) < (1ll << 30),
               "an image block must stay far below 2 GiB (32-bit buffer offsets)");
+static_assert(!(SPIO_W_F32 && SPIO_IGRAD), "the data gradient reads fp16 filters");
+// Register sets for blocks in flight: two, or one where two of fp32 blocks take too many registers.
+#ifndef SPIO_SETS
+#define SPIO_SETS 2
+#endif
+constexpr int SETS = SPIO_SETS;
 constexpr unsigned OOB = 0x80000000u;    // offset of a lane without data: beyond every descriptor
 // Cache-policy operands of the buffer instructions: streamed (2) unless several channel blocks share the
 // lines, then loaded with the default policy so that the second block finds them in L2 (128n 1392c 9x9
@@ -193,6 +199,7 @@ constexpr int fragment_set(int t, int first) {
 
 typedef __attribute__((address_space(3))) spio_uint4* lds_u4p;
 typedef __attribute__((address_space(3))) unsigned char* lds_bytep;
+typedef __attribute__((address_space(3))) spio_uint2* lds_u2p;
 
 // f(Int<I>{}) for I = BEGIN .. END-1: a loop whose index is a compile-time constant in its body by
 // construction (what is multiplied, read and stored at a step is decided per step; a loop left
@@ -222,7 +229,7 @@ SPIO_DEVICE int first_block() { return (tile_index() / GBLKS) * ITERS; }
 //      block is multiplied) -> fragments.  Every multiplying thread takes a share; every
 //      global byte is fetched once per workgroup, coalesced, as it lies in memory
 //      ([group][k or jj][r][s][8 ch]). ----
-SPIO_DEVICE void request_filters(spio_uint4 (&wraw)[WLPT], const spio_half* __restrict__ weights, int tid) {
+SPIO_DEVICE void request_filters(spio_uint4 (&wraw)[WLPT][kFilterLoads], const spio_half* __restrict__ weights, int tid) {
     const int cb = channel_block();
 #pragma unroll
     for (int l = 0; l < WLPT; ++l) {
@@ -230,16 +237,25 @@ SPIO_DEVICE void request_filters(spio_uint4 (&wraw)[WLPT], const spio_half* __re
         const int g = i / (8 * kR * kS);
         const int rem = i % (8 * kR * kS);
         const int gs = cb * GB + g < kGroups ? cb * GB + g : 0;
-        wraw[l] = reinterpret_cast<const spio_uint4*>(weights)[(long long)gs * (8 * kR * kS) + rem];
+        load_filter_unit(wraw[l], weights, (long long)gs * (8 * kR * kS) + rem);
     }
 }
-SPIO_DEVICE void stage_filters(const spio_uint4 (&wraw)[WLPT], lds_u4p lds, int tid) {
+SPIO_DEVICE void stage_filters(const spio_uint4 (&wraw)[WLPT][kFilterLoads], lds_u4p lds, int tid) {
     const lds_u4p wlds = lds + OUT_BASE_UNITS;
 #pragma unroll
     for (int l = 0; l < WLPT; ++l) {
         const int i = tid + FTHREADS * l;
-        if (i < FILTER_UNITS) wlds[i] = wraw[l];
+        if (i < FILTER_UNITS) wlds[i] = filter_unit(wraw[l]);
     }
+}
+// The rounded filters, by the first workgroup of every channel block, from the staged copy.  A thread stores
+// what it staged itself.
+SPIO_DEVICE void keep_filters(spio_uint4* __restrict__ kept_weights, lds_u4p lds, int tid) {
+    if (!(SPIO_KEEP && SPIO_W_F32) || first_block() != 0) return;
+    const int first = channel_block() * GB;
+    for (int i = tid; i < FILTER_UNITS; i += FTHREADS)
+        if (first + i / (8 * kR * kS) < kGroups)
+            kept_weights[(long long)first * (8 * kR * kS) + i] = lds[OUT_BASE_UNITS + i];
 }
 // The input buffers start as zeros: the halo columns and the slack stay zero from here on, later
 // blocks rewrite the real cells only.
@@ -314,40 +330,58 @@ SPIO_DEVICE void load_filter_fragments(spio_half8 (&wfrag)[NS][KB], lds_u4p lds,
 struct BlockMover {
     const spio_uint4* src;
     spio_uint4* dst;
-    unsigned voff;     // byte offset of the thread's cell 0 inside an image block (source and
-                       // destination blocks are laid out alike); OOB: no such group
-    int in_lds[LPT];   // 16-byte unit inside an input buffer; cells without one go to `dump`
-    int out_lds[SPT];  // byte offset inside an output buffer
+    spio_uint4* kept_src;  // SPIO_KEEP: the source rounded to fp16
+    // Where a unit is moved by two accesses (fp32) a thread takes part in two units, and moves a half of each.
+    unsigned in_voff[kSrcLoads];      // byte offset of the thread's cell 0 inside an image block (source and
+    unsigned out_voff[kDstStores];    // destination blocks are laid out alike); OOB: no such group
+    int in_lds[LPT][kSrcLoads];       // byte inside an input buffer; cells without one go to `dump`
+    int out_lds[SPT][kDstStores];     // byte inside an output buffer
     int dump;
 
     // what the loads need (so that the first block can be requested before the rest is worked out)
-    SPIO_DEVICE void init_global(spio_uint4* dst_, const spio_uint4* src_, int mtid) {
+    SPIO_DEVICE void init_global(spio_uint4* dst_, const spio_uint4* src_, spio_uint4* kept_src_, int mtid) {
         src = src_;
         dst = dst_;
-        const int cb = channel_block();
-        const int g = mtid % GB;
-        const int pix0 = mtid / GB;
-        voff = cb * GB + g < kGroups ? (unsigned)((pix0 * kGroups + cb * GB + g) * 16) : OOB;
+        kept_src = kept_src_;
+        auto offset = [&](int accesses, int j, int unit_bytes) {
+            const int cell = moved_unit(mtid, j, accesses);
+            const int g = channel_block() * GB + cell % GB;
+            return g < kGroups ? (unsigned)((cell / GB * kGroups + g) * unit_bytes + half_bytes(mtid, accesses, 16)) : OOB;
+        };
+#pragma unroll
+        for (int j = 0; j < kSrcLoads; ++j) in_voff[j] = offset(kSrcLoads, j, 8 * kSrcBytes);
+#pragma unroll
+        for (int j = 0; j < kDstStores; ++j) out_voff[j] = offset(kDstStores, j, 8 * kDstBytes);
     }
     SPIO_DEVICE void init_lds(int mtid) {
-        const int g = mtid % GB;
-        const int pix0 = mtid / GB;
-        dump = DUMP_UNIT + ((mtid & 63) >> 1);
+        dump = (DUMP_UNIT + ((mtid & 63) >> 1)) * 16 + half_bytes(mtid, kSrcLoads, 8);
 #pragma unroll
         for (int l = 0; l < LPT; ++l) {
-            const int pix = pix0 + PIXEL_STEP * l;
-            const int img = pix / (SH * SW);
-            const int row = (pix / SW) % SH;
-            const int f = pix % SW + EPX;  // column in the padded image (negative padding crops)
-            in_lds[l] = (img < NB && f >= 0 && f < WPI) ? row * ROW_UNITS + g * GS + img * WPI + f : -1;
+#pragma unroll
+            for (int j = 0; j < kSrcLoads; ++j) {
+                const int cell = moved_unit(mtid, j, kSrcLoads);
+                const int pix = cell / GB + PIXEL_STEP * l;
+                const int img = pix / (SH * SW);
+                const int row = (pix / SW) % SH;
+                const int f = pix % SW + EPX;  // column in the padded image (negative padding crops)
+                in_lds[l][j] = (img < NB && f >= 0 && f < WPI)
+                                   ? (row * ROW_UNITS + cell % GB * GS + img * WPI + f) * 16 + half_bytes(mtid, kSrcLoads, 8)
+                                   : -1;
+            }
         }
 #pragma unroll
         for (int s = 0; s < SPT; ++s) {
-            const int pix = pix0 + PIXEL_STEP * s;
-            const int img = pix / (DH * DW);
-            const int row = (pix / DW) % DH;
-            const int q = pix % DW;
-            out_lds[s] = img < NB ? row * OUT_ROW_BYTES + (img * WPI + q) * OSTRIDE + g * 16 : 0;
+#pragma unroll
+            for (int j = 0; j < kDstStores; ++j) {
+                const int cell = moved_unit(mtid, j, kDstStores);
+                const int pix = cell / GB + PIXEL_STEP * s;
+                const int img = pix / (DH * DW);
+                const int row = (pix / DW) % DH;
+                const int q = pix % DW;
+                out_lds[s][j] = img < NB ? row * OUT_ROW_BYTES + (img * WPI + q) * OSTRIDE + cell % GB * 16 +
+                                               half_bytes(mtid, kDstStores, 8)
+                                         : 0;
+            }
         }
     }
     // Image block `blk` of src / dst as a buffer descriptor.  Blocks before the workgroup's first
@@ -361,46 +395,51 @@ struct BlockMover {
         return make_rsrc(reinterpret_cast<const unsigned char*>(base) + (any ? n0 * image_bytes : 0),
                          any ? (int)(images * image_bytes) : 0);
     }
-    SPIO_DEVICE void load(spio_uint4 (&regs)[LPT], int blk, bool enabled) const {
+    SPIO_DEVICE void load(spio_uint4 (&regs)[LPT][kSrcLoads], int blk, bool enabled) const {
         const rsrc_t rs = block_rsrc(src, SRC_IMAGE_BYTES, blk, enabled);
 #pragma unroll
         for (int l = 0; l < LPT; ++l) {
-            Pack16 v;
-            v.i = __builtin_amdgcn_raw_buffer_load_b128(rs, (int)(voff + (unsigned)(CELL_STEP * l)), 0, AUX_LD);
-            regs[l] = v.u;
+#pragma unroll
+            for (int j = 0; j < kSrcLoads; ++j) {
+                Pack16 v;
+                v.i = __builtin_amdgcn_raw_buffer_load_b128(rs, (int)(in_voff[j] + (unsigned)(CELL_STEP * (kSrcBytes / 2) * l)),
+                                                            0, AUX_LD);
+                regs[l][j] = v.u;
+            }
         }
     }
-    // registers -> input buffer at 16-byte unit `base` (the dump cells lie behind the buffers:
-    // not offset by the buffer)
-    SPIO_DEVICE void to_lds(const spio_uint4 (&regs)[LPT], lds_u4p lds, int base) const {
+    // registers -> input buffer at byte `base` (the dump cells lie behind the buffers: not offset by the
+    // buffer); fp32 blocks are rounded, and block `blk` stored as fp16
+    SPIO_DEVICE void to_lds(const spio_uint4 (&regs)[LPT][kSrcLoads], lds_u4p lds, int base, int blk, bool enabled) const {
+        const rsrc_t rs = block_rsrc(kept_src, SRC_IMAGE_BYTES / 2, blk, SPIO_KEEP && enabled);
 #pragma unroll
-        for (int l = 0; l < LPT; ++l) lds[in_lds[l] < 0 ? dump : base + in_lds[l]] = regs[l];
+        for (int l = 0; l < LPT; ++l) {
+#pragma unroll
+            for (int j = 0; j < kSrcLoads; ++j) {
+                const lds_bytep to = (lds_bytep)lds + (in_lds[l][j] < 0 ? dump : base + in_lds[l][j]);
+                if (SPIO_SRC_F32) {
+                    const spio_uint2 v = narrow(regs[l][j]);
+                    *(lds_u2p)to = v;
+                    if (SPIO_KEEP)  // (half of OOB is beyond the descriptor too)
+                        __builtin_amdgcn_raw_buffer_store_b64(v, rs, (int)(in_voff[j] / 2 + (unsigned)(CELL_STEP * l)), 0, AUX_ST);
+                } else {
+                    *(lds_u4p)to = regs[l][j];
+                }
+            }
+        }
     }
     // (Constant scalar-offset operand: the form for which the compiler keeps the data registers
     //  of a 16-byte buffer store untouched for the wait states the hardware needs.)
     SPIO_DEVICE void store(int blk, bool enabled, lds_bytep out) const {
         const rsrc_t rs = block_rsrc(dst, DST_IMAGE_BYTES, blk, enabled);
-        if (SPIO_DST_F32) {
-            // the thread's offset in a block of twice the bytes; OOB stays beyond every descriptor
-            const int half = thread_id() & 1;
-            const int wide = (int)(voff == OOB ? OOB : 2 * voff);
-            auto store_half = [&](int base, int from, int s) {
-                typedef __attribute__((address_space(3))) spio_uint2* lds_u2p;
-                __builtin_amdgcn_raw_buffer_store_b128(widen(*(lds_u2p)(out + from + 8 * half)), rs,
-                                                       (int)((unsigned)base + 16 * half + (unsigned)(2 * CELL_STEP * s)),
-                                                       0, AUX_ST);
-            };
 #pragma unroll
-            for (int s = 0; s < SPT; ++s) {
-                store_half(quad_lane<0>(wide), quad_lane<0>(out_lds[s]), s);
-                store_half(quad_lane<1>(wide), quad_lane<1>(out_lds[s]), s);
-            }
-        } else {
+        for (int s = 0; s < SPT; ++s) {
 #pragma unroll
-            for (int s = 0; s < SPT; ++s) {
+            for (int j = 0; j < kDstStores; ++j) {
                 Pack16 v;
-                v.u = *(lds_u4p)(out + out_lds[s]);
-                __builtin_amdgcn_raw_buffer_store_b128(v.i, rs, (int)(voff + (unsigned)(CELL_STEP * s)), 0, AUX_ST);
+                v.u = SPIO_DST_F32 ? widen(*(lds_u2p)(out + out_lds[s][j])) : *(lds_u4p)(out + out_lds[s][j]);
+                __builtin_amdgcn_raw_buffer_store_b128(v.i, rs, (int)(out_voff[j] + (unsigned)(CELL_STEP * (kDstBytes / 2) * s)),
+                                                       0, AUX_ST);
             }
         }
         // (not in the mover waves: a scheduling fence after every block's stores costs them 8 % at
@@ -519,7 +558,6 @@ SPIO_DEVICE void multiply_block(lds_u4p in_cur, lds_bytep out_cur, const spio_ha
                     Pack8 o;
 #pragma unroll
                     for (int e = 0; e < 4; ++e) o.h[e] = (spio_half)acc[i][a][e];
-                    typedef __attribute__((address_space(3))) spio_uint2* lds_u2p;
                     *(lds_u2p)(out_cur + ll.ostage_lane[j] + (p * OUT_ROW_BYTES + 16 * i * OSTRIDE)) = o.u;
                 }
 #pragma unroll
@@ -546,7 +584,7 @@ SPIO_DEVICE void load_bias(float (&bias_reg)[4], const float* __restrict__ bias,
 template <int WS>
 SPIO_DEVICE void run(spio_uint4* __restrict__ dst, const spio_uint4* __restrict__ src,
                      const spio_half* __restrict__ weights, const float* __restrict__ bias,
-                     lds_u4p lds, int tid, int wg) {
+                     spio_uint4* __restrict__ kept_src, spio_uint4* __restrict__ kept_weights, lds_u4p lds, int tid, int wg) {
     const int lane = tid & 63;
     const lds_u4p inbuf = lds;
     const lds_bytep outbuf = (lds_bytep)(lds + OUT_BASE_UNITS);
@@ -554,23 +592,24 @@ SPIO_DEVICE void run(spio_uint4* __restrict__ dst, const spio_uint4* __restrict_
 
     // the filters first: everything up to the first multiplication waits for them (global memory
     // -> LDS -> barrier -> fragments), the image blocks are not needed before
-    spio_uint4 wraw[WLPT];
+    spio_uint4 wraw[WLPT][kFilterLoads];
     request_filters(wraw, weights, tid);
     __builtin_amdgcn_sched_barrier(0);
 
     BlockMover mv;
-    mv.init_global(dst, src, tid);
+    mv.init_global(dst, src, kept_src, tid);
     // Two register sets hold the blocks in flight: at any time the loads of two image blocks per
     // workgroup are outstanding (one block per CU does not cover the memory latency: each phase
     // would wait for its block, and the device would run at a fraction of its bandwidth).
-    spio_uint4 pre0[LPT], pre1[LPT];
+    spio_uint4 pre0[LPT][kSrcLoads], pre1[LPT][kSrcLoads];
     mv.load(pre0, first_blk, true);
-    mv.load(pre1, first_blk + 1, ITERS > 1);
+    if (SETS > 1) mv.load(pre1, first_blk + 1, ITERS > 1);
     __builtin_amdgcn_sched_barrier(0);  // both requests leave before anything waits
     mv.init_lds(tid);
 
     clear_input_buffers(lds, tid);  // while they travel
     stage_filters(wraw, lds, tid);
+    keep_filters(kept_weights, lds, tid);
     block_sync();
     spio_half8 wfrag[NS][KB];
     load_filter_fragments<WS>(wfrag, lds, wg, lane);
@@ -581,13 +620,14 @@ SPIO_DEVICE void run(spio_uint4* __restrict__ dst, const spio_uint4* __restrict_
 
     // block 0 into input buffer 0, block 2 on its way.  The barrier also keeps the first output
     // rows from being staged over filters that a slower wave is still reading.
-    mv.to_lds(pre0, inbuf, 0);
-    mv.load(pre0, first_blk + 2, ITERS > 2);
+    mv.to_lds(pre0, inbuf, 0, first_blk, true);
+    mv.load(pre0, first_blk + SETS, ITERS > SETS);
     block_sync();
 
     // One phase: block `it`.  `pre` is the register set that holds block it+1 when the phase
-    // starts (block it+2 is in flight into the other set) and receives block it+3 at its end.
-    auto phase = [&](int it, spio_uint4(&pre)[LPT]) {
+    // starts (block it+2 is in flight into the other set) and receives block it+3 at its end.  With
+    // one register set that is block it+2.
+    auto phase = [&](int it, spio_uint4(&pre)[LPT][kSrcLoads]) {
         const int cur = SPIO_DB ? (it & 1) : 0;
         const int nxt = SPIO_DB ? (cur ^ 1) : 0;
         // (a) the previous block's output out of the other output buffer
@@ -602,14 +642,14 @@ SPIO_DEVICE void run(spio_uint4* __restrict__ dst, const spio_uint4* __restrict_
             mv.store(first_blk + it, true, outbuf);
         }
         // (c) the next block, requested two phases ago, into the other input buffer
-        mv.to_lds(pre, inbuf, nxt * IN_UNITS);
+        mv.to_lds(pre, inbuf, nxt * IN_UNITS * 16, first_blk + it + 1, it + 1 < ITERS);
         // (d) the block three ahead on its way: it has two phases to arrive
-        mv.load(pre, first_blk + it + 3, it + 3 < ITERS);
+        mv.load(pre, first_blk + it + 1 + SETS, it + 1 + SETS < ITERS);
         block_sync();
     };
 #pragma nounroll
     for (int it = 0; it < ITERS; it += 2) {
-        phase(it, pre1);
+        phase(it, SETS > 1 ? pre1 : pre0);
         if (it + 1 < ITERS) phase(it + 1, pre0);
     }
     // the last block's output
@@ -619,16 +659,17 @@ SPIO_DEVICE void run(spio_uint4* __restrict__ dst, const spio_uint4* __restrict_
 // ---- SPIO_MV > 0: the two roles.  Both pass the same barriers: two in the set-up (filters
 //      staged; block 0 staged and filter fragments read), one per image block. ----
 template <int WS>
-SPIO_DEVICE void multiplier_role(const spio_half* __restrict__ weights, const float* __restrict__ bias, lds_u4p lds,
-                                 int tid, int wg) {
+SPIO_DEVICE void multiplier_role(const spio_half* __restrict__ weights, const float* __restrict__ bias,
+                                 spio_uint4* __restrict__ kept_weights, lds_u4p lds, int tid, int wg) {
     const int lane = tid & 63;
     const lds_u4p inbuf = lds;
     const lds_bytep outbuf = (lds_bytep)(lds + OUT_BASE_UNITS);
-    spio_uint4 wraw[WLPT];
+    spio_uint4 wraw[WLPT][kFilterLoads];
     request_filters(wraw, weights, tid);
     __builtin_amdgcn_sched_barrier(0);
     clear_input_buffers(lds, tid);
     stage_filters(wraw, lds, tid);
+    keep_filters(kept_weights, lds, tid);
     block_sync();
     spio_half8 wfrag[NS][KB];
     load_filter_fragments<WS>(wfrag, lds, wg, lane);
@@ -645,40 +686,41 @@ SPIO_DEVICE void multiplier_role(const spio_half* __restrict__ weights, const fl
     }
 }
 
-SPIO_DEVICE void mover_role(spio_uint4* __restrict__ dst, const spio_uint4* __restrict__ src, lds_u4p lds, int tid) {
+SPIO_DEVICE void mover_role(spio_uint4* __restrict__ dst, const spio_uint4* __restrict__ src,
+                            spio_uint4* __restrict__ kept_src, lds_u4p lds, int tid) {
     const lds_u4p inbuf = lds;
     const lds_bytep outbuf = (lds_bytep)(lds + OUT_BASE_UNITS);
     const int first_blk = first_block();
     BlockMover mv;
-    mv.init_global(dst, src, tid - 64 * WAVES);
+    mv.init_global(dst, src, kept_src, tid - 64 * WAVES);
     // Three blocks are requested before the first is multiplied (two here, the third once the
     // first is in LDS).  Every workgroup of the device starts at the same time, so the set-up is
     // a stretch in which the memory system only reads; holding the later blocks back until the
     // first has arrived starts the multiplications earlier, but the phases then ask for more
     // bandwidth than there is and the kernel is slower (measured: 16.5 against 15.0 us, 7x7 on
     // 14x14, N=256, C=256).
-    spio_uint4 pre0[LPT], pre1[LPT];
+    spio_uint4 pre0[LPT][kSrcLoads], pre1[LPT][kSrcLoads];
     mv.load(pre0, first_blk, true);
-    mv.load(pre1, first_blk + 1, ITERS > 1);
+    if (SETS > 1) mv.load(pre1, first_blk + 1, ITERS > 1);
     __builtin_amdgcn_sched_barrier(0);
     mv.init_lds(tid - 64 * WAVES);
     clear_input_buffers(lds, tid);
     block_sync();
-    mv.to_lds(pre0, inbuf, 0);
-    mv.load(pre0, first_blk + 2, ITERS > 2);
+    mv.to_lds(pre0, inbuf, 0, first_blk, true);
+    mv.load(pre0, first_blk + SETS, ITERS > SETS);
     block_sync();
     // while block `it` is multiplied: the output of block it-1 leaves, block it+1 (in `pre`,
     // requested two phases ago) enters the other input buffer, block it+3 is requested
-    auto phase = [&](int it, spio_uint4(&pre)[LPT]) {
+    auto phase = [&](int it, spio_uint4(&pre)[LPT][kSrcLoads]) {
         const int nxt = (it & 1) ^ 1;
         mv.store(first_blk + it - 1, it > 0, outbuf + nxt * OUT_BYTES);
-        mv.to_lds(pre, inbuf, nxt * IN_UNITS);
-        mv.load(pre, first_blk + it + 3, it + 3 < ITERS);
+        mv.to_lds(pre, inbuf, nxt * IN_UNITS * 16, first_blk + it + 1, it + 1 < ITERS);
+        mv.load(pre, first_blk + it + 1 + SETS, it + 1 + SETS < ITERS);
         block_sync();
     };
 #pragma nounroll
     for (int it = 0; it < ITERS; it += 2) {
-        phase(it, pre1);
+        phase(it, SETS > 1 ? pre1 : pre0);
         if (it + 1 < ITERS) phase(it + 1, pre0);
     }
     mv.store(first_blk + ITERS - 1, true, outbuf + ((ITERS - 1) & 1) * OUT_BYTES);
@@ -686,19 +728,26 @@ SPIO_DEVICE void mover_role(spio_uint4* __restrict__ dst, const spio_uint4* __re
 
 template <int WS>
 SPIO_DEVICE void dispatch(spio_uint4* __restrict__ dst, const spio_uint4* __restrict__ src,
-                          const spio_half* __restrict__ weights, const float* __restrict__ bias, lds_u4p lds,
-                          int tid, int wg) {
+                          const spio_half* __restrict__ weights, const float* __restrict__ bias,
+                          spio_uint4* __restrict__ kept_src, spio_uint4* __restrict__ kept_weights, lds_u4p lds, int tid, int wg) {
     if (MV == 0)
-        run<WS>(dst, src, weights, bias, lds, tid, wg);
+        run<WS>(dst, src, weights, bias, kept_src, kept_weights, lds, tid, wg);
     else
-        multiplier_role<WS>(weights, bias, lds, tid, wg);
+        multiplier_role<WS>(weights, bias, kept_weights, lds, tid, wg);
 }
 
 }  // namespace
 
 extern "C" __global__ void SPIO_LAUNCH_BOUNDS(THREADS)
 SPIO_KERNEL_NAME(spio_uint4* __restrict__ dst, const spio_uint4* __restrict__ src,
-                 const spio_half* __restrict__ weights, const float* __restrict__ bias) {
+                 const spio_half* __restrict__ weights, const float* __restrict__ bias
+#if SPIO_KEEP
+                 , spio_uint4* __restrict__ kept_src, spio_uint4* __restrict__ kept_weights
+#endif
+) {
+#if !SPIO_KEEP
+    spio_uint4 *const kept_src = nullptr, *const kept_weights = nullptr;
+#endif
     // One LDS block: the input buffer(s), the dump cell, the output buffer(s).  The output region
     // first holds the filters of the workgroup's groups.
     __shared__ spio_uint4 lds_block[LDS_UNITS];
@@ -707,18 +756,18 @@ SPIO_KERNEL_NAME(spio_uint4* __restrict__ dst, const spio_uint4* __restrict__ sr
     // the wave index as a scalar: whatever depends on it alone stays in scalar registers
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     if (MV > 0 && wave >= WAVES) {
-        mover_role(dst, src, lds, tid);
+        mover_role(dst, src, kept_src, lds, tid);
         return;
     }
     const int wg = wave % GB;  // group within the workgroup
     const int ws = wave / GB;  // which share of the accumulators
     if (TS == 1 || ws == 0) {
-        dispatch<0>(dst, src, weights, bias, lds, tid, wg);
+        dispatch<0>(dst, src, weights, bias, kept_src, kept_weights, lds, tid, wg);
     } else if (TS == 2 || ws == 1) {
-        dispatch<(TS > 1 ? 1 : 0)>(dst, src, weights, bias, lds, tid, wg);
+        dispatch<(TS > 1 ? 1 : 0)>(dst, src, weights, bias, kept_src, kept_weights, lds, tid, wg);
     } else if (TS == 3 || ws == 2) {
-        dispatch<(TS > 2 ? 2 : 0)>(dst, src, weights, bias, lds, tid, wg);
+        dispatch<(TS > 2 ? 2 : 0)>(dst, src, weights, bias, kept_src, kept_weights, lds, tid, wg);
     } else {
-        dispatch<(TS > 3 ? 3 : 0)>(dst, src, weights, bias, lds, tid, wg);
+        dispatch<(TS > 3 ? 3 : 0)>(dst, src, weights, bias, kept_src, kept_weights, lds, tid, wg);
     }
 }

@@ -164,10 +164,14 @@ constexpr int LDS_UNITS = STREAM_UNITS > FILTER_UNITS ? STREAM_UNITS : FILTER_UN
 static_assert(LDS_UNITS * 16 <= 160 * 1024, "LDS overflow");
 
 // Byte extents of the NB-image block a workgroup addresses through one buffer descriptor.
-constexpr long long SRC_IMAGE_BYTES = (long long)SH * SW * kC * 2;
+constexpr long long SRC_IMAGE_BYTES = (long long)SH * SW * kC * kSrcBytes;
 constexpr long long DST_IMAGE_BYTES = (long long)DH * DW * kC * kDstBytes;
 static_assert(NB * SRC_IMAGE_BYTES < (1ll << 31) && NB * DST_IMAGE_BYTES < (1ll << 31),
               "an image block must stay below 2 GiB (32-bit buffer offsets)");
+static_assert(!SPIO_KEEP || !SPIO_SRC_F32 ||
+                  (NB * SRC_IMAGE_BYTES < (1ll << 30) && EPY >= 0 && EPY < kR && EPX >= 0 && EPX < kS),
+              "the fp16 copy: offsets are halved, and every source pixel has to be staged by the block that owns it");
+static_assert(!(SPIO_W_F32 && SPIO_IGRAD), "the data gradient reads fp16 filters");
 constexpr unsigned OOB = 0x80000000u;  // offset of a lane without data: beyond every descriptor
 
 constexpr int pmod(int a, int m) { return ((a % m) + m) % m; }
@@ -213,11 +217,14 @@ SPIO_DEVICE rsrc_t make_rsrc(const void* base, int bytes) {
 typedef __attribute__((address_space(3))) spio_uint4* lds_u4p;
 typedef __attribute__((address_space(3))) unsigned char* lds_bytep;
 
+typedef __attribute__((address_space(3))) spio_uint2* lds_u2p;
+
 // One tile: ROWS output rows starting at row p0 of the NB images from n0 on, channel block cb.
+// kept_src, kept_weights: SPIO_KEEP.
 template <int ROWS>
 SPIO_DEVICE void conv_rows(spio_uint4* __restrict__ dst, const spio_uint4* __restrict__ src,
                            const spio_half* __restrict__ weights, const float* __restrict__ bias,
-                           const lds_u4p ring, const int p0, const int q0, const int n0, const int cb) {
+                           spio_uint4* __restrict__ kept_src, spio_uint4* __restrict__ kept_weights, const lds_u4p ring, const int p0, const int q0, const int n0, const int cb) {
     constexpr int STEPS = ROWS + kR - 1;
     const lds_bytep ostage = (lds_bytep)(ring + NR * RING_ROW_UNITS);
 
@@ -245,29 +252,34 @@ SPIO_DEVICE void conv_rows(spio_uint4* __restrict__ dst, const spio_uint4* __res
     // Every thread issues the same loads on every step.  Cells that hold no source data (halo
     // columns, missing groups) carry the out-of-range offset: the load returns zeros, which is
     // what the halo must hold.  Threads without a cell write to the row's dump cell.
-    unsigned in_voff[LPT];  // byte offset inside the image block; row term excluded
-    int in_lds[LPT];        // 16-byte unit inside a ring row
+    int in_voff[LPT][kSrcLoads];  // byte offset inside the image block; row term excluded
+    int in_lds[LPT][kSrcLoads];   // 16-byte unit inside a ring row (SPIO_SRC_F32: byte)
 #pragma unroll
     for (int l = 0; l < LPT; ++l) {
-        const int cell = tid + THREADS * l;
-        in_voff[l] = OOB;
-        in_lds[l] = DUMP_UNIT;
-        if (cell < IN_CELLS) {
-            const int g = cell % GB;
-            const int f = cell / GB;
-            const int img = f / WPI;
-            const int col = q0 + f % WPI - EPX;
-            in_lds[l] = g * GS + f;
-            if (col >= 0 && col < SW && cb * GB + g < kGroups)
-                in_voff[l] = (unsigned)(((img * SH * SW + col) * kGroups + cb * GB + g) * 16);
+#pragma unroll
+        for (int j = 0; j < kSrcLoads; ++j) {
+            const int cell = moved_unit(tid, j, kSrcLoads) + THREADS * l;
+            unsigned voff = OOB;
+            int unit = DUMP_UNIT;
+            if (cell < IN_CELLS) {
+                const int g = cell % GB;
+                const int f = cell / GB;
+                const int img = f / WPI;
+                const int col = q0 + f % WPI - EPX;
+                unit = g * GS + f;
+                if (col >= 0 && col < SW && cb * GB + g < kGroups)
+                    voff = (unsigned)(((img * SH * SW + col) * kGroups + cb * GB + g) * (8 * kSrcBytes));
+            }
+            in_voff[l][j] = (int)(voff + (unsigned)half_bytes(tid, kSrcLoads, 16));
+            in_lds[l][j] = SPIO_SRC_F32 ? unit * 16 + half_bytes(tid, kSrcLoads, 8) : unit;
         }
     }
-    constexpr int SRC_ROW_BYTES = SW * kC * 2;
+    constexpr int SRC_ROW_BYTES = SW * kC * kSrcBytes;
     constexpr int DST_ROW_BYTES = DW * kC * kDstBytes;
 
     // Source row `t` of this workgroup (image row p0 + t - EPY) for every cell of the thread.
     // Rows outside the image read through the empty descriptor: zeros, the vertical padding.
-    auto load_row = [&](spio_uint4(&regs)[LPT], int t) {
+    auto load_row = [&](spio_uint4(&regs)[LPT][kSrcLoads], int t) {
         const int h = p0 + t - EPY;
         const bool inside = h >= 0 && h < SH;
         const rsrc_t rs = inside ? rs_src : rs_src_none;
@@ -277,10 +289,39 @@ SPIO_DEVICE void conv_rows(spio_uint4* __restrict__ dst, const spio_uint4* __res
         const bool halo = t < kR - 1 || t >= ROWS;
 #pragma unroll
         for (int l = 0; l < LPT; ++l) {
-            Pack16 v;
-            v.i = halo ? __builtin_amdgcn_raw_buffer_load_b128(rs, (int)in_voff[l], soff, AUX_HALO)
-                       : __builtin_amdgcn_raw_buffer_load_b128(rs, (int)in_voff[l], soff, AUX_LD);
-            regs[l] = v.u;
+#pragma unroll
+            for (int j = 0; j < kSrcLoads; ++j) {
+                Pack16 v;
+                v.i = halo ? __builtin_amdgcn_raw_buffer_load_b128(rs, in_voff[l][j], soff, AUX_HALO)
+                           : __builtin_amdgcn_raw_buffer_load_b128(rs, in_voff[l][j], soff, AUX_LD);
+                regs[l][j] = v.u;
+            }
+        }
+    };
+    // A loaded row into a ring row; fp32 rows are rounded, and the ones this block owns stored as fp16:
+    // rows p0 .. p0+ROWS-1, and what follows the last block of an image.
+    const rsrc_t rs_kept = make_rsrc(reinterpret_cast<const unsigned char*>(kept_src) + (SPIO_KEEP ? n0 * SRC_IMAGE_BYTES / 2 : 0),
+                                     (int)(SPIO_KEEP ? images * (SRC_IMAGE_BYTES / 2) : 0));
+    auto row_to_ring = [&](const spio_uint4(&regs)[LPT][kSrcLoads], int t) {
+        const lds_u4p row = ring + (t % NR) * RING_ROW_UNITS;
+        if (!SPIO_SRC_F32) {
+#pragma unroll
+            for (int l = 0; l < LPT; ++l) row[in_lds[l][0]] = regs[l][0];
+            return;
+        }
+        const int h = p0 + t - EPY;
+        const bool owned = h < SH && (h < p0 + ROWS || p0 + ROWS >= DH);
+        const rsrc_t rs = owned ? rs_kept : rs_src_none;
+        const int row_off = imin(imax(h, 0), SH - 1) * (SRC_ROW_BYTES / 2);
+#pragma unroll
+        for (int l = 0; l < LPT; ++l) {
+#pragma unroll
+            for (int j = 0; j < kSrcLoads; ++j) {
+                const spio_uint2 v = narrow(regs[l][j]);
+                *(lds_u2p)((lds_bytep)row + in_lds[l][j]) = v;
+                if (SPIO_KEEP && t >= EPY && (t < EPY + ROWS || SH > DH))
+                    __builtin_amdgcn_raw_buffer_store_b64(v, rs, (int)(((unsigned)in_voff[l][j] >> 1) + (unsigned)row_off), 0, AUX_ST);
+            }
         }
     };
 
@@ -290,7 +331,7 @@ SPIO_DEVICE void conv_rows(spio_uint4* __restrict__ dst, const spio_uint4* __res
     // rows, and the first step can start as soon as source row 0 has landed.  Branch-free: dead
     // taps and idle waves load a valid address and are zeroed when the fragments are built.
     constexpr int WLPT = kIgrad ? (GB * 8 * kR * kS + THREADS - 1) / THREADS : NS * KB;
-    spio_uint4 wraw[WLPT];
+    spio_uint4 wraw[WLPT][kFilterLoads];
     if (!kIgrad) {
         // A[m = out channel ch][c] = w[8g+ch][r][s][c]: 16 contiguous bytes per lane.
         // Lane (m = lane%16, kb = lane/16): row slot j = m/8, channel m%8, column tap 4u+kb;
@@ -308,8 +349,7 @@ SPIO_DEVICE void conv_rows(spio_uint4* __restrict__ dst, const spio_uint4* __res
                 const int s = 4 * u + kb;
                 const int rr = r < kR ? r : 0;
                 const int ss = s < kS ? s : 0;
-                wraw[d * KB + u] = *reinterpret_cast<const spio_uint4*>(
-                    weights + (((long long)(8 * gsafe + ch) * kR + rr) * kS + ss) * 8);
+                load_filter_unit(wraw[d * KB + u], weights, ((long long)(8 * gsafe + ch) * kR + rr) * kS + ss);
             }
         }
     } else {
@@ -321,32 +361,37 @@ SPIO_DEVICE void conv_rows(spio_uint4* __restrict__ dst, const spio_uint4* __res
             const int g = i / (8 * kR * kS);
             const int rem = i % (8 * kR * kS);
             const int gs = cb * GB + g < kGroups ? cb * GB + g : 0;
-            wraw[l] = reinterpret_cast<const spio_uint4*>(weights)[(long long)gs * (8 * kR * kS) + rem];
+            load_filter_unit(wraw[l], weights, (long long)gs * (8 * kR * kS) + rem);
         }
     }
     __builtin_amdgcn_sched_barrier(0);  // keep the filter loads ahead of the row loads
 
     // ---- rows 0..PF-1 into registers: their latency covers the rest of the set-up ----
-    spio_uint4 pre[PF][LPT];
+    spio_uint4 pre[PF][LPT][kSrcLoads];
 #pragma unroll
     for (int t = 0; t < PF0; ++t) load_row(pre[t], imin(t, STEPS - 1));
     __builtin_amdgcn_sched_barrier(0);  // ... and the row loads ahead of everything that waits
 
     // ---- loop-invariant addressing of the cooperative row store ----
-    unsigned out_voff[SPT];  // byte offset inside the image block; row term excluded
-    int out_lds[SPT];        // byte offset inside an output-stage row
+    unsigned out_voff[SPT][kDstStores];  // byte offset inside the image block; row term excluded
+    int out_lds[SPT][kDstStores];        // byte offset inside an output-stage row
 #pragma unroll
     for (int s = 0; s < SPT; ++s) {
-        const int cell = tid + THREADS * s;
-        out_voff[s] = OOB;
-        out_lds[s] = 0;
-        if (cell < OUT_CELLS) {
-            const int g = cell % GB;
-            const int q = (cell / GB) % BQ;
-            const int img = cell / (GB * BQ);
-            out_lds[s] = (img * WPI + q) * OSTRIDE + g * 16;
-            if (cb * GB + g < kGroups && q0 + q < DW)
-                out_voff[s] = (unsigned)(((img * DH * DW + q0 + q) * kGroups + cb * GB + g) * (8 * kDstBytes));
+#pragma unroll
+        for (int j = 0; j < kDstStores; ++j) {
+            const int cell = moved_unit(tid, j, kDstStores) + THREADS * s;
+            unsigned voff = OOB;
+            int from = 0;
+            if (cell < OUT_CELLS) {
+                const int g = cell % GB;
+                const int q = (cell / GB) % BQ;
+                const int img = cell / (GB * BQ);
+                from = (img * WPI + q) * OSTRIDE + g * 16;
+                if (cb * GB + g < kGroups && q0 + q < DW)
+                    voff = (unsigned)(((img * DH * DW + q0 + q) * kGroups + cb * GB + g) * (8 * kDstBytes));
+            }
+            out_voff[s][j] = voff + (unsigned)half_bytes(tid, kDstStores, 16);
+            out_lds[s][j] = from + half_bytes(tid, kDstStores, 8);
         }
     }
 
@@ -363,7 +408,7 @@ SPIO_DEVICE void conv_rows(spio_uint4* __restrict__ dst, const spio_uint4* __res
                 const int r = (d - j + NS) % NS;
                 const int s = 4 * u + kb;
                 Pack16 v;
-                v.u = (r < kR && s < kS) ? wraw[d * KB + u] : spio_uint4{0u, 0u, 0u, 0u};
+                v.u = (r < kR && s < kS) ? filter_unit(wraw[d * KB + u]) : spio_uint4{0u, 0u, 0u, 0u};
                 wfrag[d][u] = v.h;
             }
         }
@@ -378,7 +423,7 @@ SPIO_DEVICE void conv_rows(spio_uint4* __restrict__ dst, const spio_uint4* __res
 #pragma unroll
         for (int l = 0; l < WLPT; ++l) {
             const int i = tid + THREADS * l;
-            if (i < WUNITS) wlds[i] = wraw[l];
+            if (i < WUNITS) wlds[i] = filter_unit(wraw[l]);
         }
         block_sync();
         const int kb = lane >> 4;
@@ -445,8 +490,7 @@ SPIO_DEVICE void conv_rows(spio_uint4* __restrict__ dst, const spio_uint4* __res
 
     // ---- row 0 into the ring ----
     block_sync();  // slack zeroed
-#pragma unroll
-    for (int l = 0; l < LPT; ++l) ring[in_lds[l]] = pre[0][l];
+    row_to_ring(pre[0], 0);
     block_sync();
 
     // Coalesced store of the output row staged at step `ts` (in stage buffer `obuf`): the row
@@ -466,19 +510,11 @@ SPIO_DEVICE void conv_rows(spio_uint4* __restrict__ dst, const spio_uint4* __res
 #pragma unroll
         for (int s = 0; s < SPT; ++s) {
             const lds_bytep row = ostage + obuf * OUT_ROW_BYTES;
-            if (SPIO_DST_F32) {
-                typedef __attribute__((address_space(3))) spio_uint2* lds_u2p;
-                const int half = lane & 1;
-                auto store_half = [&](int voff, int from) {
-                    __builtin_amdgcn_raw_buffer_store_b128(widen(*(lds_u2p)(row + from + 8 * half)), rs,
-                                                           (int)((unsigned)voff + 16 * half + row_off), 0, AUX_ST);
-                };
-                store_half(quad_lane<0>((int)out_voff[s]), quad_lane<0>(out_lds[s]));
-                store_half(quad_lane<1>((int)out_voff[s]), quad_lane<1>(out_lds[s]));
-            } else {
+#pragma unroll
+            for (int j = 0; j < kDstStores; ++j) {
                 Pack16 v;
-                v.u = *(lds_u4p)(row + out_lds[s]);
-                __builtin_amdgcn_raw_buffer_store_b128(v.i, rs, (int)(out_voff[s] + row_off), 0, AUX_ST);
+                v.u = SPIO_DST_F32 ? widen(*(lds_u2p)(row + out_lds[s][j])) : *(lds_u4p)(row + out_lds[s][j]);
+                __builtin_amdgcn_raw_buffer_store_b128(v.i, rs, (int)(out_voff[s][j] + row_off), 0, AUX_ST);
             }
         }
         store_group_end();
@@ -524,7 +560,6 @@ SPIO_DEVICE void conv_rows(spio_uint4* __restrict__ dst, const spio_uint4* __res
                         Pack8 o;
 #pragma unroll
                         for (int e = 0; e < 4; ++e) o.h[e] = (spio_half)acc[i][a][e];
-                        typedef __attribute__((address_space(3))) spio_uint2* lds_u2p;
                         *(lds_u2p)(ostage_lane + (te & 1) * OUT_ROW_BYTES + 16 * TS * i * OSTRIDE) = o.u;
                     }
 #pragma unroll
@@ -581,11 +616,7 @@ SPIO_DEVICE void conv_rows(spio_uint4* __restrict__ dst, const spio_uint4* __res
         if (!kLateEmit) emit_row(t);
 
         // 5. the next source row not yet in the ring (loaded earlier) into its ring row
-        if (t + 1 < STEPS) {
-#pragma unroll
-            for (int l = 0; l < LPT; ++l)
-                ring[((t + 1) % NR) * RING_ROW_UNITS + in_lds[l]] = pre[(t + 1) % PF][l];
-        }
+        if (t + 1 < STEPS) row_to_ring(pre[(t + 1) % PF], t + 1);
 
         block_sync();
     }
@@ -596,13 +627,34 @@ SPIO_DEVICE void conv_rows(spio_uint4* __restrict__ dst, const spio_uint4* __res
         block_sync();
     }
     store_output_row(STEPS - 1, (STEPS - 1) & 1);  // the last row
+
+    if (SPIO_KEEP && SPIO_W_F32 && n0 == 0 && p0 == 0 && q0 == 0 && ws == 0 && wave_active) {
+        // the rounded filters, by the first tile of the channel block: slot 0 holds filter row d of phase d
+        const int m = lane & 15;
+        const int kb = lane >> 4;
+#pragma unroll
+        for (int d = 0; d < kR; ++d)
+#pragma unroll
+            for (int u = 0; u < KB; ++u) {
+                Pack16 v;
+                v.h = wfrag[d][u];
+                if (m < 8 && 4 * u + kb < kS) kept_weights[((long long)(8 * gglob + m) * kR + d) * kS + 4 * u + kb] = v.u;
+            }
+    }
 }
 
 }  // namespace
 
 extern "C" __global__ void SPIO_LAUNCH_BOUNDS(THREADS)
 SPIO_KERNEL_NAME(spio_uint4* __restrict__ dst, const spio_uint4* __restrict__ src,
-                 const spio_half* __restrict__ weights, const float* __restrict__ bias) {
+                 const spio_half* __restrict__ weights, const float* __restrict__ bias
+#if SPIO_KEEP
+                 , spio_uint4* __restrict__ kept_src, spio_uint4* __restrict__ kept_weights
+#endif
+) {
+#if !SPIO_KEEP
+    spio_uint4 *const kept_src = nullptr, *const kept_weights = nullptr;
+#endif
     // One LDS block: the source-row ring, then the two output-stage rows.  The data-gradient
     // mode first uses the same block to stage the filters of the workgroup's groups.
     __shared__ spio_uint4 lds[LDS_UNITS];
@@ -636,10 +688,10 @@ SPIO_KERNEL_NAME(spio_uint4* __restrict__ dst, const spio_uint4* __restrict__ sr
     if (BP2 > 0) {
         const int p0 = pb * (BP + BP2);
         if (second)
-            conv_rows<(BP2 > 0 ? BP2 : 1)>(dst, src, weights, bias, ring, p0 + BP, q0, n0, cb);
+            conv_rows<(BP2 > 0 ? BP2 : 1)>(dst, src, weights, bias, kept_src, kept_weights, ring, p0 + BP, q0, n0, cb);
         else
-            conv_rows<BP>(dst, src, weights, bias, ring, p0, q0, n0, cb);
+            conv_rows<BP>(dst, src, weights, bias, kept_src, kept_weights, ring, p0, q0, n0, cb);
     } else {
-        conv_rows<BP>(dst, src, weights, bias, ring, pb * BP, q0, n0, cb);
+        conv_rows<BP>(dst, src, weights, bias, kept_src, kept_weights, ring, pb * BP, q0, n0, cb);
     }
 }

@@ -126,13 +126,12 @@ SPIO_DEVICE void store_stream(spio_uint4 v, spio_uint4* p) {
 #endif
 constexpr int kDstBytes = SPIO_DST_F32 ? 4 : 2;
 // A finished row leaves LDS as 16-byte units of 8 channels, one per lane, which widen to 32 bytes: two
-// stores.  In store j the lanes 2i and 2i+1 of a quad write the halves of the unit of the quad's lane
-// 2j + i, so that every quad fills 64 consecutive bytes; a lane that wrote its own two halves would leave
-// every second 16 bytes of a line to the other store.  quad_lane<j> is that lane's value of `v`.
-template <int J>
-SPIO_DEVICE int quad_lane(int v) {
-    return __builtin_amdgcn_update_dpp(0, v, J ? 0xFA : 0x50, 0xf, 0xf, false);  // quad_perm [2,2,3,3] / [0,0,1,1]
-}
+// stores.  In store j lane i of a wave writes half i % 2 of the unit of lane 32 j + i / 2, so that every
+// store covers whole lines (1024 consecutive bytes where the units are).  A lane that wrote its own two halves
+// would leave every second 16 bytes of a line to the other store; with the units dealt to quads of lanes every
+// access covered half of each line: 128n 384c 14x14, quads -> whole lines, fused backward that stores fp32
+// 23.4 -> 20.6 us, that also reads it 28.7 -> 23.3, forward that reads and stores it 26.5 -> 22.3.
+constexpr int kDstStores = SPIO_DST_F32 ? 2 : 1;
 SPIO_DEVICE spio_uint4 widen(spio_uint2 v) {
     union {
         spio_float4 f;
@@ -147,6 +146,48 @@ SPIO_DEVICE spio_uint4 widen(spio_uint2 v) {
     for (int e = 0; e < 4; ++e) o.f[e] = (float)i.h[e];
     return o.u;
 }
+
+// Kernels can read activations (SPIO_SRC_F32: x of the forward pass, grad_output of a backward one) and
+// weights (SPIO_W_F32, forward pass) that are fp32 and round them to fp16 on their way into LDS, as a
+// conversion beforehand would: that is a pass of 4 bytes read and 2 written per element and a launch.  With
+// SPIO_KEEP they store what they rounded as fp16 tensors too, for the backward pass or the next kernel of it:
+// the 2 written remain, the pass over the 4 and reading the 2 again do not.  128n 384c 14x14 forward and
+// backward: 68 us with conversions, 46 without (of 33 that its bytes take).
+// Loads are the float32 stores in reverse: in load j lane i reads half i % 2 of the 32-byte unit of lane
+// 32 j + i / 2.  A row in flight takes twice the registers, so half as many are in flight: as many bytes as of
+// fp16 rows.
+#ifndef SPIO_SRC_F32
+#define SPIO_SRC_F32 0
+#endif
+#ifndef SPIO_W_F32
+#define SPIO_W_F32 0
+#endif
+#ifndef SPIO_KEEP
+#define SPIO_KEEP 0
+#endif
+constexpr int kSrcBytes = SPIO_SRC_F32 ? 4 : 2;
+constexpr int kSrcLoads = SPIO_SRC_F32 ? 2 : 1;  // loads (and LDS writes) per cell of 8 channels
+constexpr int kFilterLoads = SPIO_W_F32 ? 2 : 1;
+SPIO_DEVICE spio_uint2 narrow(spio_uint4 v) {
+    union {
+        spio_uint4 u;
+        spio_float4 f;
+    } i;
+    union {
+        spio_half4 h;
+        spio_uint2 u;
+    } o;
+    i.u = v;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o.h[e] = (spio_half)i.f[e];
+    return o.u;
+}
+// The unit that thread `tid` takes part in moving by access j, and the byte of its 8 (fp16) or 16 (fp32)
+// that the thread moves where a unit is two accesses.
+SPIO_DEVICE int moved_unit(int tid, int j, int accesses) {
+    return accesses == 1 ? tid : (tid & ~63) + 32 * j + ((tid & 63) >> 1);
+}
+SPIO_DEVICE int half_bytes(int tid, int accesses, int bytes) { return accesses == 1 ? 0 : (tid & 1) * bytes; }
 
 // Closes a group of 16-byte buffer stores.  Such a store reads its data registers for a few
 // cycles after it issues; an instruction that writes one of them in the very next slot can have
@@ -195,6 +236,19 @@ union Pack8 {
     spio_half4 h;
     spio_short4 s;
 };
+
+// Eight filter values as they were loaded, as fp16.
+SPIO_DEVICE spio_uint4 filter_unit(const spio_uint4 (&raw)[kFilterLoads]) {
+    if (!SPIO_W_F32) return raw[0];
+    const spio_uint2 lo = narrow(raw[0]), hi = narrow(raw[kFilterLoads - 1]);
+    return spio_uint4{lo[0], lo[1], hi[0], hi[1]};
+}
+// Unit `i` of a filter tensor.
+SPIO_DEVICE void load_filter_unit(spio_uint4 (&raw)[kFilterLoads], const spio_half* weights, long long i) {
+    const spio_uint4* p = reinterpret_cast<const spio_uint4*>(weights) + i * kFilterLoads;
+#pragma unroll
+    for (int j = 0; j < kFilterLoads; ++j) raw[j] = p[j];
+}
 
 }  // namespace spio
 

@@ -218,102 +218,155 @@ int64_t fused_mode() {
 
 // ---- convolution ----------------------------------------------------------------------------
 
-// Bits of a key's mode: the kernel stores its activations as float32; the caller's weights, and so their
-// gradient, are float16.
-constexpr int64_t WIDE = 4, HALF_WEIGHT = 8;
-
-// `dtype`: what the caller wants; float32 comes from the kernel itself where it has such a version,
-// else the result is float16 and the caller converts it.
-Tensor conv_forward(const Conv& cv, const Tensor& x, const Tensor& w, const Tensor& bias, at::ScalarType dtype) {
-    PlanPtr plan;
-    if (dtype == at::kFloat) plan = find_plan(cv.key(FPROP, x.get_device(), WIDE));
-    if (!plan || !plan->present) {
-        dtype = at::kHalf;
-        plan = find_plan(cv.key(FPROP, x.get_device()));
-    }
-    Tensor y = empty_cl({cv.n, cv.c, cv.p(), cv.q()}, dtype, x);
-    launch(plan->main, c10::hip::getCurrentHIPStream(x.get_device()), {ptr(y), ptr(x), ptr(w), ptr(bias)});
-    return y;
-}
-
-struct ConvGrads {
-    Tensor x, w, b;
-};
-
-// The backward operator on channels_last tensors: one fused kernel where the shape uses it and
-// both gradients are wanted, else the weight and the data gradient one after the other.
-// `x_dtype`, `w_dtype`: what the caller's tensors are; a gradient is stored in that type where the kernel
-// can (a two-stage one's grad_weight), else in the operator's and the caller converts it.
-ConvGrads conv_backward(const Conv& cv, const Tensor& x, const Tensor& w, const Tensor& dy, bool need_x,
-                        bool need_w, bool need_b, at::ScalarType x_dtype, at::ScalarType w_dtype) {
-    ConvGrads g;
-    const int64_t weight_mode = w_dtype == at::kHalf ? HALF_WEIGHT : 0;
-    // the version of a kernel whose grad_input is float32, where that is wanted and there is one
-    auto wide_or = [&](const PlanPtr& plan, Kind kind, int64_t mode) {
-        const auto wide = x_dtype == at::kFloat ? find_plan(cv.key(kind, dy.get_device(), mode | WIDE)) : nullptr;
-        const bool use = wide && wide->present;
-        g.x = empty_cl({cv.n, cv.c, cv.h, cv.w}, use ? at::kFloat : at::kHalf, dy);
-        return use ? wide : plan;
-    };
-    const auto device = dy.get_device();
-    hipStream_t stream = c10::hip::getCurrentHIPStream(device);
-    // atomic kernels add into zeroed sums, two-stage ones store them whole
-    auto sums = [&](const Plan& plan, bool with_bias, bool bias_is_stored) {
-        g.w = empty_cl({cv.c, 8, cv.r, cv.s}, weight_mode && plan.second_half.function ? at::kHalf : at::kFloat, dy);
-        if (with_bias) g.b = empty_1d(cv.c, at::kFloat, dy);
-        // one launch for both: a launch is all that the fill of such small sums costs
-        zero(plan.overwrites ? Tensor() : g.w, bias_is_stored ? Tensor() : g.b, stream);
-    };
-    auto second = [&](const Plan& plan) -> const Stage& {
-        return g.w.scalar_type() == at::kHalf ? plan.second_half : plan.second;
-    };
-    PlanPtr fused;
-    if (need_x && need_w) {
-        const int64_t mode = fused_mode();
-        if (mode != 0) fused = find_plan(cv.key(BGRAD, device, mode | weight_mode));
-        if (fused && !fused->present) fused.reset();
-        if (fused) fused = wide_or(fused, BGRAD, mode | weight_mode);
-    }
-    if (fused) {
-        sums(*fused, cv.bias && need_b, fused->overwrites);
-        Tensor workspace;
-        if (fused->second.function) workspace = empty_1d(fused->workspace, at::kByte, dy);
-        const void* dw = workspace.defined() ? ptr(workspace) : ptr(g.w);
-        if (cv.bias)
-            launch(fused->main, stream, {ptr(g.x), dw, ptr(x), ptr(dy), ptr(w), ptr(g.b)});
-        else
-            launch(fused->main, stream, {ptr(g.x), dw, ptr(x), ptr(dy), ptr(w)});
-        if (workspace.defined()) launch(second(*fused), stream, {ptr(g.w), ptr(workspace), ptr(g.b)});
-    } else if (need_w) {
-        const auto plan = find_plan(cv.key(WGRAD, device, weight_mode));
-        // the second stage that stores float16 stores the bias sums as well; the other adds them with atomics
-        const bool half = weight_mode && plan->second_half.function;
-        sums(*plan, cv.bias && need_b, half);
-        Tensor workspace;
-        if (plan->second.function) workspace = empty_1d(plan->workspace, at::kByte, dy);
-        const void* dw = workspace.defined() ? ptr(workspace) : ptr(g.w);
-        if (cv.bias)
-            launch(plan->main, stream, {dw, ptr(x), ptr(dy), half ? nullptr : ptr(g.b)});
-        else
-            launch(plan->main, stream, {dw, ptr(x), ptr(dy)});
-        if (half && cv.bias)
-            launch(plan->second_half, stream, {ptr(g.w), ptr(workspace), ptr(g.b)});
-        else if (workspace.defined())
-            launch(second(*plan), stream, {ptr(g.w), ptr(workspace)});
-    }
-    if (need_b && !g.b.defined()) g.b = dy.sum({0, 2, 3}, /*keepdim=*/false, at::kFloat);
-    if (need_x && !g.x.defined()) {
-        const auto plan = wide_or(find_plan(cv.key(DGRAD, device)), DGRAD, 0);
-        launch(plan->main, stream, {ptr(g.x), ptr(dy), ptr(w), nullptr});
-    }
-    return g;
-}
+// Bits of a key's mode.  WIDE: the kernel stores its activations as float32.  HALF_WEIGHT: the caller's weights,
+// and so their gradient, are float16.  READ_F32, WEIGHT_F32: it reads a float32 source (x forward, grad_output
+// backward), float32 weights.  KEEP: it stores what it rounded of these as float16.
+constexpr int64_t WIDE = 4, HALF_WEIGHT = 8, READ_F32 = 16, WEIGHT_F32 = 32, KEEP = 64;
 
 // What the kernels read: float16, channels_last; the tensor itself where it is that already.
 Tensor to_half_cl(const Tensor& t) {
     if (t.scalar_type() == at::kHalf) return t.is_contiguous(CL) ? t : t.contiguous(CL);
     return t.to(at::kHalf, /*non_blocking=*/false, /*copy=*/false, CL).contiguous(CL);
 }
+// A float32 tensor that a kernel can read as it is, in the order and with the alignment of its 16-byte loads.
+bool readable_f32(const Tensor& t) {
+    return t.scalar_type() == at::kFloat && t.is_contiguous(CL) && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
+}
+
+struct ConvOutput {
+    Tensor y, x, w;  // x, w: the float16 tensors that the products were taken of (wanted: `keep`)
+};
+
+// The result is in the type of `x` where the kernel has such a version, else float16, for the caller to convert.
+ConvOutput conv_forward(const Conv& cv, const Tensor& x, const Tensor& w, const Tensor& bias, bool keep) {
+    const auto device = x.get_device();
+    hipStream_t stream = c10::hip::getCurrentHIPStream(device);
+    const int64_t wide = x.scalar_type() == at::kFloat ? WIDE : 0;
+    const int64_t reads = (readable_f32(x) ? READ_F32 : 0) | (readable_f32(w) ? WEIGHT_F32 : 0);
+    if (reads) {
+        const auto plan = find_plan(cv.key(FPROP, device, wide | reads | (keep ? KEEP : 0)));
+        if (plan->present) {
+            ConvOutput o;
+            o.y = empty_cl({cv.n, cv.c, cv.p(), cv.q()}, wide ? at::kFloat : at::kHalf, x);
+            const Tensor xr = reads & READ_F32 ? x : to_half_cl(x), wr = reads & WEIGHT_F32 ? w : to_half_cl(w);
+            if (keep) {
+                o.x = reads & READ_F32 ? empty_cl(x.sizes(), at::kHalf, x) : xr;
+                o.w = reads & WEIGHT_F32 ? empty_cl(w.sizes(), at::kHalf, w) : wr;
+                launch(plan->main, stream, {ptr(o.y), ptr(xr), ptr(wr), ptr(bias), ptr(o.x), ptr(o.w)});
+            } else {
+                launch(plan->main, stream, {ptr(o.y), ptr(xr), ptr(wr), ptr(bias)});
+            }
+            return o;
+        }
+    }
+    ConvOutput o{Tensor(), to_half_cl(x), to_half_cl(w)};
+    PlanPtr plan;
+    if (wide) plan = find_plan(cv.key(FPROP, device, WIDE));
+    const bool store_wide = plan && plan->present;
+    if (!store_wide) plan = find_plan(cv.key(FPROP, device));
+    o.y = empty_cl({cv.n, cv.c, cv.p(), cv.q()}, store_wide ? at::kFloat : at::kHalf, x);
+    launch(plan->main, stream, {ptr(o.y), ptr(o.x), ptr(o.w), ptr(bias)});
+    return o;
+}
+
+struct ConvGrads {
+    Tensor x, w, b;
+};
+
+// The backward operator, x and w on channels_last tensors: one fused kernel where the shape uses it and
+// both gradients are wanted, else the weight and the data gradient one after the other.
+// `x_dtype`, `w_dtype`: what the caller's tensors are; a gradient is stored in that type where the kernel
+// can (a two-stage one's grad_weight), else in the operator's and the caller converts it.
+ConvGrads conv_backward(const Conv& cv, const Tensor& x, const Tensor& w, const Tensor& grad, bool need_x,
+                        bool need_w, bool need_b, at::ScalarType x_dtype, at::ScalarType w_dtype) {
+    ConvGrads g;
+    const auto device = grad.get_device();
+    hipStream_t stream = c10::hip::getCurrentHIPStream(device);
+    const int64_t weight_mode = w_dtype == at::kHalf ? HALF_WEIGHT : 0;
+    const bool read_f32 = readable_f32(grad);
+    // grad as float16, made when a kernel that wants it comes first
+    Tensor half_grad;
+    auto dy = [&]() -> const Tensor& {
+        if (!half_grad.defined()) half_grad = to_half_cl(grad);
+        return half_grad;
+    };
+    // The version of a kernel for the caller's types: one whose grad_input is float32, one that reads a float32
+    // grad_output (and leaves a float16 copy), where these are wanted and there is one.
+    int64_t types = 0;
+    auto version = [&](const PlanPtr& plan, Kind kind, int64_t mode, int64_t keep) {
+        const int64_t wide = x_dtype == at::kFloat ? WIDE : 0;
+        for (const int64_t t : {wide | (read_f32 ? READ_F32 | keep : 0), wide}) {
+            if (t == 0) continue;
+            const auto v = find_plan(cv.key(kind, device, mode | t));
+            if (!v->present) continue;
+            types = t;
+            return v;
+        }
+        return plan;
+    };
+    auto make_grad_input = [&] { g.x = empty_cl({cv.n, cv.c, cv.h, cv.w}, types & WIDE ? at::kFloat : at::kHalf, grad); };
+    // atomic kernels add into zeroed sums, two-stage ones store them whole
+    auto sums = [&](const Plan& plan, bool with_bias, bool bias_is_stored) {
+        g.w = empty_cl({cv.c, 8, cv.r, cv.s}, weight_mode && plan.second_half.function ? at::kHalf : at::kFloat, grad);
+        if (with_bias) g.b = empty_1d(cv.c, at::kFloat, grad);
+        // one launch for both: a launch is all that the fill of such small sums costs
+        zero(plan.overwrites ? Tensor() : g.w, bias_is_stored ? Tensor() : g.b, stream);
+    };
+    auto second = [&](const Plan& plan) -> const Stage& {
+        return g.w.scalar_type() == at::kHalf ? plan.second_half : plan.second;
+    };
+    auto data_gradient = [&](int64_t keep) {
+        const auto plan = version(find_plan(cv.key(DGRAD, device)), DGRAD, 0, keep);
+        make_grad_input();
+        if (types & KEEP) half_grad = empty_cl(grad.sizes(), at::kHalf, grad);
+        if (types & KEEP)
+            launch(plan->main, stream, {ptr(g.x), ptr(grad), ptr(w), nullptr, ptr(half_grad), nullptr});
+        else
+            launch(plan->main, stream, {ptr(g.x), types & READ_F32 ? ptr(grad) : ptr(dy()), ptr(w), nullptr});
+    };
+    PlanPtr fused;
+    if (need_x && need_w) {
+        const int64_t mode = fused_mode();
+        if (mode != 0) fused = find_plan(cv.key(BGRAD, device, mode | weight_mode));
+        if (fused && !fused->present) fused.reset();
+        if (fused) fused = version(fused, BGRAD, mode | weight_mode, 0);
+    }
+    if (fused) {
+        make_grad_input();
+        sums(*fused, cv.bias && need_b, fused->overwrites);
+        Tensor workspace;
+        if (fused->second.function) workspace = empty_1d(fused->workspace, at::kByte, grad);
+        const void* dw = workspace.defined() ? ptr(workspace) : ptr(g.w);
+        const void* dy_ptr = types & READ_F32 ? ptr(grad) : ptr(dy());
+        if (cv.bias)
+            launch(fused->main, stream, {ptr(g.x), dw, ptr(x), dy_ptr, ptr(w), ptr(g.b)});
+        else
+            launch(fused->main, stream, {ptr(g.x), dw, ptr(x), dy_ptr, ptr(w)});
+        if (workspace.defined()) launch(second(*fused), stream, {ptr(g.w), ptr(workspace), ptr(g.b)});
+    } else if (need_w) {
+        // a data gradient that reads float32 goes first: it leaves the copy that the weight gradient reads
+        if (need_x && read_f32) data_gradient(KEEP);
+        const auto plan = find_plan(cv.key(WGRAD, device, weight_mode));
+        // the second stage that stores float16 stores the bias sums as well; the other adds them with atomics
+        const bool half = weight_mode && plan->second_half.function;
+        sums(*plan, cv.bias && need_b, half);
+        Tensor workspace;
+        if (plan->second.function) workspace = empty_1d(plan->workspace, at::kByte, grad);
+        const void* dw = workspace.defined() ? ptr(workspace) : ptr(g.w);
+        if (cv.bias)
+            launch(plan->main, stream, {dw, ptr(x), ptr(dy()), half ? nullptr : ptr(g.b)});
+        else
+            launch(plan->main, stream, {dw, ptr(x), ptr(dy())});
+        if (half && cv.bias)
+            launch(plan->second_half, stream, {ptr(g.w), ptr(workspace), ptr(g.b)});
+        else if (workspace.defined())
+            launch(second(*plan), stream, {ptr(g.w), ptr(workspace)});
+    }
+    if (need_b && !g.b.defined()) g.b = dy().sum({0, 2, 3}, /*keepdim=*/false, at::kFloat);
+    if (need_x && !g.x.defined()) data_gradient(0);
+    return g;
+}
+
 // Whether a saved tensor still is what the forward pass saved, up to its layout: hooks on saved tensors may
 // unpack it with other strides (a copy packed into host memory, say) or elsewhere altogether.
 bool is_again(const Tensor& t, const Tensor& grad, at::IntArrayRef sizes, at::ScalarType dtype = at::kHalf) {
@@ -343,8 +396,8 @@ struct ConvFunction : torch::autograd::Function<ConvFunction> {
     static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& w,
                           const std::optional<Tensor>& bias_arg, const Conv& cv) {
         const Tensor bias = bias_arg.value_or(Tensor());
-        const Tensor xh = to_half_cl(x), wh = to_half_cl(w), bf = to_float_1d(bias);
-        Tensor y = conv_forward(cv, xh, wh, bf, x.scalar_type());
+        const Tensor bf = to_float_1d(bias);
+        const auto [y, xh, wh] = conv_forward(cv, x, w, bf, /*keep=*/true);
         // the caller's own tensors unless their type was cast: with their history and their version, which
         // a second differentiation and a write to one of them before the backward pass are noticed by
         ctx->save_for_backward({x.scalar_type() == at::kHalf ? x : xh, w.scalar_type() == at::kHalf ? w : wh,
@@ -377,7 +430,7 @@ struct ConvFunction : torch::autograd::Function<ConvFunction> {
             g = {get(0), get(1), get(2)};
         } else {
             RECORD_FUNCTION("spio::conv2d_gw8_backward", tensors({x, w, saved[2], grads[0]}));
-            g = conv_backward(cv, to_half_cl(x), to_half_cl(w), to_half_cl(grads[0]), need_x, need_w, need_b,
+            g = conv_backward(cv, to_half_cl(x), to_half_cl(w), grads[0], need_x, need_w, need_b,
                               static_cast<at::ScalarType>(v[9]), static_cast<at::ScalarType>(v[10]));
         }
         auto typed = [&](const Tensor& t, int i) {
@@ -543,7 +596,7 @@ PyObject* conv2d_gw8(PyObject*, PyObject* const* args, Py_ssize_t nargs, PyObjec
             y = ConvFunction::apply(x, w, optional(bias), cv);
         } else {
             at::AutoDispatchBelowADInplaceOrView below;
-            y = conv_forward(cv, to_half_cl(x), to_half_cl(w), to_float_1d(bias), x.scalar_type()).to(x.scalar_type());
+            y = conv_forward(cv, x, w, to_float_1d(bias), /*keep=*/false).y.to(x.scalar_type());
         }
     }
     return THPVariable_Wrap(y);
@@ -605,6 +658,9 @@ PYBIND11_MODULE(_native, m) {
     m.attr("built_from") = "spio-built-from:" SPIO_TEXT(SPIO_BUILT_FROM);
     m.attr("WIDE") = WIDE;
     m.attr("HALF_WEIGHT") = HALF_WEIGHT;
+    m.attr("READ_F32") = READ_F32;
+    m.attr("WEIGHT_F32") = WEIGHT_F32;
+    m.attr("KEEP") = KEEP;
     m.def("configure", [](py::object make_plan, py::object backward_op, py::object norm_gradients) {
         g_make_plan = make_plan.release().ptr();
         g_backward_op = backward_op.release().ptr();

@@ -11,12 +11,13 @@ from .kernel_factory import KernelFactory
 from .kernel_cache import KernelCache
 from .kernel_params_logger import KernelParamsLogger, kernel_params_logging_is_enabled
 from .tuner import tuner, Tuner
-from .conv2d_gw8_kernel import conv2d_gw8_kernel_factory, Conv2dGw8Config
+from .conv2d_gw8_kernel import conv2d_gw8_kernel_factory, Conv2dGw8Config, fits_float32_output, reads_float32
 from .conv2d_gw8_wgrad_kernel import conv2d_gw8_wgrad_kernel_factory, Conv2dGw8WgradConfig, stored_sums
 from .conv2d_gw8_bgrad_kernel import (
     conv2d_gw8_bgrad_kernel_factory,
     Conv2dGw8BgradConfig,
     bgrad_is_supported,
+    bgrad_reads_float32,
 )
 from .layernorm_2d_kernel import (
     layernorm_2d_kernel_factory,

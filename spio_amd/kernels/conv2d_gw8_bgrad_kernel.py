@@ -246,13 +246,27 @@ def _get_configs(params: Conv2dGw8Params, device_attr=None) -> List[Conv2dGw8Bgr
     return with_joined_stores(params, configs)
 
 
-def _get_kernel_name(out_f32: bool = False) -> str:
-    return "spio_conv2d_gw8_bgrad" + ("_f32" if out_f32 else "")
+def _float32_prefetch(prefetch: int) -> int:
+    """Rows in flight where grad_output is float32: half as many.  (All of them: 128n 384c 14x14 29.7 us, half
+    28.7.)"""
+    return max(2, prefetch // 4 * 2)
+
+
+def bgrad_reads_float32(params: Conv2dGw8Params, config: Conv2dGw8BgradConfig) -> bool:
+    """Whether a configuration has a version that reads a float32 grad_output: its rows in flight take twice
+    the registers."""
+    config = replace(config, prefetch=_float32_prefetch(config.prefetch))
+    g = bgrad_geometry(params, config)
+    return g["REGISTERS"] + 4 * config.prefetch * g["LPTD"] <= MAX_REGISTERS and fits_float32_output(params, config)
+
+
+def _get_kernel_name(out_f32: bool = False, src_f32: bool = False) -> str:
+    return "spio_conv2d_gw8_bgrad" + ("_f32" if out_f32 else "") + ("_srcf32" if src_f32 else "")
 
 
 def _get_kernel_spec(params: Conv2dGw8Params, config: Conv2dGw8BgradConfig, _device_attr=None,
-                     out_f32: bool = False) -> KernelSpec:  # fmt: skip
-    """Macros and launch geometry; `out_f32`: grad_input is a float32 tensor."""
+                     out_f32: bool = False, src_f32: bool = False) -> KernelSpec:  # fmt: skip
+    """Macros and launch geometry; `out_f32`: grad_input is a float32 tensor, `src_f32`: grad_output is."""
     params.validate()
     assert _config_is_legal(params, config), f"illegal configuration {config} for {params}"
     g = bgrad_geometry(params, config)
@@ -260,9 +274,12 @@ def _get_kernel_spec(params: Conv2dGw8Params, config: Conv2dGw8BgradConfig, _dev
     if out_f32:
         assert fits_float32_output(params, config), f"no float32 output for {config} and {params}"
         defines["SPIO_DST_F32"] = 1
+    if src_f32:
+        assert bgrad_reads_float32(params, config), f"no float32 grad_output for {config} and {params}"
+        defines["SPIO_SRC_F32"] = 1
     defines.update(SPIO_GB=config.groups, SPIO_BH=g["BH"], SPIO_NB=config.block_n,
                    SPIO_ITERS=config.block_n_iters,
-                   SPIO_PF=config.prefetch, SPIO_TS=config.split,
+                   SPIO_PF=_float32_prefetch(config.prefetch) if src_f32 else config.prefetch, SPIO_TS=config.split,
                    SPIO_HALO_CACHED=config.halo_cached, SPIO_XCD_CHUNK=config.xcd_chunk,
                    SPIO_NT=config.nontemporal, SPIO_HAS_BIAS=int(params.has_bias))  # fmt: skip
     if config.block_q:

@@ -171,7 +171,14 @@ def image_geometry(params: Conv2dGw8Params, config: Conv2dGw8Config, igrad: bool
         registers = max(multiplying + 4 * wlpt, moving) + 14
     else:
         registers = multiplying + 4 * max(2 * lpt, lpt + wlpt) + lpt + spt + 14
+    # the same with fp32 source, destination and weights, by the number of blocks in flight
+    wide = [16 * lpt * sets + 2 * (lpt + spt) for sets in (1, 2)]
+    if config.movers:
+        wide_registers = [max(multiplying + 8 * wlpt, w) + 14 for w in wide]
+    else:
+        wide_registers = [multiplying + max(w, 16 * lpt + 8 * wlpt + 2 * (lpt + spt)) + 14 for w in wide]
     d.update(
+        WIDE_REGISTERS=wide_registers,
         NS=ns, NACC=nacc, APW=apw, KB=kb, WPI=wpi, F=f, WT=wt, GS=gs, THREADS=threads,
         MTHREADS=mthreads, LDS_BYTES=lds, LPT=lpt, SPT=spt, STEPS=d["DH"] + r - 1,
         GBLKS=divup(params.groups, gb), NBLKS=divup(params.n, nb),
@@ -182,11 +189,32 @@ def image_geometry(params: Conv2dGw8Params, config: Conv2dGw8Config, igrad: bool
     return d
 
 
+def _register_budget(config) -> int:
+    """Registers per lane that leave room for the workgroup's waves on a SIMD (512 in all)."""
+    return {1: 232, 2: 232, 3: 160, 4: 128}.get(divup(config.groups * config.split + config.movers, 4), 0)
+
+
+def float32_block_sets(params, config, igrad) -> int:
+    """Image blocks in flight of the whole-image kernel where they are float32: two if the registers allow it,
+    one, or none (no such version)."""
+    registers = image_geometry(params, config, igrad)["WIDE_REGISTERS"]
+    return sum(r <= _register_budget(config) for r in registers)
+
+
+def _float32_config(params, config, igrad):
+    """The configuration a version that reads float32 runs in: without mover waves where the registers allow it.
+    Rounding and keeping a block is work that all waves share then (128n 384c 14x14 forward with mover waves
+    22.3 us, without 20.4; of float16 blocks 8.6 and 10.4)."""
+    without = replace(config, movers=0)
+    if config.variant == "image" and config.movers and float32_block_sets(params, without, igrad):
+        if _image_config_is_legal(params, without, igrad):
+            return without
+    return config
+
+
 def _image_config_is_legal(params, config, igrad) -> bool:
     g = image_geometry(params, config, igrad)
     waves = config.groups * config.split + config.movers
-    # registers per lane that leave room for the workgroup's waves on a SIMD (512 in all)
-    budget = {1: 232, 2: 232, 3: 160, 4: 128}.get(divup(waves, 4), 0)
     return (
         waves <= MAX_WAVES
         and config.movers >= 0
@@ -200,7 +228,7 @@ def _image_config_is_legal(params, config, igrad) -> bool:
         and g["LPT"] <= MAX_LOADS_PER_THREAD
         and g["SPT"] <= MAX_LOADS_PER_THREAD
         and g["STEPS"] <= MAX_UNROLLED_STEPS
-        and g["REGISTERS"] <= budget
+        and g["REGISTERS"] <= _register_budget(config)
         and config.block_n * params.c * max(params.h * params.w, params.p * params.q) * 2 < 2**31
     )
 
@@ -435,15 +463,37 @@ def fits_float32_output(params: Conv2dGw8Params, config) -> bool:
     return block_n * params.c * max(params.h * params.w, params.p * params.q) * 4 < 2**30
 
 
+def reads_float32(params: Conv2dGw8Params, config, igrad: bool = False, src_f32: bool = False,
+                  w_f32: bool = False, keep: bool = False) -> bool:  # fmt: skip
+    """Whether a configuration has a version that reads float32 tensors.  The float16 copy it can leave is
+    whole only if every source pixel is staged by the workgroup that owns it: padding below the filter size."""
+    return (
+        config.variant in ("mfma", "image")
+        and fits_float32_output(params, config)
+        and not (config.variant == "image" and src_f32
+                 and not float32_block_sets(params, _float32_config(params, config, igrad), igrad))
+        and not (igrad and w_f32)
+        and not (keep and src_f32 and (params.padding_h >= params.r or params.padding_w >= params.s))
+    )
+
+
 def _get_kernel_spec(params: Conv2dGw8Params, config: Conv2dGw8Config, _device_attr=None,
-                     igrad: bool = False, out_f32: bool = False) -> KernelSpec:  # fmt: skip
+                     igrad: bool = False, out_f32: bool = False, src_f32: bool = False,
+                     w_f32: bool = False, keep: bool = False) -> KernelSpec:  # fmt: skip
     """Macros and launch geometry for one (params, config, direction); `out_f32`: the destination is a
-    float32 tensor (the same values, widened when they are stored)."""
+    float32 tensor (the same values, widened when they are stored); `src_f32`, `w_f32`: source, weights are
+    (rounded to float16 as they are read); `keep`: two more arguments, float16 tensors that receive what was
+    rounded of the two."""
     params.validate()
     defines = _shape_defines(params)
     if out_f32:
         assert fits_float32_output(params, config), f"no float32 output for {config} and {params}"
         defines["SPIO_DST_F32"] = 1
+    if src_f32:
+        config = _float32_config(params, config, igrad)
+    if src_f32 or w_f32:
+        assert reads_float32(params, config, igrad, src_f32, w_f32, keep), f"no float32 input for {config} and {params}"
+        defines.update(SPIO_SRC_F32=int(src_f32), SPIO_W_F32=int(w_f32), SPIO_KEEP=int(keep))
     defines["SPIO_IGRAD"] = int(igrad)
     defines["SPIO_HAS_BIAS"] = int(params.has_bias and not igrad)
     if config.variant == "direct":
@@ -455,6 +505,8 @@ def _get_kernel_spec(params: Conv2dGw8Params, config: Conv2dGw8Config, _device_a
     if config.variant == "image":
         assert _image_config_is_legal(params, config, igrad), f"illegal configuration {config} for {params}"
         g = image_geometry(params, config, igrad)
+        if src_f32:
+            defines["SPIO_SETS"] = float32_block_sets(params, config, igrad)
         defines.update(
             SPIO_GB=config.groups, SPIO_NB=config.block_n, SPIO_TS=config.split,
             SPIO_ITERS=config.block_n_iters, SPIO_NT=config.nontemporal,
@@ -467,16 +519,18 @@ def _get_kernel_spec(params: Conv2dGw8Params, config: Conv2dGw8Config, _device_a
         raise ValueError(f"unknown kernel variant {config.variant!r}")
     assert _mfma_config_is_legal(params, config, igrad), f"illegal configuration {config} for {params}"
     g = mfma_geometry(params, config, igrad)
+    # float32 rows: half as many in flight, which are as many bytes (and registers)
+    prefetch = max(2, config.prefetch // 2) if src_f32 else config.prefetch
     defines.update(
         SPIO_GB=config.groups, SPIO_BP=config.block_p, SPIO_NB=config.block_n,
-        SPIO_TS=config.split, SPIO_PF=config.prefetch,
+        SPIO_TS=config.split, SPIO_PF=prefetch,
         SPIO_NT=config.nontemporal, SPIO_HALO_CACHED=config.halo_cached,
         SPIO_XCD_CHUNK=config.xcd_chunk,
     )  # fmt: skip
     if config.block_p2:
         defines["SPIO_BP2"] = config.block_p2
     if config.prefetch_start:
-        defines["SPIO_PF0"] = config.prefetch_start
+        defines["SPIO_PF0"] = max(2, config.prefetch_start // 2) if src_f32 else config.prefetch_start
     if config.prefetch_rate != 1:
         defines["SPIO_PF_RATE"] = config.prefetch_rate
     if config.block_q:
@@ -486,8 +540,10 @@ def _get_kernel_spec(params: Conv2dGw8Params, config: Conv2dGw8Config, _device_a
     )
 
 
-def _get_kernel_name(igrad: bool = False, out_f32: bool = False) -> str:
-    return ("spio_conv2d_gw8_dgrad" if igrad else "spio_conv2d_gw8_fprop") + ("_f32" if out_f32 else "")
+def _get_kernel_name(igrad: bool = False, out_f32: bool = False, src_f32: bool = False, w_f32: bool = False,
+                     keep: bool = False) -> str:  # fmt: skip
+    name = ("spio_conv2d_gw8_dgrad" if igrad else "spio_conv2d_gw8_fprop") + ("_f32" if out_f32 else "")
+    return name + ("_srcf32" if src_f32 else "") + ("_wf32" if w_f32 else "") + ("_keep" if keep else "")
 
 
 def _make_test_args(params: Conv2dGw8Params, device, igrad: bool = False):

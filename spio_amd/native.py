@@ -57,23 +57,36 @@ def _stage(function, launch_params):
     return [function.handle, *launch_params.grid, *launch_params.block, launch_params.shared_mem_bytes]
 
 
-# bits of a key's mode: the kernel stores its activations as float32; the caller's weights are float16
+# bits of a key's mode: which tensors are float32 (results, source, weights), whether the kernel keeps what it
+# rounds, and that the weights are float16 (and so is their gradient)
 WIDE = 0 if _native is None else _native.WIDE
 HALF_WEIGHT = 0 if _native is None else _native.HALF_WEIGHT
+READ_F32 = 0 if _native is None else _native.READ_F32
+WEIGHT_F32 = 0 if _native is None else _native.WEIGHT_F32
+KEEP = 0 if _native is None else _native.KEEP
 
 
 def _adapted(kernel, factory, params, device, mode, **kwargs):
     """`kernel` or the version of it for the caller's types, in the configuration chosen for the plain one (it
     reads and multiplies the same); None where that has no such version."""
-    from .kernels import stored_sums
-    from .kernels.conv2d_gw8_kernel import fits_float32_output
+    from . import kernels
 
-    config = stored_sums(factory, params, kernel.config) if mode & HALF_WEIGHT else kernel.config
+    config = kernels.stored_sums(factory, params, kernel.config) if mode & HALF_WEIGHT else kernel.config
     if mode & WIDE:
-        if not fits_float32_output(params, config):
+        if not kernels.fits_float32_output(params, config):
             return None
         kwargs["out_f32"] = True
-    elif config == kernel.config:
+    if mode & (READ_F32 | WEIGHT_F32):
+        if factory is kernels.conv2d_gw8_bgrad_kernel_factory:
+            kwargs["src_f32"] = True
+            if not kernels.bgrad_reads_float32(params, config):
+                return None
+        else:
+            reads = dict(src_f32=bool(mode & READ_F32), w_f32=bool(mode & WEIGHT_F32), keep=bool(mode & KEEP))
+            if not kernels.reads_float32(params, config, kwargs.get("igrad", False), **reads):
+                return None
+            kwargs.update(reads)
+    if config == kernel.config and not mode & (WIDE | READ_F32 | WEIGHT_F32):
         return kernel
     return factory.get_kernel_in_config(params, device, config, **kwargs)
 

@@ -214,6 +214,69 @@ def test_float32_outputs_are_the_float16_ones_widened(params, configs, fused):
         activations(conv2d_gw8_bgrad_kernel_factory, config, params.input_shape, sums)
 
 
+@pytest.mark.parametrize("params,configs,fused", _F32_CASES + [
+    # more output rows than source rows and fewer, two tile heights with a ramped prefetch, an image block of
+    # several images in one register set, an idle group, a filter row only
+    (Conv2dGw8Params(n=3, c=40, h=8, w=9, padding=2, has_bias=True),
+     [Conv2dGw8Config(groups=4, block_p=4, block_p2=3, prefetch=6, prefetch_start=4, prefetch_rate=2),
+      Conv2dGw8Config(groups=4, block_p=10, variant="image", prefetch=2, block_n_iters=3, split=2)],
+     [Conv2dGw8BgradConfig(groups=4, block_h=5, block_n=3, prefetch=4, split=2, two_stage=1)]),
+    (Conv2dGw8Params(n=2, c=24, h=11, w=8, r=4, s=1, padding=0),
+     [Conv2dGw8Config(groups=3, block_p=3, block_n=2, prefetch=2, halo_cached=0)], [Conv2dGw8BgradConfig(groups=3, prefetch=2)]),
+], ids=lambda v: v.encode() if hasattr(v, "encode") else "")  # fmt: skip
+def test_float32_inputs_are_rounded_once(params, configs, fused):
+    """The versions that read float32 activations and weights compute exactly what the float16 version does
+    with the rounded tensors, and leave exactly those where they keep a copy."""
+    x, w, bias, dy = [to_gpu(t) for t in gpu_args(params)]
+    generator = torch.Generator(device="cuda").manual_seed(1)
+    x, w, dy = [t.float() * (1 + 1e-3 * torch.rand(t.shape, device="cuda", generator=generator)) for t in (x, w, dy)]
+    x, w, dy = [t.contiguous(memory_format=torch.channels_last) for t in (x, w, dy)]
+    attr = get_device_attributes(0)
+
+    def empty(shape, dtype=torch.float16):
+        return torch.full(shape, -42.0, device="cuda", dtype=dtype).contiguous(memory_format=torch.channels_last)
+
+    def run(factory, config, outs, args, **kw):
+        (kernel,) = compile_kernel_configs(factory, params, configs=[config], device_attr=attr, **kw)
+        kernel.load(0)
+        kernel(*outs, *args)
+        torch.cuda.synchronize()
+        kernel.unload()
+        return outs
+
+    for config in configs:
+        if config.variant == "direct":
+            continue
+        forward = conv2d_gw8_kernel_factory
+        (expected,) = run(forward, config, [empty(params.output_shape)], (x.half(), w.half(), bias))
+        for src in (False, True):
+            for keep in (False, True):
+                kept = (empty(params.input_shape), empty(params.weight_shape)) if keep else ()
+                (y,) = run(forward, config, [empty(params.output_shape, torch.float32 if src else torch.float16)],
+                           (x if src else x.half(), w, bias, *kept), src_f32=src, w_f32=True, keep=keep, out_f32=src)
+                assert torch.equal(y.half(), expected), (config, src, keep)
+                if keep:
+                    assert torch.equal(kept[1], w.half()), config
+                    assert torch.equal(kept[0], x.half() if src else empty(params.input_shape)), config
+        if config.variant == "image" and config.block_p != params.h:
+            continue
+        (expected,) = run(forward, config, [empty(params.input_shape)], (dy.half(), w.half(), None), igrad=True)
+        copy = empty(params.output_shape)
+        (dx,) = run(forward, config, [empty(params.input_shape)], (dy, w.half(), None, copy, None), igrad=True, src_f32=True, keep=True)
+        assert torch.equal(dx, expected) and torch.equal(copy, dy.half()), config
+    for config in fused:
+        results = []
+        for src in (False, True):
+            sums = [torch.zeros(params.weight_shape, device="cuda").contiguous(memory_format=torch.channels_last)]
+            db = (torch.zeros(params.c, device="cuda"),) if params.has_bias else ()
+            (dx, dw) = run(conv2d_gw8_bgrad_kernel_factory, config, [empty(params.input_shape), *sums],
+                           (x.half(), dy if src else dy.half(), w.half(), *db), src_f32=src)  # fmt: skip
+            results.append((dx, dw, *db))
+        assert torch.equal(results[0][0], results[1][0]), config
+        for a, b in zip(*[r[1:] for r in results]):  # float32 atomics: any order
+            assert torch.allclose(a, b, rtol=1e-5, atol=1e-5 * float(a.abs().max())), config
+
+
 def test_column_blocks():
     """Workgroups that own a block of output columns (block_q) and stage block_q + S - 1 source
     columns: widths that are and are not multiples of the block, blocks wider than what is left

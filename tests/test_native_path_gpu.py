@@ -72,6 +72,42 @@ def test_conv_under_autocast_and_in_any_layout(dtype, layout):
         _check(call, args)
 
 
+@pytest.mark.parametrize("fused", ["0", "1"])
+@pytest.mark.parametrize("p", [Conv2dGw8Params(2, 40, 13, 11, has_bias=True), Conv2dGw8Params(2, 16, 9, 9, 3),
+                               Conv2dGw8Params(9, 64, 7, 7, 2, 5, 5)], ids=lambda p: p.encode())  # fmt: skip
+def test_float32_tensors_that_kernels_read(p, fused, monkeypatch):
+    """Under autocast the kernels read float32 tensors themselves: whichever of input and weight is float32 and
+    wants a gradient, an input that is not 16-byte aligned, and one that is written to after the forward
+    pass, which used a copy of it (weights likewise)."""
+    monkeypatch.setenv("SPIO_FUSED_BACKWARD", fused)
+
+    def check(args, call):
+        def under_autocast(x, w, b):
+            with torch.autocast("cuda", dtype=torch.float16):
+                y = call(x, w, b)
+            with torch.no_grad():
+                for t in (x, w):
+                    if t.dtype == torch.float32:
+                        t.add_(1.0)
+            return y
+
+        _check(under_autocast, args)
+
+    for grads in ((True,) * 3, (True, False, False), (False, True, True), (False, False, True), (False,) * 3):
+        args, call = _conv_args(p, torch.float32, grads=grads)
+        if any(t is not None and t.requires_grad for t in args) or not any(grads):
+            check(args, call)
+    args, call = _conv_args(p, torch.float32)
+    check([args[0], args[1].detach().half().requires_grad_(), args[2]], call)
+    check([args[0].detach().half().requires_grad_(), *args[1:]], call)
+    storage = torch.randn(args[0].numel() + 1, device="cuda")
+    shifted = storage[1:].as_strided(args[0].shape, args[0].stride())
+    assert shifted.data_ptr() % 16 == 4
+    with torch.autocast("cuda", dtype=torch.float16):
+        y, expected = [call(t, args[1].detach(), args[2]) for t in (shifted, shifted.clone(memory_format=CL))]
+    assert torch.equal(y, expected)
+
+
 @pytest.mark.parametrize("weight,bias", [(True, True), (True, False), (False, True), (False, False)])
 def test_norm_matches_the_python_operator(weight, bias):
     torch.manual_seed(5)
