@@ -17,6 +17,12 @@
 // same C addresses, one after the other).  The small <name>_reduce kernel below adds the rows
 // into `sums[2][C]` (0 = grad_weight, 1 = grad_bias), which it overwrites.  HBM-bound: 4 bytes in,
 // 2 bytes out per element.
+//
+// The channel sums keep workgroups few (one or two per CU), so a wave has its own loads to wait for: the next
+// pass is requested before a pass is worked on.  With the instructions of a pass from 17.5 to 13.5 an element
+// (mixed-precision multiply-adds instead of conversions) and the second stage's loads four floats wide, both
+// stages: 128n 96c 56x56 (231 MB) 44.5 -> 41.3 us, 192c 28x28 26.6 -> 24.3, 384c 14x14 16.5 -> 15.3, 4n 96c
+// 56x56 6.9 -> 6.5; 768c 7x7 10.8, as before: two launches and a pass.
 #ifndef SPIO_LN_C
 #error "SPIO_LN_C, SPIO_LN_PIXELS, SPIO_LN_LPP, SPIO_LN_THREADS, SPIO_LN_GRID are required"
 #endif
@@ -32,6 +38,7 @@
 
 typedef _Float16 ln_half8 __attribute__((ext_vector_type(8)));
 typedef unsigned int ln_uint4 __attribute__((ext_vector_type(4)));
+typedef float ln_float4 __attribute__((ext_vector_type(4)));
 typedef __amdgpu_buffer_rsrc_t ln_rsrc;
 
 namespace {
@@ -47,6 +54,7 @@ constexpr int PPW = 64 / LPP;             // pixels per wave and pass
 constexpr int PPB = PPW * WAVES;          // pixels per workgroup and pass
 constexpr int UN = SPIO_LN_UNROLL;
 constexpr unsigned OOB = 0x80000000u;
+constexpr bool kAllLive = LPP * UPL == UNITS;  // no lane holds a unit past the pixel's last
 static_assert(C % 8 == 0 && (LPP & (LPP - 1)) == 0 && LPP <= 64 && LPP * UPL >= UNITS, "bad geometry");
 
 union Pack {
@@ -64,21 +72,39 @@ __device__ inline float lane_xor_add(float v, int m) {
     const int other = __builtin_amdgcn_ds_bpermute(((lane ^ m) << 2), __builtin_bit_cast(int, v));
     return v + __builtin_bit_cast(float, other);
 }
-// Sum over the LPP lanes of a pixel; every lane ends up with the total (as in the forward kernel).
-__device__ inline float pixel_sum(float v) {
-    if (LPP >= 2) v = dpp_add<0xB1>(v);    // quad_perm [1,0,3,2]
-    if (LPP >= 4) v = dpp_add<0x4E>(v);    // quad_perm [2,3,0,1]
-    if (LPP >= 8) v = dpp_add<0x141>(v);   // row_half_mirror
-    if (LPP >= 16) v = dpp_add<0x140>(v);  // row_mirror
+template <int CTRL>
+__device__ inline void dpp_add_all(float (&v)[UN]) {
 #pragma unroll
-    for (int m = 16; m < LPP; m <<= 1) v = lane_xor_add(v, m);
-    return v;
+    for (int u = 0; u < UN; ++u) v[u] = dpp_add<CTRL>(v[u]);
+}
+// Sums over the LPP lanes of each of UN pixels; every lane ends up with the totals (as in the forward kernel).
+__device__ inline void pixel_sums(float (&v)[UN]) {
+    if (LPP >= 2) dpp_add_all<0xB1>(v);    // quad_perm [1,0,3,2]
+    if (LPP >= 4) dpp_add_all<0x4E>(v);    // quad_perm [2,3,0,1]
+    if (LPP >= 8) dpp_add_all<0x141>(v);   // row_half_mirror
+    if (LPP >= 16) dpp_add_all<0x140>(v);  // row_mirror
+#pragma unroll
+    for (int m = 16; m < LPP; m <<= 1)
+#pragma unroll
+        for (int u = 0; u < UN; ++u) v[u] = lane_xor_add(v[u], m);
 }
 // Sum over the PPW lanes of a wave that hold the same channels (lanes sub, sub + LPP, ...).
 __device__ inline float channel_sum(float v) {
 #pragma unroll
     for (int m = LPP; m < 64; m <<= 1) v = lane_xor_add(v, m);
     return v;
+}
+
+// Eight fp32 values of a [C] vector from byte offset `off` on; zeros where that is OOB.
+__device__ inline void load_channels(float (&v)[8], const float* p, unsigned off) {
+    const ln_rsrc rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p), 0, C * 4, 0x00020000);
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        const ln_float4 q =
+            __builtin_bit_cast(ln_float4, __builtin_amdgcn_raw_buffer_load_b128(rs, (int)(off + 16 * h), 0, 0));
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[4 * h + e] = q[e];
+    }
 }
 
 }  // namespace
@@ -94,14 +120,21 @@ SPIO_KERNEL_NAME(float* __restrict__ partials, ln_uint4* __restrict__ din, const
     const int sub = lane % LPP;
     const int pix_in_pass = wave * PPW + lane / LPP;
 
+    // SGPRs of 1 and -0 that the compiler does not know for constants: (float)h * one + c and (float)h * w + zero
+    // are single mixed-precision instructions, where h + c and h * w are a conversion and another one (and the
+    // same values).
+    float one = 1.f, zero = -0.f;
+    asm("" : "+s"(one), "+s"(zero));
+
     float w[UPL][8];
     bool live[UPL];
 #pragma unroll
     for (int k = 0; k < UPL; ++k) {
         const int unit = sub + k * LPP;
-        live[k] = unit < UNITS;
+        live[k] = kAllLive || unit < UNITS;
 #pragma unroll
-        for (int e = 0; e < 8; ++e) w[k][e] = (SPIO_LN_HAS_WEIGHT && live[k]) ? weight[unit * 8 + e] : 1.f;
+        for (int e = 0; e < 8; ++e) w[k][e] = 1.f;
+        if (SPIO_LN_HAS_WEIGHT) load_channels(w[k], weight, live[k] ? unit * 32 : OOB);
     }
     float dw[UPL][8], db[UPL][8];
 #pragma unroll
@@ -109,80 +142,146 @@ SPIO_KERNEL_NAME(float* __restrict__ partials, ln_uint4* __restrict__ din, const
 #pragma unroll
         for (int e = 0; e < 8; ++e) dw[k][e] = db[k][e] = 0.f;
 
-    constexpr long long PASS_PIXELS = (long long)PPB * UN;
-    const long long passes = (PIXELS + PASS_PIXELS - 1) / PASS_PIXELS;
-    for (long long it = (long long)__builtin_amdgcn_workgroup_id_x(); it < passes; it += num_workgroups) {
-        const long long first = it * PASS_PIXELS;
-        const long long left = PIXELS - first;
-        const int npix = (int)(left < PASS_PIXELS ? left : PASS_PIXELS);
-        // 32-bit buffer offsets cover 2 GiB: the descriptors are rebased per iteration
-        const ln_rsrc rs_in = __builtin_amdgcn_make_buffer_rsrc(
-            const_cast<unsigned char*>(reinterpret_cast<const unsigned char*>(in)) + first * C * 2, 0, npix * C * 2,
-            0x00020000);
-        const ln_rsrc rs_dout = __builtin_amdgcn_make_buffer_rsrc(
-            const_cast<unsigned char*>(reinterpret_cast<const unsigned char*>(dout)) + first * C * 2, 0, npix * C * 2,
-            0x00020000);
-        const ln_rsrc rs_din = __builtin_amdgcn_make_buffer_rsrc(
-            reinterpret_cast<unsigned char*>(din) + first * C * 2, 0, npix * C * 2, 0x00020000);
-
-        Pack vx[UN][UPL], vd[UN][UPL];
-        unsigned off[UN][UPL];
+    unsigned off[UN][UPL];
 #pragma unroll
-        for (int u = 0; u < UN; ++u) {
-            const int pix = u * PPB + pix_in_pass;
+    for (int u = 0; u < UN; ++u)
+#pragma unroll
+        for (int k = 0; k < UPL; ++k)
+            off[u][k] = live[k] ? (unsigned)(((u * PPB + pix_in_pass) * UNITS + sub + k * LPP) * 16) : OOB;
+
+    constexpr long long PASS_PIXELS = (long long)PPB * UN;
+    constexpr long long PASSES = (PIXELS + PASS_PIXELS - 1) / PASS_PIXELS;
+    static_assert(num_workgroups <= PASSES, "every workgroup has a pass");
+    // 32-bit buffer offsets cover 2 GiB: the descriptors are rebased per pass.  Passes behind the last one
+    // have descriptors of size zero: loads give zeros, stores are dropped.
+    auto pass_rsrc = [&](const void* base, long long it) {
+        const long long first = it < PASSES ? it * PASS_PIXELS : 0;
+        const long long left = it < PASSES ? PIXELS - first : 0;
+        const int npix = (int)(left < PASS_PIXELS ? left : PASS_PIXELS);
+        return __builtin_amdgcn_make_buffer_rsrc(
+            const_cast<unsigned char*>(reinterpret_cast<const unsigned char*>(base)) + first * C * 2, 0, npix * C * 2,
+            0x00020000);
+    };
+    auto load_pass = [&](Pack(&vx)[UN][UPL], Pack(&vd)[UN][UPL], long long it) {
+        const ln_rsrc rs_in = pass_rsrc(in, it), rs_dout = pass_rsrc(dout, it);
+#pragma unroll
+        for (int u = 0; u < UN; ++u)
 #pragma unroll
             for (int k = 0; k < UPL; ++k) {
-                off[u][k] = live[k] ? (unsigned)((pix * UNITS + sub + k * LPP) * 16) : OOB;
                 vx[u][k].u = __builtin_amdgcn_raw_buffer_load_b128(rs_in, (int)off[u][k], 0, 2);
                 vd[u][k].u = __builtin_amdgcn_raw_buffer_load_b128(rs_dout, (int)off[u][k], 0, 2);
             }
-        }
+    };
+    // Statistics as in the forward kernel (pixels past the end and dead units load zeros: rstd is finite, every
+    // product below is zero, their stores are dropped).  The sums of all UN pixels take each step of their
+    // butterflies together: one alone would wait for every step.
+    auto work_pass = [&](const Pack(&vx)[UN][UPL], const Pack(&vd)[UN][UPL], long long it) {
+        float mean[UN], rstd[UN], m1[UN], m2[UN];
 #pragma unroll
         for (int u = 0; u < UN; ++u) {
-            // statistics as in the forward kernel (pixels past the end load zeros: rstd is finite,
-            // every product below is zero, their stores are dropped)
-            float x[UPL][8];
-            float s = 0.f;
+            float s[2] = {0.f, 0.f};  // two chains of additions: few pixels in flight wait for one
+#pragma unroll
+            for (int k = 0; k < UPL; ++k)
+#pragma unroll
+                for (int e = 0; e < 8; ++e) s[e & 1] = __builtin_fmaf((float)vx[u][k].h[e], one, s[e & 1]);
+            mean[u] = s[0] + s[1];
+        }
+        pixel_sums(mean);
+        float xhat[UN][UPL][8], g[UN][UPL][8];
+#pragma unroll
+        for (int u = 0; u < UN; ++u) {
+            float s[2] = {0.f, 0.f};
+#pragma unroll
+            for (int k = 0; k < UPL; ++k) {
+                const float nmean = live[k] ? mean[u] * (-1.0f / C) : 0.f;  // x - mean is zero in dead units
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    xhat[u][k][e] = __builtin_fmaf((float)vx[u][k].h[e], one, nmean);
+                    s[e & 1] = __builtin_fmaf(xhat[u][k][e], xhat[u][k][e], s[e & 1]);
+                }
+            }
+            rstd[u] = s[0] + s[1];
+        }
+        pixel_sums(rstd);
+        // xhat, g = dy * w, the two means, the channel sums
+#pragma unroll
+        for (int u = 0; u < UN; ++u) {
+            rstd[u] = __builtin_amdgcn_rsqf(rstd[u] * (1.0f / C) + SPIO_LN_EPS);
+            m1[u] = m2[u] = 0.f;
 #pragma unroll
             for (int k = 0; k < UPL; ++k)
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
-                    x[k][e] = (float)vx[u][k].h[e];
-                    s += x[k][e];
+                    const float dy = (float)vd[u][k].h[e];
+                    xhat[u][k][e] *= rstd[u];
+                    g[u][k][e] = SPIO_LN_HAS_WEIGHT ? __builtin_fmaf(dy, w[k][e], zero) : dy;
+                    m1[u] += g[u][k][e];
+                    m2[u] = __builtin_fmaf(g[u][k][e], xhat[u][k][e], m2[u]);
+                    dw[k][e] = __builtin_fmaf(dy, xhat[u][k][e], dw[k][e]);
+                    db[k][e] = __builtin_fmaf(dy, one, db[k][e]);
                 }
-            const float mean = pixel_sum(s) * (1.0f / C);
-            float d2 = 0.f;
+        }
+        pixel_sums(m1);
+        pixel_sums(m2);
+        const ln_rsrc rs_din = pass_rsrc(din, it);
 #pragma unroll
-            for (int k = 0; k < UPL; ++k)
-#pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    const float d = x[k][e] - mean;
-                    d2 += live[k] ? d * d : 0.f;
-                }
-            const float rstd = __builtin_amdgcn_rsqf(pixel_sum(d2) * (1.0f / C) + SPIO_LN_EPS);
-            // xhat (in place of x), g = dy * w, the two means, the channel sums
-            float g[UPL][8];
-            float sg = 0.f, sgx = 0.f;
-#pragma unroll
-            for (int k = 0; k < UPL; ++k)
-#pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    const float dy = (float)vd[u][k].h[e];  // dead units loaded zeros
-                    x[k][e] = live[k] ? (x[k][e] - mean) * rstd : 0.f;
-                    g[k][e] = dy * w[k][e];
-                    sg += g[k][e];
-                    sgx += g[k][e] * x[k][e];
-                    dw[k][e] += dy * x[k][e];
-                    db[k][e] += dy;
-                }
-            const float m1 = pixel_sum(sg) * (1.0f / C);
-            const float m2 = pixel_sum(sgx) * (1.0f / C);
+        for (int u = 0; u < UN; ++u) {
+            const float c1 = -rstd[u] * (m1[u] * (1.0f / C)), c2 = -rstd[u] * (m2[u] * (1.0f / C));
 #pragma unroll
             for (int k = 0; k < UPL; ++k) {
                 Pack o;
 #pragma unroll
-                for (int e = 0; e < 8; ++e) o.h[e] = (_Float16)(rstd * (g[k][e] - m1 - x[k][e] * m2));
+                for (int e = 0; e < 8; ++e)
+                    o.h[e] = (_Float16)__builtin_fmaf(xhat[u][k][e], c2, __builtin_fmaf(g[u][k][e], rstd[u], c1));
                 __builtin_amdgcn_raw_buffer_store_b128(o.u, rs_din, (int)off[u][k], 0, 2);
+            }
+        }
+    };
+
+    // The next pass is requested before this one is worked on.  Stores and loads leave one queue in order, so a
+    // wait for the loads of a pass counts what was issued behind them: the stores of the pass before and the
+    // loads of the next one.  The first pass has no stores before it and gets dropped ones in their place;
+    // without them the count that fits every pass would wait for the stores too.
+    Pack vx0[UN][UPL], vd0[UN][UPL], vx1[UN][UPL], vd1[UN][UPL];
+    // What a turn ends with in flight counts as used there: left unused on that way out the loads would be moved
+    // behind the branch, next to their use.
+    auto drop_pass = [&](const Pack(&vx)[UN][UPL], const Pack(&vd)[UN][UPL]) {
+#pragma unroll
+        for (int u = 0; u < UN; ++u)
+#pragma unroll
+            for (int k = 0; k < UPL; ++k) asm volatile("" ::"v"(vx[u][k].u), "v"(vd[u][k].u));
+    };
+    long long it = (long long)__builtin_amdgcn_workgroup_id_x();
+    load_pass(vx0, vd0, it);
+    if (PASSES <= num_workgroups) {
+        work_pass(vx0, vd0, it);
+    } else {
+        __builtin_amdgcn_sched_barrier(0);
+        const ln_rsrc none = pass_rsrc(din, PASSES);
+#pragma unroll
+        for (int u = 0; u < UN; ++u)
+#pragma unroll
+            for (int k = 0; k < UPL; ++k)
+                __builtin_amdgcn_raw_buffer_store_b128(ln_uint4{0u, 0u, 0u, 0u}, none, (int)off[u][k], 0, 2);
+        __builtin_amdgcn_sched_barrier(0);
+        while (true) {  // (no workgroup is without a pass)
+            load_pass(vx1, vd1, it + num_workgroups);
+            __builtin_amdgcn_sched_barrier(0);
+            work_pass(vx0, vd0, it);
+            __builtin_amdgcn_sched_barrier(0);
+            it += num_workgroups;
+            if (it >= PASSES) {
+                drop_pass(vx1, vd1);
+                break;
+            }
+            load_pass(vx0, vd0, it + num_workgroups);
+            __builtin_amdgcn_sched_barrier(0);
+            work_pass(vx1, vd1, it);
+            __builtin_amdgcn_sched_barrier(0);
+            it += num_workgroups;
+            if (it >= PASSES) {
+                drop_pass(vx0, vd0);
+                break;
             }
         }
     }
@@ -219,31 +318,32 @@ SPIO_KERNEL_NAME(float* __restrict__ partials, ln_uint4* __restrict__ din, const
 }
 
 // Second stage: sums[i] = sum over the workgroups' rows of partials[row][i], i < 2*C.  A workgroup
-// owns 32 columns; its 8 slices each add the rows r = slice, slice + 8, ... with up to 32 loads
-// in flight, and meet in LDS.  Every element has one owner: no atomics, no dependence on timing.
+// owns 32 columns, 4 to a thread; its 32 slices each add the rows r = slice, slice + 32, ... with up to 16
+// loads in flight (one round trip to memory for up to 512 rows), and meet in LDS.  Every element has one
+// owner: no atomics, no dependence on timing.
 #define SPIO_LN_CONCAT2(a, b) a##b
 #define SPIO_LN_CONCAT(a, b) SPIO_LN_CONCAT2(a, b)
 extern "C" __global__ void __attribute__((amdgpu_flat_work_group_size(256, 256)))
-SPIO_LN_CONCAT(SPIO_KERNEL_NAME, _reduce)(float* __restrict__ sums, const float* __restrict__ partials) {
+SPIO_LN_CONCAT(SPIO_KERNEL_NAME, _reduce)(float* __restrict__ sums, const ln_float4* __restrict__ partials) {
     constexpr int ROWS = SPIO_LN_GRID;
-    constexpr int COLS = 32;
+    constexpr int COLS = 8;  // float4 columns of a workgroup
     constexpr int SLICES = 256 / COLS;
-    // as many rows in flight per thread as a slice has, up to 32: one round trip to memory for up
-    // to 256 rows (with 8 in flight the stage took 1.5-2 us longer on the 7x7 and 14x14 shapes)
-    constexpr int UNR = (ROWS + SLICES - 1) / SLICES < 32 ? (ROWS + SLICES - 1) / SLICES : 32;
-    __shared__ float red[SLICES][COLS];
+    constexpr int UNR = (ROWS + SLICES - 1) / SLICES < 16 ? (ROWS + SLICES - 1) / SLICES : 16;
+    constexpr int ROW_F4 = 2 * C / 4;
+    __shared__ ln_float4 red[SLICES][COLS];
     const int tid = (int)__builtin_amdgcn_workitem_id_x();
     const int cl = tid % COLS;
     const int slice = tid / COLS;
     const int col = (int)__builtin_amdgcn_workgroup_id_x() * COLS + cl;
-    float sum = 0.f;
-    if (col < 2 * C) {
+    ln_float4 sum = ln_float4{0.f, 0.f, 0.f, 0.f};
+    if (col < ROW_F4) {
         for (int base = slice; base < ROWS; base += SLICES * UNR) {
-            float v[UNR];
+            ln_float4 v[UNR];
 #pragma unroll
             for (int i = 0; i < UNR; ++i) {
                 const int r = base + i * SLICES;
-                v[i] = r < ROWS ? partials[(long long)r * 2 * C + col] : 0.f;
+                v[i] = ln_float4{0.f, 0.f, 0.f, 0.f};
+                if (r < ROWS) v[i] = partials[(long long)r * ROW_F4 + col];
             }
 #pragma unroll
             for (int i = 0; i < UNR; ++i) sum += v[i];
@@ -253,10 +353,13 @@ SPIO_LN_CONCAT(SPIO_KERNEL_NAME, _reduce)(float* __restrict__ sums, const float*
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-    if (slice == 0 && col < 2 * C) {
+    // one wave adds the slices, a float each: thread t < 32 column t
+    const int out = (int)__builtin_amdgcn_workgroup_id_x() * COLS * 4 + tid;
+    if (tid < COLS * 4 && out < 2 * C) {
+        const float* flat = reinterpret_cast<const float*>(red) + tid;
+        float total = 0.f;
 #pragma unroll
-        for (int i = 1; i < SLICES; ++i) sum += red[i][cl];
-        sums[col] = sum;
+        for (int i = 0; i < SLICES; ++i) total += flat[i * COLS * 4];
+        sums[out] = total;
     }
 }
-

@@ -133,6 +133,42 @@ def test_every_backward_configuration_of_one_shape():
         kernel.unload()
 
 
+@pytest.mark.parametrize("pixels", [(1, 1, 1), (1, 5, 103), (1, 129, 8), (2, 32, 48), (1, 41, 101)])
+@pytest.mark.parametrize("c", [8, 96, 256])
+def test_backward_passes_of_a_workgroup(pixels, c):
+    """The backward kernel works on a pass with the next one's loads in flight: one pass in all, one for every
+    workgroup, several, a last pass of one pixel, idle lanes (c = 96) and weights that are only 4-byte aligned."""
+    attr = get_device_attributes(0)
+    n, h, w_ = pixels
+    g = torch.Generator().manual_seed(c + n * h * w_)
+    x = (torch.randn((n, c, h, w_), generator=g) * 2 + 0.5).half()
+    dy = torch.randn((n, c, h, w_), generator=g).half()
+    w = torch.randn(c + 1, generator=g)
+    eps = 1e-6
+    ex_dx, ex_dw, ex_db = _reference_backward(x, dy, w[1:], torch.zeros(c), eps)
+    xg = x.cuda().contiguous(memory_format=torch.channels_last)
+    dyg = dy.cuda().contiguous(memory_format=torch.channels_last)
+    wg = w.cuda()[1:]
+    # Channel sums of up to 4141 products of 1 and 2 in fp32, in another order: 4141 * 2^-24 * 3 of the largest.
+    close = dict(rtol=2e-3, atol=3e-2)
+    params = LayerNorm2dParams(n=n, c=c, h=h, w=w_, eps=eps, has_bias=False)
+
+    class FewUnits:  # enough passes for one workgroup without large tensors
+        multiprocessor_count = 4
+
+    for config in layernorm_2d_bwd_kernel_factory.configs(params, attr):
+        kernel = layernorm_2d_bwd_kernel_factory.make_kernel(params, config, FewUnits)
+        kernel.compile()
+        kernel.load(0)
+        dx, sums = torch.full_like(xg, -42.0), torch.full((2, c), float("nan"), device="cuda")
+        kernel(sums, dx, xg, dyg, wg)
+        torch.cuda.synchronize()
+        kernel.unload()
+        torch.testing.assert_close(dx.float().cpu(), ex_dx, rtol=4e-3, atol=4e-3, msg=str(config))
+        torch.testing.assert_close(sums[0].cpu(), ex_dw, **close, msg=str(config))
+        torch.testing.assert_close(sums[1].cpu(), ex_db, **close, msg=str(config))
+
+
 def _random_layernorm_params(seed, count):
     import random
 
