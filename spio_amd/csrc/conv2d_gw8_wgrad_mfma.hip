@@ -36,6 +36,14 @@
 //     a group to finish" was measured and rejected: the device-scope
 //     release/acquire fences it needs write back and invalidate the L2 of an
 //     XCD and cost more than the atomics they save.)
+//   * The row loads do not stop at the end of an image block: they run on into the next one while the last
+//     rows of this one are multiplied, so that only a workgroup's first block waits a memory latency for its
+//     first row.  A step (barrier, fragment reads, ring writes, MFMAs) takes about 0.4 us on a compute unit
+//     whatever is in it, so what bounds small images is the number of steps of the longest workgroup: the host
+//     deals equal shares.  Rows in the padding or past the block go through an empty descriptor and cost no
+//     traffic; the clamped loads that stood here before fetched a real row for each, PF of them per image
+//     block.  20n 1024c 27x27 5x5 48.6 -> 43.8 us, with equal shares (3 images instead of 8 and 2 blocks of two) 25.3;
+//     77n 168c 20x20 7x7 32.5 -> 21.1, 300n 88c 17x17 5x5 30.1 -> 19.6, 184n 288c 31x31 3x3 45.0 -> 41.4.
 //   * With SPIO_HAS_BIAS the kernel takes a fourth pointer, grad_bias ([K]
 //     fp32, accumulated into like grad_weight; null = not wanted), and sums dy
 //     per channel in the same pass: one more MFMA per chunk and row pair with
@@ -71,6 +79,9 @@ using namespace spio;
 #endif
 #ifndef SPIO_PIPE
 #define SPIO_PIPE 0
+#endif
+#ifndef SPIO_MAX_UNROLL
+#define SPIO_MAX_UNROLL 64
 #endif
 
 namespace {
@@ -149,7 +160,7 @@ constexpr int STEPS = (ROWS + RB - 1) / RB;  // barrier-separated steps of RB ro
 // after the last one nothing at all.  It starts at the first step with a real x row, with the dy
 // rows up to that step staged in the prologue, and stops after the last.  (Not with the bias
 // sum, which takes its row pairs at fixed steps.)
-constexpr bool kSkipPadding = PBLKS == 1 && !kDbias;
+constexpr bool kSkipPadding = PBLKS == 1 && !kDbias && (ROWS + RB - 1) / RB <= SPIO_MAX_UNROLL;
 constexpr int T_FIRST = kSkipPadding ? kPadY : 0;
 constexpr int T_END = kSkipPadding && kH + kPadY < ROWS ? kH + kPadY : ROWS;
 constexpr int S0 = T_FIRST / RB;               // first step
@@ -158,11 +169,9 @@ constexpr int LEAD = S0 * RB;                  // dy rows staged ahead of the fi
 // A workgroup that owns whole images unrolls its step loop completely, up to SPIO_MAX_UNROLL
 // steps (every condition on the step is then known at compile time); other loops run in chunks
 // of PF steps.
-#ifndef SPIO_MAX_UNROLL
-#define SPIO_MAX_UNROLL 64
-#endif
 constexpr bool kFullUnroll = PBLKS == 1 && S1 - S0 <= SPIO_MAX_UNROLL;
-constexpr int UNROLL = kFullUnroll ? (S1 - S0 + PF - 1) / PF * PF : PF;
+constexpr int SLOTS = (S1 - S0 + PF - 1) / PF * PF;  // steps of an image block, rounded up to whole rounds of the register buffers
+constexpr int UNROLL = kFullUnroll ? SLOTS : PF;
 constexpr int NPAIR = kR / 2 + 1;            // aligned dy row pairs one step can touch
 constexpr int CPW = (KC + TS - 1) / TS;      // 32-pixel chunks per wave
 
@@ -192,6 +201,27 @@ constexpr int PART_WAVE_FLOATS = kR * NBLK * 4 * 32;  // floats one wave publish
 // for channels past the last one.
 constexpr long long BIAS_PARTIALS = (long long)NBLKS * PBLKS * QBLKS * GBLKS * GB * PART_WAVE_FLOATS;
 
+
+constexpr long long X_ROW_BYTES = (long long)kW * kGroups * 16, X_IMAGE_BYTES = kH * X_ROW_BYTES;
+constexpr long long D_ROW_BYTES = (long long)kQ * kGroups * 16, D_IMAGE_BYTES = kP * D_ROW_BYTES;
+// Whether a row is read through a descriptor that begins at it, or through one of its image block with the row
+// as the scalar offset.  Unrolled loops know the row at compile time and take the former (20n 1024c 27x27 5x5
+// 23.6 us, 28.6 with scalar offsets); in others it is 64-bit arithmetic for every
+// row (64n 64c 56x56 16.1 us, with scalar offsets 14.8; 32n 48c 224x224 66.0 and 63.5).  It is also the one for
+// images that side by side exceed 32-bit offsets.
+constexpr bool kRowDescriptors = kFullUnroll || NB * X_IMAGE_BYTES + (kPadY + BH + kR) * X_ROW_BYTES >= (1ll << 31) ||
+                              NB * D_IMAGE_BYTES + (BH + kR) * D_ROW_BYTES >= (1ll << 31);
+static_assert((NB - 1) * X_IMAGE_BYTES + X_ROW_BYTES < (1ll << 31) && (NB - 1) * D_IMAGE_BYTES + D_ROW_BYTES < (1ll << 31),
+              "a row of all images side by side lies within 32-bit buffer offsets");
+constexpr int OUT_OF_RANGE = (int)0x80000000u;  // as an unsigned offset behind the end of every descriptor
+constexpr bool kSplitLines = splits_lines(GB, GBLKS);
+// Non-temporal, but for lines that channel blocks straddle (blocks that are halves of whole lines: 64n 64c
+// 56x56 14.3 us with the default policy, 13.7 non-temporal, 20n 1024c 27x27 5x5 25.6 and 23.7).
+constexpr int AUX_LD = kSplitLines && kC % 64 != 0 ? 0 : 2;
+typedef __amdgpu_buffer_rsrc_t rsrc_t;
+SPIO_DEVICE rsrc_t make_rsrc(const void* base, int bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, bytes, 0x00020000);
+}
 
 SPIO_DEVICE spio_half8 read_tr_pair(const unsigned char* lo, const unsigned char* hi) {
     typedef spio_short4 __attribute__((address_space(3))) * lds_ptr;
@@ -230,7 +260,6 @@ SPIO_KERNEL_NAME(float* __restrict__ grad_weight, const spio_uint4* __restrict__
     // then row blocks.  Where channel blocks share lines they go fastest, so that the lines are fetched
     // from memory once.
     const int b = xcd_tile<0, NUM_BLOCKS>(block_id());
-    constexpr bool kSplitLines = splits_lines(GB, GBLKS);
     constexpr int TILES = QBLKS * PBLKS;
     const int tile = kSplitLines ? (b / GBLKS) % TILES : b % TILES;
     const int cb = kSplitLines ? b % GBLKS : (b / TILES) % GBLKS;
@@ -264,113 +293,133 @@ SPIO_KERNEL_NAME(float* __restrict__ grad_weight, const spio_uint4* __restrict__
     spio_float4 accb = spio_float4{0.f, 0.f, 0.f, 0.f};
     const spio_half8 ones8 = spio_half8{1, 1, 1, 1, 1, 1, 1, 1};
     (void)ones8;
-    const long long xrow_units = (long long)kW * kGroups;
-    const long long drow_units = (long long)kQ * kGroups;
+    // ---- addressing ----
+    // Every thread issues the same loads in every slot, without branches, so that the compiler counts
+    // outstanding loads exactly and a step waits only for the rows it needs (a load under a branch makes it
+    // wait for all of them, which would serialise the prefetch).  The images are read
+    // through a buffer descriptor that ends with the last image that exists; lanes without data (halo columns, missing groups) carry an offset no descriptor reaches,
+    // and a row that nobody needs has an empty one: such loads give zeros and touch no memory.  (Threads
+    // beyond the last cell skip their LDS writes; letting them write spare cells instead, to make the
+    // writes branch-free, costs 14 % at N=256, C=256, 14x14, 7x7.)
+    int x_off[LPTX], x_lds[LPTX];
+#pragma unroll
+    for (int l = 0; l < LPTX; ++l) {
+        const int cell = tid + THREADS * l;
+        x_off[l] = OUT_OF_RANGE;
+        x_lds[l] = -1;
+        if (cell < X_CELLS) {
+            const int g = cell % GB;
+            const int f = cell / GB;
+            const int img = f / WPI;
+            const int col = q0 + f % WPI - kPadX;
+            x_lds[l] = g * GSX + x_image_offset(img) + f % WPI;
+            if (col >= 0 && col < kW && cb * GB + g < kGroups)
+                x_off[l] = (int)(img * X_IMAGE_BYTES) + (col * kGroups + cb * GB + g) * 16;
+        }
+    }
+    int d_off[LPTD], d_lds[LPTD];
+#pragma unroll
+    for (int l = 0; l < LPTD; ++l) {
+        const int cell = tid + THREADS * l;
+        d_off[l] = OUT_OF_RANGE;
+        d_lds[l] = -1;
+        if (cell < D_CELLS) {
+            const int g = cell % GB;
+            const int q = (cell / GB) % BQ;
+            const int img = cell / (GB * BQ);
+            d_lds[l] = g * GSD + d_image_offset(img) + q;
+            if (q0 + q < kQ && cb * GB + g < kGroups)
+                d_off[l] = (int)(img * D_IMAGE_BYTES) + ((q0 + q) * kGroups + cb * GB + g) * 16;
+        }
+    }
+    const spio_uint4 zero4 = spio_uint4{0u, 0u, 0u, 0u};
+
+    // Row t of the current image block (ahead = 0) or of the next one (1).
+    const int nfirst = nbk * ITERS * NB;
+    const unsigned char* xbase[2] = {};
+    const unsigned char* dbase[2] = {};
+    int images[2] = {};
+    auto enter_block = [&](int it) {
+#pragma unroll
+        for (int ahead = 0; ahead < (ITERS > 1 ? 2 : 1); ++ahead) {
+            const int n0 = nfirst + (it + ahead) * NB;
+            images[ahead] = it + ahead < ITERS ? imin(imax(kN - n0, 0), NB) : 0;
+            xbase[ahead] = reinterpret_cast<const unsigned char*>(x) + (images[ahead] > 0 ? n0 : 0) * X_IMAGE_BYTES;
+            dbase[ahead] = reinterpret_cast<const unsigned char*>(dy) + (images[ahead] > 0 ? n0 : 0) * D_IMAGE_BYTES;
+        }
+    };
+    auto load_x = [&](int ahead, int t, spio_uint4(&v)[LPTX]) {
+        const int h = p0 + t - kPadY;
+        const int n = t < ROWS && h >= 0 && h < kH ? images[ahead] : 0;
+        const rsrc_t rs = kRowDescriptors ? make_rsrc(xbase[ahead] + (n > 0 ? h : 0) * X_ROW_BYTES,
+                                                   n > 0 ? (int)((n - 1) * X_IMAGE_BYTES + X_ROW_BYTES) : 0)
+                                       : make_rsrc(xbase[ahead], (int)(n * X_IMAGE_BYTES));
+        const int row = kRowDescriptors ? 0 : h * (int)X_ROW_BYTES;
+#pragma unroll
+        for (int l = 0; l < LPTX; ++l) v[l] = __builtin_amdgcn_raw_buffer_load_b128(rs, x_off[l], row, AUX_LD);
+    };
+    auto load_dy = [&](int ahead, int t, spio_uint4(&v)[LPTD]) {
+        const int n = t < bh_eff ? images[ahead] : 0;
+        const rsrc_t rs = kRowDescriptors ? make_rsrc(dbase[ahead] + (n > 0 ? p0 + t : 0) * D_ROW_BYTES,
+                                                   n > 0 ? (int)((n - 1) * D_IMAGE_BYTES + D_ROW_BYTES) : 0)
+                                       : make_rsrc(dbase[ahead], (int)(n * D_IMAGE_BYTES));
+        const int row = kRowDescriptors ? 0 : (p0 + t) * (int)D_ROW_BYTES;
+#pragma unroll
+        for (int l = 0; l < LPTD; ++l) v[l] = __builtin_amdgcn_raw_buffer_load_b128(rs, d_off[l], row, AUX_LD);
+    };
+    // The loads run PF slots ahead of the steps and straight on into the next image block: step S0 + i is slot
+    // i, and SLOTS, a multiple of PF, holds an image block, so that the register buffer of a slot is known at
+    // compile time.
+    spio_uint4 xpre[PF][RB][LPTX], dpre[PF][RB][LPTD];
+    spio_uint4 dlead[LEAD > 0 ? LEAD : 1][LPTD];
+    auto load_slot = [&](int ahead, int slot, int buffer) {
+#pragma unroll
+        for (int rr = 0; rr < RB; ++rr) {
+            if (kFullUnroll && slot >= S1 - S0) continue;
+            const int t = slot < S1 - S0 ? (S0 + slot) * RB + rr : ROWS + BH;  // a slot without a step: no rows
+            load_x(ahead, t, xpre[buffer][rr]);
+            load_dy(ahead, t, dpre[buffer][rr]);
+        }
+    };
+    auto load_lead = [&](int ahead) {
+#pragma unroll
+        for (int i = 0; i < LEAD; ++i) load_dy(ahead, i, dlead[i]);
+    };
+    enter_block(0);
+    load_lead(0);
+#pragma unroll
+    for (int slot = 0; slot < PF; ++slot) {
+        load_slot(0, slot, slot);
+        // in the order they are needed: loads return in order, and with the first slot's requested last the
+        // first step waits for all of them (20n 1024c 27x27 5x5 25.3 us, 23.6 in order)
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    // zero both rings once, while the first loads are in flight: halo, gap and slack cells are never
+    // written again
+    for (int i = tid; i < NRX * XROW_UNITS; i += THREADS) xring[i] = zero4;
+    for (int i = tid; i < NRD * DROW_UNITS; i += THREADS) dring[i] = zero4;
+    block_sync();
 
     for (int it = 0; it < ITERS; ++it) {
-        const int n0 = (nbk * ITERS + it) * NB;
-        if (n0 >= kN) break;
+        if (nfirst + it * NB >= kN) break;
+        if (it > 0) enter_block(it);
 
-        // ---- loop-invariant addressing for this image block ----
-        // Every thread issues the same loads on every step, without branches, so that the
-        // compiler counts outstanding loads exactly and a step waits only for the rows it
-        // needs (a load under a branch makes it wait for all of them, which would serialise the
-        // prefetch).  Cells without data (halo columns, missing images or groups) and rows
-        // outside the tensor load a valid address and become zero when written to LDS.  (Threads
-        // beyond the last cell skip their LDS writes; letting them write spare cells instead, to
-        // make the writes branch-free, costs 14 % at N=256, C=256, 14x14, 7x7.)
-        int x_off[LPTX], x_lds[LPTX];
-        bool x_ok[LPTX];
-        const int x_dummy = n0 * kH * kW * kGroups;
-#pragma unroll
-        for (int l = 0; l < LPTX; ++l) {
-            const int cell = tid + THREADS * l;
-            x_off[l] = x_dummy;
-            x_ok[l] = false;
-            x_lds[l] = -1;
-            if (cell < X_CELLS) {
-                const int g = cell % GB;
-                const int f = cell / GB;
-                const int img = f / WPI;
-                const int col = q0 + f % WPI - kPadX;
-                x_lds[l] = g * GSX + x_image_offset(img) + f % WPI;
-                if (col >= 0 && col < kW && n0 + img < kN && cb * GB + g < kGroups) {
-                    x_off[l] = ((n0 + img) * kH * kW + col) * kGroups + cb * GB + g;
-                    x_ok[l] = true;
-                }
-            }
-        }
-        int d_off[LPTD], d_lds[LPTD];
-        bool d_ok[LPTD];
-        const int d_dummy = n0 * kP * kQ * kGroups;
-#pragma unroll
-        for (int l = 0; l < LPTD; ++l) {
-            const int cell = tid + THREADS * l;
-            d_off[l] = d_dummy;
-            d_ok[l] = false;
-            d_lds[l] = -1;
-            if (cell < D_CELLS) {
-                const int g = cell % GB;
-                const int q = (cell / GB) % BQ;
-                const int img = cell / (GB * BQ);
-                d_lds[l] = g * GSD + d_image_offset(img) + q;
-                if (q0 + q < kQ && n0 + img < kN && cb * GB + g < kGroups) {
-                    d_off[l] = ((n0 + img) * kP * kQ + q0 + q) * kGroups + cb * GB + g;
-                    d_ok[l] = true;
-                }
-            }
-        }
-        const spio_uint4 zero4 = spio_uint4{0u, 0u, 0u, 0u};
-
-        // ---- prologue: steps S0..S0+PF-1 into registers, step S0 (and the dy rows before it)
-        //      into LDS ----
-        spio_uint4 xpre[PF][RB][LPTX], dpre[PF][RB][LPTD];
-        spio_uint4 dlead[LEAD > 0 ? LEAD : 1][LPTD];
+        // ---- step S0 and the dy rows before it into LDS (every step ends with a barrier: the rings are free) ----
 #pragma unroll
         for (int i = 0; i < LEAD; ++i) {
-            const int pr = imin(p0 + i, kP - 1);
-#pragma unroll
-            for (int l = 0; l < LPTD; ++l) dlead[i][l] = load_stream(dy + d_off[l] + pr * drow_units);
-        }
-#pragma unroll
-        for (int sp = 0; sp < PF; ++sp) {
-#pragma unroll
-            for (int rr = 0; rr < RB; ++rr) {
-                const int t = (S0 + sp) * RB + rr;
-                const int h = imin(imax(p0 + t - kPadY, 0), kH - 1);
-#pragma unroll
-                for (int l = 0; l < LPTX; ++l) xpre[sp][rr][l] = load_stream(x + x_off[l] + h * xrow_units);
-                const int pr = imin(p0 + t, kP - 1);
-#pragma unroll
-                for (int l = 0; l < LPTD; ++l) dpre[sp][rr][l] = load_stream(dy + d_off[l] + pr * drow_units);
-            }
-        }
-        if (it == 0) {
-            // zero both rings once, while the first loads are in flight: halo, gap and slack
-            // cells are never written again
-            for (int i = tid; i < NRX * XROW_UNITS; i += THREADS) xring[i] = zero4;
-            for (int i = tid; i < NRD * DROW_UNITS; i += THREADS) dring[i] = zero4;
-        }
-        block_sync();  // rings zeroed / previous image block finished
-#pragma unroll
-        for (int i = 0; i < LEAD; ++i) {
-            const bool drow_ok = i < bh_eff;
 #pragma unroll
             for (int l = 0; l < LPTD; ++l)
-                if (d_lds[l] >= 0) dring[(i % NRD) * DROW_UNITS + d_lds[l]] = (drow_ok && d_ok[l]) ? dlead[i][l] : zero4;
+                if (d_lds[l] >= 0) dring[(i % NRD) * DROW_UNITS + d_lds[l]] = dlead[i][l];
         }
 #pragma unroll
         for (int rr = 0; rr < RB; ++rr) {
             const int t = S0 * RB + rr;
-            const int h = p0 + t - kPadY;
-            const bool xrow_ok = h >= 0 && h < kH;
 #pragma unroll
             for (int l = 0; l < LPTX; ++l)
-                if (x_lds[l] >= 0) xring[((S0 & 1) * RB + rr) * XROW_UNITS + x_lds[l]] = (xrow_ok && x_ok[l]) ? xpre[0][rr][l] : zero4;
-            const bool drow_ok = t < bh_eff;
+                if (x_lds[l] >= 0) xring[((S0 & 1) * RB + rr) * XROW_UNITS + x_lds[l]] = xpre[0][rr][l];
 #pragma unroll
             for (int l = 0; l < LPTD; ++l)
-                if (d_lds[l] >= 0) dring[(t % NRD) * DROW_UNITS + d_lds[l]] = (drow_ok && d_ok[l]) ? dpre[0][rr][l] : zero4;
+                if (d_lds[l] >= 0) dring[(t % NRD) * DROW_UNITS + d_lds[l]] = dpre[0][rr][l];
         }
         block_sync();
 
@@ -447,21 +496,17 @@ SPIO_KERNEL_NAME(float* __restrict__ grad_weight, const spio_uint4* __restrict__
                 if (m == 0 && pl.bias_pair) accb = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[ci][0], ones8, accb, 0, 0, 0);
             }
         };
-        // 2. prefetch step st+PF (its register buffer held step st, now in LDS); rows past the end
-        //    repeat a real row and are never used
-        auto prefetch_rows = [&](int st, int uf) {
-#pragma unroll
-            for (int rr = 0; rr < RB; ++rr) {
-                const int t2 = (st + PF) * RB + rr;
-                const int h = imin(imax(p0 + t2 - kPadY, 0), kH - 1);
-#pragma unroll
-                for (int l = 0; l < LPTX; ++l) xpre[uf % PF][rr][l] = load_stream(x + x_off[l] + h * xrow_units);
-                const int pr = imin(p0 + t2, kP - 1);
-#pragma unroll
-                for (int l = 0; l < LPTD; ++l) dpre[uf % PF][rr][l] = load_stream(dy + d_off[l] + pr * drow_units);
-            }
+        // 2. the slot PF ahead: its register buffer held this slot's rows, now in LDS
+        auto prefetch_rows = [&](int slot, int uf) {
+            const bool next = slot + PF >= SLOTS;
+            const int ahead = next ? slot + PF - SLOTS : slot + PF;
+            if (LEAD > 0 && ITERS > 1 && next && ahead == 0) load_lead(1);  // (the loop is unrolled)
+            if (ITERS > 1)
+                load_slot(next, ahead, uf % PF);
+            else if (!kFullUnroll || !next)
+                load_slot(0, slot + PF, uf % PF);
         };
-        // 3. the rows of step st+1 into LDS (dy rows past the block's last row become zero).  The
+        // 3. the rows of step st+1 into LDS (dy rows past the block's last row are zeros).  The
         //    ring rows written here are not read in this step, except for dy entries whose filter
         //    row is out of range and whose product is ignored.
         auto stage_x = [&](int st, int sp, int uf) {
@@ -474,8 +519,7 @@ SPIO_KERNEL_NAME(float* __restrict__ grad_weight, const spio_uint4* __restrict__
 #pragma unroll
                     for (int l = 0; l < LPTX; ++l)
                         if (x_lds[l] >= 0)
-                            xring[(((sp + 1) & 1) * RB + rr) * XROW_UNITS + x_lds[l]] =
-                                x_ok[l] ? xpre[(uf + 1) % PF][rr][l] : zero4;
+                            xring[(((sp + 1) & 1) * RB + rr) * XROW_UNITS + x_lds[l]] = xpre[(uf + 1) % PF][rr][l];
                 }
             }
         };
@@ -485,11 +529,9 @@ SPIO_KERNEL_NAME(float* __restrict__ grad_weight, const spio_uint4* __restrict__
             for (int rr = 0; rr < RB; ++rr) {
                 const int tn = (st + 1) * RB + rr;
                 const int dslot = tn % NRD;
-                const bool drow_ok = tn < bh_eff;
 #pragma unroll
                 for (int l = 0; l < LPTD; ++l)
-                    if (d_lds[l] >= 0)
-                        dring[dslot * DROW_UNITS + d_lds[l]] = (drow_ok && d_ok[l]) ? dpre[(uf + 1) % PF][rr][l] : zero4;
+                    if (d_lds[l] >= 0) dring[dslot * DROW_UNITS + d_lds[l]] = dpre[(uf + 1) % PF][rr][l];
             }
         };
 
@@ -501,11 +543,18 @@ SPIO_KERNEL_NAME(float* __restrict__ grad_weight, const spio_uint4* __restrict__
         constexpr int FSETS = SPIO_PIPE ? 2 : 1;
         constexpr int GROUPS = CPW * NPAIR;
         spio_half8 bfrag[FSETS][CPW][RB][NBLK], afrag[FSETS][CPW][NPAIR];
-        for (int sb = S0; sb < S1; sb += UNROLL) {
+        for (int sb = 0; sb < SLOTS; sb += UNROLL) {
 #pragma unroll
             for (int uf = 0; uf < UNROLL; ++uf) {
-                const int st = sb + uf;
-                if (st >= S1) break;
+                const int slot = sb + uf;
+                const int st = S0 + slot;
+                // A slot without a step has the loads only; where the loop is not unrolled it runs through the
+                // same code as the others (with nothing to read, stage or multiply), because loads on two paths
+                // would cost the exact counts.
+                if (kFullUnroll && st >= S1) {
+                    prefetch_rows(slot, uf);
+                    continue;
+                }
                 // PF is even, so the parity of the step is known at compile time: it fixes the
                 // x ring rows and, with one row per step, the parity of delta.
                 const int sp = (S0 + uf) & 1;
@@ -517,10 +566,10 @@ SPIO_KERNEL_NAME(float* __restrict__ grad_weight, const spio_uint4* __restrict__
                     for (int g = 0; g < GROUPS; ++g) {
                         const int ci = g / NPAIR, m = g % NPAIR;
                         if (pl.do_math) read_group(pl, sp, ci, m, bfrag[fs], afrag[fs]);
-                        if (g == 0) prefetch_rows(st, uf);
+                        if (g == 0) prefetch_rows(slot, uf);
                         if (g == (GROUPS > 1 ? 1 : 0)) stage_x(st, sp, uf);
                         if (g == (GROUPS > 2 ? 2 : GROUPS - 1)) stage_dy(st, uf);
-                        if (st > S0 && before.do_math) multiply_group(before, sp ^ 1, ci, m, bfrag[fs ^ 1], afrag[fs ^ 1]);
+                        if (st > S0 && st < S1 && before.do_math) multiply_group(before, sp ^ 1, ci, m, bfrag[fs ^ 1], afrag[fs ^ 1]);
                         __builtin_amdgcn_sched_barrier(0);
                     }
                 } else {
@@ -529,7 +578,7 @@ SPIO_KERNEL_NAME(float* __restrict__ grad_weight, const spio_uint4* __restrict__
 #pragma unroll
                         for (int g = 0; g < GROUPS; ++g) read_group(pl, sp, g / NPAIR, g % NPAIR, bfrag[0], afrag[0]);
                     }
-                    prefetch_rows(st, uf);
+                    prefetch_rows(slot, uf);
                     stage_x(st, sp, uf);
                     stage_dy(st, uf);
                     if (pl.do_math) {
