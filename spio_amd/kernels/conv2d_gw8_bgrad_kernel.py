@@ -18,9 +18,10 @@ from typing import Dict, List, Tuple
 
 import torch
 
-from ..util.math import divup
+from ..util.math import balanced, divup
 from .conv2d_gw8_kernel import _shape_defines, fits_float32_output, with_joined_stores
 from .conv2d_gw8_params import Conv2dGw8Params
+from .conv2d_gw8_wgrad_kernel import image_block_runs
 from .conv2d_stats import Conv2dStats
 from .kernel import KernelSpec
 from .kernel_factory import KernelFactory
@@ -170,7 +171,7 @@ def _config_is_legal(params, config) -> bool:
         and 0 <= config.block_q <= bgrad_domain(params)[1]
         and (config.block_q == 0 or (config.block_q % 32 == 0 and config.block_n == 1))
         and g["LPTD"] <= MAX_LOADS_PER_THREAD
-        and config.block_n * config.block_n_iters <= max(params.n, 1)
+        and config.block_n <= max(params.n, 1) and config.block_n * (config.block_n_iters - 1) < max(params.n, 1)
         and g["LDS_BYTES"] <= MAX_LDS_BYTES
         and g["LPTX"] <= MAX_LOADS_PER_THREAD
         and g["REGISTERS"] <= MAX_REGISTERS
@@ -185,6 +186,8 @@ def _score(params, config, num_cus) -> float:
     g = bgrad_geometry(params, config)
     group_eff = params.groups / (g["GBLKS"] * config.groups)
     quant = divup(g["NUM_BLOCKS"], num_cus) * num_cus / g["NUM_BLOCKS"]
+    quant *= g["PBLKS"] * g["BH"] / bgrad_domain(params)[0]  # the last, shorter tiles
+    quant *= g["NBLKS"] * config.block_n * config.block_n_iters / params.n
     halo = 1.0 + (2.0 / 3.0) * (params.r - 1 if g["PBLKS"] > 1 else 0) / g["BH"]
     dh, dw = bgrad_domain(params)
     stream_us = halo * 6.0 * params.n * params.c * dh * dw / 5.0e6
@@ -205,7 +208,7 @@ def _get_configs(params: Conv2dGw8Params, device_attr=None) -> List[Conv2dGw8Bgr
     # whether whole images or row blocks win depends on the shape in ways the score does not
     # capture (contiguity of the channel block, halo re-reads, workgroups per compute unit).
     dh, dw = bgrad_domain(params)
-    row_choices = [0] + sorted({bh for bh in (7, 14, 28) if bh < dh}, reverse=True)
+    row_choices = [0] + balanced(dh, [bh for bh in (7, 14, 28) if bh < dh])[::-1]
     # images side by side: powers of two, and for rows shorter than a 32-pixel chunk of the weight
     # gradient's contraction the counts that fill the chunks clearly better (as in the
     # weight-gradient kernel's configuration space)
@@ -226,7 +229,8 @@ def _get_configs(params: Conv2dGw8Params, device_attr=None) -> List[Conv2dGw8Bgr
         for bq in col_choices:
             for gb in group_choices:
                 for nb in image_counts if bq == 0 else (1,):
-                    for iters in (1, 2, 4):
+                    tiles = divup(G, gb) * divup(dh, bh or dh) * divup(dw, bq or dw)
+                    for iters in image_block_runs(divup(params.n, nb), tiles, num_cus, (1, 2, 4)):
                         for ts in (1, 2):
                             cfg = Conv2dGw8BgradConfig(groups=gb, block_h=bh, block_n=nb, block_n_iters=iters,
                                                        prefetch=4, split=ts, block_q=bq)  # fmt: skip

@@ -15,7 +15,7 @@ from typing import Dict, List
 
 import torch
 
-from ..util.math import divup
+from ..util.math import balanced, divup
 from .conv2d_gw8_params import Conv2dGw8Params
 from .conv2d_stats import Conv2dStats
 from .kernel import KernelSpec
@@ -36,7 +36,7 @@ MAX_IMAGE_CONFIGS = 10  # whole-image configurations that enter the sweep
 MOVER_WAVES = 4  # data-mover waves of the whole-image kernel where it has any: one per SIMD
 PREFETCH_CHOICES = (2, 4, 8, 10, 12, 16)
 COLUMN_BLOCK_CHOICES = (64, 128, 256)  # output columns per workgroup where rows are tiled
-MAX_GEOMETRIES = 30  # tile geometries that enter the sweep; the best few also try the other cache/XCD policies
+MAX_GEOMETRIES = 40  # tile geometries that enter the sweep; the best few also try the other cache/XCD policies
 
 
 @dataclass(frozen=True)
@@ -386,9 +386,10 @@ def _get_configs(params: Conv2dGw8Params, device_attr=None, igrad: bool = False)
     num_cus = getattr(device_attr, "multiprocessor_count", 256) or 256
     G = params.groups
     group_choices = sorted({g for g in (4, 8, 16, G) if g <= min(G, MAX_WAVES)}) or [min(G, MAX_WAVES)]
-    row_choices = sorted({bp for bp in (2, 4, 7, 8, 14, 16, 28, 32, 56, d["DH"]) if bp <= d["DH"]})
+    row_choices = balanced(d["DH"], (2, 4, 7, 8, 14, 16, 28, 32, 56, d["DH"]))
     # column blocks for wide rows only: narrower ones fit whole and pay no column halo
-    col_choices = [0] + [bq for bq in COLUMN_BLOCK_CHOICES if d["DW"] >= 2 * bq and d["DW"] > 128]
+    col_choices = [bq for bq in COLUMN_BLOCK_CHOICES if d["DW"] >= 2 * bq and d["DW"] > 128]
+    col_choices = [0] + sorted({*col_choices, *balanced(d["DW"], col_choices)})
     found = []
     for bq in col_choices:
         for gb in group_choices:
@@ -403,7 +404,14 @@ def _get_configs(params: Conv2dGw8Params, device_attr=None, igrad: bool = False)
                             if _mfma_config_is_legal(params, cfg, igrad):
                                 found.append((_mfma_score(params, cfg, igrad, num_cus), cfg))
     found.sort(key=lambda sc: sc[0])
-    configs = [cfg for _, cfg in found[:MAX_GEOMETRIES]]
+    # two prefetch distances of a geometry first, then the others: a capped sweep sees more geometries
+    head, rest = [], []
+    for _, cfg in found:
+        shape = replace(cfg, prefetch=0)
+        (head if sum(replace(h, prefetch=0) == shape for h in head[-16:]) < 2 else rest).append(cfg)
+        if len(head) >= MAX_GEOMETRIES:
+            break
+    configs = [*head[:8], *sorted(head[8:] + rest, key=lambda c: _mfma_score(params, c, igrad, num_cus))][:MAX_GEOMETRIES]
     # the memory-system policies, which the score cannot rank: halo rows with or without the
     # non-temporal hint, and how tiles are dealt to the XCDs
     leading = []  # the first four tile geometries, whatever their prefetch depth

@@ -15,7 +15,7 @@ from typing import Dict, List
 
 import torch
 
-from ..util.math import divup
+from ..util.math import balanced, divup
 from .conv2d_gw8_kernel import _shape_defines
 from .conv2d_gw8_params import Conv2dGw8Params
 from .conv2d_stats import Conv2dStats
@@ -30,8 +30,9 @@ MAX_WAVES = 16
 MAX_LDS_BYTES = 128 * 1024
 MAX_LOADS_PER_THREAD = 8
 MAX_ACCUMULATORS = 32
-MAX_GEOMETRIES = 16
+MAX_GEOMETRIES = 20
 PIPELINE_CHOICES = ((2, 1, 0), (4, 1, 0), (2, 2, 0), (2, 1, 1), (4, 1, 1))  # (prefetch, rows, pipe)
+LEADING_PIPELINES = 3  # of these, for the leading geometries at the head of the list
 
 
 @dataclass(frozen=True)
@@ -142,7 +143,7 @@ def _mfma_config_is_legal(params, config) -> bool:
         config.groups * config.split <= MAX_WAVES
         and config.split <= g["KC"]
         and config.block_h <= params.p
-        and config.block_n * config.block_n_iters <= max(params.n, 1)
+        and config.block_n <= max(params.n, 1) and config.block_n * (config.block_n_iters - 1) < max(params.n, 1)
         and g["LDS_BYTES"] <= MAX_LDS_BYTES
         and g["LPTX"] <= MAX_LOADS_PER_THREAD
         and g["ND"] * g["NBLK"] <= MAX_ACCUMULATORS
@@ -152,9 +153,26 @@ def _mfma_config_is_legal(params, config) -> bool:
         and config.pipe in (0, 1)
         and 0 <= config.block_q <= params.q
         and (g["LPTX"] + g["LPTD"]) * config.prefetch * config.rows <= 32
-        # the kernel indexes both tensors in 16-byte units with 32-bit integers
+        # one row of all images side by side lies within 32-bit buffer offsets
+        and ((config.block_n - 1) * max(params.h * params.w, params.p * params.q) + max(params.w, params.q))
+        * params.c * 2 < 2**31
+        # general bound on the tensors' 16-byte units
         and params.n * params.groups * max(params.h * params.w, params.p * params.q) < 2**31
     )
+
+
+def image_block_runs(blocks: int, tiles: int, num_cus: int, sizes) -> List[int]:
+    """Image blocks a workgroup takes one after the other: as many workgroups as `sizes` give, but with equal
+    shares, and those with which the grid of `tiles` per image block is one or two whole rounds of the device.
+
+    A round lasts as long as its longest workgroup.  Weight gradient 20n 1024c 27x27 5x5, two images a block:
+    runs of 8 are 8 and 2 blocks."""
+    runs = set(balanced(blocks, sizes))
+    for rounds in (1, 2):
+        workgroups = min(blocks, num_cus * rounds // tiles)
+        if workgroups:
+            runs.add(divup(blocks, workgroups))
+    return sorted(r for r in runs if r <= 16)
 
 
 def _mfma_score(params, config, num_cus) -> float:
@@ -163,8 +181,10 @@ def _mfma_score(params, config, num_cus) -> float:
     halo = (config.block_h + params.r - 1) / config.block_h
     traffic = 1.0 + 0.5 * (halo - 1.0) + 0.25 * (params.s - 1) / g["BQ"]
     group_eff = params.groups / (g["GBLKS"] * config.groups)
-    # compute units idle in the last round of workgroups
+    # compute units idle in the last round of workgroups, and in the last, shorter tiles
     quant = divup(g["NUM_BLOCKS"], num_cus) * num_cus / g["NUM_BLOCKS"]
+    quant *= g["PBLKS"] * config.block_h / params.p * g["NBLKS"] * config.block_n * config.block_n_iters / params.n
+    quant *= g["QBLKS"] * g["BQ"] / params.q
     # Publishing costs R*S*64 values per (workgroup, group): atomics retire at roughly 128 per
     # clock device-wide; partial stores plus the reduction kernel cost bandwidth and a launch.
     stream_bytes = 4.0 * params.n * params.c * params.h * params.w
@@ -174,8 +194,13 @@ def _mfma_score(params, config, num_cus) -> float:
         publish_us = 4.5 + 2.0 * 4.0 * values / 5.0e6
     else:
         publish_us = values / (128 * 2.1e3)
-    split_line = 1.0 if (config.groups * 16) % 128 == 0 or config.groups == params.groups else 1.12
-    return (traffic * quant * split_line / (g["PIXEL_EFF"] ** 0.3 * group_eff)) * (
+    # blocks of part of a line; they cost more where a pixel is not whole lines, so that blocks straddle them
+    # (184n 288c 31x31 3x3: 4 groups 50.4 us, 8 groups, of which the last block has half, 42.1)
+    split_line = 1.0 if (config.groups * 16) % 128 == 0 or config.groups == params.groups else (
+        1.12 if params.c % 64 == 0 else 1.2)
+    # fewer waves than SIMDs (14n 24c 167x167 3x3: 3 waves 21.1 us, 6 waves 19.4)
+    few_waves = 1.15 if g["THREADS"] < 256 else 1.0
+    return (traffic * quant * split_line * few_waves / (g["PIXEL_EFF"] ** 0.3 * group_eff)) * (
         1.0 + publish_us / stream_us
     )
 
@@ -188,7 +213,7 @@ def _get_configs(params: Conv2dGw8Params, device_attr=None) -> List[Conv2dGw8Wgr
     # (96 channels: 12 groups = 2 x 6)
     group_choices = sorted({g for g in (4, 8, 16, G, G // 2 if G % 2 == 0 and G & (G - 1) else G)
                             if 0 < g <= min(G, MAX_WAVES)}) or [min(G, MAX_WAVES)]
-    row_choices = sorted({bh for bh in (4, 7, 8, 14, 16, 28, 32, 56, params.p) if bh <= params.p})
+    row_choices = balanced(params.p, (4, 7, 8, 14, 16, 28, 32, 56, params.p))
     # Images side by side.  The contraction runs over 32-pixel chunks of the flattened row, so
     # where a padded image row is shorter than a chunk the count decides how full the chunks
     # are: besides the powers of two, the counts that fill them clearly better (7x7 images with
@@ -203,13 +228,15 @@ def _get_configs(params: Conv2dGw8Params, device_attr=None) -> List[Conv2dGw8Wgr
     # Rank the tile geometries first and keep the best few; each of them is then tried with the
     # pipeline variants (prefetch distance, rows per step), which the score cannot tell apart.
     # column blocks for wide rows only: narrower ones fit whole
-    col_choices = [0] + [bq for bq in (64, 128, 256) if params.q >= 2 * bq and params.q > 128]
+    col_choices = [bq for bq in (64, 128, 256) if params.q >= 2 * bq and params.q > 128]
+    col_choices = [0] + sorted({*col_choices, *balanced(params.q, col_choices)})
     geometries = []
     for bq in col_choices:
         for gb in group_choices:
             for nb in image_counts if bq == 0 else (1,):
-                for iters in (1, 2, 4, 8):
-                    for bh in row_choices:
+                for bh in row_choices:
+                    tiles = divup(G, gb) * divup(params.p, bh) * divup(params.q, bq or params.q)
+                    for iters in image_block_runs(divup(params.n, nb), tiles, num_cus, (1, 2, 4, 8)):
                         for two_stage in (0, 1):
                             for ts in (1, 2):
                                 cfg = Conv2dGw8WgradConfig(groups=gb, block_h=bh, block_n=nb, block_n_iters=iters,
@@ -217,14 +244,17 @@ def _get_configs(params: Conv2dGw8Params, device_attr=None) -> List[Conv2dGw8Wgr
                                 if _mfma_config_is_legal(params, cfg):
                                     geometries.append((_mfma_score(params, cfg, num_cus), cfg))
     geometries.sort(key=lambda sc: sc[0])
-    configs = []
-    for _, base in geometries[:MAX_GEOMETRIES]:
-        for pf, rows, pipe in PIPELINE_CHOICES:
+    # The head of the list, which is all that a sweep inside an operator call tries, holds three geometries:
+    # the score is not good enough to spend it on the pipelines of one.
+    head, rest = [], []
+    for i, (_, base) in enumerate(geometries[:MAX_GEOMETRIES]):
+        for j, (pf, rows, pipe) in enumerate(PIPELINE_CHOICES):
             if pf > 2 and pf * rows > base.block_h + params.r - 1:
                 continue
             cfg = replace(base, prefetch=pf, rows=rows, pipe=pipe)
             if _mfma_config_is_legal(params, cfg):
-                configs.append(cfg)
+                (head if i < 3 and j < LEADING_PIPELINES else rest).append(cfg)
+    configs = head + rest
     total_pix = params.n * params.p * params.q
     chunks = max(1, min(divup(8 * num_cus, params.groups), divup(total_pix, 64)))
     configs.append(Conv2dGw8WgradConfig(groups=1, block_h=1, block_n=1, block_n_iters=1,

@@ -20,3 +20,8 @@ def next_relative_prime(a: int, b: int) -> int:
             return r
         r += 1
     raise AssertionError(f"no number coprime to {b} in [{a}, {limit}]")
+
+
+def balanced(extent: int, sizes) -> list:
+    """Block sizes that cut `extent` into as many blocks as `sizes` do, but into nearly equal ones."""
+    return sorted({divup(extent, divup(extent, size)) for size in sizes if size <= extent})

@@ -382,6 +382,31 @@ FUSED = [p for p in SANITY if bgrad_is_supported(p) and list(conv2d_gw8_bgrad_ke
 ]
 
 
+def _runs(groups, block_h, block_n, iters, prefetch, **kw):
+    return Conv2dGw8WgradConfig(groups=groups, block_h=block_h, block_n=block_n, block_n_iters=iters, prefetch=prefetch, **kw)
+
+
+@pytest.mark.parametrize("params,configs", [
+    # whole images, the steps in the padding skipped; 9 and 14 steps against prefetch distances that do and do
+    # not divide them; 5 images in runs that end in the middle of a block of images and of a run
+    (Conv2dGw8Params(n=5, c=40, h=9, w=9, r=5, s=5, padding=2),
+     [_runs(4, 9, 2, 2, 2), _runs(4, 9, 1, 5, 4, pipe=1), _runs(5, 9, 2, 3, 8), _runs(4, 9, 3, 2, 4, rows=2)]),
+    (Conv2dGw8Params(n=7, c=64, h=14, w=14, r=7, s=7, padding=3),
+     [_runs(4, 14, 4, 2, 4, pipe=1, two_stage=1), _runs(4, 14, 2, 4, 2, rows=2), _runs(4, 14, 3, 3, 8)]),
+    # row blocks (loops that are not unrolled), the last one shorter, a bias, one with a single filter row
+    (Conv2dGw8Params(n=3, c=48, h=23, w=12, padding=1, has_bias=True),
+     [_runs(6, 8, 1, 3, 4), _runs(6, 12, 2, 2, 4, pipe=1), _runs(3, 5, 1, 2, 2, rows=2), _runs(6, 6, 2, 2, 8, split=1)]),
+    (Conv2dGw8Params(n=4, c=16, h=10, w=33, r=1, s=3, padding=(0, 1), has_bias=True),
+     [_runs(2, 4, 1, 3, 4), _runs(2, 10, 2, 2, 2, split=2)]),
+    # column blocks of equal width and a padding that crops
+    (Conv2dGw8Params(n=3, c=24, h=9, w=140, padding=0), [_runs(3, 7, 1, 3, 4, block_q=46), _runs(3, 4, 1, 2, 2, block_q=64)]),
+    # more rows than an unrolled loop takes, in one row block
+    (Conv2dGw8Params(n=2, c=16, h=70, w=8, padding=1), [_runs(2, 70, 1, 2, 4), _runs(2, 70, 1, 2, 2, pipe=1)]),
+], ids=lambda v: v.encode() if hasattr(v, "encode") else "")  # fmt: skip
+def test_weight_gradient_streams_on_into_the_next_image_block(params, configs):
+    run_grad_kernel_test(conv2d_gw8_wgrad_kernel_factory, params, configs=configs)
+
+
 @pytest.mark.parametrize("params", FUSED, ids=lambda p: p.encode())
 def test_bgrad_sanity(params):
     """Fused data + weight (+ bias) gradient kernel, first configurations of every shape."""

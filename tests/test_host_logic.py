@@ -452,3 +452,25 @@ def test_whole_image_configurations_offer_whole_rounds():
         shorter = ck.image_geometry(params, replace(first, block_n_iters=max(1, first.block_n_iters - 1)), False)
         assert g["NUM_BLOCKS"] <= 2 * 256 * resident
         assert first.block_n_iters == 1 or shorter["NUM_BLOCKS"] > g["NUM_BLOCKS"]
+
+
+def test_balanced_blocks_and_runs_of_image_blocks():
+    """Tiles cut an extent into as many blocks as the sizes asked for, nearly equal ones; runs of image blocks
+    leave no workgroup with a share much shorter than another's."""
+    from spio_amd.kernels.conv2d_gw8_wgrad_kernel import conv2d_gw8_wgrad_kernel_factory, image_block_runs
+    from spio_amd.util.math import balanced
+
+    assert balanced(57, (4, 14, 28, 57, 64)) == [4, 12, 19, 57] and balanced(56, (4, 14, 28)) == [4, 14, 28]
+    for extent in range(1, 80):
+        for size in range(1, extent + 1):
+            (block,) = balanced(extent, (size,))
+            assert block <= size and -(-extent // block) == -(-extent // size)
+    for blocks in (1, 2, 5, 10, 63, 500):
+        for tiles in (1, 32, 300):
+            runs = image_block_runs(blocks, tiles, 256, (1, 2, 4, 8))
+            assert 1 in runs or blocks == 1 and runs == [1]
+            assert all(1 <= r <= 16 for r in runs)
+    params = Conv2dGw8Params(n=20, c=1024, h=27, w=27, padding=2, r=5, s=5)
+    first = conv2d_gw8_wgrad_kernel_factory.configs(params, ATTR)[0]
+    images = first.block_n * first.block_n_iters
+    assert -(-params.n // images) * images <= params.n + 2  # runs of 8 of two images: 16 and 4
