@@ -211,6 +211,11 @@ constexpr long long D_ROW_BYTES = (long long)kQ * kGroups * 16, D_IMAGE_BYTES = 
 // images that side by side exceed 32-bit offsets.
 constexpr bool kRowDescriptors = kFullUnroll || NB * X_IMAGE_BYTES + (kPadY + BH + kR) * X_ROW_BYTES >= (1ll << 31) ||
                               NB * D_IMAGE_BYTES + (BH + kR) * D_ROW_BYTES >= (1ll << 31);
+// the first row asked for and the one that a slot without a step asks for, behind the last block
+constexpr int FIRST_ROW = -kPadY, IDLE_ROW = kP + ROWS + BH;
+static_assert(kRowDescriptors || (offset_row(FIRST_ROW, kH) >= 0 && offset_row(IDLE_ROW, kH) * X_ROW_BYTES < (1ll << 31) &&
+                                  offset_row(IDLE_ROW, kP) * D_ROW_BYTES < (1ll << 31)),
+              "row offsets stay within 32 bits, also those of rows that do not exist");
 static_assert((NB - 1) * X_IMAGE_BYTES + X_ROW_BYTES < (1ll << 31) && (NB - 1) * D_IMAGE_BYTES + D_ROW_BYTES < (1ll << 31),
               "a row of all images side by side lies within 32-bit buffer offsets");
 constexpr int OUT_OF_RANGE = (int)0x80000000u;  // as an unsigned offset behind the end of every descriptor
@@ -354,7 +359,7 @@ SPIO_KERNEL_NAME(float* __restrict__ grad_weight, const spio_uint4* __restrict__
         const rsrc_t rs = kRowDescriptors ? make_rsrc(xbase[ahead] + (n > 0 ? h : 0) * X_ROW_BYTES,
                                                    n > 0 ? (int)((n - 1) * X_IMAGE_BYTES + X_ROW_BYTES) : 0)
                                        : make_rsrc(xbase[ahead], (int)(n * X_IMAGE_BYTES));
-        const int row = kRowDescriptors ? 0 : h * (int)X_ROW_BYTES;
+        const int row = kRowDescriptors ? 0 : offset_row(h, kH) * (int)X_ROW_BYTES;
 #pragma unroll
         for (int l = 0; l < LPTX; ++l) v[l] = __builtin_amdgcn_raw_buffer_load_b128(rs, x_off[l], row, AUX_LD);
     };
@@ -363,7 +368,7 @@ SPIO_KERNEL_NAME(float* __restrict__ grad_weight, const spio_uint4* __restrict__
         const rsrc_t rs = kRowDescriptors ? make_rsrc(dbase[ahead] + (n > 0 ? p0 + t : 0) * D_ROW_BYTES,
                                                    n > 0 ? (int)((n - 1) * D_IMAGE_BYTES + D_ROW_BYTES) : 0)
                                        : make_rsrc(dbase[ahead], (int)(n * D_IMAGE_BYTES));
-        const int row = kRowDescriptors ? 0 : (p0 + t) * (int)D_ROW_BYTES;
+        const int row = kRowDescriptors ? 0 : offset_row(p0 + t, kP) * (int)D_ROW_BYTES;
 #pragma unroll
         for (int l = 0; l < LPTD; ++l) v[l] = __builtin_amdgcn_raw_buffer_load_b128(rs, d_off[l], row, AUX_LD);
     };

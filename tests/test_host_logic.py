@@ -9,10 +9,13 @@ from dataclasses import replace
 import pytest
 
 from helpers import reference_test_params
+from spio_amd.compiler.compile import compile_hip
+from spio_amd.compiler.compile_kernel import kernel_headers, read_source
 from spio_amd.hip import DeviceAttributes
 from spio_amd.kernels import (
     Conv2dGw8Config,
     Conv2dGw8Params,
+    Conv2dGw8WgradConfig,
     KernelCache,
     KernelFactory,
     KernelKey,
@@ -474,3 +477,18 @@ def test_balanced_blocks_and_runs_of_image_blocks():
     first = conv2d_gw8_wgrad_kernel_factory.configs(params, ATTR)[0]
     images = first.block_n * first.block_n_iters
     assert -(-params.n // images) * images <= params.n + 2  # runs of 8 of two images: 16 and 4
+
+
+def test_row_offsets_stay_within_32_bits():
+    """Rows in the padding and slots without a row have an offset inside the tensor: an image of almost 2 GiB,
+    where the rows a step or two behind it would overflow."""
+    params = Conv2dGw8Params(n=1, c=8, h=32748, w=4096, padding=1, r=3, s=3)
+    config = Conv2dGw8WgradConfig(groups=1, block_h=14, block_n=1, block_n_iters=1, prefetch=4, block_q=64)
+    defines = dict(conv2d_gw8_wgrad_kernel_factory.get_kernel_spec(params, config, ATTR).defines, SPIO_KERNEL_NAME="k")
+    source = read_source("conv2d_gw8_wgrad_mfma.hip") + """
+    static_assert(!kRowDescriptors, "offsets from the first row of an image");
+    static_assert(IDLE_ROW * X_ROW_BYTES >= (1ll << 31), "a row behind the image overflows");
+    static_assert(offset_row(FIRST_ROW, kH) == 0 && offset_row(0, kH) == 0 && offset_row(kH - 1, kH) == kH - 1);
+    static_assert(offset_row(IDLE_ROW, kH) == kH - 1 && offset_row(IDLE_ROW, kP) == kP - 1);
+    """
+    assert compile_hip(source, "row_offsets.hip", headers=kernel_headers(), defines=defines)
