@@ -45,6 +45,8 @@ HIPCC_DEVICE_FLAGS = [
     "-target-feature",
     "-Xclang",
     "-packed-fp32-ops",
+    "-mllvm",
+    "-pragma-unroll-threshold=200000",  # (as at run time, see compiler/compile.py)
 ]
 
 

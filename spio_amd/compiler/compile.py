@@ -17,8 +17,13 @@ from . import flags
 
 GFX_ARCH = "gfx950"
 
-# hipcc-side feature switch required for every device compilation here.
-_FEATURE_FLAGS = ["-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
+# hipcc-side feature switch required for every device compilation here, and the size up to which loops are unrolled
+# where a pragma asks for it.  The kernels index arrays of registers with the step of such a loop: one that the
+# compiler leaves rolled keeps them in memory.  The default, 16384, is below 56 steps of an ordinary tile
+# (weight gradient 64n 96c 56x56 7x7 493 -> 40 us, forward 512n 64c 56x56 with two images side by side 766 -> 82);
+# how long a loop may be is bounded where configurations are chosen.
+_FEATURE_FLAGS = ["-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+                  "-mllvm", "-pragma-unroll-threshold=200000"]  # fmt: skip
 
 
 def hiprtc_options(

@@ -8,6 +8,7 @@ pre-filled by a sentinel, and compare with the fp32 CPU oracle.
 import json
 import os
 import random
+import struct
 from dataclasses import replace
 from typing import List
 
@@ -15,7 +16,8 @@ import torch
 
 from oracle import conv2d_gw8_oracle as oracle
 from spio_amd.compiler import compile_kernel_configs
-from spio_amd.hip import get_device_attributes
+from spio_amd.compiler.compile_kernel import compile_kernel
+from spio_amd.hip import DeviceAttributes, get_device_attributes
 from spio_amd.kernels import Conv2dGw8Params, Conv2dStats
 
 DEAD_VALUE = -42.0  # every output element must be overwritten (run_test.py:23,64)
@@ -223,3 +225,23 @@ def run_bgrad_kernel_test(factory, params: Conv2dGw8Params, configs=None, seed=0
         oracle.check_close(dx, dx_e, acc_depth=d_dx, what=f"fused dgrad {what}")
         oracle.check_close(dw, dw_e, acc_depth=d_dw, what=f"fused wgrad {what}")
         kernel.unload()
+
+
+def scratch_bytes(factory, params, config, **kw) -> int:
+    """Bytes of memory a lane of a configuration's main kernel keeps registers in: the private segment size of its
+    kernel descriptor (the second word of <kernel>.kd) in the code object."""
+    spec = factory.get_kernel_spec(params, config, DeviceAttributes(), **kw)
+    code = compile_kernel(spec.source_file, dict(spec.defines, SPIO_KERNEL_NAME="k"))
+    section_table, = struct.unpack_from("<Q", code, 0x28)
+    entry, count = struct.unpack_from("<HH", code, 0x3A)
+    sections = [struct.unpack_from("<IIQQQQIIQQ", code, section_table + entry * i) for i in range(count)]
+    for _, kind, _, _, offset, size, link, _, _, each in sections:
+        if kind != 11:  # dynamic symbols
+            continue
+        for at in range(offset, offset + size, each):
+            name, _, _, section, value, _ = struct.unpack_from("<IBBHQQ", code, at)
+            start = sections[link][4] + name
+            if code[start:code.index(b"\0", start)] == b"k.kd":
+                _, _, _, address, file_offset = sections[section][:5]
+                return struct.unpack_from("<I", code, value - address + file_offset + 4)[0]
+    raise ValueError("no kernel descriptor")

@@ -8,7 +8,7 @@ from dataclasses import replace
 
 import pytest
 
-from helpers import reference_test_params
+from helpers import reference_test_params, scratch_bytes
 from spio_amd.compiler.compile import compile_hip
 from spio_amd.compiler.compile_kernel import kernel_headers, read_source
 from spio_amd.hip import DeviceAttributes
@@ -492,3 +492,23 @@ def test_row_offsets_stay_within_32_bits():
     static_assert(offset_row(IDLE_ROW, kH) == kH - 1 && offset_row(IDLE_ROW, kP) == kP - 1);
     """
     assert compile_hip(source, "row_offsets.hip", headers=kernel_headers(), defines=defines)
+
+
+@pytest.mark.parametrize("groups,prefetch,iters", [(4, 4, 1), (4, 4, 2)])
+def test_weight_gradient_of_whole_images_keeps_its_sums_in_registers(groups, prefetch, iters):
+    """Unrolled over 56 rows the step loop is long; left rolled it indexes the sums in memory."""
+    params = Conv2dGw8Params(n=64, c=96, h=56, w=56, padding=2, r=5, s=5, has_bias=True)
+    config = Conv2dGw8WgradConfig(groups=groups, block_h=56, prefetch=prefetch, block_n_iters=iters)
+    assert scratch_bytes(conv2d_gw8_wgrad_kernel_factory, params, config) == 0
+
+
+@pytest.mark.parametrize("config,kernel_size", [
+    (Conv2dGw8WgradConfig(groups=4, block_h=56, prefetch=2, two_stage=1), 7),
+    (Conv2dGw8WgradConfig(groups=8, block_h=56, block_n=2, prefetch=2), 3),
+    (Conv2dGw8Config(groups=8, block_p=56, block_n=2, prefetch=8), 3),
+])  # fmt: skip
+def test_long_loops_are_unrolled(config, kernel_size):
+    factory = conv2d_gw8_kernel_factory if isinstance(config, Conv2dGw8Config) else conv2d_gw8_wgrad_kernel_factory
+    params = Conv2dGw8Params(n=64, c=64 if kernel_size == 3 else 96, h=56, w=56, padding=kernel_size // 2,
+                             r=kernel_size, s=kernel_size, has_bias=True)  # fmt: skip
+    assert scratch_bytes(factory, params, config) == 0
