@@ -335,6 +335,21 @@ def test_column_blocks_weight_gradient_and_fused_backward():
         run_bgrad_kernel_test(conv2d_gw8_bgrad_kernel_factory, params, configs=bconfigs)
 
 
+@pytest.mark.parametrize("params,groups,images", [
+    (Conv2dGw8Params(n=5, c=40, h=9, w=8, r=5, s=5, padding=(0, 3), has_bias=False), 4, 4),
+    (Conv2dGw8Params(n=7, c=24, h=6, w=11, padding=(2, 0), has_bias=True), 2, 3),
+    (Conv2dGw8Params(n=3, c=16, h=4, w=5, r=7, s=3, padding=(3, 1), has_bias=False), 2, 2),
+    (Conv2dGw8Params(n=9, c=8, h=5, w=7, r=1, s=2, padding=0, has_bias=True), 1, 8),
+], ids=str)  # fmt: skip
+def test_weight_gradient_of_one_block_of_images(params, groups, images):
+    """One image block a workgroup, unrolled: a last block of one image, a last channel block of one group, rows in
+    the padding, threads without a cell."""
+    W = Conv2dGw8WgradConfig
+    configs = [W(groups=groups, block_h=params.p, block_n=images, **o) for o in (
+        dict(prefetch=2), dict(prefetch=2, rows=2), dict(prefetch=4, pipe=1, two_stage=1), dict(prefetch=2, rows=2, pipe=1))]
+    run_grad_kernel_test(conv2d_gw8_wgrad_kernel_factory, params, configs=configs)
+
+
 def test_weight_gradient_packed_images_skipped_padding_and_pipeline():
     """Small images under large filters: images sharing their halo columns, chunks that hold their
     own images (14x14 under 7x7: two per 32-pixel chunk; 10 wide under 3x3: three), whole-image
