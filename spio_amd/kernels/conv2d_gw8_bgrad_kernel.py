@@ -19,7 +19,7 @@ from typing import Dict, List, Tuple
 import torch
 
 from ..util.math import balanced, divup
-from .conv2d_gw8_kernel import _shape_defines, fits_float32_output, with_joined_stores
+from .conv2d_gw8_kernel import _policies_are_legal, _shape_defines, fits_float32_output, with_joined_stores
 from .conv2d_gw8_params import Conv2dGw8Params
 from .conv2d_gw8_wgrad_kernel import image_block_runs
 from .conv2d_stats import Conv2dStats
@@ -181,6 +181,15 @@ def _config_is_legal(params, config) -> bool:
     )
 
 
+def _recorded_config_is_legal(params, config) -> bool:
+    return (
+        min(config.groups, config.block_n, config.block_n_iters, config.split) >= 1
+        and config.two_stage in (0, 1)
+        and _policies_are_legal(config)
+        and _config_is_legal(params, config)
+    )
+
+
 def _score(params, config, num_cus) -> float:
     """Rough relative cost used only to order (and cap) the sweep; lower is better."""
     g = bgrad_geometry(params, config)
@@ -326,4 +335,5 @@ conv2d_gw8_bgrad_kernel_factory = KernelFactory(
     configs=_get_configs,
     kernel_spec=_get_kernel_spec,
     make_test_args=_make_test_args,
+    is_legal=_recorded_config_is_legal,
 )

@@ -315,6 +315,20 @@ def _mfma_config_is_legal(params, config, igrad) -> bool:
     )
 
 
+def _policies_are_legal(config) -> bool:
+    return config.nontemporal in (0, 1) and config.halo_cached in (0, 1) and config.xcd_chunk >= 0
+
+
+def _config_is_legal(params, config, igrad: bool = False) -> bool:
+    """Whether the row-streaming or the whole-image kernel can run a configuration."""
+    if min(config.groups, config.block_p, config.block_n, config.split, config.prefetch) < 1:
+        return False
+    if config.variant == "image":
+        return _policies_are_legal(config) and _image_config_is_legal(params, config, igrad)
+    return (config.variant == "mfma" and config.prefetch % 2 == 0 and _policies_are_legal(config)
+            and _mfma_config_is_legal(params, config, igrad))  # fmt: skip
+
+
 def _resident_workgroups(lds_bytes: int, threads: int) -> int:
     """Workgroups of one kernel a CU can hold (LDS and thread limits)."""
     return max(1, min(160 * 1024 // max(lds_bytes, 1), 2048 // threads, 8))
@@ -574,4 +588,5 @@ conv2d_gw8_kernel_factory = KernelFactory(
     configs=_get_configs,
     kernel_spec=_get_kernel_spec,
     make_test_args=_make_test_args,
+    is_legal=_config_is_legal,
 )

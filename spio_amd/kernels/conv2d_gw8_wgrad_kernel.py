@@ -161,6 +161,16 @@ def _mfma_config_is_legal(params, config) -> bool:
     )
 
 
+def _config_is_legal(params, config) -> bool:
+    """Whether the MFMA kernel can run a configuration."""
+    return (
+        config.variant == "mfma"
+        and min(config.groups, config.block_h, config.block_n, config.block_n_iters, config.split) >= 1
+        and config.two_stage in (0, 1)
+        and _mfma_config_is_legal(params, config)
+    )
+
+
 def image_block_runs(blocks: int, tiles: int, num_cus: int, sizes) -> List[int]:
     """Image blocks a workgroup takes one after the other: as many workgroups as `sizes` give, but with equal
     shares, and those with which the grid of `tiles` per image block is one or two whole rounds of the device.
@@ -347,4 +357,5 @@ conv2d_gw8_wgrad_kernel_factory = KernelFactory(
     configs=_get_configs,
     kernel_spec=_get_kernel_spec,
     make_test_args=_make_test_args,
+    is_legal=_config_is_legal,
 )

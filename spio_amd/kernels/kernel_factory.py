@@ -25,6 +25,7 @@ class KernelFactory:
         kernel_spec: Union[KernelSpec, Callable[..., KernelSpec]] = None,
         make_test_args: Callable[..., Any] = None,
         args_checker=check_channels_last,
+        is_legal: Callable[..., bool] = None,
     ):
         self.params_cls = params_cls
         self.config_cls = config_cls
@@ -34,6 +35,7 @@ class KernelFactory:
         self._kernel_spec = kernel_spec
         self._make_test_args = make_test_args
         self._args_checker = args_checker
+        self._is_legal = is_legal
         self._kernel_caches: Dict[str, KernelCache] = {}
 
     def configs(self, params, device_attr=None, **kwargs):
@@ -41,6 +43,14 @@ class KernelFactory:
         if callable(self._configs):
             return self._configs(params, device_attr, **kwargs)
         return self._configs
+
+    def is_legal(self, params, config, **kwargs) -> bool:
+        """Whether the kernel can run `config`, listed or not (a recorded one may be from a list of another time);
+        False where the family does not say."""
+        try:
+            return self._is_legal is not None and self._is_legal(params, config, **kwargs)
+        except (ArithmeticError, TypeError):  # a field of zero, of another type
+            return False
 
     def get_kernel_name(self, **kwargs) -> str:
         if callable(self._kernel_name):

@@ -196,7 +196,7 @@ class Tuner:
                     config = kernel_factory.config_cls(**record["config"])
                 except TypeError:
                     config = None
-                if config in configs:
+                if config in configs or (config and kernel_factory.is_legal(params, config, **kernel_kwargs)):
                     return compile_and_load_kernel(
                         kernel_factory, params, config, ordinal, device_attr, **kernel_kwargs
                     )

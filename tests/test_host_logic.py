@@ -13,6 +13,7 @@ from spio_amd.compiler.compile import compile_hip
 from spio_amd.compiler.compile_kernel import kernel_headers, read_source
 from spio_amd.hip import DeviceAttributes
 from spio_amd.kernels import (
+    Conv2dGw8BgradConfig,
     Conv2dGw8Config,
     Conv2dGw8Params,
     Conv2dGw8WgradConfig,
@@ -27,7 +28,7 @@ from spio_amd.kernels import (
     kernel_params_logging_is_enabled,
 )
 from spio_amd.kernels.conv2d_gw8_kernel import MAX_LDS_BYTES, image_geometry, mfma_geometry
-from spio_amd.kernels.tuner import Tuner, device_key
+from spio_amd.kernels.tuner import Tuner, config_to_dict, device_key
 
 ATTR = DeviceAttributes()
 
@@ -247,6 +248,36 @@ def test_tuner_record_store(tmp_path, monkeypatch):
     assert Tuner().lookup(ATTR, "k__x")["us"] == 12.5
     assert device_key(ATTR) == "gfx950_256cu"
     assert json.load(open(tmp_path / "db.json"))["k__x"]["config"] == {"groups": 8}
+
+
+@pytest.mark.parametrize("factory,mode,config,used", [
+    # tiles of an earlier list: heights that do not divide 56 rows evenly
+    (conv2d_gw8_kernel_factory, {}, Conv2dGw8Config(groups=8, block_p=16, prefetch=4), True),
+    (conv2d_gw8_kernel_factory, {"igrad": True}, Conv2dGw8Config(groups=8, block_p=16, prefetch=4), True),
+    (conv2d_gw8_wgrad_kernel_factory, {}, Conv2dGw8WgradConfig(groups=8, block_h=16), True),
+    (conv2d_gw8_bgrad_kernel_factory, {}, Conv2dGw8BgradConfig(groups=8, block_h=16), True),
+    # not a configuration of this kernel, or not one it can run
+    (conv2d_gw8_kernel_factory, {}, Conv2dGw8Config(groups=8, block_p=64, prefetch=4), False),
+    (conv2d_gw8_kernel_factory, {}, Conv2dGw8Config(groups=8, block_p=16, prefetch=4, halo_cached=2), False),
+    (conv2d_gw8_kernel_factory, {}, Conv2dGw8Config(groups=0, block_p=16, prefetch=4), False),
+    (conv2d_gw8_kernel_factory, {}, Conv2dGw8Config(groups=8, block_p=16, prefetch=None), False),
+    (conv2d_gw8_wgrad_kernel_factory, {}, Conv2dGw8WgradConfig(groups=8, block_h=16, block_n_iters=0), False),
+    (conv2d_gw8_bgrad_kernel_factory, {}, Conv2dGw8BgradConfig(groups=8, block_h=16, block_q=40), False),
+    (conv2d_gw8_wgrad_kernel_factory, {}, Conv2dGw8WgradConfig(variant="direct", chunks=0), False),
+])  # fmt: skip
+def test_a_recorded_choice_is_used_while_the_kernel_can_run_it(factory, mode, config, used, tmp_path, monkeypatch):
+    """Records are kept longer than the lists of candidates they were chosen from."""
+    from spio_amd.kernels import kernel_cache
+
+    monkeypatch.setenv("SPIO_TUNE_DB", str(tmp_path / "db.json"))
+    monkeypatch.setenv("SPIO_TUNE", "0")
+    params = Conv2dGw8Params(n=37, c=64, h=56, w=56)
+    tuner = Tuner()
+    tuner._store(ATTR, factory.get_full_kernel_name(params, **mode), {"config": config_to_dict(config), "us": 1.0})
+    monkeypatch.setattr(kernel_cache, "compile_and_load_kernel", lambda f, p, c, *a, **kw: c)
+    first = list(factory.configs(params, ATTR, **mode))[0]
+    assert config not in factory.configs(params, ATTR, **mode) and config != first
+    assert tuner.best_kernel(factory, params, 0, ATTR, **mode) == (config if used else first)
 
 
 def test_small_image_shapes_offer_mover_wave_configurations():
