@@ -205,17 +205,16 @@ constexpr long long BIAS_PARTIALS = (long long)NBLKS * PBLKS * QBLKS * GBLKS * G
 constexpr long long X_ROW_BYTES = (long long)kW * kGroups * 16, X_IMAGE_BYTES = kH * X_ROW_BYTES;
 constexpr long long D_ROW_BYTES = (long long)kQ * kGroups * 16, D_IMAGE_BYTES = kP * D_ROW_BYTES;
 // Whether a row is read through a descriptor that begins at it, or through one of its image block with the row
-// as the scalar offset.  Unrolled loops know the row at compile time and take the former (20n 1024c 27x27 5x5
-// 23.6 us, 28.6 with scalar offsets); in others it is 64-bit arithmetic for every
-// row (64n 64c 56x56 16.1 us, with scalar offsets 14.8; 32n 48c 224x224 66.0 and 63.5).  It is also the one for
+// in the lanes' offsets.  Unrolled loops know the row at compile time and take the former (20n 1024c 27x27 5x5
+// 23.6 us, 28.6 with one of the block); in others it is 64-bit arithmetic for every
+// row (64n 64c 56x56 16.1 us, 14.2 with one of the block; 32n 48c 224x224 66.0 and 55.7).  It is also the one for
 // images that side by side exceed 32-bit offsets.
-constexpr bool kRowDescriptors = kFullUnroll || NB * X_IMAGE_BYTES + (kPadY + BH + kR) * X_ROW_BYTES >= (1ll << 31) ||
-                              NB * D_IMAGE_BYTES + (BH + kR) * D_ROW_BYTES >= (1ll << 31);
-// the first row asked for and the one that a slot without a step asks for, behind the last block
-constexpr int FIRST_ROW = -kPadY, IDLE_ROW = kP + ROWS + BH;
-static_assert(kRowDescriptors || (offset_row(FIRST_ROW, kH) >= 0 && offset_row(IDLE_ROW, kH) * X_ROW_BYTES < (1ll << 31) &&
-                                  offset_row(IDLE_ROW, kP) * D_ROW_BYTES < (1ll << 31)),
-              "row offsets stay within 32 bits, also those of rows that do not exist");
+constexpr bool kRowDescriptors = kFullUnroll || NB * X_IMAGE_BYTES >= (1ll << 31) || NB * D_IMAGE_BYTES >= (1ll << 31);
+// What a row adds to the offsets of its lanes.  Rows above the image and behind it (padding, slots without a step)
+// have one too, which may wrap around; their loads go through an empty descriptor, which no offset is inside of.
+// (It is not the scalar offset, which the range check may leave out, and it is not clamped to rows that exist: the
+// row loop then computes every offset anew, 32n 48c 224x224 55.7 -> 66.1 us.)
+constexpr unsigned row_offset(int row, long long row_bytes) { return (unsigned)row * (unsigned)row_bytes; }
 static_assert((NB - 1) * X_IMAGE_BYTES + X_ROW_BYTES < (1ll << 31) && (NB - 1) * D_IMAGE_BYTES + D_ROW_BYTES < (1ll << 31),
               "a row of all images side by side lies within 32-bit buffer offsets");
 // Images side by side in an unrolled loop, one block of them a workgroup: plain loads.  There is no next block to
@@ -382,9 +381,10 @@ SPIO_KERNEL_NAME(float* __restrict__ grad_weight, const spio_uint4* __restrict__
         const rsrc_t rs = kRowDescriptors ? make_rsrc(xbase[ahead] + (n > 0 ? h : 0) * X_ROW_BYTES,
                                                    n > 0 ? (int)((n - 1) * X_IMAGE_BYTES + X_ROW_BYTES) : 0)
                                        : make_rsrc(xbase[ahead], (int)(n * X_IMAGE_BYTES));
-        const int row = kRowDescriptors ? 0 : offset_row(h, kH) * (int)X_ROW_BYTES;
+        const unsigned row = kRowDescriptors ? 0u : row_offset(h, X_ROW_BYTES);
 #pragma unroll
-        for (int l = 0; l < LPTX; ++l) v[l] = __builtin_amdgcn_raw_buffer_load_b128(rs, x_off[l], row, AUX_LD);
+        for (int l = 0; l < LPTX; ++l)
+            v[l] = __builtin_amdgcn_raw_buffer_load_b128(rs, (int)((unsigned)x_off[l] + row), 0, AUX_LD);
     };
     auto load_dy = [&](int ahead, int t, spio_uint4(&v)[LPTD]) {
         if (kPlainLoads) {
@@ -396,9 +396,10 @@ SPIO_KERNEL_NAME(float* __restrict__ grad_weight, const spio_uint4* __restrict__
         const rsrc_t rs = kRowDescriptors ? make_rsrc(dbase[ahead] + (n > 0 ? p0 + t : 0) * D_ROW_BYTES,
                                                    n > 0 ? (int)((n - 1) * D_IMAGE_BYTES + D_ROW_BYTES) : 0)
                                        : make_rsrc(dbase[ahead], (int)(n * D_IMAGE_BYTES));
-        const int row = kRowDescriptors ? 0 : offset_row(p0 + t, kP) * (int)D_ROW_BYTES;
+        const unsigned row = kRowDescriptors ? 0u : row_offset(p0 + t, D_ROW_BYTES);
 #pragma unroll
-        for (int l = 0; l < LPTD; ++l) v[l] = __builtin_amdgcn_raw_buffer_load_b128(rs, d_off[l], row, AUX_LD);
+        for (int l = 0; l < LPTD; ++l)
+            v[l] = __builtin_amdgcn_raw_buffer_load_b128(rs, (int)((unsigned)d_off[l] + row), 0, AUX_LD);
     };
     // The loads run PF slots ahead of the steps and straight on into the next image block: step S0 + i is slot
     // i, and SLOTS, a multiple of PF, holds an image block, so that the register buffer of a slot is known at

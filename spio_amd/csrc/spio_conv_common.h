@@ -51,10 +51,6 @@ static_assert(kP > 0 && kQ > 0, "empty output");
 #define SPIO_DEVICE __device__ inline __attribute__((always_inline))
 #define SPIO_LAUNCH_BOUNDS(threads) __attribute__((amdgpu_flat_work_group_size(threads, threads)))
 
-// The row whose offset a load of row `h` takes: rows above the tensor and behind it (padding, slots without a row)
-// go through an empty descriptor, but their offset is computed all the same and has to stay within 32 bits.
-constexpr int offset_row(int h, int rows) { return h < 0 ? 0 : h < rows ? h : rows - 1; }
-
 SPIO_DEVICE int imin(int a, int b) { return a < b ? a : b; }
 SPIO_DEVICE int imax(int a, int b) { return a > b ? a : b; }
 SPIO_DEVICE int thread_id() { return (int)__builtin_amdgcn_workitem_id_x(); }

@@ -511,16 +511,20 @@ def test_balanced_blocks_and_runs_of_image_blocks():
 
 
 def test_row_offsets_stay_within_32_bits():
-    """Rows in the padding and slots without a row have an offset inside the tensor: an image of almost 2 GiB,
+    """Rows in the padding and slots without a row have offsets without signed overflow: an image of almost 2 GiB,
     where the rows a step or two behind it would overflow."""
     params = Conv2dGw8Params(n=1, c=8, h=32748, w=4096, padding=1, r=3, s=3)
     config = Conv2dGw8WgradConfig(groups=1, block_h=14, block_n=1, block_n_iters=1, prefetch=4, block_q=64)
     defines = dict(conv2d_gw8_wgrad_kernel_factory.get_kernel_spec(params, config, ATTR).defines, SPIO_KERNEL_NAME="k")
     source = read_source("conv2d_gw8_wgrad_mfma.hip") + """
     static_assert(!kRowDescriptors, "offsets from the first row of an image");
+    constexpr int IDLE_ROW = kP + ROWS + BH;  // the row that a slot without a step asks for, behind the last block
     static_assert(IDLE_ROW * X_ROW_BYTES >= (1ll << 31), "a row behind the image overflows");
-    static_assert(offset_row(FIRST_ROW, kH) == 0 && offset_row(0, kH) == 0 && offset_row(kH - 1, kH) == kH - 1);
-    static_assert(offset_row(IDLE_ROW, kH) == kH - 1 && offset_row(IDLE_ROW, kP) == kP - 1);
+    static_assert(row_offset(IDLE_ROW, X_ROW_BYTES) == (unsigned)(IDLE_ROW * X_ROW_BYTES));
+    static_assert(row_offset(-kPadY, X_ROW_BYTES) == (unsigned)(-kPadY * X_ROW_BYTES));
+    // rows that exist: lanes with data stay below 2 GiB, lanes without above every descriptor
+    static_assert(row_offset(kH - 1, X_ROW_BYTES) == (kH - 1) * X_ROW_BYTES && NB * X_IMAGE_BYTES < (1ll << 31));
+    static_assert((unsigned)OUT_OF_RANGE + row_offset(kH - 1, X_ROW_BYTES) >= (1u << 31));
     """
     assert compile_hip(source, "row_offsets.hip", headers=kernel_headers(), defines=defines)
 
