@@ -20,9 +20,9 @@
 //
 // The channel sums keep workgroups few (one or two per CU), so a wave has its own loads to wait for: the next
 // pass is requested before a pass is worked on.  With the instructions of a pass from 17.5 to 13.5 an element
-// (mixed-precision multiply-adds instead of conversions) and the second stage's loads four floats wide, both
-// stages: 128n 96c 56x56 (231 MB) 44.5 -> 41.3 us, 192c 28x28 26.6 -> 24.3, 384c 14x14 16.5 -> 15.3, 4n 96c
-// 56x56 6.9 -> 6.5; 768c 7x7 10.8, as before: two launches and a pass.
+// (mixed-precision multiply-adds instead of conversions), both stages: 128n 96c 56x56 (231 MB) 46.9 -> 41.3 us,
+// 192c 28x28 26.2 -> 24.5, 384c 14x14 16.6 -> 15.2, 4n 96c 56x56 7.1 -> 6.4; 768c 7x7 10.9, as before: two
+// launches and a pass.
 #ifndef SPIO_LN_C
 #error "SPIO_LN_C, SPIO_LN_PIXELS, SPIO_LN_LPP, SPIO_LN_THREADS, SPIO_LN_GRID are required"
 #endif
@@ -318,32 +318,31 @@ SPIO_KERNEL_NAME(float* __restrict__ partials, ln_uint4* __restrict__ din, const
 }
 
 // Second stage: sums[i] = sum over the workgroups' rows of partials[row][i], i < 2*C.  A workgroup
-// owns 32 columns, 4 to a thread; its 32 slices each add the rows r = slice, slice + 32, ... with up to 16
-// loads in flight (one round trip to memory for up to 512 rows), and meet in LDS.  Every element has one
-// owner: no atomics, no dependence on timing.
+// owns 32 columns; its 8 slices each add the rows r = slice, slice + 8, ... with up to 32 loads
+// in flight, and meet in LDS.  Every element has one owner: no atomics, no dependence on timing.
 #define SPIO_LN_CONCAT2(a, b) a##b
 #define SPIO_LN_CONCAT(a, b) SPIO_LN_CONCAT2(a, b)
 extern "C" __global__ void __attribute__((amdgpu_flat_work_group_size(256, 256)))
-SPIO_LN_CONCAT(SPIO_KERNEL_NAME, _reduce)(float* __restrict__ sums, const ln_float4* __restrict__ partials) {
+SPIO_LN_CONCAT(SPIO_KERNEL_NAME, _reduce)(float* __restrict__ sums, const float* __restrict__ partials) {
     constexpr int ROWS = SPIO_LN_GRID;
-    constexpr int COLS = 8;  // float4 columns of a workgroup
+    constexpr int COLS = 32;
     constexpr int SLICES = 256 / COLS;
-    constexpr int UNR = (ROWS + SLICES - 1) / SLICES < 16 ? (ROWS + SLICES - 1) / SLICES : 16;
-    constexpr int ROW_F4 = 2 * C / 4;
-    __shared__ ln_float4 red[SLICES][COLS];
+    // as many rows in flight per thread as a slice has, up to 32: one round trip to memory for up
+    // to 256 rows (with 8 in flight the stage took 1.5-2 us longer on the 7x7 and 14x14 shapes)
+    constexpr int UNR = (ROWS + SLICES - 1) / SLICES < 32 ? (ROWS + SLICES - 1) / SLICES : 32;
+    __shared__ float red[SLICES][COLS];
     const int tid = (int)__builtin_amdgcn_workitem_id_x();
     const int cl = tid % COLS;
     const int slice = tid / COLS;
     const int col = (int)__builtin_amdgcn_workgroup_id_x() * COLS + cl;
-    ln_float4 sum = ln_float4{0.f, 0.f, 0.f, 0.f};
-    if (col < ROW_F4) {
+    float sum = 0.f;
+    if (col < 2 * C) {
         for (int base = slice; base < ROWS; base += SLICES * UNR) {
-            ln_float4 v[UNR];
+            float v[UNR];
 #pragma unroll
             for (int i = 0; i < UNR; ++i) {
                 const int r = base + i * SLICES;
-                v[i] = ln_float4{0.f, 0.f, 0.f, 0.f};
-                if (r < ROWS) v[i] = partials[(long long)r * ROW_F4 + col];
+                v[i] = r < ROWS ? partials[(long long)r * 2 * C + col] : 0.f;
             }
 #pragma unroll
             for (int i = 0; i < UNR; ++i) sum += v[i];
@@ -353,13 +352,9 @@ SPIO_LN_CONCAT(SPIO_KERNEL_NAME, _reduce)(float* __restrict__ sums, const ln_flo
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-    // one wave adds the slices, a float each: thread t < 32 column t
-    const int out = (int)__builtin_amdgcn_workgroup_id_x() * COLS * 4 + tid;
-    if (tid < COLS * 4 && out < 2 * C) {
-        const float* flat = reinterpret_cast<const float*>(red) + tid;
-        float total = 0.f;
+    if (slice == 0 && col < 2 * C) {
 #pragma unroll
-        for (int i = 0; i < SLICES; ++i) total += flat[i * COLS * 4];
-        sums[out] = total;
+        for (int i = 1; i < SLICES; ++i) sum += red[i][cl];
+        sums[col] = sum;
     }
 }
