@@ -547,7 +547,7 @@ SPIO_KERNEL_NAME(spio_uint4* __restrict__ grad_input, float* __restrict__ grad_w
 #pragma unroll
             for (int uu = 0; uu < UNROLL; ++uu) {
                 const int t = tb + uu;
-                if (t >= ROWS) break;
+                if (t >= ROWS) continue;  // (with a second way out of the loop the compiler leaves 12 steps rolled)
                 const int sp = uu & 1;                   // parity of t: x ring row, parity of delta
                 const int pbuf = uu % PF;                // register buffer that held row t
                 const int ph = uu % NS;                  // data-gradient phase: t mod NS

@@ -451,6 +451,16 @@ def test_bgrad_two_stage():
         run_bgrad_kernel_test(conv2d_gw8_bgrad_kernel_factory, params, configs=configs)
 
 
+@pytest.mark.parametrize("config", [
+    Conv2dGw8BgradConfig(groups=3, block_h=0, split=2, prefetch=4),
+    Conv2dGw8BgradConfig(groups=2, block_h=37, block_n_iters=2, split=2, prefetch=4, two_stage=1),
+], ids=["whole images", "two row blocks"])  # fmt: skip
+def test_bgrad_in_chunks_of_twelve_steps(config):
+    """5x5 over more rows than an unrolled loop takes; the last chunk is not full."""
+    params = Conv2dGw8Params(n=3, c=24, h=41, w=40, r=5, s=5, padding=2, has_bias=True)
+    run_bgrad_kernel_test(conv2d_gw8_bgrad_kernel_factory, params, configs=[config])
+
+
 def test_bgrad_when_the_image_size_changes():
     """Paddings other than (R-1)/2, and even filter sizes: the kernel works on a domain that holds
     both tensors at offsets that reproduce the padding.  Row blocks that lie partly or wholly

@@ -547,3 +547,10 @@ def test_long_loops_are_unrolled(config, kernel_size):
     params = Conv2dGw8Params(n=64, c=64 if kernel_size == 3 else 96, h=56, w=56, padding=kernel_size // 2,
                              r=kernel_size, s=kernel_size, has_bias=True)  # fmt: skip
     assert scratch_bytes(factory, params, config) == 0
+
+
+def test_chunks_of_twelve_steps_are_unrolled():
+    """Left rolled they index the accumulators, 720 bytes a lane, in memory; unrolled a few registers are short."""
+    params = Conv2dGw8Params.decode("62n_56c_46h_46w_2py_2px_5r_5s_b")
+    config = Conv2dGw8BgradConfig(groups=4, split=2, prefetch=4)
+    assert scratch_bytes(conv2d_gw8_bgrad_kernel_factory, params, config) <= 96
