@@ -520,11 +520,11 @@ def test_row_offsets_stay_within_32_bits():
     static_assert(!kRowDescriptors, "offsets from the first row of an image");
     constexpr int IDLE_ROW = kP + ROWS + BH;  // the row that a slot without a step asks for, behind the last block
     static_assert(IDLE_ROW * X_ROW_BYTES >= (1ll << 31), "a row behind the image overflows");
-    static_assert(row_offset(IDLE_ROW, X_ROW_BYTES) == (unsigned)(IDLE_ROW * X_ROW_BYTES));
-    static_assert(row_offset(-kPadY, X_ROW_BYTES) == (unsigned)(-kPadY * X_ROW_BYTES));
+    static_assert(ROW_OFFSET(IDLE_ROW, X_ROW_BYTES) == (unsigned)(IDLE_ROW * X_ROW_BYTES));
+    static_assert(ROW_OFFSET(-kPadY, X_ROW_BYTES) == (unsigned)(-kPadY * X_ROW_BYTES));
     // rows that exist: lanes with data stay below 2 GiB, lanes without above every descriptor
-    static_assert(row_offset(kH - 1, X_ROW_BYTES) == (kH - 1) * X_ROW_BYTES && NB * X_IMAGE_BYTES < (1ll << 31));
-    static_assert((unsigned)OUT_OF_RANGE + row_offset(kH - 1, X_ROW_BYTES) >= (1u << 31));
+    static_assert(ROW_OFFSET(kH - 1, X_ROW_BYTES) == (kH - 1) * X_ROW_BYTES && NB * X_IMAGE_BYTES < (1ll << 31));
+    static_assert((unsigned)OUT_OF_RANGE + ROW_OFFSET(kH - 1, X_ROW_BYTES) >= (1u << 31));
     """
     assert compile_hip(source, "row_offsets.hip", headers=kernel_headers(), defines=defines)
 
