@@ -19,7 +19,13 @@ from typing import Dict, List, Tuple
 import torch
 
 from ..util.math import balanced, divup
-from .conv2d_gw8_kernel import _policies_are_legal, _shape_defines, fits_float32_output, with_joined_stores
+from .conv2d_gw8_kernel import (
+    _policies_are_legal,
+    _shape_defines,
+    fits_float32_output,
+    lane_registers,
+    with_joined_stores,
+)
 from .conv2d_gw8_params import Conv2dGw8Params
 from .conv2d_gw8_wgrad_kernel import image_block_runs
 from .conv2d_stats import Conv2dStats
@@ -181,6 +187,21 @@ def _config_is_legal(params, config) -> bool:
     )
 
 
+def _fits(params, config) -> bool:
+    """Whether a lane's registers hold the sums, the filters, the rows in flight and a step's operands, or most of them.
+    The weights were fitted to what the compiler reports for 960 kernels of 76 shapes.  The line lies a quarter above
+    the registers there are, as some with 72 to 130 bytes a lane in memory are the best (128n 1392c 9x9 5x5 60 us, 76
+    without; but 32n 256c 28x28 5x5 34 and 23); those behind it, 16 waves mostly, are several times slower."""
+    g = bgrad_geometry(params, config)
+    ns, kb = 2 * divup(params.r, 2), divup(params.s, 4)
+    kept = (params.r + 1) * g["NBLK"] + 1 + g["TPW"] * (ns // 2) + ns * kb
+    operands = g["CPW"] * (g["NBLK"] + params.r // 2 + 1) + g["TPW"] * kb
+    loads = g["LPTX"] + g["LPTD"]
+    stores = divup(config.block_n * g["BQ"] * config.groups, g["THREADS"])
+    needed = 4.92 * kept + 5.76 * operands + 4.0 * config.prefetch * loads + 4.85 * (loads + stores) + 26.5
+    return needed <= 1.25 * lane_registers(config.groups * config.split)
+
+
 def _recorded_config_is_legal(params, config) -> bool:
     return (
         min(config.groups, config.block_n, config.block_n_iters, config.split) >= 1
@@ -246,7 +267,12 @@ def _get_configs(params: Conv2dGw8Params, device_attr=None) -> List[Conv2dGw8Bgr
                             if _config_is_legal(params, cfg):
                                 geometries.append((_score(params, cfg, num_cus), cfg))
         geometries.sort(key=lambda sc: sc[0])
-        configs += [cfg for _, cfg in geometries[:GEOMETRIES_PER_HEIGHT]]
+        ranked = [cfg for _, cfg in geometries]
+        # the best, and as many of those that fit the registers
+        fitting = [cfg for cfg in ranked if _fits(params, cfg)][:GEOMETRIES_PER_HEIGHT]
+        configs += ranked[:GEOMETRIES_PER_HEIGHT] + [cfg for cfg in fitting if cfg not in ranked[:GEOMETRIES_PER_HEIGHT]]
+    # what keeps much of its registers in memory comes last
+    configs.sort(key=lambda cfg: not _fits(params, cfg))
     # a shallower and a deeper pipeline for the first few: the shallow one wins where rows are short
     first = configs[:GEOMETRIES_PER_HEIGHT]
     configs += [replace(cfg, prefetch=2) for cfg in first]

@@ -138,6 +138,23 @@ def mfma_geometry(params: Conv2dGw8Params, config: Conv2dGw8Config, igrad: bool)
     return d
 
 
+def lane_registers(waves: int) -> int:
+    """Registers a lane has where `waves` waves share a compute unit's four SIMDs (512 a lane and SIMD, dealt in
+    eights).  A kernel that needs more keeps the rest in memory."""
+    return {1: 512, 2: 256, 3: 168, 4: 128}.get(divup(waves, 4), 0)
+
+
+def _mfma_fits(params, config, igrad) -> bool:
+    """Whether a lane's registers hold what the row-streaming kernel keeps in them, or all but a few: filter fragments,
+    accumulators and rows in flight.  The weights were fitted to what the compiler reports for 1771 kernels of 110
+    shapes, 1x1 to 7x7: of 100 that used memory 5 pass, with 100 bytes at most, of 1671 others 2 do not."""
+    g = mfma_geometry(params, config, igrad)
+    fragments, accumulators = 4 * g["NS"] * g["KB"], 4 * g["TPW"] * g["NACC"]
+    rows = 4 * min(config.prefetch, g["STEPS"]) * g["LPT"]
+    needed = fragments + 1.6 * accumulators + 1.3 * rows + 6
+    return needed <= 1.05 * lane_registers(config.groups * config.split)
+
+
 def image_geometry(params: Conv2dGw8Params, config: Conv2dGw8Config, igrad: bool) -> Dict[str, int]:
     """Host mirror of the compile-time constants of conv2d_gw8_image_mfma.hip."""
     d = direction_geometry(params, igrad)
@@ -417,7 +434,11 @@ def _get_configs(params: Conv2dGw8Params, device_attr=None, igrad: bool = False)
                             cfg = Conv2dGw8Config(groups=gb, block_p=bp, block_n=nb, split=ts, prefetch=pf, block_q=bq)
                             if _mfma_config_is_legal(params, cfg, igrad):
                                 found.append((_mfma_score(params, cfg, igrad, num_cus), cfg))
-    found.sort(key=lambda sc: sc[0])
+    # Those that keep part of their registers in memory (12 and 16 waves with 5x5 and 7x7 filters) after all others:
+    # they are among the slowest (32n 64c 112x112 5x5, the eight that a first use tries: 31 to 114 us, without them
+    # 31 to 46; 64n 96c 56x56 7x7 32 to 106, 31 to 40; of all configurations of these and three other shapes none of
+    # the best 14 is one)
+    found.sort(key=lambda sc: (not _mfma_fits(params, sc[1], igrad), sc[0]))
     # two prefetch distances of a geometry first, then the others: a capped sweep sees more geometries
     head, rest = [], []
     for _, cfg in found:
@@ -425,7 +446,8 @@ def _get_configs(params: Conv2dGw8Params, device_attr=None, igrad: bool = False)
         (head if sum(replace(h, prefetch=0) == shape for h in head[-16:]) < 2 else rest).append(cfg)
         if len(head) >= MAX_GEOMETRIES:
             break
-    configs = [*head[:8], *sorted(head[8:] + rest, key=lambda c: _mfma_score(params, c, igrad, num_cus))][:MAX_GEOMETRIES]
+    rank = {cfg: i for i, (_, cfg) in enumerate(found)}
+    configs = [*head[:8], *sorted(head[8:] + rest, key=rank.get)][:MAX_GEOMETRIES]
     # the memory-system policies, which the score cannot rank: halo rows with or without the
     # non-temporal hint, and how tiles are dealt to the XCDs
     leading = []  # the first four tile geometries, whatever their prefetch depth

@@ -16,7 +16,7 @@ from typing import Dict, List
 import torch
 
 from ..util.math import balanced, divup
-from .conv2d_gw8_kernel import _shape_defines
+from .conv2d_gw8_kernel import _shape_defines, lane_registers
 from .conv2d_gw8_params import Conv2dGw8Params
 from .conv2d_stats import Conv2dStats
 from .kernel import KernelSpec
@@ -161,6 +161,16 @@ def _mfma_config_is_legal(params, config) -> bool:
     )
 
 
+def _fits(params, config) -> bool:
+    """Whether a lane's registers hold the sums, the rows in flight and a step's operands (weights fitted to what the
+    compiler reports for 564 kernels: of 34 that used memory 6 pass, of 530 others 6 do not)."""
+    g = wgrad_geometry(params, config)
+    loads = g["LPTX"] + g["LPTD"]
+    operands = divup(g["KC"], config.split) * config.rows * (g["NBLK"] + params.r // 2 + 1) * (2 if config.pipe else 1)
+    needed = 5.2 * g["ND"] * g["NBLK"] + 2.84 * config.prefetch * config.rows * loads + 3.72 * operands + 12.9 * loads
+    return needed <= 1.05 * lane_registers(config.groups * config.split)
+
+
 def _config_is_legal(params, config) -> bool:
     """Whether the MFMA kernel can run a configuration."""
     return (
@@ -264,7 +274,8 @@ def _get_configs(params: Conv2dGw8Params, device_attr=None) -> List[Conv2dGw8Wgr
             cfg = replace(base, prefetch=pf, rows=rows, pipe=pipe)
             if _mfma_config_is_legal(params, cfg):
                 (head if i < 3 and j < LEADING_PIPELINES else rest).append(cfg)
-    configs = head + rest
+    # what keeps part of its registers in memory comes last (64n 96c 56x56 7x7: 500 us, 35 without)
+    configs = sorted(head + rest, key=lambda cfg: not _fits(params, cfg))
     total_pix = params.n * params.p * params.q
     chunks = max(1, min(divup(8 * num_cus, params.groups), divup(total_pix, 64)))
     configs.append(Conv2dGw8WgradConfig(groups=1, block_h=1, block_n=1, block_n_iters=1,

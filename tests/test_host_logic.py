@@ -554,3 +554,20 @@ def test_chunks_of_twelve_steps_are_unrolled():
     params = Conv2dGw8Params.decode("62n_56c_46h_46w_2py_2px_5r_5s_b")
     config = Conv2dGw8BgradConfig(groups=4, split=2, prefetch=4)
     assert scratch_bytes(conv2d_gw8_bgrad_kernel_factory, params, config) <= 96
+
+
+@pytest.mark.parametrize("shape,family,mode", [
+    ("32n_64c_112h_112w_2py_2px_5r_5s_b", "fprop", {}),
+    ("64n_96c_56h_56w_3py_3px_7r_7s_b", "fprop", {}),
+    ("64n_96c_56h_56w_3py_3px_7r_7s_b", "fprop", {"igrad": True}),
+    ("128n_1392c_9h_9w_2py_2px_5r_5s_nb", "wgrad", {}),
+    ("64n_96c_56h_56w_3py_3px_7r_7s_b", "wgrad", {}),
+    ("128n_1392c_9h_9w_2py_2px_5r_5s_nb", "bgrad", {}),
+], ids=str)  # fmt: skip
+def test_the_first_candidates_fit_the_registers(shape, family, mode):
+    """The eight that a first use tries: all but a few of their registers (bytes a lane of memory) are registers."""
+    factory = {"fprop": conv2d_gw8_kernel_factory, "wgrad": conv2d_gw8_wgrad_kernel_factory,
+               "bgrad": conv2d_gw8_bgrad_kernel_factory}[family]  # fmt: skip
+    params = Conv2dGw8Params.decode(shape)
+    for config in factory.configs(params, ATTR, **mode)[:8]:
+        assert scratch_bytes(factory, params, config, **mode) <= (140 if family == "bgrad" else 100), config
