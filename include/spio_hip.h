@@ -91,6 +91,10 @@ int spio_hip_get_function(void* module, const char* kernel_name, void** function
  * LDS limit of one kernel. */
 int spio_hip_func_set_max_dynamic_lds(void* function, int bytes);
 
+/* Bytes of memory a lane of a kernel keeps registers in that it has no room
+ * for (0: none). */
+int spio_hip_func_scratch_bytes(void* function, int* bytes);
+
 /* Replaces Function.launch (driver.pyx:171-208).  Asynchronous launch on
  * `stream` (NULL = the null stream).  `params` is an array of num_params
  * pointers, each to the storage of one kernel argument; at most 16 arguments

@@ -57,6 +57,7 @@ struct Api {
     hipError_t (*hipModuleUnload)(hipModule_t) = nullptr;
     hipError_t (*hipModuleGetFunction)(hipFunction_t*, hipModule_t, const char*) = nullptr;
     hipError_t (*hipFuncSetAttribute)(const void*, hipFuncAttribute, int) = nullptr;
+    hipError_t (*hipFuncGetAttribute)(int*, hipFunction_attribute, hipFunction_t) = nullptr;
     hipError_t (*hipModuleLaunchKernel)(hipFunction_t, unsigned, unsigned, unsigned, unsigned,
                                         unsigned, unsigned, unsigned, hipStream_t, void**,
                                         void**) = nullptr;
@@ -186,6 +187,7 @@ int spio_hip_init(const char* hip_library_path, const char* hiprtc_library_path)
     bind(h, "hipModuleUnload", &api.hipModuleUnload, &missing);
     bind(h, "hipModuleGetFunction", &api.hipModuleGetFunction, &missing);
     bind(h, "hipFuncSetAttribute", &api.hipFuncSetAttribute, &missing);
+    bind(h, "hipFuncGetAttribute", &api.hipFuncGetAttribute, &missing);
     bind(h, "hipModuleLaunchKernel", &api.hipModuleLaunchKernel, &missing);
     bind(h, "hipEventCreate", &api.hipEventCreate, &missing);
     bind(h, "hipEventDestroy", &api.hipEventDestroy, &missing);
@@ -301,6 +303,14 @@ int spio_hip_func_set_max_dynamic_lds(void* function, int bytes) {
     if (!function || bytes < 0)
         return fail(SPIO_HIP_ERR_ARGUMENT, "spio_hip_func_set_max_dynamic_lds: bad argument");
     HIP_TRY(hipFuncSetAttribute(function, hipFuncAttributeMaxDynamicSharedMemorySize, bytes));
+    return SPIO_HIP_OK;
+}
+
+int spio_hip_func_scratch_bytes(void* function, int* bytes) {
+    REQUIRE_READY();
+    if (!function || !bytes)
+        return fail(SPIO_HIP_ERR_ARGUMENT, "spio_hip_func_scratch_bytes: null argument");
+    HIP_TRY(hipFuncGetAttribute(bytes, HIP_FUNC_ATTRIBUTE_LOCAL_SIZE_BYTES, static_cast<hipFunction_t>(function)));
     return SPIO_HIP_OK;
 }
 

@@ -86,6 +86,7 @@ _SIGNATURES = {
     "spio_hip_module_unload": ([_vp], ctypes.c_int),
     "spio_hip_get_function": ([_vp, ctypes.c_char_p, ctypes.POINTER(_vp)], ctypes.c_int),
     "spio_hip_func_set_max_dynamic_lds": ([_vp, ctypes.c_int], ctypes.c_int),
+    "spio_hip_func_scratch_bytes": ([_vp, ctypes.POINTER(ctypes.c_int)], ctypes.c_int),
     "spio_hip_launch": (
         [_vp] + [ctypes.c_uint] * 7 + [_vp, ctypes.POINTER(_vp), ctypes.c_int],
         ctypes.c_int,
@@ -280,6 +281,12 @@ class Function:
     def set_max_dynamic_lds(self, nbytes: int):
         """Raise the kernel's dynamic LDS limit."""
         _check(_lib.spio_hip_func_set_max_dynamic_lds(self._handle, int(nbytes)))
+
+    def scratch_bytes(self) -> int:
+        """Bytes of memory a lane keeps registers in that it has no room for."""
+        nbytes = ctypes.c_int()
+        _check(_lib.spio_hip_func_scratch_bytes(self._handle, ctypes.byref(nbytes)))
+        return nbytes.value
 
     @staticmethod
     def marshal(args) -> Tuple[object, object]:

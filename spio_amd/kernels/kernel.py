@@ -106,6 +106,7 @@ class Kernel:
         self.function = None
         self.epilogue_function = None
         self.epilogue_half_function = None
+        self.scratch_bytes = 0  # of a loaded kernel: memory a lane keeps registers in
         self.device_ordinal: Optional[int] = None
         self.in_plans = False  # launch plans of the native call path point into the module
 
@@ -132,6 +133,7 @@ class Kernel:
             raise ValueError(f"Kernel {self.kernel_name} has not been compiled")
         self.module, self.function = load_kernel(self.kernel_name, self.code, device_ordinal)
         self.device_ordinal = device_ordinal
+        self.scratch_bytes = self.function.scratch_bytes()
         if self.kernel_spec.epilogue_suffix:
             self.epilogue_function = self.module.get_function(
                 self.kernel_name + self.kernel_spec.epilogue_suffix

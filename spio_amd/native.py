@@ -88,7 +88,15 @@ def _adapted(kernel, factory, params, device, mode, **kwargs):
             kwargs.update(reads)
     if config == kernel.config and not mode & (WIDE | READ_F32 | WEIGHT_F32):
         return kernel
-    return factory.get_kernel_in_config(params, device, config, **kwargs)
+    adapted = factory.get_kernel_in_config(params, device, config, **kwargs)
+    # Float32 rows and filters take twice the registers.  What then has to keep some in memory is slower than
+    # conversions and the plain kernel: 64n 96c 56x56 5x5 by 16 waves, forward 124 us (144 bytes a lane) and 70 with
+    # conversions, data gradient 107 (68) and 60; 117n 48c 39x39 7x7 57 (72) and 49; 49n 264c 34x34 55 (8) and 46; 24 of
+    # 27 such versions were, the others 10 per cent faster.  (Not the fused backward: 57 (68) and 73 at 128n 64c
+    # 56x56, 9 of 10 faster.)
+    if "w_f32" in kwargs and adapted.scratch_bytes > kernel.scratch_bytes:
+        return None
+    return adapted
 
 
 def _make_plan(values):

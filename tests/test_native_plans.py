@@ -110,3 +110,22 @@ def test_recorders_may_be_entered_again(recorder, monkeypatch):
             assert sum(held) == 2
         assert sum(held) == 1
     assert sum(held) == 0
+
+
+def test_versions_that_read_float32_with_registers_in_memory_are_not_used(made, monkeypatch):
+    """They are slower than a conversion and the plain kernel, in whose configuration they run."""
+    kernels, loaded = made
+    spilled = []
+
+    def compile_and_load(factory, params, config, ordinal, device_attr, **kwargs):
+        kernel = _Kernel(loaded)
+        kernel.scratch_bytes = 68 if kwargs.get("src_f32") or kwargs.get("w_f32") else 0
+        spilled.append(kernel.scratch_bytes)
+        return kernel
+
+    monkeypatch.setattr(kernel_cache, "compile_and_load_kernel", compile_and_load)
+    kind, device, *shape, mode = WIDE_FORWARD
+    for reads in (native.READ_F32, native.WEIGHT_F32, native.READ_F32 | native.WEIGHT_F32 | native.KEEP):
+        assert native._make_plan((kind, device, *shape, mode | reads)) is None
+    assert spilled == [0, 68, 68, 68]  # the plain kernel, then a version each
+    assert native._make_plan(WIDE_FORWARD) is not None
