@@ -325,8 +325,11 @@ def _get_kernel_spec(params: Conv2dGw8Params, config: Conv2dGw8WgradConfig, _dev
     return spec
 
 
-# Partial sums up to this many bytes are published in two stages where grad_weight ends as float16: twice
-# this through memory costs about what the two launches do.
+# Partial sums up to this many bytes are published in two stages where grad_weight ends as float16.  Atomics take
+# longer the more sums there are, too: forward and weight gradient, atomics -> two stages, 64n 256c 28x28 5x5 with 16
+# MB 51 -> 47 us, with 32 MB 65 -> 56, 128n 256c 14x14 7x7 with 15 MB 43 -> 36, 3x3 with 25 MB 128n 64c 56x56 64 -> 60 and
+# 64n 256c 28x28 45 -> 46.  (Chosen configurations have 15 MB at most, and those with more than 7 are two-stage
+# ones by the sweep's choice.)
 STORED_SUMS_BYTES = 32 * 1024 * 1024
 
 
