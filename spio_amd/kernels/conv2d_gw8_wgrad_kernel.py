@@ -30,7 +30,7 @@ MAX_WAVES = 16
 MAX_LDS_BYTES = 128 * 1024
 MAX_LOADS_PER_THREAD = 8
 MAX_ACCUMULATORS = 32
-MAX_GEOMETRIES = 20
+MAX_GEOMETRIES = 20  # that enter the sweep, with the pipelines about 100 candidates (20 s)
 PIPELINE_CHOICES = ((2, 1, 0), (4, 1, 0), (2, 2, 0), (2, 1, 1), (4, 1, 1))  # (prefetch, rows, pipe)
 LEADING_PIPELINES = 3  # of these, for the leading geometries at the head of the list
 
@@ -214,13 +214,12 @@ def _mfma_score(params, config, num_cus) -> float:
         publish_us = 4.5 + 2.0 * 4.0 * values / 5.0e6
     else:
         publish_us = values / (128 * 2.1e3)
-    # blocks of part of a line; they cost more where a pixel is not whole lines, so that blocks straddle them
-    # (184n 288c 31x31 3x3: 4 groups 50.4 us, 8 groups, of which the last block has half, 42.1)
+    # blocks of part of a line; they cost more where a pixel is not whole lines, so that blocks straddle them (184n
+    # 288c 31x31 3x3: 4 groups 50.4 us, 8 groups, of which the last block has half, 42.1; best of a first use over ten
+    # such shapes with 1.12 and 1.2: that one 47.0 and 41.0, 23n 1360c 29x18 22.9 and 21.2, the others equal)
     split_line = 1.0 if (config.groups * 16) % 128 == 0 or config.groups == params.groups else (
         1.12 if params.c % 64 == 0 else 1.2)
-    # fewer waves than SIMDs (14n 24c 167x167 3x3: 3 waves 21.1 us, 6 waves 19.4)
-    few_waves = 1.15 if g["THREADS"] < 256 else 1.0
-    return (traffic * quant * split_line * few_waves / (g["PIXEL_EFF"] ** 0.3 * group_eff)) * (
+    return (traffic * quant * split_line / (g["PIXEL_EFF"] ** 0.3 * group_eff)) * (
         1.0 + publish_us / stream_us
     )
 

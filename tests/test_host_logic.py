@@ -571,3 +571,9 @@ def test_the_first_candidates_fit_the_registers(shape, family, mode):
     params = Conv2dGw8Params.decode(shape)
     for config in factory.configs(params, ATTR, **mode)[:8]:
         assert scratch_bytes(factory, params, config, **mode) <= (140 if family == "bgrad" else 100), config
+
+
+def test_weight_gradient_candidates_of_few_groups_are_not_all_split():
+    """Three waves are fewer than a compute unit has SIMDs, and still the fastest (128n 24c 144x144)."""
+    params = Conv2dGw8Params.decode("128n_24c_144h_144w_1py_1px_3r_3s_nb")
+    assert any(c.split == 1 for c in conv2d_gw8_wgrad_kernel_factory.configs(params, ATTR)[:8])
