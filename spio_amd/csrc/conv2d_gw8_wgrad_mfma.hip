@@ -42,8 +42,8 @@
 //     whatever is in it, so what bounds small images is the number of steps of the longest workgroup: the host
 //     deals equal shares.  Rows in the padding or past the block go through an empty descriptor and cost no
 //     traffic; the clamped loads that stood here before fetched a real row for each, PF of them per image
-//     block.  20n 1024c 27x27 5x5 48.6 -> 43.8 us, with equal shares (3 images instead of 8 and 2 blocks of two) 25.3;
-//     77n 168c 20x20 7x7 32.5 -> 21.1, 300n 88c 17x17 5x5 30.1 -> 19.6, 184n 288c 31x31 3x3 45.0 -> 41.4.
+//     block.  20n 1024c 27x27 5x5 48.6 -> 43.8 us, with equal shares (3 images instead of 8 and 2 blocks of two) 23.4;
+//     77n 168c 20x20 7x7 32.5 -> 22.1, 300n 88c 17x17 5x5 30.1 -> 20.4, 184n 288c 31x31 3x3 45.0 -> 39.7.
 //   * With SPIO_HAS_BIAS the kernel takes a fourth pointer, grad_bias ([K]
 //     fp32, accumulated into like grad_weight; null = not wanted), and sums dy
 //     per channel in the same pass: one more MFMA per chunk and row pair with

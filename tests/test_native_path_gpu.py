@@ -5,9 +5,12 @@ tracer, a transform or a recorder has to see the call."""
 import pytest
 import torch
 
+from helpers import scratch_bytes
 from spio_amd import native
 from spio_amd.functional import conv2d_gw8, layernorm_2d
-from spio_amd.kernels import Conv2dGw8Params, KernelParamsLogger
+from spio_amd.hip import get_device_attributes
+from spio_amd.kernels import Conv2dGw8Config, Conv2dGw8Params, KernelParamsLogger, conv2d_gw8_kernel_factory
+from spio_amd.kernels.tuner import config_to_dict, tuner
 
 pytestmark = pytest.mark.gpu
 CL = torch.channels_last
@@ -115,6 +118,27 @@ def test_norm_matches_the_python_operator(weight, bias):
     w = torch.randn(48, device="cuda").requires_grad_() if weight else None
     b = torch.randn(48, device="cuda").requires_grad_() if bias else None
     _check(lambda x, w, b: layernorm_2d(x, w, b, 1e-5), [x, w, b])
+
+
+def test_float32_is_converted_where_a_version_that_reads_it_is_short_of_registers(tmp_path, monkeypatch):
+    """In a configuration of 16 waves whose float16 kernel fits the registers and whose float32 one does not."""
+    monkeypatch.setenv("SPIO_TUNE_DB", str(tmp_path / "db.json"))
+    factory, config = conv2d_gw8_kernel_factory, Conv2dGw8Config(groups=4, block_p=14, split=4, prefetch=10)
+    p = Conv2dGw8Params(2, 64, 28, 56, padding=2, r=5, s=5, has_bias=True)
+    tuner._store(get_device_attributes(0), factory.get_full_kernel_name(p), {"config": config_to_dict(config), "us": 1.0})
+    reads = dict(out_f32=True, src_f32=True, w_f32=True, keep=True)
+    for kwargs in ({}, reads):
+        kernel = factory.get_kernel_in_config(p, torch.device("cuda", 0), config, **kwargs)
+        assert kernel.scratch_bytes == scratch_bytes(factory, p, config, **kwargs)
+        assert (kernel.scratch_bytes > 0) == bool(kwargs)
+    args, call = _conv_args(p, torch.float32)
+
+    def under_autocast(*a):
+        with torch.autocast("cuda", dtype=torch.float16):
+            return call(*a)
+
+    assert factory.get_kernel(p, torch.device("cuda", 0)).config == config
+    _check(under_autocast, args)
 
 
 def test_gradients_accumulate_and_graphs_are_kept():
