@@ -30,13 +30,16 @@
 // there is no halo.  Everything else is the separate kernels' design:
 //   * rows of x and dy staged in LDS as [group][flattened pixel][8 ch], zero halo materialised
 //     once, branch-free global loads SPIO_PF steps ahead;
-//   * weight gradient: A = dy row pair, B = x (two column taps), one accumulator per (delta,
-//     tap pair), transposing LDS reads (see conv2d_gw8_wgrad_mfma.hip);
-//   * data gradient: A = flipped, group-transposed filter, B = dy (pixel n + tap kb is the
-//     16 bytes lane (n, kb) reads), rotating accumulator row slots (see conv2d_gw8_mfma.hip);
+//   * weight gradient: A = dy and dy one pixel on, B = x at two column taps, one accumulator per filter
+//     row and four column taps, transposing LDS reads (see conv2d_gw8_wgrad_mfma.hip);
+//   * data gradient: A = flipped, group-transposed filter for pairs of neighbouring pixels, B = every
+//     second dy pixel (see conv2d_gw8_mfma.hip); dx rows take turns in R sets of accumulators;
 //     a dy pixel (image i, column q) sits at flattened pixel i*WPI + q + PR, which is both its
 //     place as a source pixel of the data gradient and, shifted by PR, its place opposite x
 //     (column c at i*WPI + c + PL) in the weight gradient;
+//   * a dy row is read from LDS for the weight gradient once, when it is the newest, and its fragments stay
+//     in registers while the next R-1 x rows meet it: two ring rows of each tensor are enough;
+//   * products of rows that do not exist (above, below, of neighbouring blocks) are left out at compile time;
 //   * publishing of dw (and db) as in the weight-gradient kernel: sums staged in LDS in
 //     grad_weight order, atomics of 64 consecutive floats;
 //   * global memory through buffer instructions with the hardware bounds check as predicate
@@ -44,6 +47,14 @@
 //     such loads return zeros, such stores are dropped) and a fully unrolled step loop, so that
 //     no memory instruction sits under a branch and the compiler's count of outstanding loads and
 //     stores is exact (see conv2d_gw8_mfma.hip).
+//
+// With two rows instead of two neighbouring pixels side by side in both A operands a step had a third more
+// products and twice the LDS reads, half of the lanes idled when a row was converted, and the sums took 32
+// registers for a 3x3 filter and 128 for 7x7 (now 12 and 56).  What bounds the kernel is the chain of a step (barrier,
+// LDS reads, products, conversion) on one or two waves a SIMD, then memory.  Before -> after: 128n 64c 56x56 35.2 ->
+// 32.4 us (154 MB, 4.75 TB/s), 32n 15.4 -> 11.9, 512n 120.4 -> 112.2, 128n 96c 54.8 -> 52.9, 128n 768c 7x7 12.3 -> 9.9,
+// 31n 1472c 27x17 38.2 -> 30.6, 54n 688c 18x18 5x5 44.2 -> 28.9, 128n 1392c 9x9 5x5 59 -> 42, 3n 224c 182x182 46 -> 38,
+// 2n 1440c 161x87 1x1 68 -> 62.
 #include "spio_conv_common.h"
 
 using namespace spio;
@@ -103,53 +114,55 @@ constexpr int WAVES = GB * TS;
 constexpr int THREADS = 64 * WAVES;
 constexpr bool kDbias = SPIO_HAS_BIAS != 0;
 
-// ---- weight gradient ----
-constexpr int S2 = 2 * ((kS + 1) / 2);
-constexpr int NBLK = S2 / 2;          // column-tap pairs
-constexpr int ND = kR + 1;            // values of delta
-constexpr int NPAIR = kR / 2 + 1;     // aligned dy row pairs one x row meets
+// ---- weight gradient: column taps 4 nb .. 4 nb + 3 share one MFMA ----
+constexpr int NB4 = (kS + 3) / 4;
 // Column blocks (SPIO_BQ > 0): a workgroup owns BQ columns (of dx, and of dy for the weight
 // gradient) and stages BQ + S - 1 columns of x and of dy: the extra columns hold the neighbouring
 // blocks' pixels (the data gradient of the block's edge columns needs the neighbours' dy, the
-// weight gradient the neighbours' x), or zeros at the image's edges.  The weight gradient reads dy
-// in 32-pixel chunks from the block's first column on, so BQ is a multiple of 32: a chunk that
-// reached into the right-hand extra columns would count the neighbour's dy a second time.
+// weight gradient the neighbours' x), or zeros at the image's edges.  The weight gradient's dy
+// fragments are cleared where they reach into the extra columns, or the neighbour's dy would count twice.
 // 0 = the whole width.
 constexpr bool kColBlocks = SPIO_BQ > 0;
 constexpr int BQ = kColBlocks ? SPIO_BQ : DW;
 constexpr int QBLKS = (DW + BQ - 1) / BQ;
-static_assert(!kColBlocks || (NB == 1 && BQ % 32 == 0), "column blocks: one image per row, a multiple of 32 columns");
+static_assert(!kColBlocks || NB == 1, "column blocks: one image per row");
 constexpr int WPI = BQ + kS - 1;      // padded width of one image (block)
 constexpr int F = NB * WPI;           // flattened pixels of a staged row
 constexpr int KSPAN = (NB - 1) * WPI + BQ;
-constexpr int KC = (KSPAN + 31) / 32;     // 32-pixel chunks
+constexpr int KC = (KSPAN + 1 + 31) / 32;  // 32-pixel chunks; the first begins one pixel before the row
 constexpr int CPW = (KC + TS - 1) / TS;   // chunks per wave
-// ---- data gradient ----
-constexpr int NS = 2 * ((kR + 1) / 2);   // accumulator row slots
-constexpr int NACC = NS / 2;
-constexpr int KB = (kS + 3) / 4;         // MFMA K-steps per dy row (4 column taps each)
-constexpr int WT = (F - kS + 1 + 15) / 16;   // 16-pixel tiles of a dx row
+// ---- data gradient: a tile is 16 pairs of neighbouring pixels ----
+constexpr int KB = (kS + 1 + 3) / 4;      // MFMA K-steps per dy row (4 of a pair's S + 1 columns each)
+constexpr int WT = (F - kS + 1 + 31) / 32;   // 32-pixel tiles of a dx row
 constexpr int TPW = (WT + TS - 1) / TS;      // tiles per wave
 // ---- LDS geometry ----
-constexpr int FPX = 32 * KC + S2 - 1;  // x pixels a weight-gradient read can touch
-constexpr int GSX = FPX + ((9 - FPX % 16) + 16) % 16;  // x group stride (pixels), = 9 mod 16
-constexpr int FPD_W = PR + 32 * KC;                    // dy pixels: weight-gradient reads
-constexpr int FPD_D = 16 * WT + 4 * KB - 1;            // dy pixels: data-gradient reads
+// The pixels of a staged row lie in two planes, even ones first: lanes of the data gradient read every
+// second pixel.  The planes are 8 cells (half the banks) apart modulo 16, the groups so that the cells a
+// wave's threads write fall into different banks.  Chunks and tiles past the last one (waves share a
+// row) read and write cells that exist; they hold zeros, and nobody looks at the results.
+constexpr int plane_cells(int pixels) { return (pixels + 1) / 2 + ((8 - (pixels + 1) / 2 % 16) + 16) % 16; }
+constexpr int GS_MOD = GB > 4 ? 9 : GB > 2 ? 2 : 4;
+constexpr int group_cells(int plane, int pixels) { return plane + pixels / 2 + ((GS_MOD - (plane + pixels / 2) % 16) + 16) % 16; }
+constexpr int FPX = 32 * CPW * TS + 4 * NB4 - 2;  // x pixels a weight-gradient read can touch
+constexpr int HX = plane_cells(FPX);
+constexpr int GSX = group_cells(HX, FPX);  // x group stride
+constexpr int DL = PR > 0 ? PR : 1;  // pixel of the first dy column: at least one zero (or neighbour's) pixel before it
+constexpr int DO = DL - PR;
+constexpr int FPD_W = DL + 32 * CPW * TS;                    // dy pixels: weight-gradient reads
+constexpr int FPD_D = DO + 32 * TPW * TS + 4 * KB - 2;       // dy pixels: data-gradient reads
 constexpr int FPD = FPD_W > FPD_D ? FPD_W : FPD_D;
-constexpr int GSD = FPD + ((9 - FPD % 16) + 16) % 16;  // dy group stride, = 9 mod 16
-constexpr int NRX = 2;                                 // x ring rows
-// dy ring rows: even, >= R+1; and at least 4 when the bias is summed, because that sum reads the
-// whole row pair (t-1, t) in the step that stages row t+1 (with a one-row filter the weight
-// gradient itself needs only two rows)
-constexpr int NRD = (SPIO_HAS_BIAS && kR == 1) ? 4 : 2 * ((kR + 2) / 2);
+constexpr int HD = plane_cells(FPD);
+constexpr int GSD = group_cells(HD, FPD);  // dy group stride
+SPIO_DEVICE constexpr int pos(int pixel, int plane) { return (pixel >> 1) + (pixel & 1) * plane; }
 // ring rows carry one spare unit behind the last group: the cell that threads without a source
 // cell write their (zero) load result to
 constexpr int XROW_UNITS = GB * GSX + 1;
-constexpr int DROW_UNITS = GB * GSD + 1 + ((4 - (GB * GSD + 1) % 16) + 16) % 16;
+constexpr int DROW_UNITS = GB * GSD + 1;
 constexpr int XDUMP = GB * GSX;
 constexpr int DDUMP = GB * GSD;
-constexpr int OSTRIDE = GB * 16 + 16;        // bytes per pixel in the dx output stage
-constexpr int OUT_ROW_BYTES = 16 * WT * OSTRIDE;
+constexpr int OSTRIDE = GB * 16 + 16;        // bytes per pixel in the dx output stage, two planes as well
+constexpr int OPLANE = 16 * TPW * TS * OSTRIDE + 128;
+constexpr int OUT_ROW_BYTES = 2 * OPLANE;
 constexpr int X_CELLS = F * GB;
 constexpr int LPTX = (X_CELLS + THREADS - 1) / THREADS;
 // dy cells a workgroup loads per row: the real columns of whole rows (the halo stays zero), all
@@ -162,27 +175,20 @@ constexpr int GBLKS = (kGroups + GB - 1) / GB;
 constexpr int NBLKS = (kN + NB * ITERS - 1) / (NB * ITERS);
 constexpr int PBLKS = (DH + BH - 1) / BH;
 constexpr int NUM_BLOCKS = GBLKS * PBLKS * QBLKS * NBLKS;
-// steps: dy rows p0-PB .. p0+BH-1+PT, then PB more for the last x rows.  The bias sum takes a dy
-// row pair one step after its first row was staged, so a one-row filter needs one more step
-// when the sum is wanted.
-constexpr int ROWS = BH + PB + kR - 1 + (SPIO_HAS_BIAS && kR == 1 ? 1 : 0);
+// steps: dy rows p0-PB .. p0+BH-1+PT, then PB more for the last x rows
+constexpr int ROWS = BH + PB + kR - 1;
 
 constexpr int gcd_(int a, int b) { return b == 0 ? a : gcd_(b, a % b); }
-constexpr int LCM = NS / gcd_(NS, PF) * PF;  // lcm(NS, PF): even
+constexpr int lcm_(int a, int b) { return a / gcd_(a, b) * b; }
+constexpr int LCM = lcm_(kR, PF);  // PF is even, so this is too
 // up to SPIO_MAX_UNROLL steps the step loop is unrolled completely, longer ones run in chunks
 constexpr bool kFullUnroll = ROWS <= SPIO_MAX_UNROLL;
 constexpr int UNROLL = kFullUnroll ? (ROWS + LCM - 1) / LCM * LCM : LCM;
 constexpr int pmod(int a, int m) { return ((a % m) + m) % m; }
 
-constexpr int RING_UNITS = NRX * XROW_UNITS + NRD * DROW_UNITS;
+constexpr int RING_UNITS = 2 * XROW_UNITS + 2 * DROW_UNITS;  // two rows each: a step's and the next one's
 constexpr int STREAM_UNITS = RING_UNITS + 2 * OUT_ROW_BYTES / 16;
 constexpr int FILTER_UNITS = GB * 8 * kR * kS;  // filters staged once at the start
-// Filter rows whose row-slot halves are exchanged through the per-wave scratch in one go: all of
-// them where that fits 96 KB of LDS for the workgroup (every exchange costs an LDS round trip),
-// else one; one when waves share a group, whose sums are then added row by row.
-constexpr int RCH = (TS == 1 && WAVES * kR * NBLK * 512 <= 96 * 1024) ? kR : 1;
-constexpr int SCRATCH_FLOATS = RCH * NBLK * 128;  // per wave: row-slot halves
-constexpr int RED_FLOATS = GB * (TS - 1) * NBLK * 128;
 constexpr int GROUP_FLOATS = kR * kS * 64;
 // Two-stage publishing (SPIO_PARTIALS = 1): every workgroup stores its sums, in grad_weight order
 // (and its GB * 8 bias sums behind them), into its own block of a workspace that takes the place
@@ -192,8 +198,7 @@ constexpr int GROUP_FLOATS = kR * kS * 64;
 // other (14 ns each: 3.6 us for 256 workgroups at N=128, C=64, 56x56); nothing to zero first.
 constexpr int PART_FLOATS = GB * GROUP_FLOATS + (SPIO_HAS_BIAS ? GB * 8 : 0);  // one workgroup's block
 constexpr int NPART = NBLKS * PBLKS * QBLKS;  // blocks per channel block
-constexpr int PUBLISH_FLOATS =
-    WAVES * SCRATCH_FLOATS + RED_FLOATS + GB * GROUP_FLOATS + (SPIO_HAS_BIAS ? WAVES * 8 : 0);
+constexpr int PUBLISH_FLOATS = WAVES * GROUP_FLOATS + (SPIO_HAS_BIAS ? WAVES * 8 : 0);
 constexpr int max3(int a, int b, int c) { return a > b ? (a > c ? a : c) : (b > c ? b : c); }
 constexpr int LDS_UNITS = max3(STREAM_UNITS, FILTER_UNITS, (PUBLISH_FLOATS + 3) / 4);
 static_assert(LDS_UNITS * 16 <= 160 * 1024, "LDS overflow");
@@ -250,7 +255,7 @@ SPIO_KERNEL_NAME(spio_uint4* __restrict__ grad_input, float* __restrict__ grad_w
     // the staged filters, after the last one the reduction scratch.
     __shared__ spio_uint4 lds[LDS_UNITS];
     spio_uint4* const xring = lds;
-    spio_uint4* const dring = lds + NRX * XROW_UNITS;
+    spio_uint4* const dring = lds + 2 * XROW_UNITS;
     unsigned char* const ostage = reinterpret_cast<unsigned char*>(lds + RING_UNITS);
 
     const int tid = thread_id();
@@ -258,8 +263,8 @@ SPIO_KERNEL_NAME(spio_uint4* __restrict__ grad_input, float* __restrict__ grad_w
     // scalar wave index: conditions on it become scalar branches, so no MFMA (which ignores the
     // lane mask) is issued under an empty mask
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wg = wave % GB;
-    const int ws = wave / GB;
+    const int wg = TS == 1 ? wave : wave % GB;
+    const int ws = TS == 1 ? 0 : wave / GB;
 
     // Tile order: row blocks fastest, so that neighbours in a run of SPIO_XCD_CHUNK tiles share halo
     // rows through one XCD's L2.  Where channel blocks share lines they go fastest instead, a run
@@ -283,8 +288,9 @@ SPIO_KERNEL_NAME(spio_uint4* __restrict__ grad_input, float* __restrict__ grad_w
     const int gglob = cb * GB + wg;
     const bool wave_active = gglob < kGroups;
 
-    // ---- data-gradient filter fragments: wfrag[d][u], d = (phase - 2*acc) mod NS ----
-    // A[m = dx channel ch][jj] = w[8g+jj][R-1-r][S-1-s][ch].  The workgroup copies its groups'
+    // ---- data-gradient filter fragments: wfrag[r][u] ----
+    // A[m = 8 j + ch][(kb, jj)] = w[8g+jj][R-1-r][S-1-s][ch], s = 4 u + kb - j: pixel j of a pair meets
+    // column 4 u + kb of the pair's S + 1 source columns under tap s.  The workgroup copies its groups'
     // filters to LDS as they lie in memory and every wave reads its fragments with the
     // transposing LDS read (same scheme as the data-gradient mode of conv2d_gw8_mfma.hip).
     // The filter loads are issued here, the loads of the first rows right behind them, and only
@@ -304,29 +310,28 @@ SPIO_KERNEL_NAME(spio_uint4* __restrict__ grad_input, float* __restrict__ grad_w
         }
     }
     __builtin_amdgcn_sched_barrier(0);  // keep the filter loads ahead of the row loads
-    spio_half8 wfrag[NS][KB];
+    spio_half8 wfrag[kR][KB];
 
     // ---- lane roles ----
     // weight gradient (transposing reads): block kb = lane/16 covers pixels 8*kb..8*kb+7, source
-    // lane 4*jr + t supplies pixel jr (+4 for the second read) of unit t/2 (dy row j or column
-    // tap sj) and channel half t%2.
+    // lane 4*jr + t supplies pixel jr (+4 for the second read) of unit t/2 (dy: shift j, x: tap offset
+    // 2 sj) and channel half t%2.
     const int kb = lane >> 4;
     const int jr = (lane & 15) >> 2;
     const int tt = lane & 3;
     const int sel = tt >> 1;
-    const int xfrag_off = ((wg * GSX + 8 * kb + jr + sel) * 16) + (tt & 1) * 8;
-    const int dfrag_off = ((wg * GSD + PR + 8 * kb + jr) * 16) + (tt & 1) * 8;
-    // data gradient: D[m = 4*(lane/16)+i][n = lane%16]: pixel n, row slot lane/32, channels
+    const int xfrag_off = (wg * GSX + pos(8 * kb + jr + 2 * sel, HX)) * 16 + (tt & 1) * 8;
+    const int dfrag_off = (wg * GSD + pos(DL - 1 + 8 * kb + jr + sel, HD)) * 16 + (tt & 1) * 8;
+    // data gradient: D[m = 4*(lane/16)+i][n = lane%16]: pixel 2 n + out_j of the tile, channels
     // 4*((lane/16)&1) + i
-    const int out_j = lane >> 5;
-    const int out_kh = (lane >> 4) & 1;
-    const int out_n = lane & 15;
+    const int sfrag_unit = wg * GSD + (lane & 15) + pos(DO + kb, HD);
+    const int out_off = (lane >> 5) * OPLANE + (lane & 15) * OSTRIDE + wg * 16 + ((lane >> 4) & 1) * 8;
 
-    spio_float4 acc[ND][NBLK];  // weight gradient
+    spio_float4 acc[kR][NB4];  // weight gradient
 #pragma unroll
-    for (int d = 0; d < ND; ++d)
+    for (int r = 0; r < kR; ++r)
 #pragma unroll
-        for (int nb = 0; nb < NBLK; ++nb) acc[d][nb] = spio_float4{0.f, 0.f, 0.f, 0.f};
+        for (int nb = 0; nb < NB4; ++nb) acc[r][nb] = spio_float4{0.f, 0.f, 0.f, 0.f};
     spio_float4 accb = spio_float4{0.f, 0.f, 0.f, 0.f};  // bias gradient
     const spio_half8 ones8 = spio_half8{1, 1, 1, 1, 1, 1, 1, 1};
     (void)ones8;
@@ -362,7 +367,7 @@ SPIO_KERNEL_NAME(spio_uint4* __restrict__ grad_input, float* __restrict__ grad_w
                 const int f = cell / GB;
                 const int img = f / WPI;
                 const int col = q0 + f % WPI - PL - XOX;  // column of x
-                x_lds[l] = g * GSX + f;
+                x_lds[l] = g * GSX + pos(f, HX);
                 if (col >= 0 && col < kW && cb * GB + g < kGroups)
                     x_voff[l] = (unsigned)(((img * kH * kW + col) * kGroups + cb * GB + g) * 16);
             }
@@ -384,7 +389,7 @@ SPIO_KERNEL_NAME(spio_uint4* __restrict__ grad_input, float* __restrict__ grad_w
                     // whole rows: the cells are the real columns; column blocks: every staged column
                     const int q = kColBlocks ? q0 + (cell / GB) % WPI - PR : (cell / GB) % DW;  // domain column
                     const int img = kColBlocks ? 0 : cell / (GB * DW);
-                    unit = g * GSD + (kColBlocks ? cell / GB : img * WPI + q + PR);
+                    unit = g * GSD + pos(kColBlocks ? cell / GB + DO : img * WPI + q + DL, HD);
                     const int qd = q - DOX;  // column of dy
                     if (qd >= 0 && qd < kQ && cb * GB + g < kGroups)
                         voff = (unsigned)(((img * kP * kQ + qd) * kGroups + cb * GB + g) * (8 * kSrcBytes));
@@ -404,7 +409,8 @@ SPIO_KERNEL_NAME(spio_uint4* __restrict__ grad_input, float* __restrict__ grad_w
                     const int g = cell % GB;
                     const int q = (cell / GB) % BQ;
                     const int img = cell / (GB * BQ);
-                    from = (img * WPI + q) * OSTRIDE + g * 16;
+                    const int o = img * WPI + q;
+                    from = (o & 1) * OPLANE + (o >> 1) * OSTRIDE + g * 16;
                     const int wx = q0 + q - XOX;  // column of dx
                     if (q0 + q < DW && wx >= 0 && wx < kW && cb * GB + g < kGroups)
                         voff = (unsigned)(((img * kH * kW + wx) * kGroups + cb * GB + g) * (8 * kDstBytes));
@@ -477,14 +483,13 @@ SPIO_KERNEL_NAME(spio_uint4* __restrict__ grad_input, float* __restrict__ grad_w
             const int my_slot = (lane & 15) >> 3;
             typedef spio_short4 __attribute__((address_space(3))) * lds_ptr;
 #pragma unroll
-            for (int d = 0; d < NS; ++d) {
+            for (int r = 0; r < kR; ++r) {
 #pragma unroll
                 for (int u = 0; u < KB; ++u) {
-                    const int s = 4 * u + fkb;
-                    const int r_src = (d - src_slot + NS) % NS;
-                    const int r_mine = (d - my_slot + NS) % NS;
-                    const int rr = r_src < kR ? kR - 1 - r_src : 0;  // dead taps: any valid address
-                    const int ss = s < kS ? kS - 1 - s : 0;
+                    const int s_src = 4 * u + fkb - src_slot;
+                    const int s_mine = 4 * u + fkb - my_slot;
+                    const int rr = kR - 1 - r;
+                    const int ss = s_src >= 0 && s_src < kS ? kS - 1 - s_src : 0;  // dead taps: any valid address
                     const unsigned char* base = reinterpret_cast<const unsigned char*>(lds) +
                                                 ((((wg * 8 + fjr) * kR + rr) * kS + ss) * 16) + (ft4 & 1) * 8;
                     union {
@@ -493,8 +498,8 @@ SPIO_KERNEL_NAME(spio_uint4* __restrict__ grad_input, float* __restrict__ grad_w
                     } v;
                     v.q[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)base);
                     v.q[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)(base + 4 * kR * kS * 16));
-                    if (!(wave_active && r_mine < kR && s < kS)) v.h = spio_half8{0, 0, 0, 0, 0, 0, 0, 0};
-                    wfrag[d][u] = v.h;
+                    if (!(wave_active && s_mine >= 0 && s_mine < kS)) v.h = spio_half8{0, 0, 0, 0, 0, 0, 0, 0};
+                    wfrag[r][u] = v.h;
                 }
             }
             block_sync();  // everyone has its fragments before the rings are zero-filled
@@ -508,11 +513,19 @@ SPIO_KERNEL_NAME(spio_uint4* __restrict__ grad_input, float* __restrict__ grad_w
         dy_to_ring(dpre[0], 0);
         block_sync();
 
-        spio_float4 dacc[TPW][NACC];  // data gradient: rotating row slots
+        // Data gradient: dy row t reaches dx rows t - r (named by the step that completes them, less R-1);
+        // each has one slot of sums, t - r modulo R, from its first dy row (r = 0) to its last.
+        spio_float4 dacc[TPW][kR];
+        // Weight gradient: fragments of the last R dy rows, row t in slot t modulo R.  They are read once, when
+        // the row is the newest; rows the block does not own (halo, past the image) count as zero.
+        spio_half8 afrag[kR][CPW];
 #pragma unroll
-        for (int i = 0; i < TPW; ++i)
+        for (int r = 0; r < kR; ++r) {
 #pragma unroll
-            for (int a = 0; a < NACC; ++a) dacc[i][a] = spio_float4{0.f, 0.f, 0.f, 0.f};
+            for (int i = 0; i < TPW; ++i) dacc[i][r] = spio_float4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int ci = 0; ci < CPW; ++ci) afrag[r][ci] = spio_half8{0, 0, 0, 0, 0, 0, 0, 0};
+        }
 
         // Coalesced store of the dx row staged at step `ts` (domain row p0 - (R-1) + ts), one step
         // later.  Steps that finish no row of the block, or a domain row outside dx, store through
@@ -548,68 +561,57 @@ SPIO_KERNEL_NAME(spio_uint4* __restrict__ grad_input, float* __restrict__ grad_w
             for (int uu = 0; uu < UNROLL; ++uu) {
                 const int t = tb + uu;
                 if (t >= ROWS) continue;  // (with a second way out of the loop the compiler leaves 12 steps rolled)
-                const int sp = uu & 1;                   // parity of t: x ring row, parity of delta
+                const int sp = uu & 1;                   // parity of t: ring rows
                 const int pbuf = uu % PF;                // register buffer that held row t
-                const int ph = uu % NS;                  // data-gradient phase: t mod NS
+                const int ph = uu % kR;                  // t mod R
                 const int obuf = uu & 1;
+                // what the step has to do, known at compile time in an unrolled loop: dy rows are named by
+                // the step that staged them (row p0-PB+tau at step tau; the block owns tau in [PB, PB+bh_eff)),
+                // x row t (p0-(R-1)+t) meets dy rows t - r under filter row r, dy row t reaches the dx rows
+                // that complete at steps t .. t+R-1
+                const bool multiply_x = !kFullUnroll || t >= PB;
+                const bool read_dy = !kFullUnroll || (t >= PB && t < PB + BH);
+                const bool multiply_dy = !kFullUnroll || t < BH + kR - 1;
 
-                // 1. fragment reads: x row p0-(R-1)+t, the dy row pairs it meets (dy rows are named
-                //    by the step that staged them: row p0-PB+tau at step tau; the block owns
-                //    tau in [PB, PB+bh_eff)), and dy row p0-PB+t as the data gradient's source row
-                const int hcur = p0 - (kR - 1) + t;
-                const bool x_live = t >= PB && hcur >= XOY && hcur < XOY + kH;
-                const int dcur = p0 - PB + t;
-                const bool d_live = t < bh_eff + kR - 1 && dcur >= DOY && dcur < DOY + kP;
-                const int tbase = t - sp;
-                const int own_lo = PB, own_hi = PB + bh_eff;  // owned dy rows: [own_lo, own_hi)
-                const bool bias_pair = kDbias && sp == 1 && tbase + 1 >= own_lo && tbase < own_hi;
-                const bool do_w = wave_active && (x_live || bias_pair);
-                spio_half8 bfrag[CPW][NBLK], afrag[CPW][NPAIR];
-                if (do_w) {
+                // 1. fragment reads
+                spio_half8 bfrag[CPW][NB4];
 #pragma unroll
-                    for (int ci = 0; ci < CPW; ++ci) {
-                        const int ch = ws + TS * ci;
-                        if (TS > 1 && ch >= KC) break;
+                for (int ci = 0; ci < CPW; ++ci) {
+                    const int ch = CPW * ws + ci;
+                    if (multiply_x) {
                         const unsigned char* xrow =
                             reinterpret_cast<const unsigned char*>(xring + sp * XROW_UNITS) + xfrag_off;
 #pragma unroll
-                        for (int nb = 0; nb < NBLK; ++nb) {
-                            const unsigned char* pb0 = xrow + (32 * ch + 2 * nb) * 16;
-                            bfrag[ci][nb] = read_tr_pair(pb0, pb0 + 4 * 16);
-                        }
-#pragma unroll
-                        for (int m = 0; m < NPAIR; ++m) {
-                            const int i2 = tbase - 2 * m;  // first row of the pair (step numbering)
-                            if (i2 + 1 >= own_lo && i2 < own_hi) {
-                                const int slot = (i2 + sel + NRD) % NRD;
-                                const unsigned char* pa0 =
-                                    reinterpret_cast<const unsigned char*>(dring + slot * DROW_UNITS) +
-                                    dfrag_off + (32 * ch) * 16;
-                                spio_half8 a = read_tr_pair(pa0, pa0 + 4 * 16);
-                                // a halo row in the pair belongs to the neighbouring block; the
-                                // transposed fragment holds row j = (lane % 16) / 8 of the pair
-                                const int row = i2 + ((lane & 15) >> 3);
-                                if (row < own_lo || row >= own_hi) a = spio_half8{0, 0, 0, 0, 0, 0, 0, 0};
-                                afrag[ci][m] = a;
-                            }
+                        for (int nb = 0; nb < NB4; ++nb) {
+                            const unsigned char* pb0 = xrow + (16 * ch + 2 * nb) * 16;
+                            bfrag[ci][nb] = read_tr_pair(pb0, pb0 + 2 * 16);
                         }
                     }
+                    if (read_dy) {
+                        const unsigned char* pa0 = reinterpret_cast<const unsigned char*>(dring + sp * DROW_UNITS) +
+                                                   dfrag_off + (16 * ch) * 16;
+                        spio_half8 a = read_tr_pair(pa0, pa0 + 2 * 16);
+                        if (kColBlocks) {  // the block's own columns only (the lane holds row m = lane % 16)
+                            const int q = 32 * ch + 8 * kb + ((lane & 15) >> 3) - 1;
+#pragma unroll
+                            for (int e = 0; e < 8; ++e)
+                                if (q + e < 0 || q + e >= BQ) a[e] = 0;
+                        }
+                        if ((!kFullUnroll && t < PB) || ((!kFullUnroll || DH % BH != 0) && t >= PB + bh_eff))
+                            a = spio_half8{0, 0, 0, 0, 0, 0, 0, 0};
+                        afrag[ph][ci] = a;
+                    }
                 }
-                const bool do_d = wave_active && d_live;
                 spio_half8 sfrag[TPW][KB];
-                if (do_d) {
-                    const spio_uint4* rrow =
-                        dring + (t % NRD) * DROW_UNITS + wg * GSD + (lane & 15) + (lane >> 4);
+                if (multiply_dy) {
+                    const spio_uint4* rrow = dring + sp * DROW_UNITS + sfrag_unit;
 #pragma unroll
                     for (int i = 0; i < TPW; ++i) {
-                        const int tile = ws + TS * i;
-                        if (TS == 1 || tile < WT) {
 #pragma unroll
-                            for (int u = 0; u < KB; ++u) {
-                                Pack16 v;
-                                v.u = rrow[16 * tile + 4 * u];
-                                sfrag[i][u] = v.h;
-                            }
+                        for (int u = 0; u < KB; ++u) {
+                            Pack16 v;
+                            v.u = rrow[16 * (TPW * ws + i) + 2 * u];
+                            sfrag[i][u] = v.h;
                         }
                     }
                 }
@@ -622,81 +624,57 @@ SPIO_KERNEL_NAME(spio_uint4* __restrict__ grad_input, float* __restrict__ grad_w
                 // 3. the dx row finished in the previous step goes out
                 if (!kFullUnroll || t - 1 >= kR - 1) store_dx_row(t - 1, (uu + 1) & 1);
 
-                // 4. rows t+1 into LDS (dy rows past the last one become zero).  The ring rows
-                //    written here are not read in this step, except for dy entries of the weight
-                //    gradient whose filter row is out of range and whose product is ignored.
+                // 4. rows t+1 into LDS, where nothing of this step reads (dy rows past the last one become zero)
                 if (t + 1 < ROWS) {
 #pragma unroll
                     for (int l = 0; l < LPTX; ++l)
-                        xring[((sp + 1) & 1) * XROW_UNITS + x_lds[l]] = xpre[(uu + 1) % PF][l];
-                    dy_to_ring(dpre[(uu + 1) % PF], (t + 1) % NRD);
+                        xring[(sp ^ 1) * XROW_UNITS + x_lds[l]] = xpre[(uu + 1) % PF][l];
+                    dy_to_ring(dpre[(uu + 1) % PF], sp ^ 1);
                 }
 
-                // 5. multiply: weight gradient ...
-                if (do_w) {
-#pragma unroll
-                    for (int ci = 0; ci < CPW; ++ci) {
-                        const int ch = ws + TS * ci;
-                        if (TS > 1 && ch >= KC) break;
-#pragma unroll
-                        for (int m = 0; m < NPAIR; ++m) {
-                            const int i2 = tbase - 2 * m;
-                            if (i2 + 1 >= own_lo && i2 < own_hi) {
-                                const int d = sp + 2 * m;  // = t - i2
-                                if (d <= kR && x_live) {
-#pragma unroll
-                                    for (int nb = 0; nb < NBLK; ++nb)
-                                        acc[d][nb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
-                                            afrag[ci][m], bfrag[ci][nb], acc[d][nb], 0, 0, 0);
-                                }
-                                if (m == 0 && bias_pair)
-                                    accb = __builtin_amdgcn_mfma_f32_16x16x32_f16(afrag[ci][0], ones8, accb, 0, 0, 0);
-                            }
-                        }
-                    }
-                }
-                //    ... and data gradient: dy row t into the live dx rows
-                if (do_d) {
+                // 5. multiply: data gradient, dy row t into the dx rows that exist ...
+                if (multiply_dy) {
 #pragma unroll
                     for (int i = 0; i < TPW; ++i) {
-                        const int tile = ws + TS * i;
-                        if (TS == 1 || tile < WT) {
 #pragma unroll
-                            for (int a = 0; a < NACC; ++a) {
-                                const int d = pmod(ph - 2 * a, NS);
+                        for (int u = 0; u < KB; ++u) {
 #pragma unroll
-                                for (int u = 0; u < KB; ++u)
-                                    dacc[i][a] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
-                                        wfrag[d][u], sfrag[i][u], dacc[i][a], 0, 0, 0);
+                            for (int r = 0; r < kR; ++r) {
+                                if (kFullUnroll && (t - r < 0 || t - r >= BH)) continue;
+                                spio_float4& d = dacc[i][pmod(ph - r, kR)];
+                                const spio_float4 before = r == 0 && u == 0 ? spio_float4{0.f, 0.f, 0.f, 0.f} : d;
+                                d = __builtin_amdgcn_mfma_f32_16x16x32_f16(wfrag[r][u], sfrag[i][u], before, 0, 0, 0);
                             }
                         }
                     }
                 }
-
-                // 6. the dx row that received its last tap (row p0-(R-1)+t): stage it if the block
-                //    owns it, reset its slot
-                {
-                    const int slot = pmod(ph - (kR - 1), NS);
-                    const int a = slot >> 1;
-                    const int j = slot & 1;
-                    const bool emit = t >= kR - 1 && t < kR - 1 + bh_eff;
-                    if (wave_active && out_j == j) {
+                //    ... and weight gradient
+                if (multiply_x) {
 #pragma unroll
-                        for (int i = 0; i < TPW; ++i) {
-                            const int tile = ws + TS * i;
-                            if (TS == 1 || tile < WT) {
-                                if (emit) {
-                                    Pack8 o;
+                    for (int ci = 0; ci < CPW; ++ci) {
 #pragma unroll
-                                    for (int e = 0; e < 4; ++e) o.h[e] = (spio_half)dacc[i][a][e];
-                                    *reinterpret_cast<spio_uint2*>(ostage + obuf * OUT_ROW_BYTES +
-                                                                   (16 * tile + out_n) * OSTRIDE + wg * 16 +
-                                                                   out_kh * 8) = o.u;
-                                }
+                        for (int nb = 0; nb < NB4; ++nb) {
 #pragma unroll
-                                for (int e = 0; e < 4; ++e) dacc[i][a][e] = 0.f;
+                            for (int r = 0; r < kR; ++r) {
+                                if (kFullUnroll && (t - r < PB || t - r >= PB + BH)) continue;
+                                acc[r][nb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                                    afrag[pmod(ph - r, kR)][ci], bfrag[ci][nb], acc[r][nb], 0, 0, 0);
                             }
                         }
+                        if (kDbias && read_dy)
+                            accb = __builtin_amdgcn_mfma_f32_16x16x32_f16(afrag[ph][ci], ones8, accb, 0, 0, 0);
+                    }
+                }
+
+                // 6. the dx row that received its last tap (row p0-(R-1)+t): stage it
+                if (!kFullUnroll || (t >= kR - 1 && t < kR - 1 + BH)) {
+#pragma unroll
+                    for (int i = 0; i < TPW; ++i) {
+                        Pack8 o;
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) o.h[e] = (spio_half)dacc[i][pmod(ph - (kR - 1), kR)][e];
+                        *reinterpret_cast<spio_uint2*>(ostage + obuf * OUT_ROW_BYTES +
+                                                       16 * (TPW * ws + i) * OSTRIDE + out_off) = o.u;
                     }
                 }
                 block_sync();
@@ -705,125 +683,58 @@ SPIO_KERNEL_NAME(spio_uint4* __restrict__ grad_input, float* __restrict__ grad_w
         store_dx_row(ROWS - 1, (ROWS - 1) & 1);  // the last staged row (if it is a real one)
     }
 
-    // ---- publish grad_weight (and grad_bias): as in conv2d_gw8_wgrad_mfma.hip ----
-    // dw[k,r,s,c] = acc[delta = r] (lanes 0-31: j = 0) + acc[delta = r+1] (lanes 32-63: j = 1);
-    // the halves meet in a per-wave LDS scratch, the waves of a split group add their sums
-    // through LDS, the group's R*S*64 sums are staged in grad_weight order and added with
-    // atomics of 64 consecutive floats.
+    // ---- publish grad_weight (and grad_bias) ----
+    // Sum m = 8 j + k, n = 8 sj + c of acc[r][nb] belongs to filter row r and column 4 nb + 2 sj + 1 - j.  Every
+    // wave stages its R*S*64 sums in grad_weight order; the waves of a group share the way out (64
+    // consecutive floats at a time), where the sums of the group's waves meet.
     block_sync();  // every wave is done with the rings and the output stage
     {
-        float* scratch = reinterpret_cast<float*>(lds) + wave * SCRATCH_FLOATS;
-        float* red = reinterpret_cast<float*>(lds) + WAVES * SCRATCH_FLOATS;
-        float* gstage = reinterpret_cast<float*>(lds) + WAVES * SCRATCH_FLOATS + RED_FLOATS + wg * GROUP_FLOATS;
-        const int k4 = 4 * ((lane >> 4) & 1);
-        const int sj = (lane & 15) >> 3;
-        const int c = lane & 7;
-        if (RCH > 1) {
-            // all filter rows at once: lanes 32-63 leave their halves in the scratch as float4s, one
-            // wave-level sync, lanes 0-31 add them and stage the sums in grad_weight order
-            spio_float4* half4 = reinterpret_cast<spio_float4*>(scratch);
-            if (lane >= 32) {
+        float* const sums = reinterpret_cast<float*>(lds);
+        float* const gstage = sums + wg * GROUP_FLOATS;  // of the group's first wave
+        {
+            const int c = lane & 7;
+            const int k4 = 4 * ((lane >> 4) & 1);
+            float* const mine = sums + wave * GROUP_FLOATS;
 #pragma unroll
-                for (int r = 0; r < kR; ++r)
+            for (int nb = 0; nb < NB4; ++nb) {
+                const int s = 4 * nb + 2 * ((lane & 15) >> 3) + 1 - (lane >> 5);
+                if (s < kS) {
 #pragma unroll
-                    for (int nb = 0; nb < NBLK; ++nb) half4[(r * NBLK + nb) * 32 + (lane - 32)] = acc[r + 1][nb];
-            }
-            wave_sync();  // lanes 32-63 stored, lanes 0-31 load
-            if (wave_active && lane < 32) {
+                    for (int r = 0; r < kR; ++r)
 #pragma unroll
-                for (int r = 0; r < kR; ++r)
-#pragma unroll
-                    for (int nb = 0; nb < NBLK; ++nb) {
-                        const spio_float4 total = acc[r][nb] + half4[(r * NBLK + nb) * 32 + lane];
-                        const int s = 2 * nb + sj;
-                        if (s < kS) {
-#pragma unroll
-                            for (int e = 0; e < 4; ++e) gstage[(((k4 + e) * kR + r) * kS + s) * 8 + c] = total[e];
-                        }
-                    }
-            }
-        } else {
-#pragma unroll
-            for (int r = 0; r < kR; ++r) {
-                float total[NBLK][4];
-    #pragma unroll
-                for (int nb = 0; nb < NBLK; ++nb) {
-                    if (lane >= 32) {
-    #pragma unroll
-                        for (int e = 0; e < 4; ++e) scratch[e * 32 + (lane - 32)] = acc[r + 1][nb][e];
-                    }
-                    wave_sync();  // lanes 32-63 stored, lanes 0-31 load
-    #pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        total[nb][e] = 0.f;
-                        if (lane < 32) total[nb][e] = acc[r][nb][e] + scratch[e * 32 + lane];
-                    }
-                    wave_sync();  // the scratch is free for the next tap pair
+                        for (int e = 0; e < 4; ++e) mine[(((k4 + e) * kR + r) * kS + s) * 8 + c] = acc[r][nb][e];
                 }
-                if (TS > 1) {
-                    if (ws > 0 && lane < 32) {
-    #pragma unroll
-                        for (int nb = 0; nb < NBLK; ++nb)
-    #pragma unroll
-                            for (int e = 0; e < 4; ++e)
-                                red[(((wg * (TS - 1) + ws - 1) * NBLK + nb) * 4 + e) * 32 + lane] = total[nb][e];
-                    }
-                    block_sync();
-                    if (ws == 0 && lane < 32) {
-    #pragma unroll
-                        for (int w2 = 0; w2 < TS - 1; ++w2)
-    #pragma unroll
-                            for (int nb = 0; nb < NBLK; ++nb)
-    #pragma unroll
-                                for (int e = 0; e < 4; ++e)
-                                    total[nb][e] += red[(((wg * (TS - 1) + w2) * NBLK + nb) * 4 + e) * 32 + lane];
-                    }
-                }
-                if (wave_active && ws == 0 && lane < 32) {
-    #pragma unroll
-                    for (int nb = 0; nb < NBLK; ++nb) {
-                        const int s = 2 * nb + sj;
-                        if (s < kS) {
-    #pragma unroll
-                            for (int e = 0; e < 4; ++e) gstage[(((k4 + e) * kR + r) * kS + s) * 8 + c] = total[nb][e];
-                        }
-                    }
-                }
-                if (TS > 1) block_sync();  // the scratch is rewritten for the next filter row
             }
-}
+        }
+        if (TS > 1)
+            block_sync();
+        else
+            wave_sync();  // all lanes read what all lanes staged
+        auto total = [&](int i) {
+            float v = gstage[64 * i + lane];
+#pragma unroll
+            for (int w2 = 1; w2 < TS; ++w2) v += gstage[w2 * GB * GROUP_FLOATS + 64 * i + lane];
+            return v;
+        };
 #if SPIO_PARTIALS
         // this workgroup's block of the workspace: [group][k][r][s][c], then [group][k] bias sums
         float* const pblock = grad_weight + ((long long)cb * NPART + (nbk * PBLKS + pb) * QBLKS + q0 / BQ) * PART_FLOATS;
-        if (ws == 0) {  // groups past the last one store their zeros: the block is read whole
-            float* gout = pblock + wg * GROUP_FLOATS;
-            wave_sync();  // lanes 0-31 staged the sums, all lanes read them
+        float* const gout = pblock + wg * GROUP_FLOATS;  // groups past the last one store their zeros: the block is read whole
 #pragma unroll
-            for (int i = 0; i < kR * kS; ++i)
-                __builtin_nontemporal_store(wave_active ? gstage[64 * i + lane] : 0.f, gout + 64 * i + lane);
-        }
+        for (int i = ws; i < kR * kS; i += TS) __builtin_nontemporal_store(wave_active ? total(i) : 0.f, gout + 64 * i + lane);
 #else
-        if (wave_active && ws == 0) {
-            float* gout = grad_weight + (long long)gglob * GROUP_FLOATS;
-            wave_sync();  // lanes 0-31 staged the sums, all lanes read them
+        if (wave_active) {
+            float* const gout = grad_weight + (long long)gglob * GROUP_FLOATS;
 #pragma unroll
-            for (int i = 0; i < kR * kS; ++i) atomic_add_f32(gout + 64 * i + lane, gstage[64 * i + lane]);
+            for (int i = ws; i < kR * kS; i += TS) atomic_add_f32(gout + 64 * i + lane, total(i));
         }
 #endif
 #if SPIO_HAS_BIAS
         {
-            wave_sync();
-            if (lane >= 32) {
-#pragma unroll
-                for (int e = 0; e < 4; ++e) scratch[e * 32 + (lane - 32)] = accb[e];
-            }
-            wave_sync();
-            float* bslots = reinterpret_cast<float*>(lds) + WAVES * SCRATCH_FLOATS + RED_FLOATS +
-                            GB * GROUP_FLOATS;  // [wave][8]
+            float* bslots = sums + WAVES * GROUP_FLOATS;  // [wave][8]
             if ((lane & 47) == 0) {
 #pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    bslots[wave * 8 + k4 + e] = wave_active ? accb[e] + scratch[e * 32 + lane] : 0.f;
+                for (int e = 0; e < 4; ++e) bslots[wave * 8 + (lane >> 4) * 4 + e] = wave_active ? accb[e] : 0.f;
             }
             block_sync();
 #if SPIO_PARTIALS

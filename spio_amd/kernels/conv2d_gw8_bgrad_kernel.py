@@ -38,7 +38,10 @@ SOURCE = "conv2d_gw8_bgrad_mfma.hip"
 MAX_WAVES = 16
 MAX_LDS_BYTES = 128 * 1024
 MAX_LOADS_PER_THREAD = 4
-MAX_REGISTERS = 224  # estimated fragments + accumulators + prefetch buffers, in 32-bit registers
+MAX_REGISTERS = 256  # estimated fragments + accumulators + prefetch buffers, in 32-bit registers
+# Accumulators of the weight gradient.  The 14 of a 7x7 filter fit, but one pass is slower there than two kernels:
+# 256n 256c 14x14 55.7 us (best of 25 configurations) against 15.3 and 26.2, since both bound by the arithmetic.
+MAX_SUMS = 14
 GEOMETRIES_PER_HEIGHT = 6
 MAX_UNROLLED_STEPS = 40  # SPIO_MAX_UNROLL of the kernel: longer step loops run in chunks
 
@@ -118,46 +121,47 @@ def bgrad_geometry(params: Conv2dGw8Params, config: Conv2dGw8BgradConfig) -> Dic
     dh, dw = bgrad_domain(params)
     pb, pr = r - 1 - r // 2, s - 1 - s // 2  # the domain's padding below and right
     bh = config.block_h or dh
-    s2 = 2 * ((s + 1) // 2)
-    nblk = s2 // 2
+    nb4 = divup(s, 4)
     bq = config.block_q or dw
     wpi = bq + s - 1
     f = nb * wpi
     kspan = (nb - 1) * wpi + bq
-    kc = divup(kspan, 32)
+    kc = divup(kspan + 1, 32)
     cpw = divup(kc, ts)
-    ns = 2 * ((r + 1) // 2)
-    kb = divup(s, 4)
-    wt = divup(f - s + 1, 16)
+    kb = divup(s + 1, 4)
+    wt = divup(f - s + 1, 32)
     tpw = divup(wt, ts)
-    fpx = 32 * kc + s2 - 1
-    gsx = fpx + ((9 - fpx % 16) + 16) % 16
-    fpd = max(pr + 32 * kc, 16 * wt + 4 * kb - 1)
-    gsd = fpd + ((9 - fpd % 16) + 16) % 16
-    nrd = 4 if (params.has_bias and r == 1) else 2 * ((r + 2) // 2)
+
+    def group_cells(pixels):
+        plane = divup(pixels, 2)
+        plane += (8 - plane) % 16
+        return plane + pixels // 2 + ((9 if gb > 4 else 2 if gb > 2 else 4) - plane - pixels // 2) % 16
+
+    dl = max(pr, 1)
+    gsx = group_cells(32 * cpw * ts + 4 * nb4 - 2)
+    gsd = group_cells(max(dl + 32 * cpw * ts, dl - pr + 32 * tpw * ts + 4 * kb - 2))
     threads = 64 * gb * ts
     # every ring row carries a spare unit behind its last group (see the kernel)
-    ring_units = 2 * (gb * gsx + 1) + nrd * (gb * gsd + 1 + ((4 - (gb * gsd + 1) % 16) + 16) % 16)
-    out_row_bytes = 16 * wt * (gb * 16 + 16)
+    ring_units = 2 * (gb * gsx + 1) + 2 * (gb * gsd + 1)
+    out_row_bytes = 2 * (16 * tpw * ts * (gb * 16 + 16) + 128)
     stream_bytes = ring_units * 16 + 2 * out_row_bytes
     filter_bytes = gb * 8 * r * s * 16
-    rch = r if (ts == 1 and gb * ts * r * nblk * 512 <= 96 * 1024) else 1  # RCH of the kernel
-    publish_bytes = (gb * ts * rch * nblk * 128 + gb * (ts - 1) * nblk * 128 + gb * r * s * 64
-                     + (gb * ts * 8 if params.has_bias else 0)) * 4  # fmt: skip
+    publish_bytes = (gb * ts * r * s * 64 + (gb * ts * 8 if params.has_bias else 0)) * 4
     lptx = divup(f * gb, threads)
     lptd = divup((f if config.block_q else nb * dw) * gb, threads)  # grad_output loads per row
     registers = (
-        4 * ((r + 1) * nblk + 1)  # weight-gradient accumulators (+ bias)
-        + 4 * tpw * (ns // 2)  # data-gradient accumulators
-        + 4 * ns * kb  # filter fragments
-        + 4 * (cpw * (nblk + r // 2 + 1) + tpw * kb)  # operand fragments of one step
+        4 * (r * nb4 + 1)  # weight-gradient accumulators (+ bias)
+        + 4 * tpw * r  # data-gradient accumulators
+        + 4 * r * kb  # filter fragments
+        + 4 * r * cpw  # fragments of the last grad_output rows
+        + 4 * (cpw * nb4 + tpw * kb)  # other operand fragments of one step
         + 4 * pf * (lptx + lptd)  # prefetch buffers
     )
     g = dict(
-        NBLK=nblk, KC=kc, CPW=cpw, WT=wt, TPW=tpw, THREADS=threads,
+        NB4=nb4, KB=kb, KC=kc, CPW=cpw, WT=wt, TPW=tpw, THREADS=threads,
         LDS_BYTES=max(stream_bytes, filter_bytes, publish_bytes),
         LPTX=lptx, LPTD=lptd, REGISTERS=registers,
-        STEPS=bh + pb + r - 1 + (1 if params.has_bias and r == 1 else 0),
+        STEPS=bh + pb + r - 1,
         BH=bh, GBLKS=divup(params.groups, gb), PBLKS=divup(dh, bh), NBLKS=divup(params.n, nb * iters),
         BQ=bq, QBLKS=divup(dw, bq),
         PIXEL_EFF=(nb * bq) / (32.0 * kc),
@@ -181,6 +185,7 @@ def _config_is_legal(params, config) -> bool:
         and g["LDS_BYTES"] <= MAX_LDS_BYTES
         and g["LPTX"] <= MAX_LOADS_PER_THREAD
         and g["REGISTERS"] <= MAX_REGISTERS
+        and params.r * g["NB4"] < MAX_SUMS
         and config.prefetch >= 2
         and config.prefetch % 2 == 0
         and config.block_n * params.c * max(params.h * params.w, params.p * params.q) * 2 < 2**31
@@ -189,17 +194,15 @@ def _config_is_legal(params, config) -> bool:
 
 def _fits(params, config) -> bool:
     """Whether a lane's registers hold the sums, the filters, the rows in flight and a step's operands, or most of them.
-    The weights were fitted to what the compiler reports for 960 kernels of 76 shapes.  The line lies a quarter above
-    the registers there are, as some with 72 to 130 bytes a lane in memory are the best (128n 1392c 9x9 5x5 60 us, 76
-    without; but 32n 256c 28x28 5x5 34 and 23); those behind it, 16 waves mostly, are several times slower."""
+    The weights were fitted to what the compiler reports for 402 kernels of 67 shapes.  The line lies a tenth above the
+    registers there are: up to there the compiler keeps 20 to 130 bytes a lane in memory, if any, which costs little;
+    beyond it hundreds (16 waves mostly), which costs a multiple."""
     g = bgrad_geometry(params, config)
-    ns, kb = 2 * divup(params.r, 2), divup(params.s, 4)
-    kept = (params.r + 1) * g["NBLK"] + 1 + g["TPW"] * (ns // 2) + ns * kb
-    operands = g["CPW"] * (g["NBLK"] + params.r // 2 + 1) + g["TPW"] * kb
+    kept = params.r * (g["NB4"] + g["TPW"] + g["KB"] + g["CPW"]) + 1
+    operands = g["CPW"] * g["NB4"] + g["TPW"] * g["KB"]
     loads = g["LPTX"] + g["LPTD"]
-    stores = divup(config.block_n * g["BQ"] * config.groups, g["THREADS"])
-    needed = 4.92 * kept + 5.76 * operands + 4.0 * config.prefetch * loads + 4.85 * (loads + stores) + 26.5
-    return needed <= 1.25 * lane_registers(config.groups * config.split)
+    needed = 3.6 * kept + 13.9 * operands + 5.2 * config.prefetch * loads + 21
+    return needed <= 1.1 * lane_registers(config.groups * config.split)
 
 
 def _recorded_config_is_legal(params, config) -> bool:
@@ -245,7 +248,7 @@ def _get_configs(params: Conv2dGw8Params, device_attr=None) -> List[Conv2dGw8Bgr
     wpi = dw + params.s - 1
 
     def chunk_fill(nb):
-        return nb * dw / (32.0 * divup((nb - 1) * wpi + dw, 32))
+        return nb * dw / (32.0 * divup((nb - 1) * wpi + dw + 1, 32))
 
     image_counts = [1, 2, 4, 8]
     if wpi < 32:

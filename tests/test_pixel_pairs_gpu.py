@@ -1,0 +1,45 @@
+"""GPU parity of the kernels whose products take pairs of neighbouring pixels, where tiles and chunks of 32 pixels
+end: rows of 31 to 33 and of 64 pixels, every filter width, step loops in chunks, row blocks that do not divide the
+image.  Oracle and tolerances are those of the other kernel tests."""
+
+import pytest
+from helpers import run_bgrad_kernel_test
+
+from spio_amd.kernels import Conv2dGw8BgradConfig, Conv2dGw8Params, conv2d_gw8_bgrad_kernel_factory
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [
+    # (n, c, h, w, r, s, padding, bias)
+    (3, 24, 9, 31, 3, 3, 1, True),
+    (3, 16, 7, 32, 3, 3, 1, True),  # a chunk, which begins a pixel early, more than a tile
+    (2, 16, 6, 33, 5, 5, 2, False),
+    (2, 24, 5, 64, 3, 3, 1, True),
+    (5, 16, 11, 9, 5, 5, 2, True),  # three images and their shared halo fill a tile
+    (4, 40, 6, 14, 5, 4, (2, 1), False),
+    (3, 8, 5, 13, 1, 1, 0, True),
+    (3, 16, 8, 15, 2, 2, 1, True),
+    (2, 16, 9, 10, 3, 1, (0, 0), False),
+    (2, 16, 70, 6, 3, 3, 1, True),  # step loops in chunks
+    (2, 16, 67, 6, 5, 3, (2, 1), True),
+]
+
+
+def _params(shape):
+    n, c, h, w, r, s, padding, bias = shape
+    return Conv2dGw8Params(n=n, c=c, h=h, w=w, r=r, s=s, padding=padding, has_bias=bias)
+
+
+@pytest.mark.parametrize("shape", SHAPES, ids=str)
+def test_fused_backward(shape):
+    params = _params(shape)
+    groups, h, images = min(params.groups, 4), params.h, min(params.n, 3)
+    B = Conv2dGw8BgradConfig
+    configs = [
+        B(groups=groups, block_n=1, block_n_iters=params.n, prefetch=2),
+        B(groups=groups, block_n=images if params.w < 32 else 1, block_h=4, prefetch=4),
+        B(groups=groups, block_h=h if h < 40 else 13, block_n=2 if params.r < 5 else 1, prefetch=2, two_stage=1),
+    ]
+    if params.w > 32:
+        configs.append(B(groups=groups, block_h=5, prefetch=2, split=2))
+    run_bgrad_kernel_test(conv2d_gw8_bgrad_kernel_factory, params, configs=configs)
