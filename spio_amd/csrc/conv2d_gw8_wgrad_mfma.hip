@@ -17,20 +17,26 @@
 //     "8 channels of one pixel"; the transposing LDS read of gfx950
 //     (ds_read_b64_tr_b16) delivers exactly that from the pixel-major rows.
 //   * v_mfma_f32_16x16x32_f16 per 32-pixel chunk:
-//         A (16 x 32) = dy:  rows m = 8*j + k    (two dy rows j of an aligned row pair, 8 k)
-//         B (32 x 16) = x:   cols n = 8*sj + c   (two column taps sj, 8 c)
-//     so one MFMA yields dw for 2 filter rows x 2 filter columns.  For x row t
-//     and the dy row pair (2i, 2i+1) the filter rows are r = delta - j with
-//     delta = t - 2i in [0, R]; there is one accumulator per (delta, column-tap
-//     pair).  Entries with r or s out of range are never read.
-//   * At the end dw[k,r,s,c] = acc[delta=r] (lanes with j=0) + acc[delta=r+1]
-//     (lanes with j=1); the halves are combined through LDS.  Two ways to
+//         A (16 x 32) = dy:  rows m = 8*j + k    (the chunk, j pixels on; 8 k)
+//         B (32 x 16) = x:   cols n = 8*sj + c   (the chunk under two column taps, 2 sj; 8 c)
+//     so one MFMA yields dw for one filter row and the four filter columns 4 nb + 2 sj + 1 - j.  Both
+//     operands begin one pixel before the row: over all chunks each of the two copies of dy counts every
+//     pixel once.  x row t meets dy row t - r under filter row r: R * ceil(S/4) MFMAs per chunk and x row,
+//     as many accumulators, and nothing to combine between lanes.
+//   * A dy row is read from LDS once, when it is the newest, and its fragments stay in registers for the R
+//     x rows that meet it.
+//   * With two dy rows side by side in A, as before, there were (R+1) * ceil(S/2) accumulators (32 of a 7x7
+//     filter, now 14), 4, 9, 16 MFMAs per chunk and x row for 3x3, 5x5, 7x7 (now 3, 10, 14), R/2 + 1 reads
+//     of dy a step, and an exchange of halves through LDS at the end.  Before -> after, best of 24
+//     configurations: 128n 64c 56x56 21.0 -> 20.3 us (103 MB, 5.1 TB/s), 32n 10.0 -> 9.0, 32n 48c 224x224 55.4 -> 51.4, 256n 256c
+//     14x14 7x7 24.7 -> 21.0, 54n 688c 18x18 5x5 24.9 -> 20.9, 7n 392c 68x64 7x7 33.9 -> 25.5, 2n 56c 102x102 7x7 23.2 -> 11.4.
+//   * At the end the sums are staged in LDS in grad_weight order. Two ways to
 //     publish: SPIO_PARTIALS=0 adds into grad_weight with fp32 atomics.  Atomics
 //     of different workgroups to the same 128-byte line retire one after the
 //     other, so the sums are first staged in LDS in grad_weight order and then
 //     added with instructions that cover 64 consecutive floats (two full
 //     lines): the fewest line operations possible.  SPIO_PARTIALS=1 stores each
-//     workgroup's sums into its own partial image of a workspace with plain
+//     workgroup's sums into its own part of a partial image of a workspace with plain
 //     stores, and the small <name>_reduce kernel below stores the sum of the
 //     partial images into grad_weight (which then needs no zero fill).  (Reducing inside the kernel by "the last workgroup of
 //     a group to finish" was measured and rejected: the device-scope
@@ -46,7 +52,7 @@
 //     77n 168c 20x20 7x7 32.5 -> 22.1, 300n 88c 17x17 5x5 30.1 -> 20.4, 184n 288c 31x31 3x3 45.0 -> 39.7.
 //   * With SPIO_HAS_BIAS the kernel takes a fourth pointer, grad_bias ([K]
 //     fp32, accumulated into like grad_weight; null = not wanted), and sums dy
-//     per channel in the same pass: one more MFMA per chunk and row pair with
+//     per channel in the same pass: one more MFMA per chunk and row with
 //     an all-ones B operand (the reference runs a separate reduction,
 //     spio/functional/conv2d_gw8_function.py:134-136).
 #include "spio_conv_common.h"
@@ -96,9 +102,7 @@ constexpr int THREADS = 64 * WAVES;
 constexpr int PF = SPIO_PF;  // prefetch distance in steps (even)
 constexpr int RB = SPIO_RB;  // x rows (and dy rows) per step: 1 or 2
 
-constexpr int S2 = 2 * ((kS + 1) / 2);
-constexpr int NBLK = S2 / 2;   // column-tap pairs
-constexpr int ND = kR + 1;     // values of delta
+constexpr int NB4 = (kS + 3) / 4;  // column taps 4 nb .. 4 nb + 3 share one MFMA
 // Column blocks (SPIO_BQ > 0): a workgroup sums over BQ columns of dy and the BQ + S - 1 columns
 // of x opposite them, so rows of any width fit the rings (the reference tiles the width with a
 // fixed block of 8 columns, spio/kernels/conv2d_gw8_wgrad_kernel.py:40).  0 = the whole width.
@@ -119,29 +123,26 @@ constexpr int F = NB * WPI;
 #endif
 constexpr int GAP = kPadX > kS - 1 - kPadX ? kPadX : kS - 1 - kPadX;
 constexpr int IP = (SPIO_BQ > 0 || !SPIO_SHARED_HALO) ? WPI : BQ + GAP;  // pitch of the images in a run
-constexpr int IPC_MAX = (32 + IP - BQ) / IP;                             // whole images per 32-pixel chunk
-constexpr int KC_FLAT = ((NB - 1) * IP + BQ + 31) / 32;
+// A chunk begins one pixel before its first image: 31 of its pixels are the images'.
+constexpr int IPC_MAX = (31 + IP - BQ) / IP;                             // whole images per 32-pixel chunk
+constexpr int KC_FLAT = ((NB - 1) * IP + BQ + 1 + 31) / 32;
 constexpr int KC_PACKED = IPC_MAX > 0 ? (NB + IPC_MAX - 1) / IPC_MAX : KC_FLAT;
 constexpr bool kPacked = SPIO_SHARED_HALO && KC_PACKED < KC_FLAT;
 constexpr int IPC = kPacked ? IPC_MAX : NB;  // images per run: a chunk, or the whole row
 constexpr int KC = kPacked ? KC_PACKED : KC_FLAT;  // 32-pixel chunks
-constexpr int XCP = kPacked ? 16 * ((32 + S2 - 1 + 15) / 16) : 32;  // x cells from chunk to chunk
-constexpr int FPX = kPacked ? KC * XCP : 32 * KC + S2 - 1;         // x pixels the reads can touch
+constexpr int CPW = (KC + TS - 1) / TS;            // 32-pixel chunks per wave (past the last one: zeros)
+constexpr int XCP = kPacked ? 16 * ((32 + 4 * NB4 - 2 + 15) / 16) : 32;  // x cells from chunk to chunk
+constexpr int FPX = kPacked ? CPW * TS * XCP : 32 * CPW * TS + 4 * NB4 - 2;  // x pixels the reads can touch
 constexpr int GSX = FPX + ((9 - FPX % 16) + 16) % 16;  // x group stride (pixels), = 9 mod 16
-constexpr int FPD = 32 * KC;
+constexpr int FPD = 32 * CPW * TS + 1;                 // dy pixels, the first one a zero
 constexpr int GSD = FPD + ((9 - FPD % 16) + 16) % 16;  // dy group stride
 constexpr int d_image_offset(int img) { return (img / IPC) * 32 + (img % IPC) * IP; }
 constexpr int x_image_offset(int img) { return (img / IPC) * XCP + (img % IPC) * IP; }
-constexpr int NRX = 2 * RB;                             // x ring rows: the step's rows and the next step's
-// dy ring rows: the aligned row pairs a step multiplies (R+1 rows with one row per step, up to
-// R+2 with two) plus the rows the step writes for the next one; even.  The bias sum reads the
-// whole pair (t-1, t) in the step that stages row t+1, so it needs four rows even with a one-row
-// filter, whose weight gradient alone gets by with two.
-constexpr int NRD = ((SPIO_HAS_BIAS && kR == 1) ? 4 : 2 * ((kR + 2) / 2)) + (RB == 2 ? 2 : 0);
-constexpr int XROW_UNITS = GB * GSX;
-// dy ring rows are 64 bytes apart modulo the 256-byte bank period, so the two rows of a
-// pair that one transposing read touches fall into different banks.
-constexpr int DROW_UNITS = GB * GSD + ((4 - (GB * GSD) % 16) + 16) % 16;
+// ring rows carry spare units behind the last group, which lanes without a cell write to, each its own
+constexpr int DUMPS = 16;
+constexpr int XROW_UNITS = GB * GSX + DUMPS;
+constexpr int DROW_UNITS = GB * GSD + DUMPS;
+constexpr int XDUMP = GB * GSX, DDUMP = GB * GSD;
 constexpr int X_CELLS = F * GB;
 constexpr int LPTX = (X_CELLS + THREADS - 1) / THREADS;
 constexpr int D_CELLS = NB * BQ * GB;
@@ -151,55 +152,47 @@ constexpr int PBLKS = (kP + BH - 1) / BH;
 constexpr int NBLKS = (kN + NB * ITERS - 1) / (NB * ITERS);
 constexpr int NUM_BLOCKS = GBLKS * PBLKS * QBLKS * NBLKS;
 constexpr bool kDbias = SPIO_HAS_BIAS != 0;  // also sum grad_output per channel (grad_bias)
-// x rows a workgroup streams.  The bias sum takes a grad_output row pair one step after its
-// first row was staged, so a one-row filter needs one more step when the sum is wanted.
-constexpr int ROWS = BH + (kDbias && kR == 1 ? 2 : kR) - 1;
+constexpr int ROWS = BH + kR - 1;  // x rows a workgroup streams
 constexpr int STEPS = (ROWS + RB - 1) / RB;  // barrier-separated steps of RB rows
 // A workgroup that owns whole images (one row block) knows at compile time which of its x rows
 // lie in the padding: the steps before the first real row would only stage dy rows, the steps
 // after the last one nothing at all.  It starts at the first step with a real x row, with the dy
-// rows up to that step staged in the prologue, and stops after the last.  (Not with the bias
-// sum, which takes its row pairs at fixed steps.)
-constexpr bool kSkipPadding = PBLKS == 1 && !kDbias && (ROWS + RB - 1) / RB <= SPIO_MAX_UNROLL;
+// rows up to that step staged in the prologue, and stops after the last.  (A padding of R or more has dy rows
+// that meet no x row at all; the bias sum wants them.)
+constexpr bool kSkipPadding = PBLKS == 1 && kPadY < kR && (ROWS + RB - 1) / RB <= SPIO_MAX_UNROLL;
 constexpr int T_FIRST = kSkipPadding ? kPadY : 0;
 constexpr int T_END = kSkipPadding && kH + kPadY < ROWS ? kH + kPadY : ROWS;
 constexpr int S0 = T_FIRST / RB;               // first step
 constexpr int S1 = (T_END + RB - 1) / RB;      // one past the last step
 constexpr int LEAD = S0 * RB;                  // dy rows staged ahead of the first step's own
-// A workgroup that owns whole images unrolls its step loop completely, up to SPIO_MAX_UNROLL
-// steps (every condition on the step is then known at compile time); other loops run in chunks
-// of PF steps.
-constexpr bool kFullUnroll = PBLKS == 1 && S1 - S0 <= SPIO_MAX_UNROLL;
-constexpr int SLOTS = (S1 - S0 + PF - 1) / PF * PF;  // steps of an image block, rounded up to whole rounds of the register buffers
-constexpr int UNROLL = kFullUnroll ? SLOTS : PF;
-constexpr int NPAIR = kR / 2 + 1;            // aligned dy row pairs one step can touch
-constexpr int CPW = (KC + TS - 1) / TS;      // 32-pixel chunks per wave
+// The step loop is unrolled completely up to SPIO_MAX_UNROLL steps (which rows a step multiplies is then known at
+// compile time, and products that do not exist are left out); longer loops run in chunks that are whole rounds of
+// the row buffers and of the dy fragments.
+constexpr bool kFullUnroll = S1 - S0 <= SPIO_MAX_UNROLL;
+constexpr int gcd_(int a, int b) { return b == 0 ? a : gcd_(b, a % b); }
+constexpr int lcm_(int a, int b) { return a / gcd_(a, b) * b; }
+constexpr int NA = kR + RB - 1 + (SPIO_PIPE ? RB : 0);  // dy rows whose fragments are kept
+constexpr int ROUND = kFullUnroll ? PF : lcm_(PF, NA / gcd_(NA, RB));
+constexpr int SLOTS = (S1 - S0 + ROUND - 1) / ROUND * ROUND;  // steps of an image block, rounded up to whole rounds
+constexpr int UNROLL = kFullUnroll ? SLOTS : ROUND;
+// x ring rows: the step's rows and the next step's; dy ring rows: those, and the ones staged ahead of the first
+// step (a dy row is read once, when it is the newest, and its fragments stay in registers while x rows meet it)
+constexpr int NRX = 2 * RB;
+constexpr int NRD = LEAD + 2 * RB;
 
 // LDS: the two rings while streaming; at the end the same block holds the reduction scratch:
-// per wave NBLK*128 floats for the row-slot halves, the sums of the other waves of a split
-// group, (atomic publishing) every group's R*S*64 sums in grad_weight order, and eight
-// grad_bias sums per wave.
+// every group's R*S*64 sums in grad_weight order and eight grad_bias sums per wave.
 constexpr int RING_UNITS = NRX * XROW_UNITS + NRD * DROW_UNITS;
-// Filter rows whose row-slot halves are exchanged through the per-wave scratch in one go: all of
-// them where that fits 96 KB of LDS for the workgroup (every exchange costs an LDS round trip
-// and the waves do nothing else meanwhile), else one; one when waves share a group, whose sums
-// are then added row by row.
-constexpr int RCH = (TS == 1 && WAVES * kR * NBLK * 512 <= 96 * 1024) ? kR : 1;
-constexpr int SCRATCH_FLOATS = RCH * NBLK * 128;  // per wave
-constexpr int RED_FLOATS = GB * (TS - 1) * NBLK * 128;
 constexpr int GROUP_FLOATS = kR * kS * 64;  // grad_weight values of one group
-constexpr int PUBLISH_FLOATS = WAVES * SCRATCH_FLOATS + RED_FLOATS + (SPIO_PARTIALS ? 0 : GB * GROUP_FLOATS) +
-                               (SPIO_HAS_BIAS ? WAVES * 8 : 0);
+constexpr int PUBLISH_FLOATS = GB * GROUP_FLOATS + (SPIO_HAS_BIAS ? WAVES * 8 : 0);
 constexpr int LDS_UNITS = RING_UNITS > (PUBLISH_FLOATS + 3) / 4 ? RING_UNITS : (PUBLISH_FLOATS + 3) / 4;
 static_assert(LDS_UNITS * 16 <= 160 * 1024, "LDS overflow");
-static_assert(NRD % 2 == 0 && NRD >= kR + 1, "dy ring too small");
 static_assert(PF >= 2 && PF % 2 == 0, "prefetch distance must be even");
 static_assert(RB == 1 || RB == 2, "one or two rows per step");
-static_assert(LEAD + RB <= NRD, "the dy rows of the prologue fit the ring");
-constexpr int PART_WAVE_FLOATS = kR * NBLK * 4 * 32;  // floats one wave publishes (partial-block layout)
+// Two stages: the partial block of a workgroup is its groups' sums in grad_weight order.
 // Two stages with a bias: behind the partial blocks, every workgroup's bias sums, [block][channel], zeros
 // for channels past the last one.
-constexpr long long BIAS_PARTIALS = (long long)NBLKS * PBLKS * QBLKS * GBLKS * GB * PART_WAVE_FLOATS;
+constexpr long long BIAS_PARTIALS = (long long)NBLKS * PBLKS * QBLKS * GBLKS * GB * GROUP_FLOATS;
 
 
 constexpr long long X_ROW_BYTES = (long long)kW * kGroups * 16, X_IMAGE_BYTES = kH * X_ROW_BYTES;
@@ -209,7 +202,7 @@ constexpr long long D_ROW_BYTES = (long long)kQ * kGroups * 16, D_IMAGE_BYTES = 
 // 23.6 us, 28.6 with one of the block); in others it is 64-bit arithmetic for every
 // row (64n 64c 56x56 16.1 us, 14.2 with one of the block; 32n 48c 224x224 66.0 and 55.7).  It is also the one for
 // images that side by side exceed 32-bit offsets.
-constexpr bool kRowDescriptors = kFullUnroll || NB * X_IMAGE_BYTES >= (1ll << 31) || NB * D_IMAGE_BYTES >= (1ll << 31);
+constexpr bool kRowDescriptors = (kFullUnroll && PBLKS == 1) || NB * X_IMAGE_BYTES >= (1ll << 31) || NB * D_IMAGE_BYTES >= (1ll << 31);
 // What a row adds to the offsets of its lanes.  Rows above the image and behind it (padding, slots without a step)
 // have one too, which may wrap around; their loads go through an empty descriptor, which no offset is inside of.
 // (It is not the scalar offset, which the range check may leave out, and it is not clamped to rows that exist.  A
@@ -224,7 +217,7 @@ static_assert((NB - 1) * X_IMAGE_BYTES + X_ROW_BYTES < (1ll << 31) && (NB - 1) *
 // 18.4, 300n 88c 17x17 5x5 22.3 -> 20.4, 256n 256c 14x14 7x7 eight images 30.9 -> 27.6.  With one image it is the
 // other way round (128n 64c 56x56 21.8 and 22.2, 256n 39.0 and 41.1), as in loops that are not unrolled (32n 64c
 // 56x56 two images 10.7 and 11.0).
-constexpr bool kPlainLoads = kFullUnroll && ITERS == 1 && NB > 1;
+constexpr bool kPlainLoads = kFullUnroll && PBLKS == 1 && ITERS == 1 && NB > 1;
 constexpr int OUT_OF_RANGE = (int)0x80000000u;  // as an unsigned offset behind the end of every descriptor
 constexpr bool kSplitLines = splits_lines(GB, GBLKS);
 // Non-temporal, but for lines that channel blocks straddle (blocks that are halves of whole lines: 64n 64c
@@ -269,8 +262,8 @@ SPIO_KERNEL_NAME(float* __restrict__ grad_weight, const spio_uint4* __restrict__
     // the wave index as a scalar: conditions on it become scalar branches, so that no MFMA
     // (which ignores the lane mask) is ever issued under an empty mask
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wg = wave % GB;  // group within the workgroup
-    const int ws = wave / GB;  // which share of the 32-pixel chunks this wave multiplies
+    const int wg = TS == 1 ? wave : wave % GB;  // group within the workgroup
+    const int ws = TS == 1 ? 0 : wave / GB;  // which share of the 32-pixel chunks this wave multiplies
 
     // One contiguous range of tiles per XCD; column blocks fastest (neighbours share S - 1 columns of x),
     // then row blocks.  Where channel blocks share lines they go fastest, so that the lines are fetched
@@ -290,22 +283,22 @@ SPIO_KERNEL_NAME(float* __restrict__ grad_weight, const spio_uint4* __restrict__
 
     // lane roles inside the transposing reads: block kb = lane/16 covers pixels 8*kb..8*kb+7,
     // source lane sigma = lane%16 = 4*jr + t supplies pixel jr (+4 for the second read) of
-    // unit t/2 (dy row j or column tap sj) and channel half t%2.
+    // unit t/2 (dy: shift j, x: tap offset 2 sj) and channel half t%2.
     const int kb = lane >> 4;
     const int jr = (lane & 15) >> 2;
     const int tt = lane & 3;
-    const int sel = tt >> 1;  // j for A, sj for B
-    const int xfrag_off = ((wg * GSX + 8 * kb + jr + sel) * 16) + (tt & 1) * 8;   // bytes in an x row
-    const int dfrag_off = ((wg * GSD + 8 * kb + jr) * 16) + (tt & 1) * 8;         // bytes in a dy row
+    const int sel = tt >> 1;
+    const int xfrag_off = ((wg * GSX + 8 * kb + jr + 2 * sel) * 16) + (tt & 1) * 8;  // bytes in an x row
+    const int dfrag_off = ((wg * GSD + 8 * kb + jr + sel) * 16) + (tt & 1) * 8;      // bytes in a dy row
 
-    spio_float4 acc[ND][NBLK];
+    spio_float4 acc[kR][NB4];
 #pragma unroll
-    for (int d = 0; d < ND; ++d)
+    for (int r = 0; r < kR; ++r)
 #pragma unroll
-        for (int nb = 0; nb < NBLK; ++nb) acc[d][nb] = spio_float4{0.f, 0.f, 0.f, 0.f};
+        for (int nb = 0; nb < NB4; ++nb) acc[r][nb] = spio_float4{0.f, 0.f, 0.f, 0.f};
 
-    // grad_bias rides along as one more MFMA per chunk and row pair: dy (A) times an all-ones B
-    // gives, in every column, the sum of the 32 pixels for the 16 (row slot, channel) rows.
+    // grad_bias rides along as one more MFMA per dy row and chunk: dy (A) times an all-ones B
+    // gives, in every column, the sum of the 32 pixels for the 16 (shift, channel) rows.
     spio_float4 accb = spio_float4{0.f, 0.f, 0.f, 0.f};
     const spio_half8 ones8 = spio_half8{1, 1, 1, 1, 1, 1, 1, 1};
     (void)ones8;
@@ -314,18 +307,16 @@ SPIO_KERNEL_NAME(float* __restrict__ grad_weight, const spio_uint4* __restrict__
     // outstanding loads exactly and a step waits only for the rows it needs (a load under a branch makes it
     // wait for all of them, which would serialise the prefetch).  The images are read
     // through a buffer descriptor that ends with the last image that exists; lanes without data (halo columns, missing groups) carry an offset no descriptor reaches,
-    // and a row that nobody needs has an empty one: such loads give zeros and touch no memory.  (Threads
-    // beyond the last cell skip their LDS writes; letting them write spare cells instead, to make the
-    // writes branch-free, costs 14 % at N=256, C=256, 14x14, 7x7.)
+    // and a row that nobody needs has an empty one: such loads give zeros and touch no memory.
     const int nfirst = nbk * ITERS * NB;  // the workgroup's first image
-    // (Plain loads: lanes without data load the first pixel of a row and leave their cells as they were zeroed.)
+    // (Plain loads: lanes without data load the first pixel of a row and write it to a spare unit.)
     constexpr int NO_DATA = kPlainLoads ? 0 : OUT_OF_RANGE;
     int x_off[LPTX], x_lds[LPTX];
 #pragma unroll
     for (int l = 0; l < LPTX; ++l) {
         const int cell = tid + THREADS * l;
         x_off[l] = NO_DATA;
-        x_lds[l] = -1;
+        x_lds[l] = XDUMP + tid % DUMPS;
         if (cell < X_CELLS) {
             const int g = cell % GB;
             const int f = cell / GB;
@@ -335,7 +326,7 @@ SPIO_KERNEL_NAME(float* __restrict__ grad_weight, const spio_uint4* __restrict__
             if (col >= 0 && col < kW && cb * GB + g < kGroups && (!kPlainLoads || nfirst + img < kN))
                 x_off[l] = (int)(img * X_IMAGE_BYTES) + (col * kGroups + cb * GB + g) * 16;
             else if (kPlainLoads)
-                x_lds[l] = -1;
+                x_lds[l] = XDUMP + tid % DUMPS;
         }
     }
     int d_off[LPTD], d_lds[LPTD];
@@ -343,16 +334,16 @@ SPIO_KERNEL_NAME(float* __restrict__ grad_weight, const spio_uint4* __restrict__
     for (int l = 0; l < LPTD; ++l) {
         const int cell = tid + THREADS * l;
         d_off[l] = NO_DATA;
-        d_lds[l] = -1;
+        d_lds[l] = DDUMP + tid % DUMPS;
         if (cell < D_CELLS) {
             const int g = cell % GB;
             const int q = (cell / GB) % BQ;
             const int img = cell / (GB * BQ);
-            d_lds[l] = g * GSD + d_image_offset(img) + q;
+            d_lds[l] = g * GSD + 1 + d_image_offset(img) + q;
             if (q0 + q < kQ && cb * GB + g < kGroups && (!kPlainLoads || nfirst + img < kN))
                 d_off[l] = (int)(img * D_IMAGE_BYTES) + ((q0 + q) * kGroups + cb * GB + g) * 16;
             else if (kPlainLoads)
-                d_lds[l] = -1;
+                d_lds[l] = DDUMP + tid % DUMPS;
         }
     }
     const spio_uint4 zero4 = spio_uint4{0u, 0u, 0u, 0u};
@@ -444,93 +435,75 @@ SPIO_KERNEL_NAME(float* __restrict__ grad_weight, const spio_uint4* __restrict__
         for (int i = 0; i < LEAD; ++i) {
 #pragma unroll
             for (int l = 0; l < LPTD; ++l)
-                if (d_lds[l] >= 0) dring[(i % NRD) * DROW_UNITS + d_lds[l]] = dlead[i][l];
+                dring[(i % NRD) * DROW_UNITS + d_lds[l]] = dlead[i][l];
         }
 #pragma unroll
         for (int rr = 0; rr < RB; ++rr) {
             const int t = S0 * RB + rr;
 #pragma unroll
             for (int l = 0; l < LPTX; ++l)
-                if (x_lds[l] >= 0) xring[((S0 & 1) * RB + rr) * XROW_UNITS + x_lds[l]] = xpre[0][rr][l];
+                xring[((S0 & 1) * RB + rr) * XROW_UNITS + x_lds[l]] = xpre[0][rr][l];
 #pragma unroll
             for (int l = 0; l < LPTD; ++l)
-                if (d_lds[l] >= 0) dring[(t % NRD) * DROW_UNITS + d_lds[l]] = dpre[0][rr][l];
+                dring[(t % NRD) * DROW_UNITS + d_lds[l]] = dpre[0][rr][l];
         }
         block_sync();
 
-        // What step `st` (of parity `sp`) multiplies: x rows t+rr against the aligned dy row pairs
-        // they overlap (x row t+rr and the pair starting at row i2 meet at delta = t + rr - i2).
-        // The row pair starting at tbase is complete in LDS (its second row was staged during
-        // the previous step) when two rows go per step, and on odd steps otherwise; that is
-        // when it is added to the bias sum, once per pair.
-        struct StepPlan {
-            int tbase;
-            bool row_live[RB];
-            bool bias_pair;
-            bool do_math;
-        };
-        auto plan_step = [&](int st, int sp) {
-            StepPlan pl;
-            const int t = st * RB;  // first x row of the step, relative to the block
-            pl.tbase = RB == 2 ? t : t - sp;  // even
-            bool any_live = false;
+        // Fragments: of the x rows of a step (and, with SPIO_PIPE, of the step before), and of the last NA dy
+        // rows, row t in slot t modulo NA.  dy rows past the block are zeros, so are the ones before it.
+        constexpr int FSETS = SPIO_PIPE ? 2 : 1;
+        spio_half8 bfrag[FSETS][RB][CPW][NB4], afrag[NA][CPW];
 #pragma unroll
-            for (int rr = 0; rr < RB; ++rr) {
-                const int hcur = p0 + t + rr - kPadY;
-                pl.row_live[rr] = t + rr < ROWS && hcur >= 0 && hcur < kH;
-                any_live = any_live || pl.row_live[rr];
+        for (int a = 0; a < NA; ++a)
+#pragma unroll
+            for (int ci = 0; ci < CPW; ++ci) afrag[a][ci] = spio_half8{0, 0, 0, 0, 0, 0, 0, 0};
+        auto read_dy = [&](int t, int a, int ci) {
+            const unsigned char* pa0 = reinterpret_cast<const unsigned char*>(dring + t % NRD * DROW_UNITS) + dfrag_off +
+                                       (32 * (CPW * ws + ci)) * 16;
+            afrag[a][ci] = read_tr_pair(pa0, pa0 + 4 * 16);
+        };
+        auto sum_bias = [&](int a, int ci) {
+            if (kDbias) accb = __builtin_amdgcn_mfma_f32_16x16x32_f16(afrag[a][ci], ones8, accb, 0, 0, 0);
+        };
+        // x row t (row p0 + t - py) meets dy row t - r under filter row r
+        auto x_exists = [&](int t) {
+            return !kFullUnroll || (t < ROWS && (PBLKS > 1 || (t - kPadY >= 0 && t - kPadY < kH)));
+        };
+        // Share (rr, ci) of the fragment reads of step `st`, and of its products; `ta`: slot of dy row st * RB.
+        auto read_share = [&](int st, int sp, int ta, int rr, int ci, int fs) {
+            const int t = st * RB + rr;
+            if (x_exists(t)) {
+                const unsigned char* xrow =
+                    reinterpret_cast<const unsigned char*>(xring + (sp * RB + rr) * XROW_UNITS) + xfrag_off;
+#pragma unroll
+                for (int nb = 0; nb < NB4; ++nb) {
+                    const unsigned char* pb0 = xrow + (XCP * (CPW * ws + ci) + 4 * nb) * 16;
+                    bfrag[fs][rr][ci][nb] = read_tr_pair(pb0, pb0 + 4 * 16);
+                }
             }
-            pl.bias_pair = kDbias && (RB == 2 || sp == 1) && pl.tbase < bh_eff;
-            pl.do_math = wave_active && (any_live || pl.bias_pair);
-            return pl;
+            if (!kFullUnroll || t < BH) read_dy(t, (ta + rr) % NA, ci);
         };
-        // A step's work comes in CPW * NPAIR groups: group (ci, m) is the products of chunk ci with
-        // dy row pair m, and the share m of the chunk's fragment reads (the chunk's RB * NBLK x
-        // fragments and NPAIR dy fragments dealt round-robin over its groups).
-        constexpr int ITEMS = RB * NBLK + NPAIR;  // fragment reads (pairs of LDS reads) per chunk
-        auto read_group = [&](const StepPlan& pl, int sp, int ci, int mslot, spio_half8(&bf)[CPW][RB][NBLK],
-                              spio_half8(&af)[CPW][NPAIR]) {
-            const int ch = ws + TS * ci;
-            if (TS > 1 && ch >= KC) return;
+        auto multiply_share = [&](int st, int ta, int rr, int ci, int fs) {
+            const int t = st * RB + rr;
+            if (!kFullUnroll || t < BH) sum_bias((ta + rr) % NA, ci);
+            if (!x_exists(t)) return;
 #pragma unroll
-            for (int j = mslot; j < ITEMS; j += NPAIR) {
-                if (j < RB * NBLK) {
-                    const int rr = j / NBLK, nb = j % NBLK;
-                    const unsigned char* xrow =
-                        reinterpret_cast<const unsigned char*>(xring + (sp * RB + rr) * XROW_UNITS) + xfrag_off;
-                    const unsigned char* pb0 = xrow + (XCP * ch + 2 * nb) * 16;
-                    bf[ci][rr][nb] = read_tr_pair(pb0, pb0 + 4 * 16);
-                } else {
-                    const int m = j - RB * NBLK;
-                    const int i2 = pl.tbase - 2 * m;  // first row of the pair, relative to p0
-                    if (i2 >= 0 && i2 < bh_eff) {
-                        const int slot = (i2 + sel) % NRD;
-                        const unsigned char* pa0 =
-                            reinterpret_cast<const unsigned char*>(dring + slot * DROW_UNITS) + dfrag_off + (32 * ch) * 16;
-                        af[ci][m] = read_tr_pair(pa0, pa0 + 4 * 16);
-                    }
+            for (int nb = 0; nb < NB4; ++nb) {
+#pragma unroll
+                for (int r = 0; r < kR; ++r) {
+                    if (kFullUnroll && (t - r < 0 || t - r >= BH)) continue;
+                    acc[r][nb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(afrag[(ta + rr - r + 2 * NA) % NA][ci],
+                                                                        bfrag[fs][rr][ci][nb], acc[r][nb], 0, 0, 0);
                 }
             }
         };
-        auto multiply_group = [&](const StepPlan& pl, int sp, int ci, int m, const spio_half8(&bf)[CPW][RB][NBLK],
-                                  const spio_half8(&af)[CPW][NPAIR]) {
-            const int ch = ws + TS * ci;
-            if (TS > 1 && ch >= KC) return;
-            const int i2 = pl.tbase - 2 * m;
-            if (i2 >= 0 && i2 < bh_eff) {
 #pragma unroll
-                for (int rr = 0; rr < RB; ++rr) {
-                    const int d = (RB == 2 ? rr : sp) + 2 * m;  // = t + rr - i2
-                    if (d <= kR && pl.row_live[rr]) {
+        for (int i = 0; i < (LEAD < BH ? LEAD : BH); ++i)
 #pragma unroll
-                        for (int nb = 0; nb < NBLK; ++nb)
-                            acc[d][nb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[ci][m], bf[ci][rr][nb], acc[d][nb],
-                                                                                0, 0, 0);
-                    }
-                }
-                if (m == 0 && pl.bias_pair) accb = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[ci][0], ones8, accb, 0, 0, 0);
+            for (int ci = 0; ci < CPW; ++ci) {
+                read_dy(i, i % NA, ci);
+                sum_bias(i % NA, ci);
             }
-        };
         // 2. the slot PF ahead: its register buffer held this slot's rows, now in LDS
         auto prefetch_rows = [&](int slot, int uf) {
             const bool next = slot + PF >= SLOTS;
@@ -541,21 +514,14 @@ SPIO_KERNEL_NAME(float* __restrict__ grad_weight, const spio_uint4* __restrict__
             else if (!kFullUnroll || !next)
                 load_slot(0, slot + PF, uf % PF);
         };
-        // 3. the rows of step st+1 into LDS (dy rows past the block's last row are zeros).  The
-        //    ring rows written here are not read in this step, except for dy entries whose filter
-        //    row is out of range and whose product is ignored.
+        // 3. the rows of step st+1 into LDS (rows that do not exist are zeros), where nothing of this step reads
         auto stage_x = [&](int st, int sp, int uf) {
             if (st + 1 >= S1) return;
 #pragma unroll
             for (int rr = 0; rr < RB; ++rr) {
-                const int tn = (st + 1) * RB + rr;
-                const int hn = p0 + tn - kPadY;
-                if (tn < ROWS && hn >= 0 && hn < kH) {
 #pragma unroll
-                    for (int l = 0; l < LPTX; ++l)
-                        if (x_lds[l] >= 0)
-                            xring[(((sp + 1) & 1) * RB + rr) * XROW_UNITS + x_lds[l]] = xpre[(uf + 1) % PF][rr][l];
-                }
+                for (int l = 0; l < LPTX; ++l)
+                    xring[(((sp + 1) & 1) * RB + rr) * XROW_UNITS + x_lds[l]] = xpre[(uf + 1) % PF][rr][l];
             }
         };
         auto stage_dy = [&](int st, int uf) {
@@ -566,18 +532,15 @@ SPIO_KERNEL_NAME(float* __restrict__ grad_weight, const spio_uint4* __restrict__
                 const int dslot = tn % NRD;
 #pragma unroll
                 for (int l = 0; l < LPTD; ++l)
-                    if (d_lds[l] >= 0) dring[dslot * DROW_UNITS + d_lds[l]] = dpre[(uf + 1) % PF][rr][l];
+                    dring[dslot * DROW_UNITS + d_lds[l]] = dpre[(uf + 1) % PF][rr][l];
             }
         };
 
         // With SPIO_PIPE the products of a step are issued one step later, from a second set of
         // fragment registers, and the step's own LDS reads, row loads and ring writes are dealt
         // out between the groups of MFMAs: the matrix pipe takes 16 cycles per MFMA and the wave
-        // issues the other instructions in the slots that leaves.  (The compiler does not move
-        // the ring writes, which sit under lane masks, across the MFMAs by itself.)
-        constexpr int FSETS = SPIO_PIPE ? 2 : 1;
-        constexpr int GROUPS = CPW * NPAIR;
-        spio_half8 bfrag[FSETS][CPW][RB][NBLK], afrag[FSETS][CPW][NPAIR];
+        // issues the other instructions in the slots that leaves.
+        constexpr int SHARES = RB * CPW;
         for (int sb = 0; sb < SLOTS; sb += UNROLL) {
 #pragma unroll
             for (int uf = 0; uf < UNROLL; ++uf) {
@@ -593,32 +556,31 @@ SPIO_KERNEL_NAME(float* __restrict__ grad_weight, const spio_uint4* __restrict__
                 // PF is even, so the parity of the step is known at compile time: it fixes the
                 // x ring rows and, with one row per step, the parity of delta.
                 const int sp = (S0 + uf) & 1;
-                const StepPlan pl = plan_step(st, sp);
+                const int ta = (S0 + uf) * RB % NA;
+                const bool math = kFullUnroll || st < S1;
                 if (SPIO_PIPE) {
                     const int fs = uf & 1;
-                    const StepPlan before = plan_step(st - 1, sp ^ 1);
 #pragma unroll
-                    for (int g = 0; g < GROUPS; ++g) {
-                        const int ci = g / NPAIR, m = g % NPAIR;
-                        if (pl.do_math) read_group(pl, sp, ci, m, bfrag[fs], afrag[fs]);
+                    for (int g = 0; g < SHARES; ++g) {
+                        if (math) read_share(st, sp, ta, g / CPW, g % CPW, fs);
                         if (g == 0) prefetch_rows(slot, uf);
-                        if (g == (GROUPS > 1 ? 1 : 0)) stage_x(st, sp, uf);
-                        if (g == (GROUPS > 2 ? 2 : GROUPS - 1)) stage_dy(st, uf);
-                        if (st > S0 && st < S1 && before.do_math) multiply_group(before, sp ^ 1, ci, m, bfrag[fs ^ 1], afrag[fs ^ 1]);
+                        if (g == (SHARES > 1 ? 1 : 0)) stage_x(st, sp, uf);
+                        if (g == (SHARES > 2 ? 2 : SHARES - 1)) stage_dy(st, uf);
+                        if (st > S0 && math) multiply_share(st - 1, ta + NA - RB, g / CPW, g % CPW, fs ^ 1);
                         __builtin_amdgcn_sched_barrier(0);
                     }
                 } else {
                     // all LDS reads first, so that their latency overlaps the loads and ring writes
-                    if (pl.do_math) {
+                    if (math) {
 #pragma unroll
-                        for (int g = 0; g < GROUPS; ++g) read_group(pl, sp, g / NPAIR, g % NPAIR, bfrag[0], afrag[0]);
+                        for (int g = 0; g < SHARES; ++g) read_share(st, sp, ta, g / CPW, g % CPW, 0);
                     }
                     prefetch_rows(slot, uf);
                     stage_x(st, sp, uf);
                     stage_dy(st, uf);
-                    if (pl.do_math) {
+                    if (math) {
 #pragma unroll
-                        for (int g = 0; g < GROUPS; ++g) multiply_group(pl, sp, g / NPAIR, g % NPAIR, bfrag[0], afrag[0]);
+                        for (int g = 0; g < SHARES; ++g) multiply_share(st, ta, g / CPW, g % CPW, 0);
                     }
                 }
                 block_sync();
@@ -626,194 +588,70 @@ SPIO_KERNEL_NAME(float* __restrict__ grad_weight, const spio_uint4* __restrict__
         }
         if (SPIO_PIPE) {
             constexpr int LAST = S1 - 1;
-            const StepPlan pl = plan_step(LAST, LAST & 1);
-            if (pl.do_math) {
 #pragma unroll
-                for (int g = 0; g < GROUPS; ++g)
-                    multiply_group(pl, LAST & 1, g / NPAIR, g % NPAIR, bfrag[(LAST - S0) & 1], afrag[(LAST - S0) & 1]);
-            }
+            for (int g = 0; g < SHARES; ++g) multiply_share(LAST, LAST * RB % NA, g / CPW, g % CPW, (LAST - S0) & 1);
         }
     }
 
     // ---- publish ----
-    // dw[k,r,s,c] = acc[delta = r] (lanes 0-31: j = 0) + acc[delta = r+1] (lanes 32-63: j = 1).
-    // The j = 1 halves travel through a 512-byte per-wave LDS scratch (LDS operations of one
-    // wave execute in order, so no barrier is needed inside the wave).  With TS > 1 the waves of
-    // one group then add their sums through LDS so that only one wave per group publishes:
-    // fp32 atomics into grad_weight, or plain stores into this workgroup's partial image when a
-    // second kernel does the reduction.
-    block_sync();  // every wave is done with the rings; reuse them as scratch
+    // Sum m = 8 j + k, n = 8 sj + c of acc[r][nb] belongs to filter row r and column 4 nb + 2 sj + 1 - j.  The sums
+    // are staged in LDS in grad_weight order, where the waves of a group add theirs one after the other, and
+    // leave 64 consecutive floats at a time: fp32 atomics into grad_weight (two full 128-byte lines an
+    // instruction, which the memory system retires several times faster than the scattered half-lines of the
+    // accumulator layout), or plain stores into this workgroup's partial block when a second kernel does the
+    // reduction.
+    block_sync();  // every wave is done with the rings; reuse them
     {
-        float* scratch = reinterpret_cast<float*>(lds) + wave * SCRATCH_FLOATS;
-        float* red = reinterpret_cast<float*>(lds) + WAVES * SCRATCH_FLOATS;  // [group][ts-1][nb][e][32 lanes]
-        // this group's sums in grad_weight order [k][r][s][c] (atomic publishing only)
-        float* gstage = reinterpret_cast<float*>(lds) + WAVES * SCRATCH_FLOATS + RED_FLOATS + wg * GROUP_FLOATS;
-        (void)gstage;
+        float* const gstage = reinterpret_cast<float*>(lds) + wg * GROUP_FLOATS;
         const int k4 = 4 * ((lane >> 4) & 1);
-        const int sj = (lane & 15) >> 3;
         const int c = lane & 7;
+#pragma unroll
+        for (int w2 = 0; w2 < TS; ++w2) {
+            if (TS == 1 || ws == w2) {
+#pragma unroll
+                for (int nb = 0; nb < NB4; ++nb) {
+                    const int s = 4 * nb + 2 * ((lane & 15) >> 3) + 1 - (lane >> 5);
+                    if (s < kS) {
+#pragma unroll
+                        for (int r = 0; r < kR; ++r)
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) {
+                                float* const sum = gstage + (((k4 + e) * kR + r) * kS + s) * 8 + c;
+                                *sum = (w2 > 0 ? *sum : 0.f) + acc[r][nb][e];
+                            }
+                    }
+                }
+            }
+            if (TS > 1)
+                block_sync();
+            else
+                wave_sync();  // all lanes read what all lanes staged
+        }
 #if SPIO_PARTIALS
-        // this wave's slice of the workgroup's partial block: [r][tap pair][e][32 lanes], so that
-        // every store instruction writes 128 contiguous bytes
-        float* out = grad_weight + (((long long)((nbk * PBLKS + pb) * QBLKS + qb) * GBLKS + cb) * GB + wg) * PART_WAVE_FLOATS;
+        if (wave_active && ws == 0) {  // (nobody reads the blocks of groups past the last one)
+            spio_float4* const out = reinterpret_cast<spio_float4*>(grad_weight) +
+                (((long long)((nbk * PBLKS + pb) * QBLKS + qb) * GBLKS + cb) * GB + wg) * (GROUP_FLOATS / 4);
+            const spio_float4* const staged = reinterpret_cast<const spio_float4*>(gstage);
+#pragma unroll
+            for (int i = lane; i < GROUP_FLOATS / 4; i += 64) __builtin_nontemporal_store(staged[i], out + i);
+        }
 #else
-        float* out = grad_weight;
-#endif
-        if (RCH > 1) {
-            // All filter rows at once: lanes 32-63 leave their halves in the scratch as float4s,
-            // one wave-level sync, lanes 0-31 add them.  LDS operations of a wave execute in order,
-            // so the scratch can be rewritten right after it has been read.
-            spio_float4* half4 = reinterpret_cast<spio_float4*>(scratch);
-            if (lane >= 32) {
+        if (wave_active) {
+            float* const out = grad_weight + (long long)gglob * GROUP_FLOATS;
 #pragma unroll
-                for (int r = 0; r < kR; ++r)
-#pragma unroll
-                    for (int nb = 0; nb < NBLK; ++nb) half4[(r * NBLK + nb) * 32 + (lane - 32)] = acc[r + 1][nb];
-            }
-            wave_sync();  // lanes 32-63 stored, lanes 0-31 load
-            spio_float4 total[kR][NBLK];
-#pragma unroll
-            for (int r = 0; r < kR; ++r)
-#pragma unroll
-                for (int nb = 0; nb < NBLK; ++nb) {
-                    total[r][nb] = spio_float4{0.f, 0.f, 0.f, 0.f};
-                    if (lane < 32) total[r][nb] = acc[r][nb] + half4[(r * NBLK + nb) * 32 + lane];
-                }
-            wave_sync();  // the halves are read; the scratch becomes the staging area
-#if SPIO_PARTIALS
-            // through the scratch once more, in the partial block's order [r][tap pair][e][32
-            // lanes], so that all 64 lanes store 16 contiguous bytes each
-            if (wave_active) {
-                if (lane < 32) {
-#pragma unroll
-                    for (int r = 0; r < kR; ++r)
-#pragma unroll
-                        for (int nb = 0; nb < NBLK; ++nb)
-#pragma unroll
-                            for (int e = 0; e < 4; ++e) scratch[((r * NBLK + nb) * 4 + e) * 32 + lane] = total[r][nb][e];
-                }
-                wave_sync();  // lanes 0-31 staged, all lanes load
-                const spio_float4* stage4 = reinterpret_cast<const spio_float4*>(scratch);
-                spio_float4* out4 = reinterpret_cast<spio_float4*>(out);
-#pragma unroll
-                for (int i = lane; i < kR * NBLK * 32; i += 64) __builtin_nontemporal_store(stage4[i], out4 + i);
-            }
-#else
-            if (wave_active && lane < 32) {
-#pragma unroll
-                for (int r = 0; r < kR; ++r)
-#pragma unroll
-                    for (int nb = 0; nb < NBLK; ++nb) {
-                        const int s = 2 * nb + sj;
-                        if (s < kS) {
-#pragma unroll
-                            for (int e = 0; e < 4; ++e)
-                                gstage[(((k4 + e) * kR + r) * kS + s) * 8 + c] = total[r][nb][e];
-                        }
-                    }
-            }
-#endif
-        } else {
-#pragma unroll
-            for (int r = 0; r < kR; ++r) {
-                float total[NBLK][4];
-    #pragma unroll
-                for (int nb = 0; nb < NBLK; ++nb) {
-                    if (lane >= 32) {
-    #pragma unroll
-                        for (int e = 0; e < 4; ++e) scratch[e * 32 + (lane - 32)] = acc[r + 1][nb][e];
-                    }
-                    wave_sync();  // lanes 32-63 stored, lanes 0-31 load
-    #pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        total[nb][e] = 0.f;
-                        if (lane < 32) total[nb][e] = acc[r][nb][e] + scratch[e * 32 + lane];
-                    }
-                    wave_sync();  // the scratch is free for the next tap pair
-                }
-                if (TS > 1) {
-                    if (ws > 0 && lane < 32) {
-    #pragma unroll
-                        for (int nb = 0; nb < NBLK; ++nb)
-    #pragma unroll
-                            for (int e = 0; e < 4; ++e)
-                                red[(((wg * (TS - 1) + ws - 1) * NBLK + nb) * 4 + e) * 32 + lane] = total[nb][e];
-                    }
-                    block_sync();
-                    if (ws == 0 && lane < 32) {
-    #pragma unroll
-                        for (int w2 = 0; w2 < TS - 1; ++w2)
-    #pragma unroll
-                            for (int nb = 0; nb < NBLK; ++nb)
-    #pragma unroll
-                                for (int e = 0; e < 4; ++e)
-                                    total[nb][e] += red[(((wg * (TS - 1) + w2) * NBLK + nb) * 4 + e) * 32 + lane];
-                    }
-                }
-    #if SPIO_PARTIALS
-                // through the wave's LDS scratch once more so that all 64 lanes store 16 bytes each
-                if (wave_active && ws == 0) {
-                    float* stage = scratch;  // NBLK * 128 floats: [tap pair][e][32 lanes]
-                    if (lane < 32) {
-    #pragma unroll
-                        for (int nb = 0; nb < NBLK; ++nb)
-    #pragma unroll
-                            for (int e = 0; e < 4; ++e) stage[(nb * 4 + e) * 32 + lane] = total[nb][e];
-                    }
-                    wave_sync();  // lanes 0-31 staged, all lanes load
-                    const spio_float4* stage4 = reinterpret_cast<const spio_float4*>(stage);
-                    spio_float4* out4 = reinterpret_cast<spio_float4*>(out) + r * NBLK * 32;
-    #pragma unroll
-                    for (int i = lane; i < NBLK * 32; i += 64) __builtin_nontemporal_store(stage4[i], out4 + i);
-                    wave_sync();  // the scratch is free for the next filter row
-                }
-    #else
-                if (wave_active && ws == 0 && lane < 32) {
-    #pragma unroll
-                    for (int nb = 0; nb < NBLK; ++nb) {
-                        const int s = 2 * nb + sj;
-                        if (s < kS) {
-    #pragma unroll
-                            for (int e = 0; e < 4; ++e)
-                                gstage[(((k4 + e) * kR + r) * kS + s) * 8 + c] = total[nb][e];
-                        }
-                    }
-                }
-    #endif
-                if (TS > 1) block_sync();  // the scratch is rewritten for the next filter row
-            }
-}
-#if !SPIO_PARTIALS
-        // One wave per group adds the group's R*S*64 sums into grad_weight: every atomic
-        // instruction covers 64 consecutive floats (two full 128-byte lines), which the memory
-        // system retires several times faster than the scattered half-lines of the accumulator
-        // layout.  The wave reads back what it wrote itself, so a wave-level sync is enough.
-        if (wave_active && ws == 0) {
-            float* gout = out + (long long)gglob * GROUP_FLOATS;
-            wave_sync();  // lanes 0-31 staged the sums, all lanes read them
-#pragma unroll
-            for (int i = 0; i < kR * kS; ++i) atomic_add_f32(gout + 64 * i + lane, gstage[64 * i + lane]);
+            for (int i = ws; i < kR * kS; i += TS) atomic_add_f32(out + 64 * i + lane, gstage[64 * i + lane]);
         }
 #endif
 #if SPIO_HAS_BIAS
-        // grad_bias[8g + k] = accb of row slot 0 (lanes 0-31) + row slot 1 (lanes 32-63); every
-        // column holds the same sum, so lanes 0 and 16 carry channels 0-3 and 4-7.  All waves
-        // leave their eight sums in LDS and one wave adds the workgroup's GB*8 consecutive
+        // grad_bias[8g + k] = accb of shift 0 (every column holds the same sum): lanes 0 and 16 carry channels 0-3
+        // and 4-7.  All waves leave their eight sums in LDS and one wave adds the workgroup's GB*8 consecutive
         // values with a single atomic instruction: atomics of different workgroups to the same
         // 128-byte line retire one after the other, so their number per line is what counts.
         {
-            wave_sync();
-            if (lane >= 32) {
-#pragma unroll
-                for (int e = 0; e < 4; ++e) scratch[e * 32 + (lane - 32)] = accb[e];
-            }
-            wave_sync();
-            float* bslots = reinterpret_cast<float*>(lds) + WAVES * SCRATCH_FLOATS + RED_FLOATS +
-                            (SPIO_PARTIALS ? 0 : GB * GROUP_FLOATS);  // [wave][8]
+            float* bslots = reinterpret_cast<float*>(lds) + GB * GROUP_FLOATS;  // [wave][8]
             if ((lane & 47) == 0) {
 #pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    bslots[wave * 8 + k4 + e] = wave_active ? accb[e] + scratch[e * 32 + lane] : 0.f;
+                for (int e = 0; e < 4; ++e) bslots[wave * 8 + k4 + e] = accb[e];
             }
             block_sync();
             if (wave == 0) {
@@ -830,35 +668,32 @@ SPIO_KERNEL_NAME(float* __restrict__ grad_weight, const spio_uint4* __restrict__
         }
 #endif
     }
-
 }
 
 #if SPIO_PARTIALS
 // Second stage: grad_weight = sum over the partial blocks (stored whole: a caller that runs the
 // two-stage kernel need not zero grad_weight first).  A workgroup owns COLS float4 columns
-// of one channel block (COLS * 16 contiguous bytes of every partial block); its slices each add the blocks
+// (COLS * 16 contiguous bytes of every partial image, which is grad_weight with the missing groups behind it); its slices each add the blocks
 // p = slice, slice + SLICES, ... with UN loads in flight, the slices are added through LDS and slice 0
 // stores the total.  With 32 columns (512 bytes: half a wave per load instruction) where that gives
 // a workgroup per compute unit: with 8 columns, 3584 workgroups of 128-byte rows for a 7x7 filter on 256
 // channels, the stage took 5.9 us for 14.7 MB, with 32 5.1 us, of which about 2.2 us are what any
 // kernel costs in a stream.  With 8 where there are few columns: more workgroups, and more slices each.
 // Every element of grad_weight has exactly one
-// owner, so no atomics are needed and the sum does not depend on timing.  A column is four
-// consecutive lanes of the publishing wave, i.e. four consecutive channels c of one (k, r, s).
+// owner, so no atomics are needed and the sum does not depend on timing.
 template <class T>
 SPIO_DEVICE void reduce_partials(T* __restrict__ grad_weight, const spio_float4* __restrict__ partials) {
-    constexpr int BLOCK_F4 = GB * PART_WAVE_FLOATS / 4;  // float4 columns of one partial block
+    constexpr int IMAGE_F4 = GBLKS * GB * GROUP_FLOATS / 4;  // float4 columns of one partial image
     constexpr int NPART = NBLKS * PBLKS * QBLKS;
     constexpr int COLS = SPIO_REDUCE_COLS;
     constexpr int SLICES = 256 / COLS;
     constexpr int UN = NPART <= 4 * SLICES ? 4 : NPART <= 8 * SLICES ? 8 : 16;
-    static_assert(BLOCK_F4 % COLS == 0, "a workgroup's columns lie in one channel block");
     __shared__ spio_float4 red[SLICES][COLS];
     const int tid = thread_id();
     const int cl = tid % COLS;
     const int slice = tid / COLS;
-    const int col = (block_id() % (BLOCK_F4 / COLS)) * COLS + cl;
-    const int cb = block_id() / (BLOCK_F4 / COLS);
+    const int col = block_id() * COLS + cl;
+    const bool live = col < kGroups * GROUP_FLOATS / 4;
     spio_float4 sum = spio_float4{0.f, 0.f, 0.f, 0.f};
     for (int base = slice; base < NPART; base += SLICES * UN) {
         spio_float4 v[UN];
@@ -866,27 +701,17 @@ SPIO_DEVICE void reduce_partials(T* __restrict__ grad_weight, const spio_float4*
         for (int i = 0; i < UN; ++i) {
             const int p = base + i * SLICES;
             v[i] = spio_float4{0.f, 0.f, 0.f, 0.f};
-            if (p < NPART) v[i] = partials[((long long)p * GBLKS + cb) * BLOCK_F4 + col];
+            if (p < NPART && live) v[i] = partials[(long long)p * IMAGE_F4 + col];
         }
 #pragma unroll
         for (int i = 0; i < UN; ++i) sum += v[i];
     }
     red[slice][cl] = sum;
     block_sync();
-    if (slice == 0) {
+    if (slice == 0 && live) {
 #pragma unroll 4
         for (int i = 1; i < SLICES; ++i) sum += red[i][cl];
-        // float index inside the block -> (group, r, tap pair, e, lane)
-        const int f = 4 * col;
-        const int l32 = f & 31;
-        const int e = (f >> 5) & 3;
-        const int rn = (f >> 7) % (kR * NBLK);
-        const int g = (f >> 7) / (kR * NBLK);
-        const int r = rn / NBLK;
-        const int s = 2 * (rn % NBLK) + ((l32 & 15) >> 3);
-        const int k = 8 * (cb * GB + g) + 4 * (l32 >> 4) + e;
-        if (cb * GB + g < kGroups && s < kS)
-            store_sums(grad_weight + (((long long)k * kR + r) * kS + s) * 8 + (l32 & 7), sum);
+        store_sums(grad_weight + 4 * (long long)col, sum);
     }
 }
 extern "C" __global__ void SPIO_LAUNCH_BOUNDS(256)
@@ -935,7 +760,7 @@ SPIO_CONCAT(SPIO_KERNEL_NAME, _reduce_h)(spio_half* __restrict__ grad_weight, co
 #endif
 ) {
 #if SPIO_HAS_BIAS
-    constexpr int WEIGHT_BLOCKS = GBLKS * (GB * PART_WAVE_FLOATS / 4) / SPIO_REDUCE_COLS;
+    constexpr int WEIGHT_BLOCKS = (GBLKS * GB * GROUP_FLOATS / 4 + SPIO_REDUCE_COLS - 1) / SPIO_REDUCE_COLS;
     if (block_id() >= WEIGHT_BLOCKS) {
         reduce_bias(grad_bias, reinterpret_cast<const float*>(partials) + BIAS_PARTIALS, block_id() - WEIGHT_BLOCKS);
         return;

@@ -30,6 +30,7 @@ MAX_WAVES = 16
 MAX_LDS_BYTES = 128 * 1024
 MAX_LOADS_PER_THREAD = 8
 MAX_ACCUMULATORS = 32
+MAX_UNROLLED_STEPS = 64  # SPIO_MAX_UNROLL of the kernel: longer step loops run in chunks
 MAX_GEOMETRIES = 20  # that enter the sweep, with the pipelines about 100 candidates (20 s)
 PIPELINE_CHOICES = ((2, 1, 0), (4, 1, 0), (2, 2, 0), (2, 1, 1), (4, 1, 1))  # (prefetch, rows, pipe)
 LEADING_PIPELINES = 3  # of these, for the leading geometries at the head of the list
@@ -82,55 +83,57 @@ def image_placement(params: Conv2dGw8Params, nb: int, block_q: int = 0) -> Dict[
     Images follow one another GAP = max(px, S-1-px) zero cells apart (the right halo of one is
     the left halo of the next).  The contraction runs over 32-pixel chunks of the grad_output
     row; where a chunk holds whole images and that takes fewer chunks than the images laid end
-    to end, every chunk gets its own images (PACKED).
+    to end, every chunk gets its own images (PACKED).  A chunk begins one pixel before its first
+    image, so 31 of its pixels are the images'.
     """
     s, px = params.s, params.padding_w
-    s2 = 2 * ((s + 1) // 2)
+    nb4 = divup(s, 4)
     bq = block_q or params.q
     gap = max(px, s - 1 - px)
     ip = bq + s - 1 if block_q else bq + gap
-    ipc_max = (32 + ip - bq) // ip
-    kc_flat = divup((nb - 1) * ip + bq, 32)
+    ipc_max = (31 + ip - bq) // ip
+    kc_flat = divup((nb - 1) * ip + bq + 1, 32)
     kc_packed = divup(nb, ipc_max) if ipc_max > 0 else kc_flat
     packed = kc_packed < kc_flat
     kc = kc_packed if packed else kc_flat
-    xcp = 16 * divup(32 + s2 - 1, 16) if packed else 32
+    xcp = 16 * divup(32 + 4 * nb4 - 2, 16) if packed else 32
     return dict(IP=ip, IPC=ipc_max if packed else nb, KC=kc, PACKED=int(packed), XCP=xcp,
-                FPX=kc * xcp if packed else 32 * kc + s2 - 1)  # fmt: skip
+                FPX=kc * xcp if packed else 32 * kc + 4 * nb4 - 2)  # fmt: skip
 
 
 def wgrad_geometry(params: Conv2dGw8Params, config: Conv2dGw8WgradConfig) -> Dict[str, int]:
     """Host mirror of the compile-time constants of conv2d_gw8_wgrad_mfma.hip."""
     r, s = params.r, params.s
     gb, bh, nb, iters, ts = config.groups, config.block_h, config.block_n, config.block_n_iters, config.split
-    s2 = 2 * ((s + 1) // 2)
+    nb4 = divup(s, 4)
     bq = config.block_q or params.q
     wpi = bq + s - 1
     f = nb * wpi
     place = image_placement(params, nb, config.block_q)
-    kc, fpx = place["KC"], place["FPX"]
+    kc = place["KC"]
+    chunks = divup(kc, ts) * ts  # past the last one: zeros
+    fpx = place["FPX"] + (chunks - kc) * place["XCP"]
     gsx = fpx + ((9 - fpx % 16) + 16) % 16
-    fpd = 32 * kc
+    fpd = 32 * chunks + 1
     gsd = fpd + ((9 - fpd % 16) + 16) % 16
     rb = config.rows
-    nrx = 2 * rb
-    nrd = (4 if (params.has_bias and r == 1) else 2 * ((r + 2) // 2)) + (2 if rb == 2 else 0)
+    pblks = divup(params.p, bh)
+    rows = bh + r - 1
+    skip = pblks == 1 and params.padding_h < r and divup(rows, rb) <= MAX_UNROLLED_STEPS  # kSkipPadding of the kernel
+    lead = params.padding_h // rb * rb if skip else 0
     threads = 64 * gb * ts
-    lds_rings = (nrx * gb * gsx + nrd * (gb * gsd + ((4 - (gb * gsd) % 16) + 16) % 16)) * 16
-    # the same LDS block holds the reduction scratch at the end: per-wave row-slot halves, the
-    # sums of the other waves of a split group, and (atomic publishing) every group's R*S*64 sums
-    rch = r if (ts == 1 and gb * ts * r * (s2 // 2) * 512 <= 96 * 1024) else 1  # RCH of the kernel
-    lds_scratch = (gb * ts * rch * (s2 // 2) * 128 + gb * (ts - 1) * (s2 // 2) * 128
-                   + (0 if config.two_stage else gb * r * s * 64)
-                   + (gb * ts * 8 if params.has_bias else 0)) * 4  # fmt: skip
+    # rows carry 16 spare units behind the last group
+    lds_rings = (2 * rb * (gb * gsx + 16) + (lead + 2 * rb) * (gb * gsd + 16)) * 16
+    # the same LDS block holds every group's R*S*64 sums at the end
+    lds_scratch = (gb * r * s * 64 + (gb * ts * 8 if params.has_bias else 0)) * 4
     g = dict(
-        NBLK=s2 // 2, ND=r + 1, WPI=wpi, F=f, KC=kc, GSX=gsx, GSD=gsd, NRD=nrd, THREADS=threads,
+        NB4=nb4, WPI=wpi, F=f, KC=kc, CPW=chunks // ts, GSX=gsx, GSD=gsd, THREADS=threads,
         LDS_BYTES=max(lds_rings, lds_scratch), RING_BYTES=lds_rings, SCRATCH_BYTES=lds_scratch,
         LPTX=divup(f * gb, threads), LPTD=divup(nb * bq * gb, threads),
         BQ=bq, QBLKS=divup(params.q, bq),
-        GBLKS=divup(params.groups, gb), PBLKS=divup(params.p, bh),
+        GBLKS=divup(params.groups, gb), PBLKS=pblks,
         NBLKS=divup(params.n, nb * iters),
-        STEPS=divup(bh + (2 if params.has_bias and r == 1 else r) - 1, rb),
+        STEPS=divup(rows, rb),
         PIXEL_EFF=(nb * bq) / (32.0 * kc), IPC=place["IPC"], PACKED=place["PACKED"],
     )  # fmt: skip
     g["NUM_BLOCKS"] = g["GBLKS"] * g["PBLKS"] * g["QBLKS"] * g["NBLKS"]
@@ -146,7 +149,7 @@ def _mfma_config_is_legal(params, config) -> bool:
         and config.block_n <= max(params.n, 1) and config.block_n * (config.block_n_iters - 1) < max(params.n, 1)
         and g["LDS_BYTES"] <= MAX_LDS_BYTES
         and g["LPTX"] <= MAX_LOADS_PER_THREAD
-        and g["ND"] * g["NBLK"] <= MAX_ACCUMULATORS
+        and params.r * g["NB4"] <= MAX_ACCUMULATORS
         and config.prefetch >= 2
         and config.prefetch % 2 == 0
         and config.rows in (1, 2)
@@ -162,13 +165,15 @@ def _mfma_config_is_legal(params, config) -> bool:
 
 
 def _fits(params, config) -> bool:
-    """Whether a lane's registers hold the sums, the rows in flight and a step's operands (weights fitted to what the
-    compiler reports for 564 kernels: of 34 that used memory 6 pass, of 530 others 6 do not)."""
+    """Whether a lane's registers hold the sums, the last grad_output rows, the rows in flight and a step's operands
+    (weights fitted to what the compiler reports for 480 kernels of 80 shapes: of 9 that used memory 3 pass, all by
+    16 bytes or less but one, of 471 others 3 do not)."""
     g = wgrad_geometry(params, config)
     loads = g["LPTX"] + g["LPTD"]
-    operands = divup(g["KC"], config.split) * config.rows * (g["NBLK"] + params.r // 2 + 1) * (2 if config.pipe else 1)
-    needed = 5.2 * g["ND"] * g["NBLK"] + 2.84 * config.prefetch * config.rows * loads + 3.72 * operands + 12.9 * loads
-    return needed <= 1.05 * lane_registers(config.groups * config.split)
+    operands = g["CPW"] * config.rows * (g["NB4"] + 1) * (2 if config.pipe else 1)
+    needed = (4.1 * params.r * g["NB4"] + 3.6 * params.r * g["CPW"] + 2.0 * operands
+              + 2.9 * config.prefetch * config.rows * loads + 3.7 * loads + 23)  # fmt: skip
+    return needed <= 1.02 * lane_registers(config.groups * config.split)
 
 
 def _config_is_legal(params, config) -> bool:
@@ -247,7 +252,8 @@ def _get_configs(params: Conv2dGw8Params, device_attr=None) -> List[Conv2dGw8Wgr
     # Rank the tile geometries first and keep the best few; each of them is then tried with the
     # pipeline variants (prefetch distance, rows per step), which the score cannot tell apart.
     # column blocks for wide rows only: narrower ones fit whole
-    col_choices = [bq for bq in (64, 128, 256) if params.q >= 2 * bq and params.q > 128]
+    # (one less than whole chunks, which begin a pixel before the block)
+    col_choices = [bq for bq in (63, 127, 255) if params.q >= 2 * bq and params.q > 128]
     col_choices = [0] + sorted({*col_choices, *balanced(params.q, col_choices)})
     geometries = []
     for bq in col_choices:
@@ -307,10 +313,9 @@ def _get_kernel_spec(params: Conv2dGw8Params, config: Conv2dGw8WgradConfig, _dev
     spec = KernelSpec(defines, LaunchParams(grid=g["NUM_BLOCKS"], block=g["THREADS"]), MFMA_SOURCE, notes=g)
     if config.two_stage:
         num_partials = g["NBLKS"] * g["PBLKS"] * g["QBLKS"]
-        # float4 columns of the partial blocks of one (image block, row block): per wave
-        # [r][tap pair][4][32 lanes] floats
-        cols = g["GBLKS"] * config.groups * params.r * g["NBLK"] * 32
-        # columns per workgroup of the second stage (cols is a multiple of 32 per channel block)
+        # float4 columns of a partial image: grad_weight, and the groups missing in the last channel block
+        cols = g["GBLKS"] * config.groups * params.r * params.s * 16
+        # columns per workgroup of the second stage
         reduce_cols = 32 if cols >= 32 * 256 else 8
         defines.update(SPIO_PARTIALS=1, SPIO_REDUCE_COLS=reduce_cols)
         bias_floats = num_partials * g["GBLKS"] * config.groups * 8 if params.has_bias else 0
@@ -318,9 +323,9 @@ def _get_kernel_spec(params: Conv2dGw8Params, config: Conv2dGw8WgradConfig, _dev
         spec.epilogue_suffix = "_reduce"
         spec.epilogue_half_suffix = "_reduce_h"  # with a bias it takes grad_bias as well and stores it
         spec.overwrites_output = True  # the second stage stores grad_weight whole
-        spec.epilogue_launch_params = LaunchParams(grid=cols // reduce_cols, block=256)
+        spec.epilogue_launch_params = LaunchParams(grid=divup(cols, reduce_cols), block=256)
         bias_blocks = g["GBLKS"] if params.has_bias else 0
-        spec.epilogue_half_launch_params = LaunchParams(grid=cols // reduce_cols + bias_blocks, block=256)
+        spec.epilogue_half_launch_params = LaunchParams(grid=divup(cols, reduce_cols) + bias_blocks, block=256)
     return spec
 
 

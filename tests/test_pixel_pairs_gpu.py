@@ -3,9 +3,15 @@ end: rows of 31 to 33 and of 64 pixels, every filter width, step loops in chunks
 image.  Oracle and tolerances are those of the other kernel tests."""
 
 import pytest
-from helpers import run_bgrad_kernel_test
+from helpers import run_bgrad_kernel_test, run_grad_kernel_test
 
-from spio_amd.kernels import Conv2dGw8BgradConfig, Conv2dGw8Params, conv2d_gw8_bgrad_kernel_factory
+from spio_amd.kernels import (
+    Conv2dGw8BgradConfig,
+    Conv2dGw8Params,
+    Conv2dGw8WgradConfig,
+    conv2d_gw8_bgrad_kernel_factory,
+    conv2d_gw8_wgrad_kernel_factory,
+)
 
 pytestmark = pytest.mark.gpu
 
@@ -43,3 +49,20 @@ def test_fused_backward(shape):
     if params.w > 32:
         configs.append(B(groups=groups, block_h=5, prefetch=2, split=2))
     run_bgrad_kernel_test(conv2d_gw8_bgrad_kernel_factory, params, configs=configs)
+
+
+@pytest.mark.parametrize("shape", [*SHAPES, (2, 16, 8, 15, 7, 7, 3, True), (2, 8, 6, 7, 3, 3, 4, True)], ids=str)
+def test_weight_gradient(shape):
+    """Also a filter of 14 accumulators, and padding that leaves grad_output rows which meet no input row."""
+    params = _params(shape)
+    groups, images = min(params.groups, 4), min(params.n, 3)
+    W = Conv2dGw8WgradConfig
+    configs = [
+        W(groups=groups, block_h=params.p, block_n=images, prefetch=2),
+        W(groups=groups, block_h=params.p, block_n=1, block_n_iters=params.n, prefetch=2, rows=2, pipe=1, two_stage=1),
+        W(groups=groups, block_h=4, block_n=2, prefetch=4, pipe=1),
+        W(groups=groups, block_h=3, block_n=1, prefetch=2, rows=2, two_stage=1),
+    ]
+    if params.w > 32:
+        configs.append(W(groups=groups, block_h=params.p, block_n=1, prefetch=2, split=2))
+    run_grad_kernel_test(conv2d_gw8_wgrad_kernel_factory, params, configs=configs)
