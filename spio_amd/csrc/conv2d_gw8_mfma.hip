@@ -15,18 +15,19 @@
 //     pixels of the NB images laid side by side, each image padded to
 //     WPI = DW+S-1 columns so that the zero halo is materialised once and a
 //     tap is a plain pixel offset.
-//   * One wave owns one group.  Per 16-pixel tile and source row it issues
-//     one 16-byte LDS read per lane and ceil(R/2)*ceil(S/4) MFMAs
-//     v_mfma_f32_16x16x32_f16 with
-//         A (16 x 32) = filter:  rows m = 8*j + k   (two output-row slots j, 8 out channels k)
-//                               cols  = 8*kb + c   (four column taps kb, 8 in channels c)
-//         B (32 x 16) = source:  col n = pixel, rows = (tap kb, channel c)
-//     Lane (n, kb) of B is exactly the 16 bytes of pixel n+kb, so the fragment
-//     needs no shuffling.  The two row slots of A belong to two *different*
-//     output rows: a source row contributes to R output rows, which live in
-//     NS = 2*ceil(R/2) accumulator slots that rotate (slot = output row mod
-//     NS); the filter row used for a slot at a step follows from the phase,
-//     so accumulators never move between lanes.
+//   * One wave owns one group.  Per tile of 16 pairs of neighbouring pixels and
+//     source row it issues ceil((S+1)/4) 16-byte LDS reads per lane and R times
+//     as many MFMAs v_mfma_f32_16x16x32_f16 with
+//         A (16 x 32) = filter:  rows m = 8*j + k   (pixel j of a pair, 8 out channels k)
+//                               cols  = 8*kb + c   (column kb of four of a pair's S+1 source
+//                                                   columns, which meets tap kb - j; 8 in channels c)
+//         B (32 x 16) = source:  col n = pair, rows = (column kb, channel c)
+//     Lane (n, kb) of B is exactly the 16 bytes of pixel 2n+kb, so the fragment
+//     needs no shuffling; even and odd pixels of a staged row lie in two planes,
+//     so that its reads are free of bank conflicts.  A source row contributes to
+//     R output rows, which live in R accumulators that take turns (accumulator =
+//     output row mod R); products of rows that the tile does not own are left out
+//     at compile time.
 //   * A finished output row is converted to fp16, staged through LDS into
 //     pixel-major order and stored with one coalesced 16-byte store per lane.
 //   * One workgroup barrier per step; global loads run SPIO_PF rows ahead of
@@ -41,6 +42,15 @@
 //     is for that row only.  (A wait counter covers loads and stores alike; a
 //     count merged over paths that issue different numbers of them degrades
 //     to the smallest, i.e. to waiting for rows that are not needed yet.)
+//
+// What bounds it: 3x3 filters memory (128n 64c 56x56: 103 MB at 6.0 TB/s), larger ones the chain of a step (barrier,
+// LDS reads, products) on two to four waves a SIMD.  The rows of A were two output rows, two slots of accumulators
+// each; with two neighbouring pixels a 5x5 or 7x7 filter takes 5/6 and 7/8 of the products (3x3: 3/4), every filter
+// half of the fragment reads and conversions, and all lanes convert.  Before -> after, best of the first 16
+// configurations: 128n 64c 56x56 18.9 -> 17.1 us, 32n 48c 224x224 58.4 -> 55.6, 1n 64c 56x56 2.9 -> 2.7, 60n 200c 33x33
+// 20.3 -> 17.2, 300n 1000c 9x12 34.7 -> 31.1, 13n 280c 63x93 5x5 32.1 -> 27.1, 4n 424c 84x84 5x5 23.1 -> 17.8, 2n 600c
+// 147x147 7x7 55.7 -> 45.8; equal: 59n 456c 60x60 (lines shared by channel blocks), 128n 24c 144x144 47.2 -> 47.9, 4x4
+// filters (twice the products of before, 16n 64c 50x50 5.6 -> 5.8 and 5.5 -> 5.4).
 #include "spio_conv_common.h"
 
 using namespace spio;
@@ -112,15 +122,7 @@ constexpr int PF_RATE = SPIO_PF_RATE;
 constexpr int WAVES = GB * TS;
 constexpr int THREADS = 64 * WAVES;
 
-constexpr int NS = 2 * ((kR + 1) / 2);  // accumulator row slots
-// With an odd filter height every slot rests for one step between two output rows: the finished
-// row can then be converted and staged one step after its last tap (see the step loop).
-#ifndef SPIO_LATE_EMIT
-#define SPIO_LATE_EMIT 1
-#endif
-constexpr bool kLateEmit = SPIO_LATE_EMIT && NS > kR;
-constexpr int NACC = NS / 2;            // accumulators (pairs of slots) per tile
-constexpr int KB = (kS + 3) / 4;        // MFMA K-steps per source row (4 column taps each)
+constexpr int KB = (kS + 1 + 3) / 4;  // MFMA K-steps per source row (4 of a pair's S + 1 columns each)
 // Column blocks (SPIO_BQ > 0): a workgroup owns BQ output columns of its rows and stages the
 // BQ + S - 1 source columns they need; the S - 1 extra columns hold the neighbouring blocks'
 // pixels, or zeros at the image's edges (reference: block_q / block_w = block_q + S - 1,
@@ -130,15 +132,22 @@ constexpr int BQ = SPIO_BQ > 0 ? SPIO_BQ : DW;
 constexpr int QBLKS = (DW + BQ - 1) / BQ;
 constexpr int WPI = BQ + kS - 1;        // padded width of one image (block) in LDS
 constexpr int F = NB * WPI;             // flattened pixels of a staged row
-constexpr int WT = (F - kS + 1 + 15) / 16;  // 16-pixel tiles per row
-constexpr int TPW = (WT + TS - 1) / TS;     // tiles per wave
-constexpr int FP = 16 * WT + 4 * KB - 1;    // pixels any fragment read can touch
-constexpr int GS = FP + ((9 - FP % 16) + 16) % 16;  // group stride in pixels, = 9 mod 16
+constexpr int WT = (F - kS + 1 + 31) / 32;  // 32-pixel tiles per row
+// Tiles per wave.  Those past the last one (waves share a row) read and write cells that exist; they hold
+// zeros, and nobody looks at the results.
+constexpr int TPW = (WT + TS - 1) / TS;
+constexpr int FP = 32 * TPW * TS + 4 * KB - 2;  // pixels any fragment read can touch
+// The planes of even and odd pixels are 8 cells (half the banks) apart modulo 16, the groups 9, so that the
+// cells a wave's threads write fall into different banks.
+constexpr int PLANE = (FP + 1) / 2 + ((8 - (FP + 1) / 2 % 16) + 16) % 16;
+constexpr int GS = PLANE + FP / 2 + ((9 - (PLANE + FP / 2) % 16) + 16) % 16;  // group stride in cells
+SPIO_DEVICE constexpr int pos(int pixel) { return (pixel >> 1) + (pixel & 1) * PLANE; }
 constexpr int NR = 2;                               // ring rows
 constexpr int RING_ROW_UNITS = GB * GS + 1;         // 16-byte units per ring row (+1: dump cell)
 constexpr int DUMP_UNIT = GB * GS;                  // where lanes without a cell write
 constexpr int OSTRIDE = GB * 16 + 16;               // bytes per pixel in the output stage
-constexpr int OUT_ROW_BYTES = 16 * WT * OSTRIDE;
+constexpr int OPLANE = 16 * TPW * TS * OSTRIDE + 128;  // even pixels, then odd ones, as in the ring
+constexpr int OUT_ROW_BYTES = 2 * OPLANE;
 constexpr int IN_CELLS = F * GB;
 constexpr int LPT = (IN_CELLS + THREADS - 1) / THREADS;  // source cells per thread per row
 constexpr int OUT_CELLS = NB * BQ * GB;
@@ -174,7 +183,6 @@ static_assert(!SPIO_KEEP || !SPIO_SRC_F32 ||
 static_assert(!(SPIO_W_F32 && SPIO_IGRAD), "the data gradient reads fp16 filters");
 constexpr unsigned OOB = 0x80000000u;  // offset of a lane without data: beyond every descriptor
 
-constexpr int pmod(int a, int m) { return ((a % m) + m) % m; }
 constexpr int cmin(int a, int b) { return a < b ? a : b; }
 // Source rows requested once step t of `steps` has issued its loads (t = -1: before the first step).
 constexpr int rows_requested(int t, int steps) { return cmin(cmin(steps, t + 1 + PF), PF0 + PF_RATE * (t + 1)); }
@@ -266,7 +274,7 @@ SPIO_DEVICE void conv_rows(spio_uint4* __restrict__ dst, const spio_uint4* __res
                 const int f = cell / GB;
                 const int img = f / WPI;
                 const int col = q0 + f % WPI - EPX;
-                unit = g * GS + f;
+                unit = g * GS + pos(f);
                 if (col >= 0 && col < SW && cb * GB + g < kGroups)
                     voff = (unsigned)(((img * SH * SW + col) * kGroups + cb * GB + g) * (8 * kSrcBytes));
             }
@@ -330,26 +338,24 @@ SPIO_DEVICE void conv_rows(spio_uint4* __restrict__ dst, const spio_uint4* __res
     // multiplication waits for: the filters (a few loads per lane) go ahead of the PF source
     // rows, and the first step can start as soon as source row 0 has landed.  Branch-free: dead
     // taps and idle waves load a valid address and are zeroed when the fragments are built.
-    constexpr int WLPT = kIgrad ? (GB * 8 * kR * kS + THREADS - 1) / THREADS : NS * KB;
+    constexpr int WLPT = kIgrad ? (GB * 8 * kR * kS + THREADS - 1) / THREADS : kR * KB;
     spio_uint4 wraw[WLPT][kFilterLoads];
     if (!kIgrad) {
         // A[m = out channel ch][c] = w[8g+ch][r][s][c]: 16 contiguous bytes per lane.
-        // Lane (m = lane%16, kb = lane/16): row slot j = m/8, channel m%8, column tap 4u+kb;
-        // the filter row of slot j at distance d is r = (d - j) mod NS (none if r >= R).
+        // Lane (m = lane%16, kb = lane/16): pixel j = m/8 of a pair, channel m%8, column 4u+kb of the
+        // pair's S+1, which this pixel meets under tap 4u+kb-j.
         const int m = lane & 15;
         const int kb = lane >> 4;
         const int j = m >> 3;
         const int ch = m & 7;
         const int gsafe = wave_active ? gglob : 0;
 #pragma unroll
-        for (int d = 0; d < NS; ++d) {
+        for (int r = 0; r < kR; ++r) {
 #pragma unroll
             for (int u = 0; u < KB; ++u) {
-                const int r = (d - j + NS) % NS;
-                const int s = 4 * u + kb;
-                const int rr = r < kR ? r : 0;
-                const int ss = s < kS ? s : 0;
-                load_filter_unit(wraw[d * KB + u], weights, ((long long)(8 * gsafe + ch) * kR + rr) * kS + ss);
+                const int s = 4 * u + kb - j;
+                const int ss = s >= 0 && s < kS ? s : 0;
+                load_filter_unit(wraw[r * KB + u], weights, ((long long)(8 * gsafe + ch) * kR + r) * kS + ss);
             }
         }
     } else {
@@ -386,7 +392,8 @@ SPIO_DEVICE void conv_rows(spio_uint4* __restrict__ dst, const spio_uint4* __res
                 const int g = cell % GB;
                 const int q = (cell / GB) % BQ;
                 const int img = cell / (GB * BQ);
-                from = (img * WPI + q) * OSTRIDE + g * 16;
+                const int o = img * WPI + q;
+                from = (o & 1) * OPLANE + (o >> 1) * OSTRIDE + g * 16;
                 if (cb * GB + g < kGroups && q0 + q < DW)
                     voff = (unsigned)(((img * DH * DW + q0 + q) * kGroups + cb * GB + g) * (8 * kDstBytes));
             }
@@ -395,21 +402,20 @@ SPIO_DEVICE void conv_rows(spio_uint4* __restrict__ dst, const spio_uint4* __res
         }
     }
 
-    // ---- filter fragments: wfrag[d][u], d = (phase - 2*acc) mod NS ----
-    spio_half8 wfrag[NS][KB];
+    // ---- filter fragments: wfrag[r][u] ----
+    spio_half8 wfrag[kR][KB];
     if (!kIgrad) {
         const int m = lane & 15;
         const int kb = lane >> 4;
         const int j = m >> 3;
 #pragma unroll
-        for (int d = 0; d < NS; ++d) {
+        for (int r = 0; r < kR; ++r) {
 #pragma unroll
             for (int u = 0; u < KB; ++u) {
-                const int r = (d - j + NS) % NS;
-                const int s = 4 * u + kb;
+                const int s = 4 * u + kb - j;
                 Pack16 v;
-                v.u = (r < kR && s < kS) ? filter_unit(wraw[d * KB + u]) : spio_uint4{0u, 0u, 0u, 0u};
-                wfrag[d][u] = v.h;
+                v.u = (s >= 0 && s < kS) ? filter_unit(wraw[r * KB + u]) : spio_uint4{0u, 0u, 0u, 0u};
+                wfrag[r][u] = v.h;
             }
         }
     } else {
@@ -417,7 +423,7 @@ SPIO_DEVICE void conv_rows(spio_uint4* __restrict__ dst, const spio_uint4* __res
         // the group.  The workgroup copies its groups' filters to LDS as they lie in memory
         // ([jj][r][s][8 ch]) and every wave reads its fragments with the transposing LDS read:
         // in a 16-lane block source lane 4*jr+t supplies 4 channels (half t%2) of row jj = jr for
-        // the row slot t/2, and result lane i receives rows jj = 0..3 of column i = 8*slot + ch.
+        // pixel t/2 of a pair, and result lane i receives rows jj = 0..3 of column i = 8*pixel + ch.
         constexpr int WUNITS = GB * 8 * kR * kS;
         const lds_u4p wlds = ring;  // ring and output stage are not in use yet
 #pragma unroll
@@ -429,19 +435,18 @@ SPIO_DEVICE void conv_rows(spio_uint4* __restrict__ dst, const spio_uint4* __res
         const int kb = lane >> 4;
         const int jr = (lane & 15) >> 2;
         const int t4 = lane & 3;
-        const int src_slot = t4 >> 1;        // slot whose data this lane fetches
-        const int my_slot = (lane & 15) >> 3;  // slot of the fragment row this lane receives
+        const int src_pixel = t4 >> 1;          // of a pair: whose data this lane fetches
+        const int my_pixel = (lane & 15) >> 3;  // whose fragment row this lane receives
         typedef spio_short4 __attribute__((address_space(3))) * lds_ptr;
 #pragma unroll
-        for (int d = 0; d < NS; ++d) {
+        for (int r = 0; r < kR; ++r) {
 #pragma unroll
             for (int u = 0; u < KB; ++u) {
-                const int s = 4 * u + kb;
-                const int r_src = (d - src_slot + NS) % NS;
-                const int r_mine = (d - my_slot + NS) % NS;
+                const int s_src = 4 * u + kb - src_pixel;
+                const int s_mine = 4 * u + kb - my_pixel;
                 // clamp the address of dead taps; their result is discarded below
-                const int rr = r_src < kR ? kR - 1 - r_src : 0;
-                const int ss = s < kS ? kS - 1 - s : 0;
+                const int rr = kR - 1 - r;
+                const int ss = s_src >= 0 && s_src < kS ? kS - 1 - s_src : 0;
                 const lds_bytep base = (lds_bytep)wlds + ((((wg * 8 + jr) * kR + rr) * kS + ss) * 16) + (t4 & 1) * 8;
                 union {
                     spio_short4 q[2];
@@ -449,42 +454,36 @@ SPIO_DEVICE void conv_rows(spio_uint4* __restrict__ dst, const spio_uint4* __res
                 } v;
                 v.q[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)base);
                 v.q[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)(base + 4 * kR * kS * 16));
-                if (!(r_mine < kR && s < kS)) v.h = spio_half8{0, 0, 0, 0, 0, 0, 0, 0};
-                wfrag[d][u] = v.h;
+                if (!(s_mine >= 0 && s_mine < kS)) v.h = spio_half8{0, 0, 0, 0, 0, 0, 0, 0};
+                wfrag[r][u] = v.h;
             }
         }
         block_sync();  // everyone has its fragments before the ring is zero-filled
     }
 
-    // Accumulator lane layout: D[m = 4*(lane/16)+i][n = lane%16]: pixel n = lane%16,
-    // row slot j = lane/32, channels 4*((lane/16)&1) + i.
-    const int out_j = lane >> 5;
+    // Accumulator lane layout: D[m = 4*(lane/16)+i][n = lane%16]: pixel 2*(lane%16) + lane/32 of the
+    // tile, channels 4*((lane/16)&1) + i.
     const int out_kh = (lane >> 4) & 1;
-    const int out_n = lane & 15;
     // this lane's place in a staged output row (tile 0 of the wave) and in a ring row
-    const lds_bytep ostage_lane = ostage + (16 * ws + out_n) * OSTRIDE + wg * 16 + out_kh * 8;
-    const int frag_unit = wg * GS + (lane & 15) + (lane >> 4);
-    float bias_reg[4] = {0.f, 0.f, 0.f, 0.f};
+    const lds_bytep ostage_lane =
+        ostage + (lane >> 5) * OPLANE + (16 * TPW * ws + (lane & 15)) * OSTRIDE + wg * 16 + out_kh * 8;
+    const int frag_unit = wg * GS + 16 * TPW * ws + (lane & 15) + pos(lane >> 4);
+    spio_float4 bias_reg = spio_float4{0.f, 0.f, 0.f, 0.f};
     if (kHasBias && wave_active) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) bias_reg[i] = bias[8 * gglob + 4 * out_kh + i];
     }
-    spio_float4 acc[TPW][NACC];
-#pragma unroll
-    for (int i = 0; i < TPW; ++i)
-#pragma unroll
-        for (int a = 0; a < NACC; ++a)
-            acc[i][a] = spio_float4{bias_reg[0], bias_reg[1], bias_reg[2], bias_reg[3]};
+    spio_float4 acc[TPW][kR];  // output row t of the tile in accumulator t mod R, from step t to step t + R - 1
 
     // ---- zero the slack cells behind each group's pixels once: fragment reads of the last
     //      tiles touch them (they meet zero filter taps, so they must be finite), nothing ever
     //      writes them ----
     {
-        constexpr int SLACK = GS - F;
+        constexpr int SLACK = FP - F;
         for (int i = tid; i < NR * GB * SLACK; i += THREADS) {
             const int row = i / (GB * SLACK);
             const int g = (i / SLACK) % GB;
-            ring[row * RING_ROW_UNITS + g * GS + F + i % SLACK] = spio_uint4{0u, 0u, 0u, 0u};
+            ring[row * RING_ROW_UNITS + g * GS + pos(F + i % SLACK)] = spio_uint4{0u, 0u, 0u, 0u};
         }
     }
 
@@ -528,117 +527,86 @@ SPIO_DEVICE void conv_rows(spio_uint4* __restrict__ dst, const spio_uint4* __res
         return h >= 0 && h < SH;
     };
     spio_half8 bfrag[TPW][KB];
-    auto read_fragments = [&](spio_half8(&frag)[TPW][KB], int ring_row) {
+    auto read_fragments = [&](int ring_row) {
         const lds_u4p rrow = ring + ring_row * RING_ROW_UNITS + frag_unit;
 #pragma unroll
         for (int i = 0; i < TPW; ++i) {
-            const int tile = ws + TS * i;
-            if (TS == 1 || tile < WT) {
 #pragma unroll
-                for (int u = 0; u < KB; ++u) {
-                    Pack16 v;
-                    v.u = rrow[16 * TS * i + 16 * ws + 4 * u];
-                    frag[i][u] = v.h;
-                }
+            for (int u = 0; u < KB; ++u) {
+                Pack16 v;
+                v.u = rrow[16 * i + 2 * u];
+                bfrag[i][u] = v.h;
             }
         }
     };
-    // Stages the output row that received its last tap at step `te` (stage buffer te mod 2) and
-    // resets its slot to the bias.  The row sits in one half of the lanes (slot j = lane / 32).
-    // (Letting the other half convert along and write into spare bytes, which removes the
-    // lane-dependent branch, is slower: 1-6 % at the benchmark shapes.)
+    // Stages the output row that received its last tap at step `te` (stage buffer te mod 2).
     auto emit_row = [&](int te) {
-        const int slot = pmod(te % NS - (kR - 1), NS);
-        const int a = slot >> 1;
-        const int j = slot & 1;
-        if (out_j == j) {
 #pragma unroll
-            for (int i = 0; i < TPW; ++i) {
-                const int tile = ws + TS * i;
-                if (TS == 1 || tile < WT) {
-                    if (te >= kR - 1) {
-                        Pack8 o;
+        for (int i = 0; i < TPW; ++i) {
+            Pack8 o;
 #pragma unroll
-                        for (int e = 0; e < 4; ++e) o.h[e] = (spio_half)acc[i][a][e];
-                        *(lds_u2p)(ostage_lane + (te & 1) * OUT_ROW_BYTES + 16 * TS * i * OSTRIDE) = o.u;
-                    }
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) acc[i][a][e] = bias_reg[e];
-                }
-            }
-        }
-    };
-    auto multiply_tile = [&](int ph, int i) {
-        const int tile = ws + TS * i;
-        if (TS == 1 || tile < WT) {
-#pragma unroll
-            for (int a = 0; a < NACC; ++a) {
-                const int d = pmod(ph - 2 * a, NS);
-#pragma unroll
-                for (int u = 0; u < KB; ++u)
-                    acc[i][a] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wfrag[d][u], bfrag[i][u], acc[i][a], 0, 0, 0);
-            }
+            for (int e = 0; e < 4; ++e) o.h[e] = (spio_half)acc[i][(te + 1) % kR][e];
+            *(lds_u2p)(ostage_lane + (te & 1) * OUT_ROW_BYTES + 16 * i * OSTRIDE) = o.u;
         }
     };
 #pragma unroll
-    for (int t = 0; t < STEPS; ++t) {
-        const int ph = t % NS;    // all of these are compile-time constants after unrolling
-
+    for (int t = 0; t < STEPS; ++t) {  // everything that depends on t is a compile-time constant after unrolling
         // 1. prefetch the next source rows, at most up to row t+PF (whose register buffer is
         //    free: row t is in LDS)
 #pragma unroll
         for (int r = rows_requested(t - 1, STEPS); r < rows_requested(t, STEPS); ++r) load_row(pre[r % PF], r);
 
-        // 2. fragment reads of this step's row; a finished output row is stored while they are
-        //    in flight
+        // 2. fragment reads of this step's row.  While they are in flight the row staged in the previous step
+        //    goes out, and the row that received its last tap in the previous step is converted and staged:
+        //    its results are long complete, while behind this step's MFMAs it would have to wait.  Its accumulator is
+        //    the one that this step's newest row begins in, below.
         const bool row_live = row_is_live(t);
-        if (row_live) read_fragments(bfrag, t % NR);
-        if (kLateEmit) {
-            // The row that received its last tap in the previous step is converted and staged
-            // now, ahead of this step's multiplications: its results are long complete, and the
-            // conversion runs while the fragment reads are on their way instead of behind the
-            // MFMAs it would have to wait for.  Its slot rests during this step (NS > R: the
-            // slot's filter row is out of range, its A rows are zero), so the values are still
-            // there, and the reset takes effect before the slot's next row begins.  The row
-            // staged in the previous step goes out.
-            if (t >= kR + 1) store_output_row(t - 2, t & 1);
-            if (t >= 1) emit_row(t - 1);  // (before the first finished row: resets only)
-        } else {
-            if (t >= kR) store_output_row(t - 1, (t + 1) & 1);
-        }
-        // 3. multiply source row t into the live output rows
+        if (row_live) read_fragments(t % NR);
+        if (t >= kR + 1) store_output_row(t - 2, t & 1);
+        if (t >= kR) emit_row(t - 1);
+
+        // 3. multiply source row t into the output rows t - r of the tile; row t starts from the bias
         if (row_live) {
 #pragma unroll
-            for (int i = 0; i < TPW; ++i) multiply_tile(ph, i);
+            for (int i = 0; i < TPW; ++i) {
+#pragma unroll
+                for (int u = 0; u < KB; ++u) {
+#pragma unroll
+                    for (int r = 0; r < kR; ++r) {
+                        if (t - r < 0 || t - r >= ROWS) continue;
+                        spio_float4& d = acc[i][(t - r) % kR];
+                        d = __builtin_amdgcn_mfma_f32_16x16x32_f16(wfrag[r][u], bfrag[i][u],
+                                                                   r == 0 && u == 0 ? bias_reg : d, 0, 0, 0);
+                    }
+                }
+            }
+        } else if (t < ROWS) {
+#pragma unroll
+            for (int i = 0; i < TPW; ++i) acc[i][t % kR] = bias_reg;
         }
 
-        // 4. the row that received its last tap: stage it, reset its slot
-        if (!kLateEmit) emit_row(t);
-
-        // 5. the next source row not yet in the ring (loaded earlier) into its ring row
+        // 4. the next source row not yet in the ring (loaded earlier) into its ring row
         if (t + 1 < STEPS) row_to_ring(pre[(t + 1) % PF], t + 1);
 
         block_sync();
     }
-    if (kLateEmit) {
-        // the row staged in the last step goes out, the last row is staged and follows
-        if (STEPS >= kR + 1) store_output_row(STEPS - 2, STEPS & 1);
-        emit_row(STEPS - 1);
-        block_sync();
-    }
+    // the row staged in the last step goes out, the last row is staged and follows
+    if (STEPS >= kR + 1) store_output_row(STEPS - 2, STEPS & 1);
+    emit_row(STEPS - 1);
+    block_sync();
     store_output_row(STEPS - 1, (STEPS - 1) & 1);  // the last row
 
     if (SPIO_KEEP && SPIO_W_F32 && n0 == 0 && p0 == 0 && q0 == 0 && ws == 0 && wave_active) {
-        // the rounded filters, by the first tile of the channel block: slot 0 holds filter row d of phase d
+        // the rounded filters, by the first tile of the channel block: the first pixel's rows of the fragments
         const int m = lane & 15;
         const int kb = lane >> 4;
 #pragma unroll
-        for (int d = 0; d < kR; ++d)
+        for (int r = 0; r < kR; ++r)
 #pragma unroll
             for (int u = 0; u < KB; ++u) {
                 Pack16 v;
-                v.h = wfrag[d][u];
-                if (m < 8 && 4 * u + kb < kS) kept_weights[((long long)(8 * gglob + m) * kR + d) * kS + 4 * u + kb] = v.u;
+                v.h = wfrag[r][u];
+                if (m < 8 && 4 * u + kb < kS) kept_weights[((long long)(8 * gglob + m) * kR + r) * kS + 4 * u + kb] = v.u;
             }
     }
 }

@@ -10,7 +10,6 @@ the fields mean on the device.
 """
 
 from dataclasses import dataclass, replace
-from math import gcd
 from typing import Dict, List
 
 import torch
@@ -30,7 +29,7 @@ MAX_WAVES = 16
 MAX_LDS_BYTES = 128 * 1024
 MAX_UNROLLED_STEPS = 64  # SPIO_MAX_UNROLL of the kernel: up to here the step loop is fully unrolled
 MAX_LOADS_PER_THREAD = 8
-MAX_ACCUMULATORS = 16
+MAX_ACCUMULATORS = 18
 DEVICE_LDS_BYTES = 160 * 1024
 MAX_IMAGE_CONFIGS = 10  # whole-image configurations that enter the sweep
 MOVER_WAVES = 4  # data-mover waves of the whole-image kernel where it has any: one per SIMD
@@ -110,29 +109,31 @@ def mfma_geometry(params: Conv2dGw8Params, config: Conv2dGw8Config, igrad: bool)
     """Host mirror of the compile-time constants of conv2d_gw8_mfma.hip."""
     d = direction_geometry(params, igrad)
     r, s = params.r, params.s
-    gb, bp, nb, ts, pf = config.groups, config.block_p, config.block_n, config.split, config.prefetch
+    gb, bp, nb, ts = config.groups, config.block_p, config.block_n, config.split
     bp2 = config.block_p2
     bq = config.block_q or d["DW"]
-    ns = 2 * ((r + 1) // 2)
-    kb = (s + 3) // 4
+    kb = (s + 4) // 4
     wpi = bq + s - 1
     f = nb * wpi
-    wt = divup(f - s + 1, 16)
-    fp = 16 * wt + 4 * kb - 1
-    gs = fp + ((9 - fp % 16) + 16) % 16
+    tiles = divup(f - s + 1, 32)  # a product takes 16 pairs of pixels
+    tpw = divup(tiles, ts)
+    fp = 32 * tpw * ts + 4 * kb - 2
+    plane = fp // 2 + (8 - fp // 2) % 16
+    gs = plane + fp // 2 + (9 - (plane + fp // 2)) % 16
     threads = 64 * gb * ts
     ostride = gb * 16 + 16
-    lds = 2 * (gb * gs + 1) * 16 + 2 * 16 * wt * ostride  # ring rows (+ dump cell) and two output-stage rows
+    # ring rows (+ dump cell) and two output-stage rows
+    lds = 2 * (gb * gs + 1) * 16 + 4 * (16 * tpw * ts * ostride + 128)
     if igrad:  # the data gradient stages its groups' filters in the same block first
         lds = max(lds, gb * 8 * r * s * 16)
     d.update(
-        NS=ns, NACC=ns // 2, KB=kb, WPI=wpi, F=f, WT=wt, TPW=divup(wt, ts), GS=gs,
+        KB=kb, WPI=wpi, F=f, WT=2 * tiles, TPW=tpw, GS=gs,
         THREADS=threads, LDS_BYTES=lds, LPT=divup(f * gb, threads),
         SPT=divup(nb * bq * gb, threads), BQ=bq, QBLKS=divup(d["DW"], bq),
         GBLKS=divup(params.groups, gb), NBLKS=divup(params.n, nb),
         # two tile heights: PBLKS (block_p, block_p2) pairs per image, one workgroup per tile
         PBLKS=divup(d["DH"], bp + bp2) if bp2 else divup(d["DH"], bp),
-        STEPS=max(bp, bp2) + r - 1, UNROLL=ns // gcd(ns, pf) * pf,
+        STEPS=max(bp, bp2) + r - 1,
     )  # fmt: skip
     d["NUM_BLOCKS"] = (2 if bp2 else 1) * d["GBLKS"] * d["PBLKS"] * d["QBLKS"] * d["NBLKS"]
     return d
@@ -149,7 +150,7 @@ def _mfma_fits(params, config, igrad) -> bool:
     accumulators and rows in flight.  The weights were fitted to what the compiler reports for 1771 kernels of 110
     shapes, 1x1 to 7x7: of 100 that used memory 5 pass, with 100 bytes at most, of 1671 others 2 do not."""
     g = mfma_geometry(params, config, igrad)
-    fragments, accumulators = 4 * g["NS"] * g["KB"], 4 * g["TPW"] * g["NACC"]
+    fragments, accumulators = 4 * params.r * g["KB"], 4 * g["TPW"] * params.r
     rows = 4 * min(config.prefetch, g["STEPS"]) * g["LPT"]
     needed = fragments + 1.6 * accumulators + 1.3 * rows + 6
     return needed <= 1.05 * lane_registers(config.groups * config.split)
@@ -323,7 +324,7 @@ def _mfma_config_is_legal(params, config, igrad) -> bool:
         and 0 <= config.block_q <= g["DW"]
         and g["LDS_BYTES"] <= MAX_LDS_BYTES
         and g["LPT"] <= MAX_LOADS_PER_THREAD
-        and g["TPW"] * g["NACC"] <= MAX_ACCUMULATORS
+        and g["TPW"] * params.r <= MAX_ACCUMULATORS
         and config.prefetch >= 2
         # the step loop is always unrolled completely (exact counts of outstanding loads/stores)
         and g["STEPS"] <= MAX_UNROLLED_STEPS
@@ -427,6 +428,8 @@ def _get_configs(params: Conv2dGw8Params, device_attr=None, igrad: bool = False)
         for gb in group_choices:
             for nb in (1, 2, 4, 8) if bq == 0 else (1,):
                 for ts in (1, 2, 4):
+                    if nb * ((bq or d["DW"]) + params.s - 1) - params.s + 1 <= 32 * (ts // 2):
+                        continue  # a wave without a tile
                     for bp in row_choices:
                         steps = bp + params.r - 1
                         for pf in PREFETCH_CHOICES:

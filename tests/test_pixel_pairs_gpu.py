@@ -3,13 +3,15 @@ end: rows of 31 to 33 and of 64 pixels, every filter width, step loops in chunks
 image.  Oracle and tolerances are those of the other kernel tests."""
 
 import pytest
-from helpers import run_bgrad_kernel_test, run_grad_kernel_test
+from helpers import run_bgrad_kernel_test, run_grad_kernel_test, run_kernel_test
 
 from spio_amd.kernels import (
     Conv2dGw8BgradConfig,
+    Conv2dGw8Config,
     Conv2dGw8Params,
     Conv2dGw8WgradConfig,
     conv2d_gw8_bgrad_kernel_factory,
+    conv2d_gw8_kernel_factory,
     conv2d_gw8_wgrad_kernel_factory,
 )
 
@@ -66,3 +68,24 @@ def test_weight_gradient(shape):
     if params.w > 32:
         configs.append(W(groups=groups, block_h=params.p, block_n=1, prefetch=2, split=2))
     run_grad_kernel_test(conv2d_gw8_wgrad_kernel_factory, params, configs=configs)
+
+
+@pytest.mark.parametrize("shape", [*SHAPES, (2, 16, 8, 15, 7, 7, 3, True), (2, 8, 6, 7, 3, 3, 4, True)], ids=str)
+@pytest.mark.parametrize("igrad", [False, True])
+def test_forward_and_data_gradient(shape, igrad):
+    """Also a filter of seven accumulators, and padding that makes rows without any input (they are the bias alone)."""
+    params = _params(shape)
+    groups, images, rows = min(params.groups, 4), min(params.n, 3), params.h if igrad else params.p
+    C = Conv2dGw8Config
+    configs = [
+        C(groups=groups, block_p=min(rows, 40), block_n=images if params.w < 32 else 1, prefetch=2),
+        C(groups=groups, block_p=min(rows, 4), block_n=1, prefetch=4),
+        C(groups=1, block_p=min(rows, 3), block_n=1, prefetch=2, split=2),
+        C(groups=groups, block_p=min(rows, 3), block_p2=1, block_n=1, prefetch=2),
+    ]
+    if params.w >= 31:
+        configs.append(C(groups=groups, block_p=min(rows, 5), block_q=17, prefetch=2))
+    if igrad:
+        run_grad_kernel_test(conv2d_gw8_kernel_factory, params, configs=configs, igrad=True)
+    else:
+        run_kernel_test(conv2d_gw8_kernel_factory, params, configs=configs)
