@@ -185,6 +185,13 @@ constexpr int LCM = lcm_(kR, PF);  // PF is even, so this is too
 constexpr bool kFullUnroll = ROWS <= SPIO_MAX_UNROLL;
 constexpr int UNROLL = kFullUnroll ? (ROWS + LCM - 1) / LCM * LCM : LCM;
 constexpr int pmod(int a, int m) { return ((a % m) + m) % m; }
+// Where a workgroup has one block of whole rows, a finished dx row is converted and staged in the step after its last
+// tap, while that step's fragment reads are on their way, instead of behind the products it would have to wait for.  Its
+// sums are the ones that the step begins a new row in.  Before -> after in the same configuration: 1n 64c 56x56 5.8 ->
+// 5.4 us, 8n 7.2 -> 6.8, 32n 11.9 -> 11.3, 128n in 28-row blocks 34.0 -> 31.5, 16n 64c 50x50 2x2 13.5 -> 10.5, 128n 128c 28x28
+// 19.3 -> 18.8.  Elsewhere it gives nothing or takes registers that there are not: several blocks 16n 64c 128x512 79 -> 82,
+// column blocks 1n 400c 211x211 37.7 -> 41.3, 5x5 4n 424c 84x84 61.6 -> 65.2, 1x1 8n 248c 42x42 10.3 -> 11.0.
+constexpr bool kLateStage = ITERS == 1 && !kColBlocks && (kR == 2 || kR == 3);
 
 constexpr int RING_UNITS = 2 * XROW_UNITS + 2 * DROW_UNITS;  // two rows each: a step's and the next one's
 constexpr int STREAM_UNITS = RING_UNITS + 2 * OUT_ROW_BYTES / 16;
@@ -527,8 +534,18 @@ SPIO_KERNEL_NAME(spio_uint4* __restrict__ grad_input, float* __restrict__ grad_w
             for (int ci = 0; ci < CPW; ++ci) afrag[r][ci] = spio_half8{0, 0, 0, 0, 0, 0, 0, 0};
         }
 
-        // Coalesced store of the dx row staged at step `ts` (domain row p0 - (R-1) + ts), one step
-        // later.  Steps that finish no row of the block, or a domain row outside dx, store through
+        // A finished dx row, from sums `slot` into the output stage.
+        auto stage_dx_row = [&](int slot, int obuf) {
+#pragma unroll
+            for (int i = 0; i < TPW; ++i) {
+                Pack8 o;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) o.h[e] = (spio_half)dacc[i][slot][e];
+                *reinterpret_cast<spio_uint2*>(ostage + obuf * OUT_ROW_BYTES + 16 * (TPW * ws + i) * OSTRIDE + out_off) = o.u;
+            }
+        };
+        // Coalesced store of the dx row that received its last tap at step `ts` (domain row p0 - (R-1) + ts), one step
+        // after it was staged.  Steps that finish no row of the block, or a domain row outside dx, store through
         // the empty descriptor: the
         // instructions are issued all the same and the hardware drops them.
         auto store_dx_row = [&](int ts, int obuf) {
@@ -564,7 +581,6 @@ SPIO_KERNEL_NAME(spio_uint4* __restrict__ grad_input, float* __restrict__ grad_w
                 const int sp = uu & 1;                   // parity of t: ring rows
                 const int pbuf = uu % PF;                // register buffer that held row t
                 const int ph = uu % kR;                  // t mod R
-                const int obuf = uu & 1;
                 // what the step has to do, known at compile time in an unrolled loop: dy rows are named by
                 // the step that staged them (row p0-PB+tau at step tau; the block owns tau in [PB, PB+bh_eff)),
                 // x row t (p0-(R-1)+t) meets dy rows t - r under filter row r, dy row t reaches the dx rows
@@ -621,8 +637,13 @@ SPIO_KERNEL_NAME(spio_uint4* __restrict__ grad_input, float* __restrict__ grad_w
                 //    them out.
                 if (!kFullUnroll || t + PF < ROWS) load_rows(xpre[pbuf], dpre[pbuf], t + PF);
 
-                // 3. the dx row finished in the previous step goes out
-                if (!kFullUnroll || t - 1 >= kR - 1) store_dx_row(t - 1, (uu + 1) & 1);
+                // 3. the dx row staged in the previous step goes out, one that was finished then is staged
+                if (kLateStage) {
+                    if (!kFullUnroll || t - 2 >= kR - 1) store_dx_row(t - 2, uu & 1);
+                    if (!kFullUnroll || (t - 1 >= kR - 1 && t - 1 < kR - 1 + BH)) stage_dx_row(ph, (uu + 1) & 1);
+                } else {
+                    if (!kFullUnroll || t - 1 >= kR - 1) store_dx_row(t - 1, (uu + 1) & 1);
+                }
 
                 // 4. rows t+1 into LDS, where nothing of this step reads (dy rows past the last one become zero)
                 if (t + 1 < ROWS) {
@@ -667,20 +688,20 @@ SPIO_KERNEL_NAME(spio_uint4* __restrict__ grad_input, float* __restrict__ grad_w
                 }
 
                 // 6. the dx row that received its last tap (row p0-(R-1)+t): stage it
-                if (!kFullUnroll || (t >= kR - 1 && t < kR - 1 + BH)) {
-#pragma unroll
-                    for (int i = 0; i < TPW; ++i) {
-                        Pack8 o;
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) o.h[e] = (spio_half)dacc[i][pmod(ph - (kR - 1), kR)][e];
-                        *reinterpret_cast<spio_uint2*>(ostage + obuf * OUT_ROW_BYTES +
-                                                       16 * (TPW * ws + i) * OSTRIDE + out_off) = o.u;
-                    }
-                }
+                if (!kLateStage && (!kFullUnroll || (t >= kR - 1 && t < kR - 1 + BH)))
+                    stage_dx_row(pmod(ph - (kR - 1), kR), uu & 1);
                 block_sync();
             }
         }
-        store_dx_row(ROWS - 1, (ROWS - 1) & 1);  // the last staged row (if it is a real one)
+        // the row staged in the last step and one finished in it (if they are real ones)
+        if (kLateStage) {
+            store_dx_row(ROWS - 2, ROWS & 1);
+            if (PB == 0) {
+                stage_dx_row(ROWS % kR, (ROWS - 1) & 1);
+                block_sync();
+            }
+        }
+        if (!kLateStage || PB == 0) store_dx_row(ROWS - 1, (ROWS - 1) & 1);
     }
 
     // ---- publish grad_weight (and grad_bias) ----
