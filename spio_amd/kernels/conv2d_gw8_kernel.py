@@ -418,7 +418,10 @@ def _get_configs(params: Conv2dGw8Params, device_attr=None, igrad: bool = False)
     d = direction_geometry(params, igrad)
     num_cus = getattr(device_attr, "multiprocessor_count", 256) or 256
     G = params.groups
-    group_choices = sorted({g for g in (4, 8, 16, G) if g <= min(G, MAX_WAVES)}) or [min(G, MAX_WAVES)]
+    # Where a pixel is not whole lines also the smallest blocks of one size that make up three or four lines: fewer
+    # boundaries lie inside lines, and the last block is not nearly empty.
+    even_blocks = {divup(G, divup(G, most)) for most in (12, 16)} if G % 8 else set()
+    group_choices = sorted({g for g in {4, 8, 16, G} | even_blocks if g <= min(G, MAX_WAVES)}) or [min(G, MAX_WAVES)]
     row_choices = balanced(d["DH"], (2, 4, 7, 8, 14, 16, 28, 32, 56, d["DH"]))
     # column blocks for wide rows only: narrower ones fit whole and pay no column halo
     col_choices = [bq for bq in COLUMN_BLOCK_CHOICES if d["DW"] >= 2 * bq and d["DW"] > 128]
@@ -452,6 +455,16 @@ def _get_configs(params: Conv2dGw8Params, device_attr=None, igrad: bool = False)
         if len(head) >= MAX_GEOMETRIES:
             break
     rank = {cfg: i for i, (_, cfg) in enumerate(found)}
+    if G % 8:
+        # Which number of groups is best depends on how lines are shared, which the score does not see: the best geometry
+        # of each first (of 16 no more than the others: it was the best of none).  First use of 8, before -> after:
+        # 59n 456c 60x60 110 -> 88 us, 64n 144c 56x56 36.5 -> 28.2, 50n 152c 41x41 16.5 -> 13.1, 60n 200c 33x33 17.2 -> 14.7,
+        # 7n 168c 159x159 33.2 -> 30.0, 4n 424c 84x84 5x5 20.7 -> 16.7, 2n 600c 147x147 7x7 47 -> 38; 8n 88c 61x40, 48c
+        # 224x224, 648c 56x97 5x5 equal.
+        tried = dict.fromkeys(cfg.groups for _, cfg in found if cfg.groups in even_blocks or cfg.groups != 16)
+        leaders = [next(cfg for _, cfg in found if cfg.groups == g) for g in tried]
+        head = leaders + [cfg for cfg in head if cfg not in leaders]
+        rest = [cfg for cfg in rest if cfg not in leaders]
     configs = [*head[:8], *sorted(head[8:] + rest, key=rank.get)][:MAX_GEOMETRIES]
     # the memory-system policies, which the score cannot rank: halo rows with or without the
     # non-temporal hint, and how tiles are dealt to the XCDs

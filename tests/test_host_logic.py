@@ -577,3 +577,22 @@ def test_weight_gradient_candidates_of_few_groups_are_not_all_split():
     """Three waves are fewer than a compute unit has SIMDs, and still the fastest (128n 24c 144x144)."""
     params = Conv2dGw8Params.decode("128n_24c_144h_144w_1py_1px_3r_3s_nb")
     assert any(c.split == 1 for c in conv2d_gw8_wgrad_kernel_factory.configs(params, ATTR)[:8])
+
+
+@pytest.mark.parametrize("groups", [9, 13, 19, 25, 53, 71])
+def test_capped_sweeps_try_every_number_of_groups_where_lines_are_shared(groups):
+    """Pixels that are not whole lines: among the first eight row-streaming geometries is one of every block of groups
+    that is offered, up to sixteen groups, blocks of one size among them; where a pixel is whole lines there are no others
+    than 4, 8, 16 and all."""
+    from spio_amd.kernels.tuner import _leading
+
+    def row_streaming(c):
+        configs = list(conv2d_gw8_kernel_factory.configs(Conv2dGw8Params(n=16, c=c, h=40, w=40, padding=1), DeviceAttributes()))
+        return [cfg for cfg in configs if cfg.variant == "mfma"]
+
+    configs = row_streaming(8 * groups)
+    first = configs[:_leading(configs, 8)]
+    even = {-(-groups // -(-groups // most)) for most in (12, 16)}
+    assert even <= {cfg.groups for cfg in configs}
+    assert {cfg.groups for cfg in configs} - {16} <= {cfg.groups for cfg in first}
+    assert {cfg.groups for cfg in row_streaming(8 * 24)} <= {4, 8, 16, 24}

@@ -70,7 +70,10 @@ def test_weight_gradient(shape):
     run_grad_kernel_test(conv2d_gw8_wgrad_kernel_factory, params, configs=configs)
 
 
-@pytest.mark.parametrize("shape", [*SHAPES, (2, 16, 8, 15, 7, 7, 3, True), (2, 8, 6, 7, 3, 3, 4, True)], ids=str)
+FORWARD_SHAPES = [*SHAPES, (2, 16, 8, 15, 7, 7, 3, True), (2, 8, 6, 7, 3, 3, 4, True), (2, 104, 6, 33, 3, 3, 1, True)]
+
+
+@pytest.mark.parametrize("shape", FORWARD_SHAPES, ids=str)
 @pytest.mark.parametrize("igrad", [False, True])
 def test_forward_and_data_gradient(shape, igrad):
     """Also a filter of seven accumulators, and padding that makes rows without any input (they are the bias alone)."""
@@ -85,6 +88,8 @@ def test_forward_and_data_gradient(shape, igrad):
     ]
     if params.w >= 31:
         configs.append(C(groups=groups, block_p=min(rows, 5), block_q=17, prefetch=2))
+    if params.groups > 8:  # two blocks, the second with a group less
+        configs.append(C(groups=7, block_p=min(rows, 4), prefetch=2))
     if igrad:
         run_grad_kernel_test(conv2d_gw8_kernel_factory, params, configs=configs, igrad=True)
     else:
