@@ -627,6 +627,7 @@ SPIO_KERNEL_NAME(spio_uint4* __restrict__ grad_input, float* __restrict__ grad_w
                         for (int u = 0; u < KB; ++u) {
                             Pack16 v;
                             v.u = rrow[16 * (TPW * ws + i) + 2 * u];
+                            if (in_no_window(u, kb)) v.u = zero4;
                             sfrag[i][u] = v.h;
                         }
                     }

@@ -535,6 +535,7 @@ SPIO_DEVICE void conv_rows(spio_uint4* __restrict__ dst, const spio_uint4* __res
             for (int u = 0; u < KB; ++u) {
                 Pack16 v;
                 v.u = rrow[16 * i + 2 * u];
+                if (in_no_window(u, lane >> 4)) v.u = spio_uint4{0u, 0u, 0u, 0u};
                 bfrag[i][u] = v.h;
             }
         }

@@ -97,6 +97,12 @@ SPIO_DEVICE int xcd_tile(int id) {
 // Run length where channel blocks share lines and go fastest in the tile order: whole pixels.
 constexpr int line_run(int run, int gblks) { return run <= 1 ? run : (run + gblks - 1) / gblks * gblks; }
 
+// Whether column 4 u + kb of a pair's source columns is in the filter window of neither pixel.  The pair meets S + 1
+// columns and a product takes four, so the last one has up to three more; their taps are zeros, but zero times an
+// infinity is not.  The lanes that hold them multiply zeros instead: an infinite or NaN source pixel then reaches, as NaN,
+// no output beyond its window but the one next to it that is the other of a pair.
+SPIO_DEVICE bool in_no_window(int u, int kb) { return (kS + 1) % 4 != 0 && 4 * u + kb > kS; }
+
 // Streaming accesses: activations are touched once per kernel, so they are
 // loaded and stored with the non-temporal hint (measured on MI355X: a plain
 // 16-byte-per-lane copy gains about 10% from it).
