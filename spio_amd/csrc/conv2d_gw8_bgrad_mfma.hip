@@ -160,7 +160,7 @@ constexpr int XROW_UNITS = GB * GSX + 1;
 constexpr int DROW_UNITS = GB * GSD + 1;
 constexpr int XDUMP = GB * GSX;
 constexpr int DDUMP = GB * GSD;
-constexpr int OSTRIDE = GB * 16 + 16;        // bytes per pixel in the dx output stage, two planes as well
+constexpr int OSTRIDE = stage_pitch(GB);     // bytes per pixel in the dx output stage, two planes as well
 constexpr int OPLANE = 16 * TPW * TS * OSTRIDE + 128;
 constexpr int OUT_ROW_BYTES = 2 * OPLANE;
 constexpr int X_CELLS = F * GB;

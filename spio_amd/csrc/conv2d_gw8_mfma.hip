@@ -145,7 +145,7 @@ SPIO_DEVICE constexpr int pos(int pixel) { return (pixel >> 1) + (pixel & 1) * P
 constexpr int NR = 2;                               // ring rows
 constexpr int RING_ROW_UNITS = GB * GS + 1;         // 16-byte units per ring row (+1: dump cell)
 constexpr int DUMP_UNIT = GB * GS;                  // where lanes without a cell write
-constexpr int OSTRIDE = GB * 16 + 16;               // bytes per pixel in the output stage
+constexpr int OSTRIDE = stage_pitch(GB);            // bytes per pixel in the output stage
 constexpr int OPLANE = 16 * TPW * TS * OSTRIDE + 128;  // even pixels, then odd ones, as in the ring
 constexpr int OUT_ROW_BYTES = 2 * OPLANE;
 constexpr int IN_CELLS = F * GB;

@@ -131,6 +131,13 @@ SPIO_DEVICE void store_stream(spio_uint4 v, spio_uint4* p) {
 #define SPIO_DST_F32 0
 #endif
 constexpr int kDstBytes = SPIO_DST_F32 ? 4 : 2;
+// Bytes from pixel to pixel where a finished row is staged in LDS, `groups` units of 16 bytes and a spare one, or two: an
+// odd number, so that the 8 bytes that 16 lanes store for as many pixels lie in different banks.  An even one folds them
+// onto those of 8, 4, 2 pixels or one, which all lanes of a wave run into since a tile is pairs of pixels and every lane converts.
+// With one spare unit -> odd: forward 32n 56c 112x112 (7 groups, a pitch of 128) 21.8 -> 15.6 us, 128n 24c 144x144 (3, 64)
+// 46.1 -> 45.0, in tiles of 24 whole rows 53.2 -> 48.1, 64n 40c 56x56 5x5 (5, 96) equal.
+constexpr int stage_pitch(int groups) { return 16 * (groups + 1 + groups % 2); }
+
 // A finished row leaves LDS as 16-byte units of 8 channels, one per lane, which widen to 32 bytes: two
 // stores.  In store j lane i of a wave writes half i % 2 of the unit of lane 32 j + i / 2, so that every
 // store covers whole lines (1024 consecutive bytes where the units are).  A lane that wrote its own two halves

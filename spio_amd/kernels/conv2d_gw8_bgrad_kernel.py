@@ -24,6 +24,7 @@ from .conv2d_gw8_kernel import (
     _shape_defines,
     fits_float32_output,
     lane_registers,
+    stage_pitch,
     with_joined_stores,
 )
 from .conv2d_gw8_params import Conv2dGw8Params
@@ -143,7 +144,7 @@ def bgrad_geometry(params: Conv2dGw8Params, config: Conv2dGw8BgradConfig) -> Dic
     threads = 64 * gb * ts
     # every ring row carries a spare unit behind its last group (see the kernel)
     ring_units = 2 * (gb * gsx + 1) + 2 * (gb * gsd + 1)
-    out_row_bytes = 2 * (16 * tpw * ts * (gb * 16 + 16) + 128)
+    out_row_bytes = 2 * (16 * tpw * ts * stage_pitch(gb) + 128)
     stream_bytes = ring_units * 16 + 2 * out_row_bytes
     filter_bytes = gb * 8 * r * s * 16
     publish_bytes = (gb * ts * r * s * 64 + (gb * ts * 8 if params.has_bias else 0)) * 4

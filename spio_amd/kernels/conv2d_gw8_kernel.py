@@ -105,6 +105,11 @@ def direction_geometry(params: Conv2dGw8Params, igrad: bool) -> Dict[str, int]:
                 EPY=params.padding_h, EPX=params.padding_w)  # fmt: skip
 
 
+def stage_pitch(groups: int) -> int:
+    """Bytes from pixel to pixel of a finished row in LDS: an odd number of 16-byte units (spio_conv_common.h)."""
+    return 16 * (groups + 1 + groups % 2)
+
+
 def mfma_geometry(params: Conv2dGw8Params, config: Conv2dGw8Config, igrad: bool) -> Dict[str, int]:
     """Host mirror of the compile-time constants of conv2d_gw8_mfma.hip."""
     d = direction_geometry(params, igrad)
@@ -121,7 +126,7 @@ def mfma_geometry(params: Conv2dGw8Params, config: Conv2dGw8Config, igrad: bool)
     plane = fp // 2 + (8 - fp // 2) % 16
     gs = plane + fp // 2 + (9 - (plane + fp // 2)) % 16
     threads = 64 * gb * ts
-    ostride = gb * 16 + 16
+    ostride = stage_pitch(gb)
     # ring rows (+ dump cell) and two output-stage rows
     lds = 2 * (gb * gs + 1) * 16 + 4 * (16 * tpw * ts * ostride + 128)
     if igrad:  # the data gradient stages its groups' filters in the same block first

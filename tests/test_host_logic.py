@@ -596,3 +596,28 @@ def test_capped_sweeps_try_every_number_of_groups_where_lines_are_shared(groups)
     assert even <= {cfg.groups for cfg in configs}
     assert {cfg.groups for cfg in configs} - {16} <= {cfg.groups for cfg in first}
     assert {cfg.groups for cfg in row_streaming(8 * 24)} <= {4, 8, 16, 24}
+
+
+
+@pytest.mark.parametrize("groups", [1, 2, 3, 4, 5, 7, 8, 11, 12, 15])
+def test_a_tile_stages_its_pixels_in_different_banks(groups):
+    """16 lanes store 8 bytes each for as many pixels of a finished row: their 16-byte columns of the 256 bytes that the
+    banks span are all different, in both kernels whose lanes all convert."""
+    params = Conv2dGw8Params(n=2, c=8 * groups, h=9, w=40)
+    for source, factory, config in (
+        ("conv2d_gw8_mfma.hip", conv2d_gw8_kernel_factory, Conv2dGw8Config(groups=groups, block_p=4, prefetch=2)),
+        ("conv2d_gw8_bgrad_mfma.hip", conv2d_gw8_bgrad_kernel_factory, Conv2dGw8BgradConfig(groups=groups, block_h=4, prefetch=2)),
+    ):
+        spec = factory.get_kernel_spec(params, config, ATTR)
+        pixels = """
+        constexpr bool distinct() {
+            bool taken[16] = {};
+            for (int i = 0; i < 16; ++i) {
+                if (taken[i * OSTRIDE / 16 % 16]) return false;
+                taken[i * OSTRIDE / 16 % 16] = true;
+            }
+            return OSTRIDE % 16 == 0 && OSTRIDE > GB * 16;
+        }
+        static_assert(distinct());
+        """ + f"static_assert(LDS_UNITS * 16 == {spec.notes['LDS_BYTES']});"
+        assert compile_hip(read_source(source) + pixels, source, headers=kernel_headers(), defines=dict(spec.defines, SPIO_KERNEL_NAME="k"))
