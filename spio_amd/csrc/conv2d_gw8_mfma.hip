@@ -480,10 +480,11 @@ SPIO_DEVICE void conv_rows(spio_uint4* __restrict__ dst, const spio_uint4* __res
     //      writes them ----
     {
         constexpr int SLACK = FP - F;
+        constexpr int PER_GROUP = SLACK > 0 ? SLACK : 1;  // (none behind rows of whole tiles under 3- and 7-wide filters)
         for (int i = tid; i < NR * GB * SLACK; i += THREADS) {
-            const int row = i / (GB * SLACK);
-            const int g = (i / SLACK) % GB;
-            ring[row * RING_ROW_UNITS + g * GS + pos(F + i % SLACK)] = spio_uint4{0u, 0u, 0u, 0u};
+            const int row = i / (GB * PER_GROUP);
+            const int g = i / PER_GROUP % GB;
+            ring[row * RING_ROW_UNITS + g * GS + pos(F + i % PER_GROUP)] = spio_uint4{0u, 0u, 0u, 0u};
         }
     }
 

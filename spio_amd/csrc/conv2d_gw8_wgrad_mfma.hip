@@ -554,7 +554,7 @@ SPIO_KERNEL_NAME(float* __restrict__ grad_weight, const spio_uint4* __restrict__
                     continue;
                 }
                 // PF is even, so the parity of the step is known at compile time: it fixes the
-                // x ring rows and, with one row per step, the parity of delta.
+                // x ring rows.
                 const int sp = (S0 + uf) & 1;
                 const int ta = (S0 + uf) * RB % NA;
                 const bool math = kFullUnroll || st < S1;

@@ -621,3 +621,16 @@ def test_a_tile_stages_its_pixels_in_different_banks(groups):
         static_assert(distinct());
         """ + f"static_assert(LDS_UNITS * 16 == {spec.notes['LDS_BYTES']});"
         assert compile_hip(read_source(source) + pixels, source, headers=kernel_headers(), defines=dict(spec.defines, SPIO_KERNEL_NAME="k"))
+
+
+
+@pytest.mark.parametrize("shape", ["3n_24c_9h_32w_1py_1px_3r_3s_nb", "2n_64c_9h_64w_3py_3px_7r_7s_b"])
+@pytest.mark.parametrize("igrad", [False, True])
+def test_rows_of_whole_tiles_have_no_slack_cells(shape, igrad):
+    """Where the pixels that fragment reads touch end with the row there is nothing behind it to zero, and nothing divides
+    by how many cells that is."""
+    params = Conv2dGw8Params.decode(shape)
+    spec = conv2d_gw8_kernel_factory.get_kernel_spec(params, Conv2dGw8Config(groups=3, block_p=4), ATTR, igrad=igrad)
+    source = read_source("conv2d_gw8_mfma.hip") + "static_assert(FP == F);"
+    assert compile_hip(source, "slack.hip", headers=kernel_headers(), defines=dict(spec.defines, SPIO_KERNEL_NAME="k"),
+                       extra_options=["-Werror=division-by-zero"])  # fmt: skip
