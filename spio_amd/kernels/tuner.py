@@ -41,11 +41,14 @@ from ..util.logger import logger_enabled
 
 _PACKAGE_RECORDS = os.path.join(os.path.dirname(os.path.abspath(__file__)), "tuned")
 
-# Rotate the timed launches over buffer sets totalling at least this many bytes
-# so that the sweep ranks configurations by their HBM behaviour, not by hits in
-# the 256 MB memory-side cache.
-ROTATION_BYTES = 600 * 1024 * 1024
-MAX_ROTATION_SETS = 8
+# The timed launches rotate over buffer sets of together four times the 256 MB memory-side cache, so that a sweep ranks
+# configurations by what they get from memory: blocks of half lines or stores past L2 can be the fastest while
+# everything is in that cache and are not from memory.  (With eight sets, 206 and 309 MB, the forward kernels of 32n 64c
+# 56x56 and 128n 384c 14x14 were chosen at 5.4 and 7.5 us, and took 7.4 and 12.7 from memory where other configurations take
+# 6.4 and 8.6.)  A single set of that size rotates by itself; of sets below 8 MB, whose kernels take little more than
+# a launch, there are not that many.
+ROTATION_BYTES = 4 * 256 * 1024 * 1024
+MAX_ROTATION_SETS = 128
 DEFAULT_ON_MISS_CONFIGS = 8
 FINALISTS = 6  # leaders of a sweep that are timed again before one is chosen
 
@@ -68,6 +71,11 @@ def _leading(configs, count: int) -> int:
                 return i
             count -= 1
     return len(configs)
+
+
+def _rotation_sets(set_bytes: int) -> int:
+    """Buffer sets of `set_bytes` that a sweep's launches rotate over."""
+    return max(1, min(MAX_ROTATION_SETS, -(-ROTATION_BYTES // max(set_bytes, 1))))
 
 
 def _stream_is_capturing() -> bool:
@@ -227,10 +235,13 @@ class Tuner:
         device = torch.device("cuda", ordinal)
         first = kernel_factory.make_test_args(params, device, **kernel_kwargs)
         set_bytes = sum(a.numel() * a.element_size() for a in first if hasattr(a, "numel"))
-        nsets = max(1, min(MAX_ROTATION_SETS, -(-ROTATION_BYTES // max(set_bytes, 1))))
-        arg_sets = [first] + [
-            kernel_factory.make_test_args(params, device, **kernel_kwargs) for _ in range(nsets - 1)
-        ]
+        arg_sets = [first]
+        for _ in range(_rotation_sets(set_bytes) - 1):
+            try:
+                arg_sets.append(kernel_factory.make_test_args(params, device, **kernel_kwargs))
+            except torch.OutOfMemoryError:  # what the program has left of the card has to do
+                break
+        iters = max(iters, len(arg_sets))  # each timing comes by every set, or the next one finds them where it left them
         results = []
         timed = []
         for kernel in kernels:

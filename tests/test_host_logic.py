@@ -634,3 +634,17 @@ def test_rows_of_whole_tiles_have_no_slack_cells(shape, igrad):
     source = read_source("conv2d_gw8_mfma.hip") + "static_assert(FP == F);"
     assert compile_hip(source, "slack.hip", headers=kernel_headers(), defines=dict(spec.defines, SPIO_KERNEL_NAME="k"),
                        extra_options=["-Werror=division-by-zero"])  # fmt: skip
+
+
+
+@pytest.mark.parametrize("megabytes", [0.1, 4, 8, 13, 25.7, 38.6, 77, 150, 500, 1023, 1024, 20000])
+def test_sweeps_time_from_memory(megabytes):
+    """Launches rotate over four times the memory-side cache, whatever the size of a set (very small ones excepted), and
+    over no more than one set beyond that."""
+    from spio_amd.kernels.tuner import _rotation_sets
+
+    size, cache = int(megabytes * 2**20), 256 * 2**20
+    sets = _rotation_sets(size)
+    assert 1 <= sets <= 128
+    assert sets * size >= 4 * cache or sets == 128 and megabytes < 8
+    assert (sets - 1) * size < 4 * cache
