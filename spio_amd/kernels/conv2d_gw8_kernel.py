@@ -152,8 +152,9 @@ def lane_registers(waves: int) -> int:
 
 def _mfma_fits(params, config, igrad) -> bool:
     """Whether a lane's registers hold what the row-streaming kernel keeps in them, or all but a few: filter fragments,
-    accumulators and rows in flight.  The weights were fitted to what the compiler reports for 1771 kernels of 110
-    shapes, 1x1 to 7x7: of 100 that used memory 5 pass, with 100 bytes at most, of 1671 others 2 do not."""
+    accumulators and rows in flight.  Against what the compiler reports for 5370 kernels of 207 shapes, 1x1 to 7x7: of
+    318 that used memory 13 pass, 12 of them with 76 bytes or less, of 5052 others 124 do not.  (Fitted again, with terms for
+    a step's operands and for addresses, 12 and 95.)"""
     g = mfma_geometry(params, config, igrad)
     fragments, accumulators = 4 * params.r * g["KB"], 4 * g["TPW"] * params.r
     rows = 4 * min(config.prefetch, g["STEPS"]) * g["LPT"]
@@ -462,12 +463,15 @@ def _get_configs(params: Conv2dGw8Params, device_attr=None, igrad: bool = False)
     rank = {cfg: i for i, (_, cfg) in enumerate(found)}
     if G % 8:
         # Which number of groups is best depends on how lines are shared, which the score does not see: the best geometry
-        # of each first (of 16 no more than the others: it was the best of none).  First use of 8, before -> after:
+        # of each whose registers fit first (of 16 no more than the others: it was the best of none).  First use of 8, before -> after:
         # 59n 456c 60x60 110 -> 88 us, 64n 144c 56x56 36.5 -> 28.2, 50n 152c 41x41 16.5 -> 13.1, 60n 200c 33x33 17.2 -> 14.7,
         # 7n 168c 159x159 33.2 -> 30.0, 4n 424c 84x84 5x5 20.7 -> 16.7, 2n 600c 147x147 7x7 47 -> 38; 8n 88c 61x40, 48c
         # 224x224, 648c 56x97 5x5 equal.
+        # (A number of groups whose registers do not fit gives nothing there, and is left where the order above puts it: with
+        # its best first 4n 424c 84x84 5x5 17.3, without 17.1, 2n 600c 147x147 7x7 32.7 and 32.3, 60n 216c 56x56 7x7 53.8 and 54.2.)
         tried = dict.fromkeys(cfg.groups for _, cfg in found if cfg.groups in even_blocks or cfg.groups != 16)
-        leaders = [next(cfg for _, cfg in found if cfg.groups == g) for g in tried]
+        leaders = [next((cfg for _, cfg in found if cfg.groups == g and _mfma_fits(params, cfg, igrad)), None) for g in tried]
+        leaders = [cfg for cfg in leaders if cfg]
         head = leaders + [cfg for cfg in head if cfg not in leaders]
         rest = [cfg for cfg in rest if cfg not in leaders]
     configs = [*head[:8], *sorted(head[8:] + rest, key=rank.get)][:MAX_GEOMETRIES]

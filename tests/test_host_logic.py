@@ -648,3 +648,21 @@ def test_sweeps_time_from_memory(megabytes):
     assert 1 <= sets <= 128
     assert sets * size >= 4 * cache or sets == 128 and megabytes < 8
     assert (sets - 1) * size < 4 * cache
+
+
+
+@pytest.mark.parametrize("igrad", [False, True])
+@pytest.mark.parametrize("filter_size", [3, 5, 7])
+@pytest.mark.parametrize("n,c,hw", [(60, 216, 56), (16, 72, 112), (4, 424, 84), (16, 200, 33), (64, 104, 28), (8, 600, 49)])
+def test_capped_sweeps_leave_out_what_keeps_registers_in_memory(n, c, hw, filter_size, igrad):
+    """Also where the best geometry of every number of groups comes first: a number of groups whose registers do not fit
+    has none there."""
+    from spio_amd.kernels.conv2d_gw8_kernel import _mfma_fits
+    from spio_amd.kernels.tuner import _leading
+
+    params = Conv2dGw8Params(n=n, c=c, h=hw, w=hw, r=filter_size, s=filter_size, padding=filter_size // 2)
+    configs = list(conv2d_gw8_kernel_factory.configs(params, DeviceAttributes(), igrad=igrad))
+    rows = [cfg for cfg in configs if cfg.variant == "mfma"]
+    assert len({replace(cfg, prefetch=0) for cfg in rows if _mfma_fits(params, cfg, igrad)}) >= 8
+    first = configs[:_leading(configs, 8)]
+    assert all(_mfma_fits(params, cfg, igrad) for cfg in first if cfg.variant == "mfma")
