@@ -61,7 +61,7 @@ def fused_backward_kernel(params: Conv2dGw8Params, device):
         if mode not in ("1", "true", "on", "yes"):
             # the separate kernels, tuned or looked up the same way, for the comparison
             conv2d_gw8_kernel_factory.get_kernel(params, device, igrad=True)
-            conv2d_gw8_wgrad_kernel_factory.get_kernel(params, device)
+            wgrad = conv2d_gw8_wgrad_kernel_factory.get_kernel(params, device)
             times = [
                 (tuner.lookup(attr, f.get_full_kernel_name(params, **kw)) or {}).get("us")
                 for f, kw in ((conv2d_gw8_bgrad_kernel_factory, {}),
@@ -72,8 +72,11 @@ def fused_backward_kernel(params: Conv2dGw8Params, device):
                 # one launch instead of two: the second launch costs about what an empty kernel
                 # does in a back-to-back stream (measured at N=32, C=64, 56x56: the step with the
                 # fused kernel takes 25.6 us, with the two separate ones, whose times add up to
-                # 0.5 us less, 30.3 us)
-                if times[0] >= times[1] + times[2] + LAUNCH_GAP_US:
+                # 0.5 us less, 30.3 us).  A kernel whose sums are added into cleared tensors has a launch before it that its
+                # time does not hold; one of two stages, which are both in it, has none.  (128n 1392c 9x9 5x5: 43.7
+                # fused against 19.3 and, in two stages, 22.6; as they run for float16 weights 48.5 and 39 us.)
+                clears = [0 if k.kernel_spec.overwrites_output else LAUNCH_GAP_US for k in (fused, wgrad)]
+                if times[0] + clears[0] >= times[1] + times[2] + clears[1] + LAUNCH_GAP_US:
                     fused = None
             elif fused.kernel_spec.launch_params.grid[0] < 0.75 * attr.multiprocessor_count:
                 fused = None  # no measurements: too few workgroups to fill the device

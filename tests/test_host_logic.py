@@ -666,3 +666,40 @@ def test_capped_sweeps_leave_out_what_keeps_registers_in_memory(n, c, hw, filter
     assert len({replace(cfg, prefetch=0) for cfg in rows if _mfma_fits(params, cfg, igrad)}) >= 8
     first = configs[:_leading(configs, 8)]
     assert all(_mfma_fits(params, cfg, igrad) for cfg in first if cfg.variant == "mfma")
+
+
+
+@pytest.mark.parametrize("two_stage,fused", [((False, False), True), ((False, True), False), ((True, True), True), ((True, False), True)])
+def test_the_launch_that_clears_the_sums_counts_in_the_choice_of_backward_kernels(two_stage, fused, monkeypatch):
+    """Recorded times hold both stages of a kernel that stores its sums, and not the launch before one that adds them."""
+    import types
+
+    import torch
+
+    from spio_amd.functional import conv2d_gw8_function as op
+
+    times = {"bgrad": 43.7, "dgrad": 19.3, "wgrad": 22.6}  # less than 2.2 us apart with the launch between the two
+
+    class Factory:
+        def __init__(self, name, overwrites=False):
+            self.name, self.overwrites = name, overwrites
+
+        def configs(self, *_args):
+            return [None]
+
+        def get_kernel(self, *_args, **_kw):
+            return types.SimpleNamespace(kernel_spec=types.SimpleNamespace(overwrites_output=self.overwrites), name=self.name)
+
+        def get_full_kernel_name(self, _params, **_kw):
+            return self.name
+
+    monkeypatch.setenv("SPIO_FUSED_BACKWARD", "auto")
+    monkeypatch.setattr(op, "get_device_attributes", lambda _ordinal: ATTR)
+    monkeypatch.setattr(op, "conv2d_gw8_bgrad_kernel_factory", Factory("bgrad", two_stage[0]))
+    monkeypatch.setattr(op, "conv2d_gw8_kernel_factory", Factory("dgrad"))
+    monkeypatch.setattr(op, "conv2d_gw8_wgrad_kernel_factory", Factory("wgrad", two_stage[1]))
+    monkeypatch.setattr(op.tuner, "lookup", lambda _attr, name: {"us": times[name]})
+    monkeypatch.setattr(op, "_fused_choice", {})
+    params = Conv2dGw8Params(n=128, c=1392, h=9, w=9, r=5, s=5, padding=2)
+    chosen = op.fused_backward_kernel(params, torch.device("cuda", 0))
+    assert (chosen is not None) == fused
