@@ -259,18 +259,22 @@ class Tuner:
             raise ValueError(f"every configuration of {name} failed: {results}")
         timed.sort(key=lambda mk: mk[0])
         # The first pass is short; candidates within a few per cent of each other are ranked by
-        # noise.  Time the leaders again, longer and several times, and order them by the median.
+        # noise.  Time the leaders again, longer and several times, and order them by the median.  In turn: the first
+        # tens of milliseconds after a pause read up to 5 % slow, which one after the other the leader would bear alone.
         finalists = [mk for mk in timed[:FINALISTS] if mk[0] <= 1.15 * timed[0][0]]
         if len(finalists) > 1:
-            refined = []
-            for _, kernel in finalists:
+            leaders = [kernel for _, kernel in finalists]
+            for kernel in leaders:
                 kernel.load(device_ordinal=ordinal, clear_code=False)
-                runs = sorted(kernel.time(arg_sets, warmup=2, iters=max(iters, 30)) for _ in range(5))
+            rounds = [[kernel.time(arg_sets, warmup=2, iters=max(iters, 30)) for kernel in leaders] for _ in range(6)][1:]
+            refined = []
+            for i, kernel in enumerate(leaders):
                 kernel.unload()
-                refined.append((runs[2], kernel))
+                median = sorted(times[i] for times in rounds)[2]
+                refined.append((median, kernel))
                 for r in results:
                     if r.get("config") == config_to_dict(kernel.config) and "us" in r:
-                        r["us"] = runs[2] * 1e3
+                        r["us"] = median * 1e3
             refined.sort(key=lambda mk: mk[0])
             timed = refined + timed[len(finalists):]
         best = self._first_valid(kernel_factory, params, timed, first, ordinal, results)
