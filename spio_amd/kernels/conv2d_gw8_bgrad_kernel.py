@@ -60,7 +60,7 @@ class Conv2dGw8BgradConfig:
         block_n_iters: image blocks a workgroup processes before it publishes grad_weight.
         prefetch: rows of global loads in flight ahead of the computed row (even).
         split: waves per group; they share the 32-pixel chunks (weight gradient) and the
-            16-pixel tiles (data gradient) of a row.
+            32-pixel tiles (data gradient) of a row.
         halo_cached: 1 = rows shared with the neighbouring row blocks are loaded with the default
             cache policy (the second reader can hit in L2), the others with the non-temporal hint.
         xcd_chunk: consecutive tiles that go to the same XCD before the next run goes to the next
@@ -70,7 +70,7 @@ class Conv2dGw8BgradConfig:
             which then need no zero fill; 0 = workgroups add into zeroed tensors with fp32
             atomics.  Atomic additions of different workgroups to one line retire one after the
             other, and in a one-round grid all workgroups publish at the same time.
-        block_q: columns per workgroup (0: the whole width; else a multiple of 32 with
+        block_q: columns per workgroup (0: the whole width; else a multiple of 32, or one less, with
             block_n = 1).  The workgroup stages block_q + S - 1 columns of x and of grad_output, so
             rows of any width fit.
         nontemporal: 1 = store grad_input with the non-temporal hint.
@@ -180,7 +180,7 @@ def _config_is_legal(params, config) -> bool:
         and config.split <= min(g["KC"], g["WT"])
         and 0 <= config.block_h <= bgrad_domain(params)[0]
         and 0 <= config.block_q <= bgrad_domain(params)[1]
-        and (config.block_q == 0 or (config.block_q % 32 == 0 and config.block_n == 1))
+        and (config.block_q == 0 or (config.block_q % 32 in (0, 31) and config.block_n == 1))
         and g["LPTD"] <= MAX_LOADS_PER_THREAD
         and config.block_n <= max(params.n, 1) and config.block_n * (config.block_n_iters - 1) < max(params.n, 1)
         and g["LDS_BYTES"] <= MAX_LDS_BYTES
@@ -221,6 +221,7 @@ def _score(params, config, num_cus) -> float:
     group_eff = params.groups / (g["GBLKS"] * config.groups)
     quant = divup(g["NUM_BLOCKS"], num_cus) * num_cus / g["NUM_BLOCKS"]
     quant *= g["PBLKS"] * g["BH"] / bgrad_domain(params)[0]  # the last, shorter tiles
+    quant *= g["QBLKS"] * g["BQ"] / bgrad_domain(params)[1]
     quant *= g["NBLKS"] * config.block_n * config.block_n_iters / params.n
     halo = 1.0 + (2.0 / 3.0) * (params.r - 1 if g["PBLKS"] > 1 else 0) / g["BH"]
     dh, dw = bgrad_domain(params)
@@ -255,8 +256,11 @@ def _get_configs(params: Conv2dGw8Params, device_attr=None) -> List[Conv2dGw8Bgr
     if wpi < 32:
         best = max(chunk_fill(nb) for nb in image_counts)
         image_counts += [nb for nb in (3, 5, 6, 7) if chunk_fill(nb) > best + 0.05]
-    # column blocks for wide rows only: narrower ones fit whole
-    col_choices = [0] + [bq for bq in (64, 128) if dw >= 2 * bq and dw > 128]
+    # Column blocks for wide rows only: narrower ones fit whole.  A chunk of the weight gradient begins a pixel before the
+    # block, so 64 columns take three and 63 two.  Which is better depends on the shape, best of 24 configurations with 64 and
+    # 63: 4n 96c 100x300 5x5 43.8 and 31.6 us, 32n 64c 224x224 116.6 and 115.3, 8n 64c 64x1024 42.1 and 41.5, but 16n 64c
+    # 128x512 76.9 and 78.8, 8n 24c 144x256 20.1 and 21.0 (127 columns are no better than 128 anywhere).
+    col_choices = [0] + [bq for bq in (63, 64, 128) if dw >= 2 * bq and dw > 128]
     configs = []
     for bh in row_choices:
         geometries = []

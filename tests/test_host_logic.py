@@ -82,6 +82,7 @@ def test_model_shapes_and_wide_rows_get_mfma_kernels(capsys):
     MFMA configuration in every family, the fused backward kernel included for 3x3 and 5x5
     filters; a request that has only the any-shape kernel says so on first use."""
     from helpers import GOLDEN
+    from spio_amd.kernels.conv2d_gw8_bgrad_kernel import bgrad_geometry
 
     with open(os.path.join(GOLDEN, "conv2d_gw8_model_shapes.json"), encoding="utf-8") as f:
         rows = json.load(f)
@@ -100,7 +101,10 @@ def test_model_shapes_and_wide_rows_get_mfma_kernels(capsys):
     for params in wide:
         if params.r <= 5:
             configs = list(conv2d_gw8_bgrad_kernel_factory.configs(params, ATTR))
-            assert configs and all(c.block_q % 32 == 0 for c in configs), f"fused backward: none for {params.encode()}"
+            assert configs and all(c.block_q % 32 in (0, 31) for c in configs), f"fused backward: none for {params.encode()}"
+            # among the first are column blocks that take the weight gradient no more chunks than the data gradient tiles
+            g = [bgrad_geometry(params, c) for c in configs[:8] if c.block_q]
+            assert any(x["KC"] <= x["WT"] for x in g), f"fused backward: a chunk more than tiles for {params.encode()}"
             if params.w >= 512:
                 assert all(c.block_q > 0 for c in configs)
 
@@ -703,7 +707,6 @@ def test_the_launch_that_clears_the_sums_counts_in_the_choice_of_backward_kernel
     params = Conv2dGw8Params(n=128, c=1392, h=9, w=9, r=5, s=5, padding=2)
     chosen = op.fused_backward_kernel(params, torch.device("cuda", 0))
     assert (chosen is not None) == fused
-
 
 
 def test_finalists_of_a_sweep_are_timed_in_turn(tmp_path, monkeypatch):

@@ -94,3 +94,17 @@ def test_forward_and_data_gradient(shape, igrad):
         run_grad_kernel_test(conv2d_gw8_kernel_factory, params, configs=configs, igrad=True)
     else:
         run_kernel_test(conv2d_gw8_kernel_factory, params, configs=configs)
+
+
+@pytest.mark.parametrize("shape", [(2, 24, 7, 140, 3, 3, 1, True), (1, 16, 9, 95, 5, 5, 2, False), (2, 8, 6, 63, 2, 4, 1, True)], ids=str)
+def test_fused_backward_in_column_blocks_of_whole_chunks(shape):
+    """Column blocks one short of 32-pixel tiles, whose chunks begin a pixel before the block; the last block is
+    narrower, or a whole one."""
+    params = _params(shape)
+    B = Conv2dGw8BgradConfig
+    configs = [
+        B(groups=2 if params.groups > 1 else 1, block_h=3, block_q=31, prefetch=2),
+        B(groups=1, block_q=63, prefetch=4, split=2, two_stage=1),
+        B(groups=params.groups, block_h=4, block_q=63, block_n_iters=params.n, prefetch=2),
+    ]
+    run_bgrad_kernel_test(conv2d_gw8_bgrad_kernel_factory, params, configs=configs)
