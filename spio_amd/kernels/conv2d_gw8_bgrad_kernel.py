@@ -261,7 +261,7 @@ def _get_configs(params: Conv2dGw8Params, device_attr=None) -> List[Conv2dGw8Bgr
     # 63: 4n 96c 100x300 5x5 43.8 and 31.6 us, 32n 64c 224x224 116.6 and 115.3, 8n 64c 64x1024 42.1 and 41.5, but 16n 64c
     # 128x512 76.9 and 78.8, 8n 24c 144x256 20.1 and 21.0 (127 columns are no better than 128 anywhere).
     col_choices = [0] + [bq for bq in (63, 64, 128) if dw >= 2 * bq and dw > 128]
-    configs = []
+    configs, of_each = [], []
     for bh in row_choices:
         geometries = []
         for bq in col_choices:
@@ -279,6 +279,10 @@ def _get_configs(params: Conv2dGw8Params, device_attr=None) -> List[Conv2dGw8Bgr
         # the best, and as many of those that fit the registers
         fitting = [cfg for cfg in ranked if _fits(params, cfg)][:GEOMETRIES_PER_HEIGHT]
         configs += ranked[:GEOMETRIES_PER_HEIGHT] + [cfg for cfg in fitting if cfg not in ranked[:GEOMETRIES_PER_HEIGHT]]
+        of_each += [cfg for gb in group_choices for cfg in [c for c in ranked if c.groups == gb and _fits(params, c)][:2]]
+    # ... and, where a sweep has time for them, two of every number of groups: the score has many ties, which one number
+    # can fill (128n 384c 14x14 from memory: 8 groups in blocks of four images 15.0 us, the best of the others 17.0)
+    configs += [cfg for cfg in of_each if cfg not in configs]
     # what keeps much of its registers in memory comes last
     configs.sort(key=lambda cfg: not _fits(params, cfg))
     # a shallower and a deeper pipeline for the first few: the shallow one wins where rows are short
