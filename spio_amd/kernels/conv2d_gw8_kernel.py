@@ -132,7 +132,7 @@ def mfma_geometry(params: Conv2dGw8Params, config: Conv2dGw8Config, igrad: bool)
     if igrad:  # the data gradient stages its groups' filters in the same block first
         lds = max(lds, gb * 8 * r * s * 16)
     d.update(
-        KB=kb, WPI=wpi, F=f, WT=2 * tiles, TPW=tpw, GS=gs,
+        KB=kb, WPI=wpi, F=f, WT=2 * tiles, TPW=tpw, GS=gs,  # WT in 16 pixels, as the image kernel's; the kernel's own is tiles
         THREADS=threads, LDS_BYTES=lds, LPT=divup(f * gb, threads),
         SPT=divup(nb * bq * gb, threads), BQ=bq, QBLKS=divup(d["DW"], bq),
         GBLKS=divup(params.groups, gb), NBLKS=divup(params.n, nb),
@@ -424,8 +424,8 @@ def _get_configs(params: Conv2dGw8Params, device_attr=None, igrad: bool = False)
     d = direction_geometry(params, igrad)
     num_cus = getattr(device_attr, "multiprocessor_count", 256) or 256
     G = params.groups
-    # Where a pixel is not whole lines also the smallest blocks of one size that make up three or four lines: fewer
-    # boundaries lie inside lines, and the last block is not nearly empty.
+    # Where a pixel is not whole lines also the groups in the fewest blocks of 12 or of 16 at most (one and a half lines
+    # of 128 bytes, or two), all of one size: fewer boundaries lie inside lines, and the last block is not nearly empty.
     even_blocks = {divup(G, divup(G, most)) for most in (12, 16)} if G % 8 else set()
     group_choices = sorted({g for g in {4, 8, 16, G} | even_blocks if g <= min(G, MAX_WAVES)}) or [min(G, MAX_WAVES)]
     row_choices = balanced(d["DH"], (2, 4, 7, 8, 14, 16, 28, 32, 56, d["DH"]))
@@ -438,7 +438,7 @@ def _get_configs(params: Conv2dGw8Params, device_attr=None, igrad: bool = False)
             for nb in (1, 2, 4, 8) if bq == 0 else (1,):
                 for ts in (1, 2, 4):
                     if nb * ((bq or d["DW"]) + params.s - 1) - params.s + 1 <= 32 * (ts // 2):
-                        continue  # a wave without a tile
+                        continue  # half of the waves or more without a tile (one of four may be: 3 tiles, 1 a wave)
                     for bp in row_choices:
                         steps = bp + params.r - 1
                         for pf in PREFETCH_CHOICES:

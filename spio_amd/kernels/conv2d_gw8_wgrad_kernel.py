@@ -48,8 +48,8 @@ class Conv2dGw8WgradConfig:
         chunks: (direct variant only) pixel chunks per group.
         prefetch: steps of global loads in flight ahead of the computed step (even).
         rows: rows of x (and of grad_output) a workgroup multiplies between two barriers,
-            1 or 2; two rows share their grad_output fragments and halve the barriers at the
-            price of a deeper LDS ring.
+            1 or 2; two rows halve the barriers at the price of a deeper LDS ring (grad_output
+            fragments stay in registers across rows with either).
         split: waves sharing the 32-pixel chunks of one group; their sums are added in LDS
             before publishing, so bigger workgroups do not publish more.
         two_stage: 1 = workgroups store partial sums to a workspace and a second kernel
