@@ -43,7 +43,7 @@ MAX_REGISTERS = 256  # estimated fragments + accumulators + prefetch buffers, in
 # Accumulators of the weight gradient.  The 14 of a 7x7 filter fit, but one pass is mostly slower there than two kernels, which
 # the arithmetic bounds.  Fused against data and weight gradient and the 2.2 us of a launch, best of 16 each: 256n 256c 14x14
 # 55.4 and 39.8 us, 64n 96c 56x56 59.4 and 52.4, 128n 192c 28x28 54.7 and 55.2, 32n 128c 56x56 36.0 and 40.9; 16n 64c 112x112
-# has no configuration that fits.
+# has none of whole rows.
 MAX_SUMS = 14
 GEOMETRIES_PER_HEIGHT = 6
 MAX_UNROLLED_STEPS = 40  # SPIO_MAX_UNROLL of the kernel: longer step loops run in chunks
