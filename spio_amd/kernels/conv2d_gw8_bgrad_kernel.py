@@ -72,10 +72,13 @@ class Conv2dGw8BgradConfig:
             which then need no zero fill; 0 = workgroups add into zeroed tensors with fp32
             atomics.  Atomic additions of different workgroups to one line retire one after the
             other, and in a one-round grid all workgroups publish at the same time.
-        block_q: columns per workgroup (0: the whole width; else a multiple of 32, or one less, with
+        block_q: columns per workgroup (0: the whole width; else a multiple of 32 with
             block_n = 1).  The workgroup stages block_q + S - 1 columns of x and of grad_output, so
             rows of any width fit.
         nontemporal: 1 = store grad_input with the non-temporal hint.
+        narrow: 1 = a workgroup has one column less than block_q.  The weight gradient's 32-pixel
+            chunks begin a pixel before the block, so block_q columns take one more of them than
+            block_q / 32 and block_q - 1 do not.
     """
 
     groups: int = 4
@@ -89,6 +92,7 @@ class Conv2dGw8BgradConfig:
     block_q: int = 0
     two_stage: int = 0
     nontemporal: int = 1
+    narrow: int = 0
 
 
 def bgrad_is_supported(params: Conv2dGw8Params) -> bool:
@@ -125,7 +129,7 @@ def bgrad_geometry(params: Conv2dGw8Params, config: Conv2dGw8BgradConfig) -> Dic
     pb, pr = r - 1 - r // 2, s - 1 - s // 2  # the domain's padding below and right
     bh = config.block_h or dh
     nb4 = divup(s, 4)
-    bq = config.block_q or dw
+    bq = config.block_q - config.narrow if config.block_q else dw
     wpi = bq + s - 1
     f = nb * wpi
     kspan = (nb - 1) * wpi + bq
@@ -181,8 +185,9 @@ def _config_is_legal(params, config) -> bool:
         config.groups * config.split <= MAX_WAVES
         and config.split <= min(g["KC"], g["WT"])
         and 0 <= config.block_h <= bgrad_domain(params)[0]
-        and 0 <= config.block_q <= bgrad_domain(params)[1]
-        and (config.block_q == 0 or (config.block_q % 32 in (0, 31) and config.block_n == 1))
+        and 0 <= config.block_q <= bgrad_domain(params)[1] + config.narrow
+        and (config.block_q == 0 or (config.block_q % 32 == 0 and config.block_n == 1))
+        and 0 <= config.narrow <= min(config.block_q, 1)
         and g["LPTD"] <= MAX_LOADS_PER_THREAD
         and config.block_n <= max(params.n, 1) and config.block_n * (config.block_n_iters - 1) < max(params.n, 1)
         and g["LDS_BYTES"] <= MAX_LDS_BYTES
@@ -262,18 +267,18 @@ def _get_configs(params: Conv2dGw8Params, device_attr=None) -> List[Conv2dGw8Bgr
     # block, so 64 columns take three and 63 two.  Which is better depends on the shape, best of 24 configurations with 64 and
     # 63: 4n 96c 100x300 5x5 43.8 and 31.6 us, 32n 64c 224x224 116.6 and 115.3, 8n 64c 64x1024 42.1 and 41.5, but 16n 64c
     # 128x512 76.9 and 78.8, 8n 24c 144x256 20.1 and 21.0 (127 columns are no better than 128 anywhere).
-    col_choices = [0] + [bq for bq in (63, 64, 128) if dw >= 2 * bq and dw > 128]
+    col_choices = [(0, 0)] + [(bq, less) for bq, less in ((64, 1), (64, 0), (128, 0)) if dw >= 2 * (bq - less) and dw > 128]
     configs, of_each = [], []
     for bh in row_choices:
         geometries = []
-        for bq in col_choices:
+        for bq, less in col_choices:
             for gb in group_choices:
                 for nb in image_counts if bq == 0 else (1,):
                     tiles = divup(G, gb) * divup(dh, bh or dh) * divup(dw, bq or dw)
                     for iters in image_block_runs(divup(params.n, nb), tiles, num_cus, (1, 2, 4)):
                         for ts in (1, 2):
                             cfg = Conv2dGw8BgradConfig(groups=gb, block_h=bh, block_n=nb, block_n_iters=iters,
-                                                       prefetch=4, split=ts, block_q=bq)  # fmt: skip
+                                                       prefetch=4, split=ts, block_q=bq, narrow=less)  # fmt: skip
                             if _config_is_legal(params, cfg):
                                 geometries.append((_score(params, cfg, num_cus), cfg))
         geometries.sort(key=lambda sc: sc[0])
@@ -336,7 +341,7 @@ def _get_kernel_spec(params: Conv2dGw8Params, config: Conv2dGw8BgradConfig, _dev
                    SPIO_HALO_CACHED=config.halo_cached, SPIO_XCD_CHUNK=config.xcd_chunk,
                    SPIO_NT=config.nontemporal, SPIO_HAS_BIAS=int(params.has_bias))  # fmt: skip
     if config.block_q:
-        defines["SPIO_BQ"] = config.block_q
+        defines["SPIO_BQ"] = config.block_q - config.narrow
     spec = KernelSpec(defines, LaunchParams(grid=g["NUM_BLOCKS"], block=g["THREADS"]), SOURCE, notes=g)
     if config.two_stage:
         # one block per workgroup: its groups' grad_weight values, then its 8 bias sums per group

@@ -82,7 +82,6 @@ def test_model_shapes_and_wide_rows_get_mfma_kernels(capsys):
     MFMA configuration in every family, the fused backward kernel included for 3x3 and 5x5
     filters; a request that has only the any-shape kernel says so on first use."""
     from helpers import GOLDEN
-    from spio_amd.kernels.conv2d_gw8_bgrad_kernel import bgrad_geometry
 
     with open(os.path.join(GOLDEN, "conv2d_gw8_model_shapes.json"), encoding="utf-8") as f:
         rows = json.load(f)
@@ -101,10 +100,7 @@ def test_model_shapes_and_wide_rows_get_mfma_kernels(capsys):
     for params in wide:
         if params.r <= 5:
             configs = list(conv2d_gw8_bgrad_kernel_factory.configs(params, ATTR))
-            assert configs and all(c.block_q % 32 in (0, 31) for c in configs), f"fused backward: none for {params.encode()}"
-            # among the first are column blocks that take the weight gradient no more chunks than the data gradient tiles
-            g = [bgrad_geometry(params, c) for c in configs[:8] if c.block_q]
-            assert any(x["KC"] <= x["WT"] for x in g), f"fused backward: a chunk more than tiles for {params.encode()}"
+            assert configs and all(c.block_q % 32 == 0 for c in configs), f"fused backward: none for {params.encode()}"
             if params.w >= 512:
                 assert all(c.block_q > 0 for c in configs)
 
@@ -741,3 +737,21 @@ def test_finalists_of_a_sweep_are_timed_in_turn(tmp_path, monkeypatch):
     record = str(tmp_path / "db.json")
     best = Tuner().sweep(factory, None, 0, ATTR, configs=[k.config for k in kernels], record_path=record)
     assert best.config.groups == 4 and json.load(open(record))["k__x"]["us"] == pytest.approx(10.0)
+
+
+@pytest.mark.parametrize("n,c,h,w,filter_size", [(32, 64, 224, 224, 3), (16, 64, 128, 512, 3), (8, 64, 64, 1024, 3), (4, 96, 100, 300, 5)])
+def test_wide_rows_get_column_blocks_of_whole_chunks(n, c, h, w, filter_size):
+    """Among the first configurations are column blocks that take the weight gradient no more 32-pixel chunks than the data
+    gradient 32-pixel tiles; a block is one column narrower only where rows are split."""
+    from spio_amd.kernels.conv2d_gw8_bgrad_kernel import bgrad_geometry
+
+    params = Conv2dGw8Params(n=n, c=c, h=h, w=w, r=filter_size, s=filter_size, padding=filter_size // 2)
+    first = list(conv2d_gw8_bgrad_kernel_factory.configs(params, ATTR))[:8]
+    geometries = [bgrad_geometry(params, cfg) for cfg in first if cfg.block_q]
+    assert any(g["KC"] <= g["WT"] for g in geometries)
+    narrow = next(cfg for cfg in first if cfg.narrow)
+    g = bgrad_geometry(params, narrow)
+    assert g["BQ"] == narrow.block_q - 1 and g["QBLKS"] * g["BQ"] >= w > (g["QBLKS"] - 1) * g["BQ"]
+    assert conv2d_gw8_bgrad_kernel_factory.get_kernel_spec(params, narrow, ATTR).defines["SPIO_BQ"] == g["BQ"]
+    for other in (replace(narrow, block_q=0), replace(narrow, narrow=2), replace(narrow, narrow=-1)):
+        assert not conv2d_gw8_bgrad_kernel_factory.is_legal(params, other)

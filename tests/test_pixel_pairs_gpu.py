@@ -103,8 +103,8 @@ def test_fused_backward_in_column_blocks_of_whole_chunks(shape):
     params = _params(shape)
     B = Conv2dGw8BgradConfig
     configs = [
-        B(groups=2 if params.groups > 1 else 1, block_h=3, block_q=31, prefetch=2),
-        B(groups=1, block_q=63, prefetch=4, split=2, two_stage=1),
-        B(groups=params.groups, block_h=4, block_q=63, block_n_iters=params.n, prefetch=2),
+        B(groups=2 if params.groups > 1 else 1, block_h=3, block_q=32, narrow=1, prefetch=2),
+        B(groups=1, block_q=64, narrow=1, prefetch=4, split=2, two_stage=1),
+        B(groups=params.groups, block_h=4, block_q=64, narrow=1, block_n_iters=params.n, prefetch=2),
     ]
     run_bgrad_kernel_test(conv2d_gw8_bgrad_kernel_factory, params, configs=configs)
