@@ -239,7 +239,8 @@ class Tuner:
         for _ in range(_rotation_sets(set_bytes) - 1):
             try:
                 arg_sets.append(kernel_factory.make_test_args(params, device, **kernel_kwargs))
-            except torch.OutOfMemoryError:  # what the program has left of the card has to do
+            except torch.OutOfMemoryError:  # what the program has left of the card has to do, half of it for
+                del arg_sets[max(1, len(arg_sets) // 2):]  # workspaces and code objects
                 break
         iters = max(iters, len(arg_sets))  # each timing comes by every set, or the next one finds them where it left them
         results = []
@@ -277,6 +278,7 @@ class Tuner:
                         r["us"] = median * 1e3
             refined.sort(key=lambda mk: mk[0])
             timed = refined + timed[len(finalists):]
+        del arg_sets[1:]  # the check takes copies of the first
         best = self._first_valid(kernel_factory, params, timed, first, ordinal, results)
         del arg_sets, first
         for _, kernel in timed:

@@ -755,3 +755,54 @@ def test_wide_rows_get_column_blocks_of_whole_chunks(n, c, h, w, filter_size):
     assert conv2d_gw8_bgrad_kernel_factory.get_kernel_spec(params, narrow, ATTR).defines["SPIO_BQ"] == g["BQ"]
     for other in (replace(narrow, block_q=0), replace(narrow, narrow=2), replace(narrow, narrow=-1)):
         assert not conv2d_gw8_bgrad_kernel_factory.is_legal(params, other)
+
+
+@pytest.mark.parametrize("fitting", [1, 2, 3, 9, 40])
+def test_sweeps_leave_memory_where_little_is_left(fitting, tmp_path, monkeypatch):
+    """Where fewer sets fit than a sweep rotates over it does with half of them: kernels allocate workspaces while they are
+    timed.  The check of the winner comes when all but the first are given back."""
+    import sys
+    import types
+    import weakref
+
+    import torch
+
+    module = sys.modules[Tuner.__module__]
+    live, seen = weakref.WeakSet(), []
+
+    class FakeTensor:
+        def numel(self):
+            return 10**6
+
+        def element_size(self):
+            return 1
+
+    class FakeKernel:
+        kernel_name, code, config = "k__x", b"", Conv2dGw8Config(groups=4)
+
+        def load(self, **_kw):
+            pass
+
+        def unload(self):
+            pass
+
+        def time(self, sets, warmup, iters):
+            seen.append((len(sets), len(live)))
+            return 1e-3
+
+    def make_test_args(*_args, **_kw):
+        if len(live) == fitting:
+            raise torch.OutOfMemoryError
+        tensor = FakeTensor()
+        live.add(tensor)
+        return (tensor,)
+
+    def first_valid(_self, _factory, _params, timed, *_args):
+        seen.append((1, len(live)))
+        return timed[0]
+
+    monkeypatch.setattr(module, "compile_kernel_configs", lambda *_a, **_kw: [FakeKernel()])
+    monkeypatch.setattr(Tuner, "_first_valid", first_valid)
+    factory = types.SimpleNamespace(get_full_kernel_name=lambda *_a, **_kw: "k__x", make_test_args=make_test_args)
+    Tuner().sweep(factory, None, 0, ATTR, configs=[FakeKernel.config], record_path=str(tmp_path / "db.json"))
+    assert seen == [(max(1, fitting // 2),) * 2, (1, 1)]
