@@ -13,8 +13,13 @@ import torch
 from ..compiler.compile_kernel import compile_kernel, load_kernel
 from ..compiler import flags
 from ..hip.driver import launch_sequence_timed
+from ..util.math import divup
 from ..util.memory_format import check_channels_last
 from .launch_params import LaunchParams
+
+# Timed launches of a two-stage kernel take turns with workspaces of about this size in all, four times the memory-side
+# cache, not with one for each of up to 128 sets of arguments.
+WORKSPACE_ROTATION_BYTES = 4 * 256 * 1024 * 1024
 
 
 @dataclass
@@ -248,9 +253,17 @@ class Kernel:
                 lp.grid, lp.block, prepared, lp.shared_mem_bytes, stream, warmup, iters
             )
         ep = spec.epilogue_launch_params
+        workspaces = []
+        for _ in range(min(len(prepared), divup(WORKSPACE_ROTATION_BYTES, max(spec.workspace_bytes, 1)))):
+            try:
+                workspaces.append(self._workspace(device))
+            except torch.OutOfMemoryError:  # one will do
+                if not workspaces:
+                    raise
+                break
         sets = []
-        for kargs in prepared:
-            ws = self._workspace(device)
+        for i, kargs in enumerate(prepared):
+            ws = workspaces[i % len(workspaces)]
             main_args, epilogue_args = self._stage_args(kargs, ws)
             sets.append([
                 (self.function, lp.grid, lp.block, lp.shared_mem_bytes, list(main_args)),

@@ -806,3 +806,41 @@ def test_sweeps_leave_memory_where_little_is_left(fitting, tmp_path, monkeypatch
     factory = types.SimpleNamespace(get_full_kernel_name=lambda *_a, **_kw: "k__x", make_test_args=make_test_args)
     Tuner().sweep(factory, None, 0, ATTR, configs=[FakeKernel.config], record_path=str(tmp_path / "db.json"))
     assert seen == [(max(1, fitting // 2),) * 2, (1, 1)]
+
+
+@pytest.mark.parametrize("sets,workspace,free,expected", [(4, 1000, 100, 4), (128, 10**6, 10**9, 128), (128, 20 << 20, 10**9, 52),
+                                                          (8, 3 << 30, 10**9, 1), (128, 20 << 20, 5, 5), (3, 1000, 0, None)])  # fmt: skip
+def test_timed_two_stage_kernels_share_workspaces(sets, workspace, free, expected, monkeypatch):
+    """One for each set of arguments up to 1 GB together, or as many as there is memory for: one at least."""
+    import sys
+    import types
+
+    import torch
+
+    params = Conv2dGw8Params(n=4, c=16, h=14, w=14)
+    config = Conv2dGw8WgradConfig(groups=2, block_h=14, prefetch=2, two_stage=1)
+    kernel = conv2d_gw8_wgrad_kernel_factory.make_kernel(params, config=config, device_attr=ATTR)
+    module = sys.modules[type(kernel).__module__]
+    kernel.function = kernel.epilogue_function = object()
+    kernel.kernel_spec = replace(kernel.kernel_spec, workspace_bytes=workspace)
+    made, launched = [], []
+
+    def make_workspace(_self, _device):
+        if len(made) == free:
+            raise torch.OutOfMemoryError
+        made.append(object())
+        return made[-1]
+
+    monkeypatch.setattr(type(kernel), "_workspace", make_workspace)
+    monkeypatch.setattr(type(kernel), "_prepare", lambda _self, _args: None)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda _device: types.SimpleNamespace(cuda_stream=0))
+    monkeypatch.setattr(module, "launch_sequence_timed", lambda s, *_args: launched.extend(s) or 1.0)
+    args = [("grad_weight%d" % i, "x", "grad_output") for i in range(sets)]
+    if expected is None:
+        with pytest.raises(torch.OutOfMemoryError):
+            kernel.time(args)
+        return
+    assert kernel.time(args) == 1.0
+    assert len(made) == expected and len(launched) == sets
+    for i, ((*_, main), (*_, second)) in enumerate(launched):
+        assert made[i % expected] in main and made[i % expected] in second and args[i][0] in second
